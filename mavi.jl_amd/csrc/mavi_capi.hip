@@ -148,7 +148,7 @@ static void sys_free(mavi_sys *s) {
     dfree(s->key); dfree(s->rank); dfree(s->src); dfree(s->scell); dfree(s->sid); dfree(s->slot_of);
     dfree(s->cnt); dfree(s->start); dfree(s->scan_state); dfree(s->scan_ticket); dfree(s->flags); dfree(s->counter);
     dfree(s->stamp); dfree(s->epoch); dfree(s->perm); dfree(s->needc);
-    dfree(s->active_ids); dfree(s->pos_id); dfree(s->vel_id); dfree(s->force_id);
+    dfree(s->active_ids); dfree(s->pos_id); dfree(s->vel_id); dfree(s->force_id); dfree(s->ang_id);
     dfree(s->pol); dfree(s->areas); dfree(s->cms); dfree(s->cms_next); dfree(s->cpos);
     dfree(s->rtype); dfree(s->types); dfree(s->inter); dfree(s->noise); dfree(s->red);
     dfree(s->walls); dfree(s->lines); dfree(s->neigh_cnt); dfree(s->neigh_list);
@@ -426,6 +426,7 @@ int mavi_sys_create(mavi_ctx *ctx, const mavi_sys_desc *d, mavi_sys **out) {
     if (!rings) ALLOC(s->vel_id, P.n);
     ALLOC(s->force_id, P.n);
     if (rings) {
+    if (is_active(s)) ALLOC(s->ang_id, P.n);
         ALLOC(s->active_ids, P.na);
         ALLOC(s->pol, P.nrings);
         ALLOC(s->areas, P.nrings);
@@ -488,10 +489,13 @@ int mavi_sys_upload(mavi_sys *s, const double *pos, const double *vel, const dou
     HIPCHK(ctx, hipMemcpyAsync(s->pos_id, pos, bytes, hipMemcpyHostToDevice, ctx->stream));
     if (is_active(s)) {
         // pol_angle (n) -> the x components of the velocity staging
-        HIPCHK(ctx, hipMemsetAsync(s->vel_id, 0, bytes, ctx->stream));
-        if (pol)
-            HIPCHK(ctx, hipMemcpy2DAsync(s->vel_id, sizeof(double2), pol, sizeof(double), sizeof(double),
-                                         (size_t)s->P.n, hipMemcpyHostToDevice, ctx->stream));
+        if (pol) {
+            HIPCHK(ctx, hipMemcpyAsync(s->ang_id, pol, sizeof(double) * (size_t)s->P.n, hipMemcpyHostToDevice,
+                                       ctx->stream));
+            HIPCHK(ctx, mavi::launch_spread_angles(s, ctx->stream));
+        } else {
+            HIPCHK(ctx, hipMemsetAsync(s->vel_id, 0, bytes, ctx->stream));
+        }
     } else if (vel && s->vel_id) {
         HIPCHK(ctx, hipMemcpyAsync(s->vel_id, vel, bytes, hipMemcpyHostToDevice, ctx->stream));
     }
@@ -523,9 +527,11 @@ int mavi_sys_download(mavi_sys *s, double *pos, double *vel, double *pol) {
     const size_t bytes = sizeof(double2) * (size_t)s->P.n;
     if (pos) HIPCHK(ctx, hipMemcpyAsync(pos, s->pos_id, bytes, hipMemcpyDeviceToHost, ctx->stream));
     if (is_active(s)) {
-        if (pol)
-            HIPCHK(ctx, hipMemcpy2DAsync(pol, sizeof(double), s->vel_id, sizeof(double2), sizeof(double),
-                                         (size_t)s->P.n, hipMemcpyDeviceToHost, ctx->stream));
+        if (pol) {
+            HIPCHK(ctx, mavi::launch_pack_angles(s, ctx->stream));
+            HIPCHK(ctx, hipMemcpyAsync(pol, s->ang_id, sizeof(double) * (size_t)s->P.n, hipMemcpyDeviceToHost,
+                                       ctx->stream));
+        }
     } else if (vel && s->vel_id) {
         HIPCHK(ctx, hipMemcpyAsync(vel, s->vel_id, bytes, hipMemcpyDeviceToHost, ctx->stream));
     }

@@ -276,6 +276,7 @@ struct mavi_sys {
     std::vector<int64_t> vids, vuids;   // VarRingsIds.ids (1-based, stale tail kept), uids
     int64_t vnum_active = 0;
     std::vector<HostSource> vsrc;
+    double *ang_id = nullptr;               // self-propelled: the angles packed for the host copies
     int32_t nsinks = 0, nboxes = 0;
     std::vector<double> pol_draws;      // uniform draws for random spawn polarisations
     int64_t pol_used = 0;
@@ -396,6 +397,9 @@ hipError_t launch_active_step(mavi_sys *s, const double *noise_dev, hipStream_t 
 // inputs (RingRates): per slot u = v0 p + mu F, per ring the rate of its area
 // (in units of the target area) and the alignment angle; it clears *gate.
 hipError_t launch_rings_forces(mavi_sys *s, hipStream_t st, const RingRates *rates = nullptr);
+// self-propelled: ang_id -> the x components of vel_id (y zero), and back
+hipError_t launch_spread_angles(mavi_sys *s, hipStream_t st);
+hipError_t launch_pack_angles(mavi_sys *s, hipStream_t st);
 hipError_t launch_rings_init(mavi_sys *s, hipStream_t st);
 hipError_t launch_ring_neigh(mavi_sys *s, hipStream_t st);
 // check_invasions!: ring boxes and the ring grid, then the crossing tests;

@@ -218,3 +218,24 @@ def test_unsupported_configurations(gpu_ctx):
     b = Batch()
     with pytest.raises(mv.UnsupportedOnGPU):
         b.add(system.state, sp, dyn, ic)
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 1000])
+def test_angles_survive_the_host_copies(gpu_ctx, n):
+    """Upload and download move the angles through a packed array: every
+    value comes back as it was, and pol = NULL sets all angles to zero."""
+    import mavi_hip as mv
+
+    say(f"[angles] n={n}")
+    rng = np.random.default_rng(n)
+    sp = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=50.0, height=40.0))
+    ic = mv.IntCfg(dt=1e-3, chunks_cfg=mv.ChunksCfg(num_cols=10, num_rows=8), device=mv.GPU())
+    dyn = mv.RunTumbleCfg(vo=1.0, sigma=1.0, epsilon=1.0, tumble_rate=1.0)
+    pos, ang = rng.uniform(0.0, 40.0, size=(n, 2)), rng.normal(scale=100.0, size=n)
+    s = mv.System(state=mv.SelfPropelledState(pos=pos, pol_angle=ang), space_cfg=sp, dynamic_cfg=dyn, int_cfg=ic)
+    s.state.pol_angle[:] = -1.0
+    s.download()
+    assert np.array_equal(s.state.pol_angle, ang) and np.array_equal(s.state.pos, pos)
+    s.dev.upload(s.state.pos)
+    s.download()
+    assert np.array_equal(s.state.pol_angle, np.zeros(n))
