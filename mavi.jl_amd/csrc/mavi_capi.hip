@@ -138,6 +138,7 @@ static void sys_free(mavi_sys *s) {
     (void)hipSetDevice(s->ctx->device);
     (void)hipStreamSynchronize(s->ctx->stream);
     mavi::nl_free(s);
+    mavi::rl_free(s);
     if (s->graph2) (void)hipGraphExecDestroy(s->graph2);
     for (int c = 0; c < 2; c++) {
         dfree(s->P_[c]);
@@ -425,8 +426,8 @@ int mavi_sys_create(mavi_ctx *ctx, const mavi_sys_desc *d, mavi_sys **out) {
     ALLOC(s->pos_id, P.n);
     if (!rings) ALLOC(s->vel_id, P.n);
     ALLOC(s->force_id, P.n);
-    if (rings) {
     if (is_active(s)) ALLOC(s->ang_id, P.n);
+    if (rings) {
         ALLOC(s->active_ids, P.na);
         ALLOC(s->pol, P.nrings);
         ALLOC(s->areas, P.nrings);
@@ -468,6 +469,7 @@ int mavi_sys_create(mavi_ctx *ctx, const mavi_sys_desc *d, mavi_sys **out) {
     // neighbour lists for finite-range plain systems (at most 2^31 list entries)
     if (e == hipSuccess && mavi::nl_eligible(s) && (int64_t)s->P.na * 64 < (int64_t)INT32_MAX)
         e = mavi::nl_alloc(s, ctx->stream);
+    if (e == hipSuccess && mavi::rl_eligible(s)) e = mavi::rl_alloc(s, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     s->seed = h.seed;
     if (e != hipSuccess) {
@@ -503,6 +505,8 @@ int mavi_sys_upload(mavi_sys *s, const double *pos, const double *vel, const dou
         HIPCHK(ctx, hipMemcpyAsync(s->pol, pol, sizeof(double) * s->P.nrings, hipMemcpyHostToDevice, ctx->stream));
     s->cur = 0;
     if (s->nl) s->nl->valid = false;  // a new state in id order
+    mavi::rl_invalidate(s);
+    if (s->rl) s->rl->step_hist[0] = s->rl->step_hist[1] = s->rl->step_hist[2] = 0.0;  // its steps may be longer
     HIPCHK(ctx, mavi::drop_keys(s, ctx->stream));
     HIPCHK(ctx, mavi::launch_iota_state(s, ctx->stream));
     if (s->P.potential == MAVI_POT_RINGS) HIPCHK(ctx, mavi::launch_rings_init(s, ctx->stream));
@@ -984,6 +988,8 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
     return MAVI_OK;
 }
 
+constexpr int64_t kRlMinCall = 8;
+
 static int steps_impl(mavi_sys *s, int64_t nsteps, const double *noise_host) {
     mavi_ctx *ctx = s->ctx;
     if (nsteps < 0) return set_err(ctx, MAVI_E_BADARG, "nsteps < 0");
@@ -1009,6 +1015,34 @@ static int steps_impl(mavi_sys *s, int64_t nsteps, const double *noise_host) {
         }
         nsteps = left;  // lists disabled (a list overflowed): the chunk gather runs the rest
     }
+    // Rings on lists: the same bits as the gather, so the choice is free.  A
+    // call that has to build them needs kRlMinCall steps to win the build
+    // back (a build and its checks cost about six gather steps' launches).
+    if (!noise_host && mavi::rl_active(s) && (nsteps >= kRlMinCall || (nsteps > 0 && s->rl->valid))) {
+        while (nsteps > 0) {
+            // up to and including the next step that checks invasions
+            const int64_t until = s->inv_sched ? std::max<int64_t>(s->inv_every - s->inv_since, 0) + 1 : nsteps;
+            const int64_t seg = std::min(nsteps, until);
+            int64_t left = 0;
+            const int rc = mavi::rl_steps(s, seg, &left);
+            if (rc != MAVI_OK) return rc;
+            const int64_t ran = seg - left;
+            nsteps -= ran;
+            if (s->inv_sched) {
+                const bool due = ran > 0 && s->inv_since + ran - 1 >= s->inv_every;
+                s->inv_since = due ? 1 : s->inv_since + ran;
+                const int rc2 = due ? run_invasions(s) : MAVI_OK;
+                if (rc2 != MAVI_OK) return rc2;
+            }
+            if (left > 0) break;  // the chunk gather runs the rest
+        }
+        if (nsteps == 0) {
+            const int rc = sync_staging(s, true);
+            if (rc != MAVI_OK) return rc;
+            return check_flags(s);
+        }
+    }
+    mavi::rl_invalidate(s);  // (a captured graph moves the state without passing launch_bin's host side)
     if (noise_host) {
         // draws per step: one per ring (rings), one (Szabo) or two (RTP) per particle
         const int64_t nr = s->P.potential == MAVI_POT_RINGS ? s->P.nrings
@@ -1455,6 +1489,13 @@ int mavi_prof_get(mavi_sys *s, int which, double *ms_total, int64_t *launches) {
 
 int mavi_nlist_info(mavi_sys *s, int64_t *info) {
     if (!s || !info) return MAVI_E_BADARG;
+    if (const RList *R = s->rl) {
+        info[0] = 1;
+        info[1] = mavi::rl_active(s) ? 1 : 0;
+        info[2] = R->rebuilds;
+        info[3] = R->rollbacks;
+        return MAVI_OK;
+    }
     const NList *N = s->nl;
     info[0] = N ? 1 : 0;
     info[1] = (N && N->on && !N->disabled) ? 1 : 0;
@@ -1496,7 +1537,8 @@ int mavi_sys_noise_set(mavi_sys *s, uint64_t seed, uint64_t counter) {
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     const unsigned long long c = counter;
     HIPCHK(ctx, hipMemcpy(s->counter, &c, sizeof(c), hipMemcpyHostToDevice));
-    if (seed != s->seed && s->graph2) {  // the captured graph holds the seed
+    if (seed != s->seed) mavi::rl_drop_graph(s);  // the captured graphs hold the seed
+    if (seed != s->seed && s->graph2) {
         (void)hipGraphExecDestroy(s->graph2);
         s->graph2 = nullptr;
     }
@@ -1528,6 +1570,10 @@ int mavi_sys_set_option(mavi_sys *s, int32_t option, int32_t value) {
                 s->nl->on = value != 0;
                 s->nl->valid = false;
             }
+            if (s->rl) {
+                s->rl->on = value != 0;
+                mavi::rl_invalidate(s);
+            }
             changed = true;
             break;
         case MAVI_OPT_NLIST_SKIN:
@@ -1536,12 +1582,17 @@ int mavi_sys_set_option(mavi_sys *s, int32_t option, int32_t value) {
                 nl_drop_graph(s);
                 mavi::nl_set_skin(s, value == 0 ? 0.15 : value / 1000.0);
             }
+            if (s->rl) (void)mavi::rl_set_skin(s, value == 0 ? kRlSkin : value / 1000.0);
             break;
         case MAVI_OPT_NLIST_BLOCK:
             if (value < 0 || value > 4096) return set_err(s->ctx, MAVI_E_BADARG, "block: 0 (default) .. 4096 steps");
             if (s->nl) {
                 s->nl->block = (int32_t)value;
                 s->nl->block_now = value == 0 ? kNlBlockCap : (int32_t)value;
+            }
+            if (s->rl) {
+                s->rl->block = (int32_t)value;
+                s->rl->block_now = value == 0 ? kNlBlockCap : (int32_t)value;
             }
             break;
         default:
@@ -1589,6 +1640,7 @@ int mavi_autotune(mavi_sys *s, int32_t trial_steps, double *best_us, int32_t *sh
             r = hipMemcpyAsync(s->pol, pol0, sizeof(double) * s->P.nrings, hipMemcpyDeviceToDevice, st);
         s->cur = 0;
         s->f_valid = false;
+        mavi::rl_invalidate(s);
         if (r == hipSuccess) r = mavi::drop_keys(s, st);
         if (r == hipSuccess) r = mavi::launch_iota_state(s, st);
         if (r == hipSuccess && s->P.potential == MAVI_POT_RINGS) r = mavi::launch_rings_init(s, st);
@@ -1600,6 +1652,8 @@ int mavi_autotune(mavi_sys *s, int32_t trial_steps, double *best_us, int32_t *sh
     int bw = s->wg, bl = s->lds_tiles, bt = s->two_phase;
     const bool saved_prof = s->prof;
     s->prof = false;
+    const bool saved_rl = s->rl && s->rl->on;
+    if (s->rl) s->rl->on = false;  // the shapes are the gather's
     for (int lds = 0; lds < 2 && e == hipSuccess; lds++) {
         if (lds && s->P.cols == 0) continue;
         for (int tp = 0; tp < 2 && e == hipSuccess; tp++) {
@@ -1628,6 +1682,7 @@ int mavi_autotune(mavi_sys *s, int32_t trial_steps, double *best_us, int32_t *sh
         }
     }
     s->prof = saved_prof;
+    if (s->rl) s->rl->on = saved_rl;
     mavi_sys_set_tile(s, bw);
     mavi_sys_set_option(s, MAVI_OPT_LDS_TILES, bl);
     mavi_sys_set_option(s, MAVI_OPT_TWO_PHASE, bt);

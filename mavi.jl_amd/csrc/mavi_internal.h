@@ -213,6 +213,47 @@ struct NList {
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // six steps from ph = 0 on state copy 0 / 1 (a rebuild's sort flips it)
 };
 
+constexpr double kRlSkin = 0.3;      // default list skin of rings (fraction of the widest range)
+constexpr int kRlGraphSteps = 8;     // steps per captured graph (even)
+
+// Verlet lists of a rings system with a fixed population (mavi_rlist.hip).
+struct RList {
+    bool on = true;           // option MAVI_OPT_NLIST
+    bool fits = false;        // the list grid has at least 3 x 3 cells
+    bool disabled = false;    // a list or a chunk overflowed: the chunk gather takes over
+    bool ordered = false;     // the state lies in ring order, both copies' ids too
+    bool valid = false;       // lists complete for the current state
+    bool uniform = false;     // one interaction for all type pairs
+    double rl2 = 0.0;         // list radius squared (range + skin)^2, with margin
+    double half_skin = 0.0;   // displacement bound
+    int32_t block = 0;        // steps between host checks (option; 0: as many as the bound allows, at most kNlBlockCap)
+    int32_t block_now = kNlBlockCap;
+    double step_hist[3] = {0.0, 0.0, 0.0};  // the largest step of each of the last three blocks
+    int32_t step_i = 0;
+    double d_start = 0.0;     // largest displacement from the build of the next block's first positions
+    SysParams G{};            // list grid (cells >= range + skin)
+    int ph = 0;               // counter word of the current step
+    int32_t *head = nullptr;  // int4 per slot: the first four entries, -1 past the end
+    int32_t *more = nullptr;  // further entries
+    uint8_t *count = nullptr;
+    int32_t *key = nullptr;   // reference chunk of each slot
+    int32_t *ccnt = nullptr;  // particles per reference chunk
+    double2 *xb = nullptr;    // positions at build
+    double2 *psnap = nullptr, *csnap = nullptr, *nsnap = nullptr;  // block-start positions, cms, cms_next
+    double *polsnap = nullptr;
+    uint32_t *fsnap = nullptr;
+    double2 *polcs = nullptr; // cos, sin of the polarisations
+    uint32_t *bmax = nullptr; // per wave of the step kernel
+    int32_t nbmax = 0;
+    uint32_t *status = nullptr;
+    unsigned long long *counter = nullptr;  // two words, alternating between steps
+    unsigned long long *out = nullptr, *host = nullptr;  // block-end maxima and status, pinned copy
+    unsigned long long *scan_ticket = nullptr, *scan_state = nullptr;
+    int32_t scan_words = 0;
+    int64_t rebuilds = 0, rollbacks = 0;
+    hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [state copy][counter word]
+};
+
 struct mavi_sys {
     mavi_ctx *ctx = nullptr;
     int refs = 0;          // learned propagators bound to this system
@@ -235,6 +276,7 @@ struct mavi_sys {
     unsigned long long *counter = nullptr;  // device step counter (rotational noise)
     int32_t *active_ids = nullptr;          // na ids ascending
     double2 *pos_id = nullptr, *vel_id = nullptr, *force_id = nullptr;
+    double *ang_id = nullptr;               // self-propelled: the angles packed for the host copies
     int32_t nscan_blocks = 0;
     // rings
     double *pol = nullptr, *areas = nullptr;
@@ -276,7 +318,6 @@ struct mavi_sys {
     std::vector<int64_t> vids, vuids;   // VarRingsIds.ids (1-based, stale tail kept), uids
     int64_t vnum_active = 0;
     std::vector<HostSource> vsrc;
-    double *ang_id = nullptr;               // self-propelled: the angles packed for the host copies
     int32_t nsinks = 0, nboxes = 0;
     std::vector<double> pol_draws;      // uniform draws for random spawn polarisations
     int64_t pol_used = 0;
@@ -305,6 +346,7 @@ struct mavi_sys {
     bool f_valid = false;       // F holds the last step's second evaluation
     bool keys_ready = false;    // the last second evaluation left key/rank/cnt for the next binning
     NList *nl = nullptr;        // neighbour lists (finite-range plain systems), null if not eligible
+    RList *rl = nullptr;        // lists of a rings system, null if not eligible
     // graphs of two steps (state starting in copy 0)
     hipGraphExec_t graph2 = nullptr;
     bool use_graphs = true;
@@ -355,6 +397,9 @@ namespace mavi {
 // resolved once per device with that device current
 hipError_t noalloc_scratch_setup(int device);
 hipError_t launch_iota_state(mavi_sys *s, hipStream_t st);          // id-order staging -> state copy cur
+// self-propelled: ang_id -> the x components of vel_id (y zero), and back
+hipError_t launch_spread_angles(mavi_sys *s, hipStream_t st);
+hipError_t launch_pack_angles(mavi_sys *s, hipStream_t st);
 hipError_t launch_unpermute(mavi_sys *s, bool vel, bool force, hipStream_t st);  // state -> staging
 // binning + permutation (cur flips); count_step advances the step counter
 // of the device rotational noise (a step's binning, not a lone update_chunks!)
@@ -384,6 +429,23 @@ hipError_t nl_measure(mavi_sys *s, hipStream_t st);
 // evaluated drift
 hipError_t nl_settle(mavi_sys *s, hipStream_t st);
 void nl_set_skin(mavi_sys *s, double skin_frac);
+// Lists of a rings system (mavi_rlist.hip).  rl_active: the next steps may run
+// on them; rl_steps: up to nsteps steps (*left > 0: the chunk gather runs the
+// rest); rl_invalidate: the state was moved or reordered by other kernels.
+bool rl_eligible(const mavi_sys *s);
+hipError_t rl_alloc(mavi_sys *s, hipStream_t st);
+void rl_free(mavi_sys *s);
+bool rl_set_skin(mavi_sys *s, double skin_frac);
+void rl_drop_graph(mavi_sys *s);
+bool rl_active(const mavi_sys *s);
+int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left);
+inline void rl_invalidate(mavi_sys *s) {
+    if (s->rl) s->rl->valid = s->rl->ordered = false;
+}
+// Counting sort of the slots on another grid over the same space, the state
+// left where it is: s->src, s->scell, s->start.
+hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,
+                             hipStream_t st);
 hipError_t launch_export_chunks(mavi_sys *s, int64_t *d_cp, int64_t *d_counts, hipStream_t st);
 hipError_t launch_forces_only(mavi_sys *s, hipStream_t st);
 // One newton_step!; reuse = the previous call was a Verlet step of this
@@ -397,9 +459,6 @@ hipError_t launch_active_step(mavi_sys *s, const double *noise_dev, hipStream_t 
 // inputs (RingRates): per slot u = v0 p + mu F, per ring the rate of its area
 // (in units of the target area) and the alignment angle; it clears *gate.
 hipError_t launch_rings_forces(mavi_sys *s, hipStream_t st, const RingRates *rates = nullptr);
-// self-propelled: ang_id -> the x components of vel_id (y zero), and back
-hipError_t launch_spread_angles(mavi_sys *s, hipStream_t st);
-hipError_t launch_pack_angles(mavi_sys *s, hipStream_t st);
 hipError_t launch_rings_init(mavi_sys *s, hipStream_t st);
 hipError_t launch_ring_neigh(mavi_sys *s, hipStream_t st);
 // check_invasions!: ring boxes and the ring grid, then the crossing tests;

@@ -1150,6 +1150,7 @@ hipError_t launch_bin(mavi_sys *s, hipStream_t st, bool count_step, bool stamp, 
     const SysParams &P = over ? *over : s->P;
     if (P.cols == 0) return hipSuccess;  // chunks = nothing: the state order stays the active id order
     if (s->nl) s->nl->valid = false;     // a new slot order: lists index slots
+    rl_invalidate(s);
     ProfScope ps(s, MAVI_PROF_BIN, st);
     const int c = s->cur, nc = 1 - c;
     // stamps need the previous binning's chunk of every slot (scell)
@@ -1176,6 +1177,18 @@ hipError_t launch_bin(mavi_sys *s, hipStream_t st, bool count_step, bool stamp, 
     }
     s->cur = nc;
     s->sorted = true;
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,
+                             hipStream_t st) {
+    ProfScope ps(s, MAVI_PROF_BIN, st);
+    const int c = s->cur, n = G.ncell + 1;
+    hipLaunchKernelGGL(k_bin_count, dim3(nblk(G.na, 256)), dim3(256), 0, st, G, s->P_[c], s->key, s->rank, s->cnt,
+                       s->flags, s->scell, nullptr, s->epoch);
+    launch_scan(s->cnt, n, s->start, ticket, state, s->flags, st);
+    hipLaunchKernelGGL(k_scatter, dim3(nblk(G.na > n ? G.na : n, 256)), dim3(256), 0, st, G, s->key, s->rank,
+                       s->start, s->src, s->scell, s->ID_[c], s->sid, s->cnt, nullptr, nullptr, s->epoch, s->needc);
     return hipGetLastError();
 }
 

@@ -899,6 +899,7 @@ int mavi_learned_run(mavi_learned *l, int64_t nmacro, int32_t use_net, int64_t *
         // a learned step moves the particles outside the kernels that keep
         // the chunk keys: its binning starts from scratch (also when captured)
         HIPCHK(ctx, mavi::drop_keys(s, st));
+        mavi::rl_invalidate(s);
         HIPCHK(ctx, mavi::launch_fill_i32((int32_t *)l->ctl, 0, 2, st));
         for (int64_t j = 0; j < m; j++) {
             if (s->use_graphs && !s->prof) {

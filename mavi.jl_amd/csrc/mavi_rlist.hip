@@ -1,0 +1,883 @@
+// mavi_rlist.hip -- Verlet lists for Rings step! (src/rings/integration.jl:
+// 522-543) of a fixed ring population on a periodic chunk grid whose chunks
+// are at least the interaction range wide: one kernel per step instead of a
+// binning (three launches), the pair gather and the ring update.
+//
+// State.  While the lists run the state lies in ring order (slot = position of
+// the particle's id among the active ids), so a ring's particles are
+// consecutive and every kernel reads and writes them with unit stride; the two
+// state copies ping-pong, because a ring's neighbours read its old positions.
+//
+// Pairs.  Each particle lists the others within range + skin that it can
+// interact with (not its bonded neighbours), found on a grid of cells at least
+// that wide.  The lists stay complete while no particle has moved more than
+// half the skin since the build; the host checks that once per block of steps
+// (the same bound as the neighbour lists of plain systems, mavi_nlist.hip) and
+// rolls an overrun block back.
+//
+// Same bits as the gather.  calc_forces! visits the pairs of adjacent chunks
+// of the step's own binning; every pair within range is among them, and the
+// gather adds a particle's pairs by chunk row, chunk column (the visiting order
+// at the periodic edges included) and id.  One or two pairs in range add to
+// the same value in any order; for three or more the contributions are put in
+// that order first, from the exact chunks of the positions.  Everything else
+// of the step is ring_lanes' arithmetic term by term, so a trajectory does not
+// depend on whether the lists run, when they were built or how it was split
+// into calls, and a batch replica stays bit-identical to the system alone.
+//
+// Errors.  Chunks and chunk counts of the reference grid follow every particle
+// (out of box, non-finite); a count that may have passed the capacity, or a
+// list that is too long, hands the block to the gather, which checks exactly.
+#include <math.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "mavi_device.h"
+#include "mavi_host.h"
+
+namespace {
+
+constexpr int kRlHead = 4;    // list entries in the particle's int4
+constexpr int kRlMax = 16;    // list entries per particle
+constexpr int kRlWG = 256;    // step workgroup: four waves of floor(64 / nmax) rings
+constexpr uint32_t kRlOverflow = 1u;  // a list longer than kRlMax
+constexpr uint32_t kRlCapacity = 2u;  // a chunk count may have passed the capacity
+
+// A list entry: partner slot (26 bits), its ring type (5 bits); the sign bit
+// marks the end (-1).  Same-ring partners are told apart by their slots.
+constexpr int kRlSlotBits = 26;
+constexpr int32_t kRlSlotMask = (1 << kRlSlotBits) - 1;
+
+struct RLArgs {
+    const double2 *Pin;
+    double2 *Pout;
+    double2 *F;                 // last step of a call only
+    const int32_t *slot_of;     // null: slot = id (every ring full)
+    const int4 *head;
+    const int32_t *more;        // entries kRlHead.. of slot q: more[e * na + q]
+    const uint8_t *count;
+    int32_t *key;               // reference chunk (row << 16 | col) of each slot
+    int32_t *ccnt;
+    double *pol;
+    double2 *polcs;             // cos, sin of each ring's polarisation
+    double *areas;
+    double2 *cms, *cms_next, *cpos;
+    const int32_t *rtype;
+    const RingType *types;
+    const RingInter *inter;     // matrix of interactions; null: `uni` for every pair
+    RingInter uni;
+    uint32_t *bmax;             // per wave: high word of the largest squared step, rounded up
+    uint32_t *flags, *status;
+    uint64_t seed;
+    const unsigned long long *cin;  // the step counter before this step
+    unsigned long long *cout;
+};
+
+__device__ __forceinline__ void lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// calc_diff with the image arithmetic only where some lane of the wave needs
+// it (min_image is the identity for |dr| <= half the box).
+__device__ __forceinline__ double2 wave_diff(const SysParams &P, double2 a, double2 b) {
+    double dx = a.x - b.x, dy = a.y - b.y;
+    if (__any(fabs(dx) > P.halfL || fabs(dy) > P.halfH)) {
+        dx = min_image(dx, P.L, P.halfL);
+        dy = min_image(dy, P.H, P.halfH);
+    }
+    return make_double2(dx, dy);
+}
+
+// Place of partner chunk (rj, cj) in the gather's order around (ri, ci): its
+// rows from -1 to 1, in a row the columns in slot order, except that at the
+// periodic column edges the wrapped column comes last.
+__device__ __forceinline__ uint32_t visit_rank(const SysParams &P, int ri, int ci, int rj, int cj) {
+    int d = rj - ri + 1;
+    if (d < 0) d += P.rows;
+    else if (d > 2) d -= P.rows;
+    int c = cj - ci + 1;
+    if (ci == 0) c = cj > 1 ? 2 : cj;                                     // 0, 1, then cols - 1
+    else if (ci == P.cols - 1) c = cj == 0 ? 2 : cj - (P.cols - 2);        // cols - 2, cols - 1, then 0
+    return (uint32_t)(d * 3 + c);
+}
+
+__device__ __forceinline__ RingInter rl_inter(const SysParams &P, const RLArgs &A, int ti, int32_t e) {
+    return A.inter ? A.inter[ti + P.ntypes * (e >> kRlSlotBits)] : A.uni;
+}
+
+// calc_interaction_force (src/rings/integration.jl:47-77) of a listed pair in
+// range (never bonded neighbours).
+__device__ __forceinline__ double2 rl_force(const RingInter &I, double2 d, double r2, bool same) {
+    const double dist = sqrt(r2);
+    double fmod;
+    if (r2 < I.eq2) fmod = -I.k_rep * (dist / I.dist_eq - 1.0);
+    else fmod = same ? 0.0 : -I.k_atr * (dist / I.dist_eq - 1.0);
+    const double q = fmod / dist;
+    return make_double2(q * d.x, q * d.y);
+}
+
+__device__ __forceinline__ unsigned long long visit_key(const SysParams &P, int ri, int ci, double2 pj, int j) {
+    uint32_t flag = 0;
+    int32_t rj, cj;
+    cell_rc(P, P.rows, P.cols, P.cl, P.ch, pj.x, pj.y, &flag, MAVI_FLAG_OUT_OF_BOX, &rj, &cj);
+    return ((unsigned long long)visit_rank(P, ri, ci, rj, cj) << 32) | (uint32_t)j;
+}
+
+// The sum of a particle with a long list, by repeated selection of the next
+// pair in the gather's order.
+__device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs &A, int q, int t0, int t1, int ti,
+                                            double2 x, int ri, int ci) {
+    const int n = A.count[q];
+    const int4 h = A.head[q];
+    double2 f = make_double2(0.0, 0.0);
+    unsigned long long prev = 0ull;
+    bool first = true;
+    for (;;) {
+        unsigned long long best = ~0ull;
+        int32_t be = -1;
+        for (int e = 0; e < n; e++) {
+            const int32_t w = e == 0 ? h.x : e == 1 ? h.y : e == 2 ? h.z : e == 3 ? h.w : A.more[(int64_t)(e - kRlHead) * P.na + q];
+            const int j = w & kRlSlotMask;
+            const double2 pj = A.Pin[j];
+            const double2 d = cdiff(P, x, pj);
+            const double r2 = d.x * d.x + d.y * d.y;
+            if (r2 > rl_inter(P, A, ti, w).max2) continue;
+            const unsigned long long k = visit_key(P, ri, ci, pj, j);
+            if ((first || k > prev) && k < best) {
+                best = k;
+                be = w;
+            }
+        }
+        if (be < 0) return f;
+        const int j = be & kRlSlotMask;
+        const double2 d = cdiff(P, x, A.Pin[j]);
+        const double2 c = rl_force(rl_inter(P, A, ti, be), d, d.x * d.x + d.y * d.y, j >= t0 && j < t1);
+        f.x += c.x;
+        f.y += c.y;
+        prev = best;
+        first = false;
+    }
+}
+
+// One Rings step! of the rings of this workgroup.  LAST: the last step of a
+// call, which leaves the forces and the continuous positions (every step
+// recomputes both before it uses them).
+//
+// Bound: FP64 VALU issue and the length of its dependent chain.  The ring's
+// left-to-right sums (unwrap, centre of mass, shoelace, mean velocity) run
+// once per ring and component on a few lanes (2 or 3 per ring) instead of as
+// masked loops of every lane, and the scalar work of a ring (noise, asin,
+// sincos of the new angle) once per workgroup on one lane per ring: as part of
+// every wave it was a third of the ring kernel's instructions.  45.9 us at
+// 800k particles (806 VALU instructions per wave) against 97 us for the five
+// launches it replaces (scan 12.1, scatter 8.7, finalize 11.1, pairs 26.2, ring
+// update 38.1); 11.8 against 33 us at 2k particles.
+template <bool LAST>
+__global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
+    __shared__ double2 s_a[kRlWG + 32], s_b[kRlWG + 32], s_c[kRlWG + 32];
+    __shared__ double s_t[kRlWG + 32];
+    __shared__ double s_r[4][64 * 3];  // per ring of a wave: sums
+    const int lane = (int)lane_id(), wave = (int)(threadIdx.x >> 6);
+    const int per = 64 / P.nmax;
+    const int grp = lane / P.nmax, i = lane - grp * P.nmax;
+    const int block = xcd_block();
+    const int r = (block * 4 + wave) * per + grp;
+    const bool ring_ok = grp < per && r < P.nrings;
+    const int rr = ring_ok ? r : 0;
+    const int t = P.typed ? A.rtype[rr] : 0;
+    const RingType *T = A.types + t;
+    const int np = T->np;
+    const bool act = ring_ok && i < np;
+    const int id = rr * P.nmax + i;
+    const int q = act ? (A.slot_of ? A.slot_of[id] : id) : 0;
+    const int t0 = q - i, t1 = t0 + np;  // the ring's slots
+    const double2 x = act ? A.Pin[q] : make_double2(0.0, 0.0);
+    int4 h = act ? A.head[q] : make_int4(-1, -1, -1, -1);
+    const int32_t ko = act ? A.key[q] : 0;
+    const double2 pcs = A.polcs[rr];
+    const unsigned long long step = A.cin[0] + 1ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) A.cout[0] = step;
+
+    // ---- pairs within range: the head's four entries
+    const int32_t ent[kRlHead] = {h.x, h.y, h.z, h.w};
+    double2 pj[kRlHead];
+#pragma unroll
+    for (int e = 0; e < kRlHead; e++)
+        pj[e] = ent[e] >= 0 ? A.Pin[ent[e] & kRlSlotMask] : x;
+
+    // neighbours along the ring and the unwrap's steps, meanwhile
+    const int me = (int)threadIdx.x, tb = me - i, wb = wave * 64;
+    const int inext = (i == np - 1) ? 0 : i + 1;
+    const int iprev = (i == 0) ? np - 1 : i - 1;
+    s_a[me] = x;
+    lds_sync();
+    const double2 xn = s_a[tb + inext];
+    const double2 xp = s_a[tb + iprev];
+    const double2 dprev = wave_diff(P, x, xp);
+    s_b[me] = i == 0 ? x : dprev;
+    lds_sync();
+    // ring sizes for the serial lanes: lane l < 3 per works for ring l / 2 or l / 3
+    const int np2 = __shfl(np, min(lane >> 1, per - 1) * P.nmax, 64);
+    const int np3 = __shfl(np, min(lane / 3, per - 1) * P.nmax, 64);
+    if (lane < 2 * per) {
+        // c_0 = x_0, c_k = c_{k-1} + calc_diff(x_k, x_{k-1}), one lane per component
+        const int o = 2 * (wb + (lane >> 1) * P.nmax) + (lane & 1);
+        const double *src = (const double *)s_b + o;
+        double *dst = (double *)s_c + o;
+        double c = src[0];
+        dst[0] = c;
+#pragma unroll 4
+        for (int k = 1; k < np2; k++) {
+            c = c + src[2 * k];
+            dst[2 * k] = c;
+        }
+    }
+    lds_sync();
+    const double2 c = s_c[me], cn = s_c[tb + inext];
+    if (LAST && act) A.cpos[id] = c;
+    s_t[me] = c.x * cn.y - c.y * cn.x;
+    lds_sync();
+    if (lane < 3 * per) {
+        // centre of mass and shoelace sums in ring order, one lane per sum
+        const int g = lane / 3, which = lane - 3 * g;
+        const double *src = which == 2 ? s_t + wb + g * P.nmax : (const double *)(s_c + wb + g * P.nmax) + which;
+        const int stride = which == 2 ? 1 : 2;
+        double s = 0.0;
+#pragma unroll 4
+        for (int k = 0; k < np3; k++) s += src[k * stride];
+        s_r[wave][lane] = s;
+    }
+
+    // ---- pair forces
+    double2 f[kRlHead];
+    bool in[kRlHead];
+    int m = 0;
+#pragma unroll
+    for (int e = 0; e < kRlHead; e++) {
+        f[e] = make_double2(0.0, 0.0);
+        in[e] = false;
+        if (!__any(ent[e] >= 0)) continue;
+        const double2 d = wave_diff(P, x, pj[e]);
+        const double r2 = d.x * d.x + d.y * d.y;
+        const RingInter I = rl_inter(P, A, t, ent[e] >= 0 ? ent[e] : 0);
+        in[e] = ent[e] >= 0 && !(r2 > I.max2);
+        if (in[e]) {
+            const int j = ent[e] & kRlSlotMask;
+            f[e] = rl_force(I, d, r2, j >= t0 && j < t1);
+            m++;
+        }
+    }
+    const bool longer = ent[kRlHead - 1] >= 0 && A.count[q] > kRlHead;
+    const bool order = m > 2 && !longer;
+    if (__any(order || longer)) {
+        const int ri = ko >> 16, ci = ko & 0xffff;
+        if (longer) {
+            f[0] = rl_long_sum(P, A, q, t0, t1, t, x, ri, ci);
+            f[1] = f[2] = f[3] = make_double2(0.0, 0.0);
+        } else if (order) {
+            unsigned long long k[kRlHead];
+#pragma unroll
+            for (int e = 0; e < kRlHead; e++)
+                k[e] = in[e] ? visit_key(P, ri, ci, pj[e], ent[e] & kRlSlotMask) : ~0ull;
+            auto cmpx = [&](int a, int b) {
+                const bool sw = k[b] < k[a];
+                const unsigned long long ka = sw ? k[b] : k[a], kb = sw ? k[a] : k[b];
+                const double2 fa = sw ? f[b] : f[a], fb = sw ? f[a] : f[b];
+                k[a] = ka;
+                k[b] = kb;
+                f[a] = fa;
+                f[b] = fb;
+            };
+            cmpx(0, 1);
+            cmpx(2, 3);
+            cmpx(0, 2);
+            cmpx(1, 3);
+            cmpx(1, 2);
+        }
+    }
+    double2 Fi = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int e = 0; e < kRlHead; e++) {
+        Fi.x += f[e].x;
+        Fi.y += f[e].y;
+    }
+
+    // ---- springs and area force
+    const double2 ds = wave_diff(P, x, xn);
+    const double dist = sqrt(ds.x * ds.x + ds.y * ds.y);
+    const double sq = -T->kspring * (dist - T->lspring) / dist;
+    const double2 fi = make_double2(sq * ds.x, sq * ds.y);
+    s_b[me] = fi;  // the unwrap's reads of s_b are done
+    lds_sync();
+    const double2 fprev = s_b[tb + iprev];
+    const double area = s_r[wave][min(grp, per - 1) * 3 + 2] / 2.0;
+    if (ring_ok && i == 0) {
+        const double *s = &s_r[wave][grp * 3];
+        A.cms[r] = A.cms_next[r];  // update_cms! reads the previous continuous positions
+        A.cms_next[r] = make_double2(s[0] / (double)np, s[1] / (double)np);
+        A.areas[r] = area;
+    }
+    double area0 = (double)np * T->lspring / T->p0;
+    area0 = area0 * area0;
+    const double fa = T->karea * (area - area0);
+    const double2 da = wave_diff(P, xn, xp);
+    if (i == 0) {
+        Fi.x += fi.x;
+        Fi.y += fi.y;
+        Fi.x -= fprev.x;
+        Fi.y -= fprev.y;
+    } else {
+        Fi.x -= fprev.x;
+        Fi.y -= fprev.y;
+        Fi.x += fi.x;
+        Fi.y += fi.y;
+    }
+    Fi.x -= fa * (da.y / 2.0);
+    Fi.y -= fa * (-da.x / 2.0);
+    if (LAST && act) A.F[q] = Fi;
+
+    // ---- update!
+    const double vx = T->vo * pcs.x + T->mu * Fi.x;
+    const double vy = T->vo * pcs.y + T->mu * Fi.y;
+    s_a[me] = make_double2(vx, vy);  // the neighbour reads of s_a are done
+    lds_sync();
+    if (lane < 2 * per) {
+        const double *src = (const double *)s_a + 2 * (wb + (lane >> 1) * P.nmax) + (lane & 1);
+        double s = 0.0;
+#pragma unroll 4
+        for (int k = 0; k < np2; k++) s += src[2 * k];
+        s_r[wave][lane] = s;  // the area's reads are done
+    }
+    double l2 = 0.0;
+    if (act) {
+        double px = x.x + vx * P.dt, py = x.y + vy * P.dt;
+        const double lx = px - x.x, ly = py - x.y;
+        l2 = lx * lx + ly * ly;
+        periodic_wrap(P, px, py);
+        A.Pout[q] = make_double2(px, py);
+        // the chunk of the new position; still clear inside the old one (by
+        // more than the rounding of the chunk edges): the same
+        const int r0 = ko >> 16, c0 = ko & 0xffff;
+        const double ax = px - P.blx, ay = (-py + P.bly) + P.H;
+        const double mg = 1e-12 * (P.L + P.H);
+        if (!(ax >= (double)c0 * P.cl + mg && ax <= (double)(c0 + 1) * P.cl - mg && ay >= (double)r0 * P.ch + mg &&
+              ay <= (double)(r0 + 1) * P.ch - mg)) {
+            uint32_t flag = 0;
+            int32_t rn, cc;
+            cell_rc(P, P.rows, P.cols, P.cl, P.ch, px, py, &flag, MAVI_FLAG_OUT_OF_BOX, &rn, &cc);
+            if (flag) atomicOr(A.flags, flag);
+            const int32_t kn = (rn << 16) | cc;
+            if (kn != ko) {
+                A.key[q] = kn;
+                atomicSub(&A.ccnt[r0 * P.cols + c0], 1);
+                if (atomicAdd(&A.ccnt[rn * P.cols + cc], 1) + 1 > P.nc) atomicOr(A.status, kRlCapacity);
+            }
+        }
+    }
+    // largest squared step since the block began (high word, rounded up; a
+    // non-finite step keeps the largest word)
+    uint32_t hi = l2 == l2 ? min((uint32_t)__double2hiint(l2) + 1u, 0x7ff00000u) : 0x7ff00000u;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+    if (lane == 0) {
+        uint32_t *slot = A.bmax + block * 4 + wave;
+        if (hi > *slot) *slot = hi;
+    }
+
+    // ---- polarisations: one lane per ring of the workgroup
+    __syncthreads();
+    if (wave != 0) return;
+    for (int k = lane; k < 4 * per; k += 64) {
+        const int w = k / per, g = k - w * per;
+        const int rg = (block * 4 + w) * per + g;
+        if (rg >= P.nrings) break;
+        const RingType *R = A.types + (P.typed ? A.rtype[rg] : 0);
+        const double vcx = s_r[w][2 * g] / (double)R->np, vcy = s_r[w][2 * g + 1] / (double)R->np;
+        const double2 cs = A.polcs[rg];
+        const double speed = sqrt(vcx * vcx + vcy * vcy);
+        double cr = 0.0;
+        if (speed != 0.0) {
+            cr = (cs.x * vcy - cs.y * vcx) / speed;
+            if (fabs(cr) > 1.0) cr = cr > 0.0 ? 1.0 : -1.0;
+        }
+        const double z = R->rot != 0.0 ? philox_normal(A.seed, step, (uint32_t)rg) : 0.0;
+        const double d_theta = 1.0 / R->relax * asin(cr) * P.dt + sqrt(2.0 * R->rot * P.dt) * z;
+        const double th = A.pol[rg] + d_theta;
+        double sn, cn2;
+        sincos(th, &sn, &cn2);
+        A.pol[rg] = th;
+        A.polcs[rg] = make_double2(cn2, sn);
+    }
+}
+
+// The lists: one thread per particle, in cell order of the list grid (src[t]:
+// the slot at place t), over the 3x3 cells around its own.
+__global__ __launch_bounds__(256) void k_rl_build(SysParams G, SysParams P, const double2 *__restrict__ pos,
+                                                  const int32_t *__restrict__ ID, const int32_t *__restrict__ rtype,
+                                                  const RingType *__restrict__ types,
+                                                  const int32_t *__restrict__ src, const int32_t *__restrict__ scell,
+                                                  const int32_t *__restrict__ start, double rl2,
+                                                  int4 *__restrict__ head, int32_t *__restrict__ more,
+                                                  uint8_t *__restrict__ count, uint32_t *__restrict__ status) {
+    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    if (t >= P.na) return;
+    const int q = src[t], c = scell[t];
+    const double2 x = pos[q];
+    const int id = ID[q], ring = id / P.nmax;
+    const int np = types[P.typed ? rtype[ring] : 0].np;
+    const int row = c / G.cols, col = c - row * G.cols;
+    int32_t h[kRlHead] = {-1, -1, -1, -1};
+    int n = 0;
+    auto run = [&](int a, int b) {
+        for (int u = a; u < b; u++) {
+            const int j = src[u];
+            if (j == q) continue;
+            const double2 d = cdiff(P, x, pos[j]);
+            if (!(d.x * d.x + d.y * d.y <= rl2)) continue;
+            const int idj = ID[j], rj = idj / P.nmax;
+            if (rj == ring) {
+                const int diff = abs(id - idj);
+                if (diff == 1 || diff == np - 1) continue;  // bonded neighbours do not interact
+            }
+            const int32_t e = j | ((P.typed ? rtype[rj] : 0) << kRlSlotBits);
+#pragma unroll
+            for (int s = 0; s < kRlHead; s++) h[s] = n == s ? e : h[s];
+            if (n >= kRlHead && n < kRlMax) more[(int64_t)(n - kRlHead) * P.na + q] = e;
+            n++;
+        }
+    };
+    for (int d = -1; d <= 1; d++) {
+        int rw = row + d;
+        rw = rw < 0 ? rw + G.rows : (rw >= G.rows ? rw - G.rows : rw);
+        const int32_t *sr = start + rw * G.cols;
+        if (col > 0 && col < G.cols - 1) {
+            run(sr[col - 1], sr[col + 2]);
+        } else {
+            run(sr[col == 0 ? 0 : col - 1], sr[col == 0 ? 2 : G.cols]);
+            run(sr[col == 0 ? G.cols - 1 : 0], sr[col == 0 ? G.cols : 1]);
+        }
+    }
+    if (n > kRlMax) {
+        atomicOr(status, kRlOverflow);
+        n = kRlMax;
+    }
+    head[q] = make_int4(h[0], h[1], h[2], h[3]);
+    count[q] = (uint8_t)n;
+}
+
+// After a build: reference chunks and counts (capacity as the binning checks
+// it), the build positions, cos and sin of the polarisations.
+__global__ void k_rl_keys(SysParams P, const double2 *__restrict__ pos, int32_t *__restrict__ key,
+                          int32_t *__restrict__ ccnt, double2 *__restrict__ xb, const double *__restrict__ pol,
+                          double2 *__restrict__ polcs, uint32_t *__restrict__ flags) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool valid = s < P.na;
+    uint32_t flag = 0;
+    int32_t r = 0, c = 0, k = -1;
+    double2 p = make_double2(0.0, 0.0);
+    if (valid) {
+        p = pos[s];
+        cell_rc(P, P.rows, P.cols, P.cl, P.ch, p.x, p.y, &flag, MAVI_FLAG_OUT_OF_BOX, &r, &c);
+        k = r * P.cols + c;
+    }
+    const int32_t rank = wave_arrival_rank(valid, k, ccnt);
+    if (valid && rank + 1 > P.nc) flag |= MAVI_FLAG_OVERFLOW;
+    if (flag) atomicOr(flags, flag);
+    if (s < P.nrings) {
+        double sn, cs;
+        sincos(pol[s], &sn, &cs);
+        polcs[s] = make_double2(cs, sn);
+    }
+    if (!valid) return;
+    key[s] = (r << 16) | c;
+    xb[s] = p;
+}
+
+// Block start: the state to roll back to, the step maxima cleared, the step
+// counter taken over.
+struct RLSnap {
+    double2 *pos, *cms, *cms_next;
+    double *pol;
+    uint32_t *flags;
+};
+__global__ void k_rl_block_start(int32_t na, int32_t nrings, const double2 *__restrict__ pos,
+                                 const double *__restrict__ pol, const double2 *__restrict__ cms,
+                                 const double2 *__restrict__ cms_next, RLSnap S, uint32_t *__restrict__ bmax,
+                                 int32_t nbmax, unsigned long long *__restrict__ out, uint32_t *__restrict__ status,
+                                 const uint32_t *__restrict__ flags, const unsigned long long *__restrict__ counter,
+                                 unsigned long long *__restrict__ c0) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < na) S.pos[i] = pos[i];
+    if (i < nrings) {
+        S.pol[i] = pol[i];
+        S.cms[i] = cms[i];
+        S.cms_next[i] = cms_next[i];
+    }
+    if (i < nbmax) bmax[i] = 0u;
+    if (i == 0) {
+        *S.flags = *flags;
+        out[0] = out[1] = 0ull;
+        *c0 = *counter;
+    }
+}
+
+// Block end: out[0] <- the largest squared step (bits), out[1] <- the largest
+// squared displacement from the build, out[2] <- the status.  At most 64
+// workgroups, so the maxima of one word take few atomics.
+constexpr int kRlMeasureBlocks = 64;
+__global__ __launch_bounds__(1024) void k_rl_measure(SysParams P, const double2 *__restrict__ pos,
+                                                     const double2 *__restrict__ xb,
+                                                     const uint32_t *__restrict__ bmax, int32_t nbmax,
+                                                     const uint32_t *__restrict__ status,
+                                                     unsigned long long *__restrict__ out) {
+    double d2 = 0.0;
+    uint32_t hi = 0u;
+    const int g = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (int s = g; s < P.na; s += stride) {
+        const double2 d = cdiff(P, pos[s], xb[s]);
+        const double v = d.x * d.x + d.y * d.y;
+        d2 = v == v ? fmax(d2, v) : INFINITY;
+    }
+    for (int s = g; s < nbmax; s += stride) hi = max(hi, bmax[s]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        d2 = fmax(d2, __shfl_xor(d2, o, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+    }
+    if (lane_id() == 0) {
+        atomicMax(&out[0], (unsigned long long)hi << 32);
+        atomicMax(&out[1], (unsigned long long)__double_as_longlong(d2));
+    }
+    if (g == 0) out[2] = *status;
+}
+
+__global__ void k_rl_copy_counter(const unsigned long long *__restrict__ src, unsigned long long *__restrict__ dst) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) dst[0] = src[0];
+}
+
+__global__ void k_rl_restore(int32_t na, int32_t nrings, RLSnap S, double2 *__restrict__ pos, double *__restrict__ pol,
+                             double2 *__restrict__ cms, double2 *__restrict__ cms_next, uint32_t *__restrict__ flags,
+                             uint32_t *__restrict__ status) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < na) pos[i] = S.pos[i];
+    if (i < nrings) {
+        pol[i] = S.pol[i];
+        cms[i] = S.cms[i];
+        cms_next[i] = S.cms_next[i];
+    }
+    if (i == 0) {
+        *flags = *S.flags;
+        *status = 0u;
+    }
+}
+
+int rl_waves(const SysParams &P) {
+    const int per = 64 / P.nmax;
+    return nblk(nblk(P.nrings, per), 4) * 4;
+}
+
+RLSnap rl_snap(const RList &N) { return RLSnap{N.psnap, N.csnap, N.nsnap, N.polsnap, N.fsnap}; }
+
+hipError_t rl_step(mavi_sys *s, bool last, hipStream_t st) {
+    RList &N = *s->rl;
+    ProfScope ps(s, MAVI_PROF_RINGS, st);
+    RLArgs A{};
+    const int c = s->cur;
+    A.Pin = s->P_[c];
+    A.Pout = s->P_[1 - c];
+    A.F = s->F;
+    A.slot_of = s->P.na == s->P.n ? nullptr : s->slot_of;
+    A.head = (const int4 *)N.head;
+    A.more = N.more;
+    A.count = N.count;
+    A.key = N.key;
+    A.ccnt = N.ccnt;
+    A.pol = s->pol;
+    A.polcs = N.polcs;
+    A.areas = s->areas;
+    A.cms = s->cms;
+    A.cms_next = s->cms_next;
+    A.cpos = s->cpos;
+    A.rtype = s->rtype;
+    A.types = s->types;
+    A.inter = N.uniform ? nullptr : s->inter;
+    A.uni = s->host_inter[0];
+    A.bmax = N.bmax;
+    A.flags = s->flags;
+    A.status = N.status;
+    A.seed = s->seed;
+    A.cin = N.counter + N.ph;
+    A.cout = N.counter + (1 - N.ph);
+    const dim3 grid(rl_waves(s->P) / 4);
+    if (last) hipLaunchKernelGGL(k_rl_step<true>, grid, dim3(kRlWG), 0, st, s->P, A);
+    else hipLaunchKernelGGL(k_rl_step<false>, grid, dim3(kRlWG), 0, st, s->P, A);
+    N.ph = 1 - N.ph;
+    s->cur = 1 - c;
+    return hipGetLastError();
+}
+
+// Eight steps from (copy, counter word) captured once.
+hipError_t rl_graph(mavi_sys *s, hipStream_t st, hipGraphExec_t *out) {
+    RList &N = *s->rl;
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return e;
+    const int c0 = s->cur, ph0 = N.ph;
+    hipError_t e1 = hipSuccess;
+    for (int k = 0; k < kRlGraphSteps && e1 == hipSuccess; k++) e1 = rl_step(s, false, st);
+    e = hipStreamEndCapture(st, &g);
+    s->cur = c0;
+    N.ph = ph0;
+    if (e1 != hipSuccess) e = e1;
+    if (e == hipSuccess) e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
+    if (g) (void)hipGraphDestroy(g);
+    return e;
+}
+
+// State in ring order (both copies' ids, slot_of the identity over active ids).
+hipError_t rl_ring_order(mavi_sys *s, hipStream_t st) {
+    RList &N = *s->rl;
+    if (N.ordered) return hipSuccess;
+    hipError_t e = mavi::launch_unpermute(s, false, false, st);
+    s->cur = 0;
+    if (e == hipSuccess) e = mavi::launch_iota_state(s, st);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(s->ID_[1], s->ID_[0], sizeof(int32_t) * (size_t)s->P.na, hipMemcpyDeviceToDevice, st);
+    s->sorted = false;
+    N.ordered = e == hipSuccess;
+    return e;
+}
+
+hipError_t rl_rebuild(mavi_sys *s, hipStream_t st) {
+    RList &N = *s->rl;
+    const SysParams &P = s->P;
+    hipError_t e = mavi::drop_keys(s, st);
+    if (e == hipSuccess) e = rl_ring_order(s, st);
+    if (e == hipSuccess) e = mavi::launch_cell_order(s, N.G, N.scan_ticket, N.scan_state, st);
+    if (e != hipSuccess) return e;
+    ProfScope ps(s, MAVI_PROF_BIN, st);
+    const int c = s->cur;
+    hipLaunchKernelGGL(k_rl_build, dim3(nblk(P.na, 256)), dim3(256), 0, st, N.G, P, s->P_[c], s->ID_[c], s->rtype,
+                       s->types, s->src, s->scell, s->start, N.rl2, (int4 *)N.head, N.more, N.count, N.status);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = mavi::launch_fill_i32(N.ccnt, 0, P.ncell, st)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_rl_keys, dim3(nblk(std::max(P.na, P.nrings), 256)), dim3(256), 0, st, P, s->P_[c], N.key,
+                       N.ccnt, N.xb, s->pol, N.polcs, s->flags);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    N.valid = true;
+    N.d_start = 0.0;
+    N.rebuilds++;
+    return hipSuccess;
+}
+
+double rl_step_est(const RList &N) { return std::max(N.step_hist[0], std::max(N.step_hist[1], N.step_hist[2])); }
+
+// Steps from a block start that keep d_start + (steps - 1) x step within
+// half_skin, at a step 1.08 times the estimate.
+int64_t rl_room(const RList &N) {
+    const double r = (N.half_skin - N.d_start) / (1.08 * rl_step_est(N));
+    if (!(r < 1e9)) return INT64_MAX;
+    return (int64_t)floor(r) + 1;
+}
+
+constexpr int64_t kRlMinBlock = 6;  // shorter blocks cost more than the rebuild they put off
+
+}  // namespace
+
+namespace mavi {
+
+bool rl_eligible(const mavi_sys *s) {
+    const SysParams &P = s->P;
+    if (P.potential != MAVI_POT_RINGS || P.nwalls > 0 || !P.periodic || P.na <= 0 || P.nmax > 32) return false;
+    if (P.na > kRlSlotMask || P.ntypes > 32) return false;
+    if (P.cols < 3 || P.rows < 3 || P.rows > 32767 || P.cols > 65535) return false;
+    const double range = sqrt(s->list2);
+    if (!(range > 0.0) || !(range < INFINITY)) return false;
+    // every pair within range is in adjacent chunks at the binned positions
+    return P.cl >= range * (1.0 + 1e-12) && P.ch >= range * (1.0 + 1e-12);
+}
+
+// skin as a fraction of the range; false: the box holds fewer than three cells
+// of the list grid a side
+bool rl_set_skin(mavi_sys *s, double skin_frac) {
+    RList &N = *s->rl;
+    const SysParams &P = s->P;
+    const double range = sqrt(s->list2), skin = skin_frac * range;
+    const double rl = (range + skin) * (1.0 + 1e-9);
+    N.rl2 = rl * rl;
+    N.half_skin = 0.5 * skin * (1.0 - 1e-9);
+    SysParams G = P;
+    G.cols = P.cl >= rl ? P.cols : (int32_t)floor(P.L / rl);
+    G.rows = P.ch >= rl ? P.rows : (int32_t)floor(P.H / rl);
+    G.cl = P.L / (double)std::max(G.cols, 1);
+    G.ch = P.H / (double)std::max(G.rows, 1);
+    G.ncell = G.cols * G.rows;
+    G.nc = P.na;
+    N.G = G;
+    N.valid = false;
+    N.fits = G.cols >= 3 && G.rows >= 3;
+    return N.fits;
+}
+
+hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
+    s->rl = new RList();
+    RList &N = *s->rl;
+    rl_set_skin(s, kRlSkin);
+    const int64_t na = s->P.na, nr = s->P.nrings;
+    N.uniform = true;
+    for (const RingInter &I : s->host_inter) {
+        const RingInter &J = s->host_inter[0];
+        N.uniform = N.uniform && I.k_rep == J.k_rep && I.k_atr == J.k_atr && I.dist_eq == J.dist_eq &&
+                    I.dist_max == J.dist_max;
+    }
+    N.nbmax = rl_waves(s->P);
+    N.scan_words = (s->P.ncell + 1 + kScanTileMin - 1) / kScanTileMin + 1;
+    hipError_t e = dalloc(&N.head, 4 * na, st);
+    if (e == hipSuccess) e = dalloc(&N.more, (int64_t)(kRlMax - kRlHead) * na, st);
+    if (e == hipSuccess) e = dalloc(&N.count, na, st);
+    if (e == hipSuccess) e = dalloc(&N.key, na, st);
+    if (e == hipSuccess) e = dalloc(&N.ccnt, (int64_t)s->P.ncell, st);
+    if (e == hipSuccess) e = dalloc(&N.xb, na, st);
+    if (e == hipSuccess) e = dalloc(&N.psnap, na, st);
+    if (e == hipSuccess) e = dalloc(&N.csnap, nr, st);
+    if (e == hipSuccess) e = dalloc(&N.nsnap, nr, st);
+    if (e == hipSuccess) e = dalloc(&N.polsnap, nr, st);
+    if (e == hipSuccess) e = dalloc(&N.fsnap, 1, st);
+    if (e == hipSuccess) e = dalloc(&N.polcs, nr, st);
+    if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
+    if (e == hipSuccess) e = dalloc(&N.status, 1, st);
+    if (e == hipSuccess) e = dalloc(&N.counter, 2, st);
+    if (e == hipSuccess) e = dalloc(&N.out, 3, st);
+    if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);
+    if (e == hipSuccess) e = dalloc(&N.scan_state, N.scan_words, st);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&N.host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
+    return e;
+}
+
+void rl_drop_graph(mavi_sys *s) {
+    if (!s->rl) return;
+    for (auto &row : s->rl->graph)
+        for (auto &g : row) {
+            if (!g) continue;
+            (void)hipStreamSynchronize(s->ctx->stream);
+            (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
+}
+
+void rl_free(mavi_sys *s) {
+    if (!s->rl) return;
+    RList &N = *s->rl;
+    rl_drop_graph(s);
+    dfree(N.head); dfree(N.more); dfree(N.count); dfree(N.key); dfree(N.ccnt); dfree(N.xb); dfree(N.psnap);
+    dfree(N.csnap); dfree(N.nsnap); dfree(N.polsnap); dfree(N.fsnap); dfree(N.polcs); dfree(N.bmax); dfree(N.status);
+    dfree(N.counter); dfree(N.out); dfree(N.scan_ticket); dfree(N.scan_state);
+    if (N.host) (void)hipHostFree(N.host);
+    delete s->rl;
+    s->rl = nullptr;
+}
+
+bool rl_active(const mavi_sys *s) {
+    return s->rl && s->rl->on && s->rl->fits && !s->rl->disabled && !s->neigh_on && !s->var;
+}
+
+int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
+    mavi_ctx *ctx = s->ctx;
+    hipStream_t st = ctx->stream;
+    RList &N = *s->rl;
+    const SysParams &P = s->P;
+    *left = 0;
+    const int span = std::max(std::max(P.na, P.nrings), N.nbmax);
+    int64_t k = 0;
+    while (k < nsteps) {
+        const bool fresh = !N.valid;
+        if (fresh) HIPCHK(ctx, rl_rebuild(s, st));
+        int64_t want = N.block_now;
+        if (N.block == 0) {
+            if (rl_step_est(N) > 0.0) want = std::min(want, std::max<int64_t>(1, rl_room(N)));
+            else want = std::min<int64_t>(want, 8);  // no step length measured yet
+        }
+        const int64_t blk = std::min<int64_t>(want, nsteps - k);
+        const int cur0 = s->cur;
+        N.ph = 0;
+        hipLaunchKernelGGL(k_rl_block_start, dim3(nblk(span, 256)), dim3(256), 0, st, P.na, P.nrings, s->P_[s->cur],
+                           s->pol, s->cms, s->cms_next, rl_snap(N), N.bmax, N.nbmax, N.out, N.status, s->flags,
+                           s->counter, N.counter);
+        HIPCHK(ctx, hipGetLastError());
+        const bool graphs = s->use_graphs && !s->prof;
+        const bool ends = k + blk == nsteps;  // the block's last step leaves the call's outputs
+        const int64_t plain = ends ? blk - 1 : blk;
+        int64_t done = 0;
+        while (done < plain) {
+            if (graphs && done + kRlGraphSteps <= plain) {
+                hipGraphExec_t &g = N.graph[s->cur][N.ph];
+                if (!g) HIPCHK(ctx, rl_graph(s, st, &g));
+                HIPCHK(ctx, hipGraphLaunch(g, st));
+                done += kRlGraphSteps;  // an even number: the copies and the counter words are where they were
+            } else {
+                HIPCHK(ctx, rl_step(s, false, st));
+                done++;
+            }
+        }
+        if (ends) HIPCHK(ctx, rl_step(s, true, st));
+        const int mb = std::min(nblk(std::max(P.na, N.nbmax), 1024), kRlMeasureBlocks);
+        hipLaunchKernelGGL(k_rl_measure, dim3(mb), dim3(1024), 0, st, P, s->P_[s->cur], N.xb, N.bmax, N.nbmax,
+                           N.status, N.out);
+        HIPCHK(ctx, hipGetLastError());
+        HIPCHK(ctx, hipMemcpyAsync(N.host, N.out, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+        HIPCHK(ctx, hipStreamSynchronize(st));
+        const double step = sqrt(__builtin_bit_cast(double, N.host[0]));
+        const double d_end = sqrt(__builtin_bit_cast(double, N.host[1]));
+        const uint32_t status = (uint32_t)N.host[2];
+        N.step_hist[N.step_i] = step;
+        N.step_i = (N.step_i + 1) % 3;
+        // The block evaluated y_0 .. y_{T-1} and moved to y_T: y_t is within
+        // min(d_start + t step, d_end + (T - t) step) of its build position.
+        const double T = (double)blk;
+        const bool finite = std::isfinite(step) && std::isfinite(d_end);
+        const double bound = std::min(N.d_start + (T - 1.0) * step, 0.5 * (N.d_start + d_end + T * step));
+        if (status || !finite || !(bound <= N.half_skin)) {
+            s->cur = cur0;
+            hipLaunchKernelGGL(k_rl_restore, dim3(nblk(span, 256)), dim3(256), 0, st, P.na, P.nrings, rl_snap(N),
+                               s->P_[s->cur], s->pol, s->cms, s->cms_next, s->flags, N.status);
+            HIPCHK(ctx, hipGetLastError());
+            N.valid = false;
+            N.rollbacks++;
+            // (one step from a fresh build evaluates the build positions: its
+            // bound is 0, so a block can always shrink to one that passes)
+            if (status || !finite) {
+                // the chunk gather takes over, for good if a list or a chunk
+                // overflowed, for this call if the state is not finite
+                N.disabled = status != 0;
+                if (!finite) N.step_hist[0] = N.step_hist[1] = N.step_hist[2] = 0.0;
+                *left = nsteps - k;
+                return MAVI_OK;
+            }
+            if (N.block != 0 && N.block_now > 1) N.block_now = std::max(1, N.block_now / 2);
+            continue;
+        }
+        hipLaunchKernelGGL(k_rl_copy_counter, dim3(1), dim3(64), 0, st, N.counter + N.ph, s->counter);
+        HIPCHK(ctx, hipGetLastError());
+        k += blk;
+        N.d_start = d_end;
+        if (N.block == 0) {
+            if (rl_room(N) < kRlMinBlock) N.valid = false;
+            // steps so long that a fresh list would serve only a few: the gather
+            if (!N.valid && 1.08 * rl_step_est(N) * (double)kRlMinBlock > N.half_skin && k < nsteps) {
+                *left = nsteps - k;
+                return MAVI_OK;
+            }
+        } else if (d_end + 1.2 * step * (double)N.block_now > N.half_skin) {
+            N.valid = false;
+        }
+        const int32_t cap = N.block == 0 ? kNlBlockCap : N.block;
+        if (N.block_now < cap) N.block_now = std::min(cap, 2 * N.block_now);
+    }
+    s->sorted = false;  // not in chunk order
+    return MAVI_OK;
+}
+
+}  // namespace mavi

@@ -1,0 +1,188 @@
+"""Rings step! on Verlet lists (one kernel per step, mavi_rlist.hip) against
+the chunk gather (MAVI_OPT_NLIST 0): the lists add a particle's pairs in the
+gather's order, so positions, polarisations, forces, areas, centres of mass and
+continuous positions are the same bits, whatever the box, the ring sizes, the
+length of the lists, the rebuild times and the split into calls.  The gather
+itself is checked against the oracle in test_gpu_rings.py."""
+import sys
+
+import numpy as np
+import pytest
+
+from test_gpu_rings import normal_case, types_case
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def mixture(**kw):
+    from mavi_hip import workloads as wl
+
+    return wl.rings_mixture(**kw)
+
+
+def squeezed(case, factor, dt):
+    """The case shrunk: many pairs in range of a particle, long lists."""
+    import mavi_hip as mv
+    from mavi_hip import rings
+
+    state, space, cfg, ic = case
+    g = space.geometry_cfg
+    L, H = g.length * factor, g.height * factor
+    state = rings.RingsState(rings_pos=state.rings_pos * factor, pol=state.pol, num_particles=state.num_particles,
+                             types=state.types)
+    reach = 1.2
+    space = mv.SpaceCfg(geometry_cfg=mv.RectangleCfg(length=L, height=H), wall_type=mv.PeriodicWalls())
+    ic = mv.IntCfg(dt=dt, chunks_cfg=mv.ChunksCfg(int(L // reach - 1e-9), int(H // reach - 1e-9)), device=mv.GPU())
+    return state, space, cfg, ic
+
+
+CASES = {
+    "normal": lambda: normal_case(True),
+    "normal_ragged": lambda: normal_case(True, n=21, cols=7, rows=5, seed=3),
+    "smallest_rings": lambda: normal_case(True, n=4, cols=6, rows=7, seed=4),
+    "largest_rings": lambda: normal_case(True, n=32, cols=5, rows=3, seed=5),
+    "few_cells": lambda: normal_case(True, n=9, cols=2, rows=2, seed=6),
+    "types": lambda: types_case(True),
+    "mixture": lambda: mixture(nrings=120, seed=8),
+    "dense": lambda: squeezed(normal_case(True, n=10, cols=9, rows=8), 0.62, 1e-4),
+    "dense_types": lambda: squeezed(types_case(True), 0.7, 1e-4),
+}
+
+
+def make(case, lists, seed=11):
+    from mavi_hip import _lib, rings
+
+    state, space, cfg, ic = CASES[case]()
+    s = rings.RingsSystem(state=state, space_cfg=space, dynamic_cfg=cfg, int_cfg=ic, seed=seed)
+    if not lists:
+        s.dev.set_option(_lib.MAVI_OPT_NLIST, 0)
+    return s
+
+
+def same(tag, a, b):
+    for s in (a, b):
+        s.download()
+    for what, x, y in (("pos", a.state.pos, b.state.pos), ("pol", a.state.pol, b.state.pol),
+                       ("forces", a.forces, b.forces), ("areas", a.areas, b.areas), ("cms", a.cms, b.cms),
+                       ("continuos_pos", a.continuos_pos, b.continuos_pos)):
+        assert np.array_equal(x, y), (tag, what, float(np.abs(np.asarray(x) - np.asarray(y)).max()))
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_same_bits_as_the_gather(gpu_ctx, case):
+    a, b = make(case, True), make(case, False)
+    info = a.dev.nlist_info()
+    say(f"[rings lists] {case} {info}")
+    assert info["eligible"] and not b.dev.nlist_info()["active"]
+    for k in (8, 61, 1, 30):
+        a.advance(k)
+        b.advance(k)
+        same((case, k), a, b)
+    say(f"[rings lists] {case} {a.dev.nlist_info()}")
+    assert a.dev.nlist_info()["rebuilds"] >= 1 or case == "few_cells"
+
+
+@pytest.mark.parametrize("skin,block,graphs", [(0, 0, 0), (50, 64, 1), (100, 7, 1), (600, 0, 1), (1000, 1, 1)])
+def test_skins_blocks_and_rollbacks(gpu_ctx, skin, block, graphs):
+    """Rebuild times, rolled-back blocks (a skin too thin for its fixed
+    block) and direct launches change nothing."""
+    from mavi_hip import _lib
+
+    a, b = make("normal", True), make("normal", False)
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, skin)
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_BLOCK, block)
+    a.dev.set_option(_lib.MAVI_OPT_GRAPHS, graphs)
+    a.advance(100)
+    b.advance(100)
+    info = a.dev.nlist_info()
+    say(f"[rings lists] skin {skin} block {block} graphs {graphs} {info}")
+    if block == 64:
+        assert info["rollbacks"] >= 1
+    same((skin, block), a, b)
+
+
+def test_long_lists_hand_over(gpu_ctx):
+    """Lists of more than 16 partners switch off; the gather runs the steps."""
+    from mavi_hip import _lib
+
+    a, b = make("dense", True), make("dense", False)
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, 2000)
+    a.advance(40)
+    b.advance(40)
+    info = a.dev.nlist_info()
+    say(f"[rings lists overflow] {info}")
+    assert not info["active"]
+    same("overflow", a, b)
+
+
+def test_state_changes_between_runs(gpu_ctx):
+    """Between list runs: a new state, forces!, a binning, the noise stream
+    moved and reseeded, an invasion schedule, contact neighbours on and off."""
+    from mavi_hip import rings
+
+    a, b = make("mixture", True), make("mixture", False)
+    rng = np.random.default_rng(5)
+    for s in (a, b):
+        s.advance(40)
+    pos = np.mod(a.state.pos + rng.uniform(-0.01, 0.01, size=a.state.pos.shape), a.space_cfg.geometry_cfg.length)
+    for s in (a, b):
+        s.state.pos[...] = pos
+        s.upload()
+        s.advance(20)
+    same("new state", a, b)
+    for s in (a, b):
+        s.dev.forces()
+        s.advance(12)
+        s.dev.bin()
+        s.advance(12)
+        s.dev.set_noise_state(77, 1000)
+        s.advance(16)
+    same("forces, bin, noise", a, b)
+    assert a.dev.noise_state() == b.dev.noise_state()
+    grid = rings.ring_chunks_grid(a.state, a.space_cfg, a.dynamic_cfg, type(a.int_cfg.chunks_cfg)(8, 8))
+    for s in (a, b):
+        s.dev.rings_invasions_cfg(True, 7, *grid)
+        s.advance(45)
+    assert np.array_equal(a.dev.rings_invasions(), b.dev.rings_invasions())
+    same("invasions", a, b)
+    for s in (a, b):
+        s.dev.rings_neighbors_cfg(True, 1.1, False)
+        s.advance(10)
+    for x, y in zip(a.dev.rings_neighbors(), b.dev.rings_neighbors()):
+        assert np.array_equal(x, y)
+    for s in (a, b):
+        s.dev.rings_neighbors_cfg(False)
+        s.advance(9)
+    same("neighbours", a, b)
+
+
+def test_errors_are_the_gathers(gpu_ctx):
+    """A chunk over its capacity and a non-finite position fail the same way."""
+    import mavi_hip as mv
+    from mavi_hip import _lib, rings
+
+    state, space, cfg, ic = CASES["normal"]()
+    d, chunks, keep = rings.describe(state, space, cfg, ic, 1)
+    d.nc = 1
+    for lists in (1, 0):
+        dev = _lib.DeviceSystem(gpu_ctx, d, keep=keep)
+        dev.set_option(_lib.MAVI_OPT_NLIST, lists)
+        dev.upload(state.pos, None, state.pol)
+        with pytest.raises(mv.CellOverflowError):
+            dev.step(20)
+    d.nc = chunks.nc
+    bad = state.pos.copy()
+    bad[17] = np.nan
+    for lists in (1, 0):
+        dev = _lib.DeviceSystem(gpu_ctx, d, keep=keep)
+        dev.set_option(_lib.MAVI_OPT_NLIST, lists)
+        dev.upload(bad, None, state.pol)
+        with pytest.raises(mv.MaviError):
+            dev.step(20)
+        dev.upload(state.pos, None, state.pol)  # a good state runs again
+        dev.step(20)
