@@ -22,6 +22,7 @@ constexpr int64_t kMlpParams = kOffB3 + kMlpOut;
 static_assert(kMlpParams == MAVI_MLP_NPARAMS, "parameter count of the C ABI");
 
 constexpr int kSplitRows = 256;  // rows per split-K partial of a weight gradient
+constexpr int kMaxSplits = 64;   // largest minibatch: kMaxSplits * kSplitRows rows
 
 struct mavi_mlp {
     mavi_ctx *ctx = nullptr;
@@ -32,24 +33,25 @@ struct mavi_mlp {
     int64_t adam_t = 0;
     uint16_t *w[4] = {nullptr, nullptr, nullptr, nullptr};  // BF16 W_l^T (W3 padded to 16 rows)
     float *b3 = nullptr;                                     // output bias padded to 16
-    float *ws = nullptr;                                     // split-K partials
-    int64_t ws_cap = 0;
+    uint16_t *wt[2] = {nullptr, nullptr};                    // BF16 W_1, W_2 (in x out), for the backward pass
     int fused_grid = 256;
-    // training work arrays, sized for work_cap rows
+    // layer-by-layer forward, sized for work_cap rows
     int work_cap = 0;
-    float *Z[3] = {nullptr, nullptr, nullptr};
     uint16_t *H[3] = {nullptr, nullptr, nullptr};
-    uint16_t *dZa = nullptr, *dZb = nullptr, *dY = nullptr;
-    float *Yw = nullptr, *loss_part = nullptr;
+    float *Yw = nullptr;
+    // training pass, sized for train_cap rows: feature-major arrays, loss
+    // partials, split-K partials of every parameter
+    int64_t train_cap = 0;
+    uint16_t *XT = nullptr, *HT[3] = {nullptr, nullptr, nullptr}, *dZT[3] = {nullptr, nullptr, nullptr}, *dYT = nullptr;
+    float *loss_part = nullptr, *ws = nullptr;
+    // rows handed in by mavi_mlp_loss_grad
+    int rows_cap = 0;
     uint16_t *Xw = nullptr;
     float *Tw = nullptr;
-    // device data set (features, targets) and the minibatch gathered from it
+    // device data set (features, targets)
     uint16_t *dsX = nullptr;
     float *dsT = nullptr;
     int64_t ds_count = 0, ds_cap = 0;
-    uint16_t *bX = nullptr;
-    float *bT = nullptr;
-    int b_cap = 0;
     float *loss_hist = nullptr;
     int64_t loss_hist_cap = 0;
 };
@@ -63,8 +65,6 @@ namespace mavi {
 hipError_t ensure_work(mavi_mlp *p, int M);
 hipError_t mlp_forward_fused(mavi_mlp *p, const uint16_t *X, int M, float *Y, hipStream_t st);
 hipError_t mlp_forward_gemm(mavi_mlp *p, const uint16_t *X, int M, hipStream_t st);
-hipError_t mlp_loss_grad_dev(mavi_mlp *p, const uint16_t *X, const float *T, int M, hipStream_t st);
-hipError_t mlp_adam_step(mavi_mlp *p, float lr, hipStream_t st);
 hipError_t mlp_sync_weights(mavi_mlp *p, hipStream_t st);
 double mlp_loss_value(mavi_mlp *p, int M, hipStream_t st, hipError_t *err);
 hipError_t mlp_dataset_reserve(mavi_mlp *p, int64_t cap);

@@ -3,15 +3,18 @@
 // the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16).
 //
 //   inference  k_mlp_fused: one persistent kernel, all weights resident in LDS
-//              (117 KB), 8 wavefronts per CU (two per SIMD, so one wave's
+//              (117 KB), 12 wavefronts per CU (three per SIMD, so one wave's
 //              activation epilogue overlaps another's MFMAs), each running
-//              16-row tiles through the four layers; activations go through
-//              a per-wave LDS tile between layers
-//   training   k_gemm<TA, TB, EPI>: LDS-staged 64x64x32 tiles with optional
-//              transposed operands and fused epilogues (bias + GELU keeping
-//              the pre-activation, GELU backward, split-K partials), plus
-//              loss/dY, two-stage column sums (bias gradients), split-K reduction and
-//              Adam kernels
+//              16-row tiles through the four layers; activations stay in
+//              registers
+//   training   three launches per step: k_train_pass (minibatch rows, forward,
+//              loss and backward of 32 rows per workgroup; activations and
+//              gradients written transposed), k_train_wgrad (weight and bias
+//              gradients of a 32x32 block over 256 rows per wave, both operands
+//              read straight into MFMA registers), k_train_update (sum of the
+//              row chunks, Adam, BF16 copies)
+//   check      k_gemm<TA, TB, EPI>: LDS-staged 64x64x32 tiles with optional
+//              transposed operands; the layer-by-layer forward and the tile test
 //
 // Parameters (FP32 master copy, flat): for layer l = 0..3, W_l^T (out x in,
 // row-major) followed by b_l.  BF16 copies of W_l^T feed the matrix cores.
@@ -78,13 +81,11 @@ __device__ __forceinline__ void wave_sync() {
 // fragment reads fall on distinct banks).  Wave w owns the 32x32 quarter
 // (w/2, w%2) as 2x2 MFMA blocks.  blockIdx.z is the split-K index.
 // ---------------------------------------------------------------------------
-enum { EPI_F32 = 0, EPI_BIAS_GELU = 1, EPI_BIAS = 2, EPI_GELU_BWD = 3 };
+enum { EPI_F32 = 0, EPI_BIAS_GELU = 1, EPI_BIAS = 2 };
 
 struct Epi {
     const float *bias;  // EPI_BIAS_GELU, EPI_BIAS
-    float *Z;           // pre-activation: written (BIAS_GELU) / read (GELU_BWD)
-    int ldz;
-    uint16_t *H;        // BF16 output (BIAS_GELU: GELU(z); GELU_BWD: dZ)
+    uint16_t *H;        // BIAS_GELU: BF16 output GELU(z)
     int ldh;
 };
 
@@ -165,95 +166,39 @@ __global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const uint16_
                     C[(int64_t)m * ldc + n] = x;
                 } else if constexpr (EPI == EPI_BIAS) {
                     C[(int64_t)m * ldc + n] = x + ep.bias[n];
-                } else if constexpr (EPI == EPI_BIAS_GELU) {
-                    const float z = x + ep.bias[n];
-                    ep.Z[(int64_t)m * ep.ldz + n] = z;
-                    ep.H[(int64_t)m * ep.ldh + n] = f2bf(gelu(z));
                 } else {
-                    const float z = ep.Z[(int64_t)m * ep.ldz + n];
-                    ep.H[(int64_t)m * ep.ldh + n] = f2bf(x * gelu_grad(z));
+                    ep.H[(int64_t)m * ep.ldh + n] = f2bf(gelu(x + ep.bias[n]));
                 }
             }
         }
 }
 
-// out[i] = scale * sum_z ws[z * stride + i] for i < count (fixed order over z).
-__global__ void k_split_reduce(const float *__restrict__ ws, int nsplit, int64_t stride, int64_t count,
-                               float *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float s = 0.f;
-    for (int z = 0; z < nsplit; z++) s += ws[z * stride + i];
-    out[i] = s;
-}
-
-// Column sums of H (BF16 [M][N], FP32 sums in a fixed order), first stage:
-// block (x, y) sums rows [256 y, 256 y + 256) of columns [64 x, 64 x + 64)
-// into part[y][n]; k_split_reduce then adds the row chunks in order.
-constexpr int kColRows = 256;
-__global__ void k_colsum_part(const uint16_t *__restrict__ H, int M, int N, int ldh, float *__restrict__ part) {
-    __shared__ float red[4][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + c;
-    const int m0 = blockIdx.y * kColRows;
-    float s = 0.f;
-    if (n < N)
-        for (int m = m0 + g; m < min(M, m0 + kColRows); m += 4) s += bf2f(H[(int64_t)m * ldh + n]);
-    red[g][c] = s;
-    __syncthreads();
-    if (g == 0 && n < N) part[(int64_t)blockIdx.y * N + n] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
-}
-
-// Mean-squared error L = 1/(2M) sum_m sum_o (Y - T)^2 over the 2 outputs;
-// dY = (Y - T) / M as BF16 into the 16-wide padded gradient (columns 2..15
-// stay zero).  Block partial sums of the squared error go to part[].
-__global__ void k_loss(const float *__restrict__ Y, const float *__restrict__ T, int M, uint16_t *__restrict__ dY,
-                       float *__restrict__ part) {
-    __shared__ float red[256];
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    float s = 0.f;
-    if (m < M) {
-        const float inv = 1.0f / (float)M;
-        for (int o = 0; o < kMlpOut; o++) {
-            const float d = Y[(int64_t)m * kMlpOutPad + o] - T[(int64_t)m * kMlpOut + o];
-            s += d * d;
-            dY[(int64_t)m * kMlpOutPad + o] = f2bf(d * inv);
-        }
+// BF16 copies of one parameter: W_l^T (out x in; W3 padded to 16 rows), the
+// transposes W_1, W_2 (in x out) of the backward pass, the padded output bias.
+struct BfWeights {
+    uint16_t *w0, *w1, *w2, *w3, *t1, *t2;
+    float *b3;
+};
+__device__ __forceinline__ void store_param(const BfWeights &W, int i, float v) {
+    if (i < kOffB0) {
+        W.w0[i] = f2bf(v);
+    } else if (i >= kOffW1 && i < kOffB1) {
+        const int j = i - (int)kOffW1;
+        W.w1[j] = f2bf(v);
+        W.t1[(j % kMlpHid) * kMlpHid + j / kMlpHid] = f2bf(v);
+    } else if (i >= kOffW2 && i < kOffB2) {
+        const int j = i - (int)kOffW2;
+        W.w2[j] = f2bf(v);
+        W.t2[(j % kMlpHid) * kMlpHid + j / kMlpHid] = f2bf(v);
+    } else if (i >= kOffW3 && i < kOffB3) {
+        W.w3[i - kOffW3] = f2bf(v);
+    } else if (i >= kOffB3) {
+        W.b3[i - kOffB3] = v;
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
-
-// Adam on the FP32 master parameters (step t counted from 1).
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m1,
-                       float *__restrict__ m2, int64_t n, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = b;
-    p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
-}
-
-// FP32 master -> BF16 weights (W0t..W3t, W3t padded to 16 rows) and the
-// padded output bias.
-__global__ void k_sync_weights(const float *__restrict__ p, uint16_t *__restrict__ w0, uint16_t *__restrict__ w1,
-                               uint16_t *__restrict__ w2, uint16_t *__restrict__ w3, float *__restrict__ b3) {
+__global__ void k_sync_weights(const float *__restrict__ p, BfWeights W) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < kMlpHid * kMlpIn) w0[i] = f2bf(p[kOffW0 + i]);
-    if (i < kMlpHid * kMlpHid) {
-        w1[i] = f2bf(p[kOffW1 + i]);
-        w2[i] = f2bf(p[kOffW2 + i]);
-    }
-    if (i < kMlpOutPad * kMlpHid) w3[i] = (i < kMlpOut * kMlpHid) ? f2bf(p[kOffW3 + i]) : (uint16_t)0;
-    if (i < kMlpOutPad) b3[i] = (i < kMlpOut) ? p[kOffB3 + i] : 0.f;
+    if (i < kMlpParams) store_param(W, i, p[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -421,8 +366,12 @@ __global__ __launch_bounds__(64 * kFusedWaves) void k_mlp_fused(
     }
 }
 
-// Minibatch rows drawn uniformly (with replacement) from the data set by a
-// splitmix64 hash of (seed, step, row): one thread per 16-byte chunk.
+// ---------------------------------------------------------------------------
+// Training
+// ---------------------------------------------------------------------------
+
+// Minibatch rows are drawn uniformly (with replacement) from the data set by a
+// splitmix64 hash of (seed, step, row).
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     z += 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -430,27 +379,329 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-__global__ void k_gather_batch(const uint16_t *__restrict__ dsX, const float *__restrict__ dsT, int64_t count,
-                               uint64_t seed, int64_t step, int batch, uint16_t *__restrict__ bX,
-                               float *__restrict__ bT) {
-    constexpr int kChunks = kMlpIn / 8;
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (int64_t)batch * kChunks) return;
-    const int j = (int)(q / kChunks), c = (int)(q % kChunks);
-    const uint64_t h = mix64(seed ^ mix64(((uint64_t)step << 32) ^ (uint64_t)j));
-    const int64_t src = (int64_t)(h % (uint64_t)count);
-    *reinterpret_cast<uint4 *>(bX + (int64_t)j * kMlpIn + c * 8) =
-        *reinterpret_cast<const uint4 *>(dsX + src * kMlpIn + c * 8);
-    if (c == 0)
-        for (int o = 0; o < kMlpOut; o++) bT[(int64_t)j * kMlpOut + o] = dsT[src * kMlpOut + o];
+struct TrainIn {
+    const uint16_t *X;  // rows of features
+    const float *T;     // and targets
+    int64_t count;      // > 0: minibatch drawn from `count` rows by (seed, step); 0: row j is row j
+    uint64_t seed;
+    int64_t step;
+};
+
+// Transposed (feature-major) BF16 arrays of one pass over Mp rows (M padded to
+// whole row chunks; the padding's gradients are zero).
+struct TrainT {
+    uint16_t *X, *H[3], *dZ[3], *dY;
+    int Mp;
+};
+
+constexpr int kTrRows = 32;                // rows per workgroup of the training pass
+constexpr int kTrPX = kMlpIn + 8, kTrPA = kMlpHid + 8;
+
+// One [32 rows][COLS] LDS tile to feature-major global rows, 16 bytes (8 rows)
+// per thread and piece.
+template <int COLS, int PITCH>
+__device__ __forceinline__ void store_transposed(const uint16_t *tile, uint16_t *__restrict__ dst, int64_t Mp, int m0,
+                                                 int t) {
+    for (int q = t; q < COLS * (kTrRows / 8); q += 256) {
+        const int col = q >> 2, r0 = (q & 3) * 8;
+        uint16_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = tile[(r0 + j) * PITCH + col];
+        *reinterpret_cast<uint4 *>(dst + col * Mp + m0 + r0) =
+            make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16,
+                       v[6] | (uint32_t)v[7] << 16);
+    }
 }
 
-// loss[0] = sum of the block partials / (2M), in a fixed order.
-__global__ void k_loss_finish(const float *__restrict__ part, int nb, int M, float *__restrict__ loss) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float s = 0.f;
-    for (int i = 0; i < nb; i++) s += part[i];
-    loss[0] = s / (2.0f * (float)M);
+// Forward, loss and backward of 32 rows.  Wave w owns hidden units 32 w ..
+// 32 w + 31 of every layer: it reads only their weights (from L2, a layer
+// ahead of their use, no LDS copy), keeps their pre-activations in registers
+// for the backward pass and exchanges BF16 activations and gradients with the
+// other waves through two LDS tiles.  BF16 rounding where the layer-by-layer
+// oracle rounds: weights, hidden activations, dY and dZ.
+// Bound: the latency of the seven dependent layers (one workgroup per CU at
+// 8192 rows).  The GEMM chain it replaces took 15 launches and about 95 us at
+// 8192 rows, its operands staged with 2-byte loads.
+__global__ __launch_bounds__(256) void k_train_pass(TrainIn in, int M, const uint16_t *__restrict__ w0,
+                                                    const uint16_t *__restrict__ w1, const uint16_t *__restrict__ w2,
+                                                    const uint16_t *__restrict__ w3, const uint16_t *__restrict__ t1,
+                                                    const uint16_t *__restrict__ t2, const float *__restrict__ params,
+                                                    const float *__restrict__ b3, TrainT O,
+                                                    float *__restrict__ loss_part) {
+    __shared__ __attribute__((aligned(16))) uint16_t sx[kTrRows * kTrPX];
+    __shared__ __attribute__((aligned(16))) uint16_t sa[2][kTrRows * kTrPA];
+    __shared__ float st[kTrRows][2], sdy[kTrRows][2];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int fr = lane & 15, g = lane >> 4, fk = g * 8;
+    const int m0 = blockIdx.x * kTrRows;
+
+    // this wave's fragments of a layer's weights (rows 32 w + 16 f + fr)
+    auto load_w = [&](const uint16_t *W, int kin, int ks, int f) { return ld8(W + (32 * w + 16 * f + fr) * kin + ks * 32 + fk); };
+    bf16x8 wf[kMlpIn / 32][2], wn[kMlpHid / 32][2];
+#pragma unroll
+    for (int ks = 0; ks < kMlpIn / 32; ks++)
+#pragma unroll
+        for (int f = 0; f < 2; f++) wf[ks][f] = load_w(w0, kMlpIn, ks, f);
+
+    // the rows
+    for (int q = t; q < kTrRows * (kMlpIn / 8); q += 256) {
+        const int j = q / (kMlpIn / 8), c = (q % (kMlpIn / 8)) * 8;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (m0 + j < M) {
+            int64_t row = m0 + j;
+            if (in.count > 0)
+                row = (int64_t)(mix64(in.seed ^ mix64(((uint64_t)in.step << 32) ^ (uint64_t)row)) % (uint64_t)in.count);
+            v = *reinterpret_cast<const uint4 *>(in.X + row * kMlpIn + c);
+            if (c == 0) {
+                st[j][0] = in.T[row * kMlpOut];
+                st[j][1] = in.T[row * kMlpOut + 1];
+            }
+        }
+        *reinterpret_cast<uint4 *>(&sx[j * kTrPX + c]) = v;
+    }
+    __syncthreads();
+
+    f32x4 acc[2][2], z[3][2][2];  // [f][row tile]
+    auto clear = [&]() {
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    // 4 consecutive units of row 16 u + fr into an activation tile
+    auto put = [&](uint16_t *tile, int f, int u, float a, float b, float c, float d) {
+        *reinterpret_cast<uint2 *>(&tile[(16 * u + fr) * kTrPA + 32 * w + 16 * f + 4 * g]) = make_uint2(f2bf2(a, b), f2bf2(c, d));
+    };
+    auto forward_out = [&](int l, const float *bias, uint16_t *tile) {
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+            const float4 b = *reinterpret_cast<const float4 *>(bias + 32 * w + 16 * f + 4 * g);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const f32x4 v = f32x4{acc[f][u][0] + b.x, acc[f][u][1] + b.y, acc[f][u][2] + b.z, acc[f][u][3] + b.w};
+                z[l][f][u] = v;
+                put(tile, f, u, gelu(v[0]), gelu(v[1]), gelu(v[2]), gelu(v[3]));
+            }
+        }
+    };
+    auto backward_out = [&](int l, uint16_t *tile) {
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const f32x4 a = acc[f][u], v = z[l][f][u];
+                put(tile, f, u, a[0] * gelu_grad(v[0]), a[1] * gelu_grad(v[1]), a[2] * gelu_grad(v[2]), a[3] * gelu_grad(v[3]));
+            }
+    };
+    auto prefetch = [&](const uint16_t *W) {
+#pragma unroll
+        for (int ks = 0; ks < kMlpHid / 32; ks++)
+#pragma unroll
+            for (int f = 0; f < 2; f++) wn[ks][f] = load_w(W, kMlpHid, ks, f);
+    };
+    // a hidden layer's products (its weights in wn)
+    auto hidden = [&](const uint16_t *tile) {
+        clear();
+#pragma unroll
+        for (int ks = 0; ks < kMlpHid / 32; ks++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const bf16x8 h = ld8(&tile[(16 * u + fr) * kTrPA + ks * 32 + fk]);
+#pragma unroll
+                for (int f = 0; f < 2; f++) acc[f][u] = mfma16(wn[ks][f], h, acc[f][u]);
+            }
+    };
+
+    // layer 0
+    prefetch(w1);
+    clear();
+#pragma unroll
+    for (int ks = 0; ks < kMlpIn / 32; ks++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const bf16x8 x = ld8(&sx[(16 * u + fr) * kTrPX + ks * 32 + fk]);
+#pragma unroll
+            for (int f = 0; f < 2; f++) acc[f][u] = mfma16(wf[ks][f], x, acc[f][u]);
+        }
+    store_transposed<kMlpIn, kTrPX>(sx, O.X, O.Mp, m0, t);
+    forward_out(0, params + kOffB0, sa[0]);
+    __syncthreads();
+    // layers 1 and 2
+    hidden(sa[0]);
+    prefetch(w2);
+    store_transposed<kMlpHid, kTrPA>(sa[0], O.H[0], O.Mp, m0, t);
+    forward_out(1, params + kOffB1, sa[1]);
+    __syncthreads();
+    hidden(sa[1]);
+    prefetch(t2);
+    store_transposed<kMlpHid, kTrPA>(sa[1], O.H[1], O.Mp, m0, t);
+    forward_out(2, params + kOffB2, sa[0]);
+    __syncthreads();
+    // output layer: waves 0 and 1, one 16-row tile each (outputs 0 and 1 of
+    // row fr in the lanes with g = 0); L = 1/(2M) sum (Y - T)^2, dY = (Y - T)/M
+    store_transposed<kMlpHid, kTrPA>(sa[0], O.H[2], O.Mp, m0, t);
+    if (w < 2) {
+        f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < kMlpHid / 32; ks++)
+            o = mfma16(ld8(w3 + fr * kMlpHid + ks * 32 + fk), ld8(&sa[0][(16 * w + fr) * kTrPA + ks * 32 + fk]), o);
+        float s = 0.f;
+        if (g == 0) {
+            const int j = 16 * w + fr;
+            const bool ok = m0 + j < M;
+            const float inv = 1.0f / (float)M;
+#pragma unroll
+            for (int c = 0; c < kMlpOut; c++) {
+                const float d = ok ? o[c] + b3[c] - st[j][c] : 0.f;
+                s += d * d;
+                const uint16_t h = f2bf(d * inv);
+                sdy[j][c] = bf2f(h);
+                O.dY[(int64_t)c * O.Mp + m0 + j] = h;
+            }
+        }
+#pragma unroll
+        for (int d = 8; d > 0; d >>= 1) s += __shfl_xor(s, d, 16);
+        if (lane == 0) loss_part[2 * blockIdx.x + w] = s;
+    }
+    __syncthreads();
+    // dZ2 = (dY W3) * gelu'(Z2)
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+        const int n = 32 * w + 16 * f + 4 * g;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const float d0 = sdy[16 * u + fr][0], d1 = sdy[16 * u + fr][1];
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[f][u][i] = d0 * bf2f(w3[n + i]) + d1 * bf2f(w3[kMlpHid + n + i]);
+        }
+    }
+    backward_out(2, sa[1]);
+    __syncthreads();
+    // dZ1 = (dZ2 W2) * gelu'(Z1), dZ0 = (dZ1 W1) * gelu'(Z0)
+    hidden(sa[1]);
+    prefetch(t1);
+    store_transposed<kMlpHid, kTrPA>(sa[1], O.dZ[2], O.Mp, m0, t);
+    backward_out(1, sa[0]);
+    __syncthreads();
+    hidden(sa[0]);
+    store_transposed<kMlpHid, kTrPA>(sa[0], O.dZ[1], O.Mp, m0, t);
+    backward_out(0, sa[1]);
+    __syncthreads();
+    store_transposed<kMlpHid, kTrPA>(sa[1], O.dZ[0], O.Mp, m0, t);
+}
+
+// Weight gradients dW_l^T[n][k] = sum_m dZ_l[m][n] Hin_l[m][k] and bias
+// gradients sum_m dZ_l[m][n], over row chunk blockIdx.y (kSplitRows rows):
+// one wave per 32x32 block (56 blocks over the four layers), both operands
+// feature-major, so a lane's 8 consecutive rows are one 16-byte load and
+// there is no staging.  The chunks' partial sums go to ws[chunk][parameter].
+constexpr int kWgTiles = 4 * 5 + 4 * 4 + 4 * 4 + 4;
+__global__ __launch_bounds__(256) void k_train_wgrad(TrainT I, float *__restrict__ ws) {
+    const int lane = threadIdx.x & 63;
+    int tile = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    static_assert(kWgTiles % 4 == 0, "whole workgroups");
+    const int fr = lane & 15, g = lane >> 4;
+    const int64_t Mp = I.Mp;
+    float *out = ws + (int64_t)blockIdx.y * kMlpParams;
+    const uint16_t *A, *B;
+    int kin = kMlpHid, n0, k0, rows = 32;
+    int64_t woff, boff;
+    if (tile < 20) {
+        kin = kMlpIn;
+        n0 = tile / 5 * 32;
+        k0 = tile % 5 * 32;
+        A = I.dZ[0], B = I.X, woff = kOffW0, boff = kOffB0;
+    } else if (tile < 36) {
+        n0 = (tile - 20) / 4 * 32;
+        k0 = tile % 4 * 32;
+        A = I.dZ[1], B = I.H[0], woff = kOffW1, boff = kOffB1;
+    } else if (tile < 52) {
+        n0 = (tile - 36) / 4 * 32;
+        k0 = tile % 4 * 32;
+        A = I.dZ[2], B = I.H[1], woff = kOffW2, boff = kOffB2;
+    } else {
+        n0 = 0;
+        k0 = (tile - 52) * 32;
+        rows = kMlpOut;
+        A = I.dY, B = I.H[2], woff = kOffW3, boff = kOffB3;
+    }
+    const bf16x8 zero = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+    const bool a0 = fr < rows, a1 = fr + 16 < rows;
+    const int64_t m = (int64_t)blockIdx.y * kSplitRows + g * 8;
+    const uint16_t *pa0 = A + (n0 + (a0 ? fr : 0)) * Mp + m, *pa1 = A + (n0 + (a1 ? fr + 16 : 0)) * Mp + m;
+    const uint16_t *pb0 = B + (k0 + fr) * Mp + m, *pb1 = pb0 + 16 * Mp;
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bs0 = 0.f, bs1 = 0.f;
+#pragma unroll
+    for (int s = 0; s < kSplitRows / 32; s++) {
+        const bf16x8 x0 = a0 ? ld8(pa0 + s * 32) : zero, x1 = a1 ? ld8(pa1 + s * 32) : zero;
+        const bf16x8 y0 = ld8(pb0 + s * 32), y1 = ld8(pb1 + s * 32);
+        acc[0][0] = mfma16(x0, y0, acc[0][0]);
+        acc[0][1] = mfma16(x0, y1, acc[0][1]);
+        acc[1][0] = mfma16(x1, y0, acc[1][0]);
+        acc[1][1] = mfma16(x1, y1, acc[1][1]);
+        if (k0 == 0) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                bs0 += (float)x0[e];
+                bs1 += (float)x1[e];
+            }
+        }
+    }
+    // D layout: lane holds column fr of a 16x16 block, rows 4 g + r
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int n = 16 * i + 4 * g + r;
+            if (n >= rows) continue;
+#pragma unroll
+            for (int j = 0; j < 2; j++) out[woff + (int64_t)(n0 + n) * kin + k0 + 16 * j + fr] = acc[i][j][r];
+        }
+    if (k0 == 0) {
+        bs0 += __shfl_xor(bs0, 16, 64);
+        bs1 += __shfl_xor(bs1, 16, 64);
+        bs0 += __shfl_xor(bs0, 32, 64);
+        bs1 += __shfl_xor(bs1, 32, 64);
+        if (g == 0 && a0) out[boff + n0 + fr] = bs0;
+        if (g == 0 && a1) out[boff + n0 + fr + 16] = bs1;
+    }
+}
+
+// grad <- the sum of the row chunks (in order); with lr > 0 the Adam step on
+// the FP32 master parameters and the BF16 copies; loss[0] <- the sum of the
+// squared errors / (2M) (first workgroup, fixed order).
+__global__ __launch_bounds__(256) void k_train_update(const float *__restrict__ ws, int nsplit, float *__restrict__ p,
+                                                      float *__restrict__ grad, float *__restrict__ m1,
+                                                      float *__restrict__ m2, float lr, float b1, float b2, float eps,
+                                                      float c1, float c2, BfWeights W,
+                                                      const float *__restrict__ loss_part, int nloss, int M,
+                                                      float *__restrict__ loss) {
+    if (blockIdx.x == 0 && threadIdx.x < 64 && loss) {
+        float s = 0.f;
+        for (int i = threadIdx.x; i < nloss; i += 64) s += loss_part[i];
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+        if (threadIdx.x == 0) loss[0] = s / (2.0f * (float)M);
+    }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= kMlpParams) return;
+    float gi = 0.f;
+#pragma unroll 8
+    for (int z = 0; z < nsplit; z++) gi += ws[(int64_t)z * kMlpParams + i];
+    grad[i] = gi;
+    if (!(lr > 0.f)) return;
+    const float a = b1 * m1[i] + (1.0f - b1) * gi;
+    const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
+    m1[i] = a;
+    m2[i] = b;
+    const float v = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+    p[i] = v;
+    store_param(W, i, v);
 }
 
 }  // namespace
@@ -489,41 +740,56 @@ hipError_t mlp_forward_fused(mavi_mlp *p, const uint16_t *X, int M, float *Y, hi
     return hipGetLastError();
 }
 
+static BfWeights bf_weights(mavi_mlp *p) {
+    return BfWeights{p->w[0], p->w[1], p->w[2], p->w[3], p->wt[0], p->wt[1], p->b3};
+}
+
 hipError_t mlp_sync_weights(mavi_mlp *p, hipStream_t st) {
-    hipLaunchKernelGGL(k_sync_weights, dim3((kMlpHid * kMlpIn + 255) / 256), dim3(256), 0, st, p->params, p->w[0],
-                       p->w[1], p->w[2], p->w[3], p->b3);
+    hipLaunchKernelGGL(k_sync_weights, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, p->params, bf_weights(p));
     return hipGetLastError();
 }
 
+// Work arrays of the layer-by-layer forward.
 hipError_t ensure_work(mavi_mlp *p, int M) {
     if (M <= p->work_cap) return hipSuccess;
     hipStream_t st = p->ctx->stream;
     (void)hipStreamSynchronize(st);
-    for (int l = 0; l < 3; l++) {
-        dfree(p->Z[l]);
-        dfree(p->H[l]);
-    }
-    dfree(p->dZa); dfree(p->dZb); dfree(p->Yw); dfree(p->dY); dfree(p->loss_part); dfree(p->Xw); dfree(p->Tw);
+    for (auto &h : p->H) dfree(h);
+    dfree(p->Yw);
     p->work_cap = 0;
-    const int64_t m = M;
     hipError_t e = hipSuccess;
-    for (int l = 0; l < 3 && e == hipSuccess; l++) {
-        e = dalloc(&p->Z[l], m * kMlpHid, st);
-        if (e == hipSuccess) e = dalloc(&p->H[l], m * kMlpHid, st);
-    }
-    if (e == hipSuccess) e = dalloc(&p->dZa, m * kMlpHid, st);
-    if (e == hipSuccess) e = dalloc(&p->dZb, m * kMlpHid, st);
-    if (e == hipSuccess) e = dalloc(&p->Yw, m * kMlpOutPad, st);
-    if (e == hipSuccess) e = dalloc(&p->dY, m * kMlpOutPad, st);
-    if (e == hipSuccess) e = dalloc(&p->loss_part, (m + 255) / 256, st);
-    if (e == hipSuccess) e = dalloc(&p->Xw, m * kMlpIn, st);
-    if (e == hipSuccess) e = dalloc(&p->Tw, m * kMlpOut, st);
+    for (int l = 0; l < 3 && e == hipSuccess; l++) e = dalloc(&p->H[l], (int64_t)M * kMlpHid, st);
+    if (e == hipSuccess) e = dalloc(&p->Yw, (int64_t)M * kMlpOutPad, st);
     if (e == hipSuccess) p->work_cap = M;
     return e;
 }
 
-// Training forward over M rows of X (BF16 [M][160], device): keeps the
-// pre-activations Z_l and BF16 activations H_l, output in p->Yw [M][16].
+// Work arrays of a training pass (feature-major, M padded to whole chunks).
+hipError_t ensure_train(mavi_mlp *p, int M) {
+    const int64_t Mp = (int64_t)(M + kSplitRows - 1) / kSplitRows * kSplitRows;
+    if (Mp <= p->train_cap) return hipSuccess;
+    hipStream_t st = p->ctx->stream;
+    (void)hipStreamSynchronize(st);
+    dfree(p->XT); dfree(p->dYT); dfree(p->loss_part); dfree(p->ws);
+    for (int l = 0; l < 3; l++) {
+        dfree(p->HT[l]);
+        dfree(p->dZT[l]);
+    }
+    p->train_cap = 0;
+    hipError_t e = dalloc(&p->XT, Mp * kMlpIn, st);
+    if (e == hipSuccess) e = dalloc(&p->dYT, Mp * kMlpOut, st);
+    for (int l = 0; l < 3 && e == hipSuccess; l++) {
+        e = dalloc(&p->HT[l], Mp * kMlpHid, st);
+        if (e == hipSuccess) e = dalloc(&p->dZT[l], Mp * kMlpHid, st);
+    }
+    if (e == hipSuccess) e = dalloc(&p->loss_part, 2 * Mp / kTrRows, st);
+    if (e == hipSuccess) e = dalloc(&p->ws, Mp / kSplitRows * kMlpParams, st);
+    if (e == hipSuccess) p->train_cap = Mp;
+    return e;
+}
+
+// Layer-by-layer forward over M rows of X (BF16 [M][160], device): BF16
+// activations H_l, output in p->Yw [M][16].
 hipError_t mlp_forward_gemm(mavi_mlp *p, const uint16_t *X, int M, hipStream_t st) {
     hipError_t e = ensure_work(p, M);
     if (e != hipSuccess) return e;
@@ -532,93 +798,45 @@ hipError_t mlp_forward_gemm(mavi_mlp *p, const uint16_t *X, int M, hipStream_t s
     int kin = kMlpIn;
     const int64_t boff[3] = {kOffB0, kOffB1, kOffB2};
     for (int l = 0; l < 3; l++) {
-        Epi ep{prm + boff[l], p->Z[l], kMlpHid, p->H[l], kMlpHid};
+        Epi ep{prm + boff[l], p->H[l], kMlpHid};
         if ((e = gemm_t<false, true, EPI_BIAS_GELU>(st, M, kMlpHid, kin, in, kin, p->w[l], kin, nullptr, 0, 0, 0,
                                                     ep)) != hipSuccess)
             return e;
         in = p->H[l];
         kin = kMlpHid;
     }
-    Epi ep{p->b3, nullptr, 0, nullptr, 0};
+    Epi ep{p->b3, nullptr, 0};
     return gemm_t<false, true, EPI_BIAS>(st, M, kMlpOutPad, kMlpHid, p->H[2], kMlpHid, p->w[3], kMlpHid, p->Yw,
                                          kMlpOutPad, 0, 0, ep);
 }
 
-// One forward + backward pass over M rows (X BF16 [M][160], T [M][2], both
-// on the device): loss partials in p->loss_part, gradients in p->grad.
-hipError_t mlp_loss_grad_dev(mavi_mlp *p, const uint16_t *X, const float *T, int M, hipStream_t st) {
-    hipError_t e = mlp_forward_gemm(p, X, M, st);
+// One forward + backward pass over M rows of `in` (device): loss partials in
+// p->loss_part, gradients in p->grad, and with lr > 0 the Adam step.
+static hipError_t mlp_pass(mavi_mlp *p, const TrainIn &in, int M, float lr, float *loss, hipStream_t st) {
+    hipError_t e = ensure_train(p, M);
     if (e != hipSuccess) return e;
-    const int64_t boff[3] = {kOffB0, kOffB1, kOffB2};
-    Epi ep{};
-    hipLaunchKernelGGL(k_loss, dim3((M + 255) / 256), dim3(256), 0, st, p->Yw, T, M, p->dY, p->loss_part);
+    const int nsplit = (M + kSplitRows - 1) / kSplitRows, Mp = nsplit * kSplitRows;
+    TrainT O{p->XT, {p->HT[0], p->HT[1], p->HT[2]}, {p->dZT[0], p->dZT[1], p->dZT[2]}, p->dYT, Mp};
+    hipLaunchKernelGGL(k_train_pass, dim3(Mp / kTrRows), dim3(256), 0, st, in, M, p->w[0], p->w[1], p->w[2], p->w[3],
+                       p->wt[0], p->wt[1], p->params, p->b3, O, p->loss_part);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-
-    // backward.  Weight gradients: split-K over rows, chunks of kSplitRows.
-    const int kc = kSplitRows;
-    const int nsplit = (M + kc - 1) / kc;
-    auto wgrad = [&](const uint16_t *dZ, int ldz_, int nout, const uint16_t *Hin, int kin_, int64_t off,
-                     int64_t count) -> hipError_t {
-        if ((int64_t)nsplit * nout * kin_ > p->ws_cap) return hipErrorInvalidValue;
-        Epi none{};
-        hipError_t r = gemm_t<true, false, EPI_F32>(st, nout, kin_, M, dZ, ldz_, Hin, kin_, p->ws, kin_, kc,
-                                                    (int64_t)nout * kin_, none);
-        if (r != hipSuccess) return r;
-        hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, p->ws, nsplit,
-                           (int64_t)nout * kin_, count, p->grad + off);
-        return hipGetLastError();
-    };
-    auto bgrad = [&](const uint16_t *dZ, int ld, int n, int64_t off) -> hipError_t {
-        const int nchunk = (M + kColRows - 1) / kColRows;
-        if ((int64_t)nchunk * n > p->ws_cap) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_colsum_part, dim3((n + 63) / 64, nchunk), dim3(256), 0, st, dZ, M, n, ld, p->ws);
-        hipLaunchKernelGGL(k_split_reduce, dim3((n + 255) / 256), dim3(256), 0, st, p->ws, nchunk, (int64_t)n,
-                           (int64_t)n, p->grad + off);
-        return hipGetLastError();
-    };
-    // output layer: dW3t = dY^T H2 (rows 0..1 of the 16-row padded product), db3 = colsum dY
-    if ((e = wgrad(p->dY, kMlpOutPad, kMlpOutPad, p->H[2], kMlpHid, kOffW3, (int64_t)kMlpOut * kMlpHid)) !=
-        hipSuccess)
-        return e;
-    if ((e = bgrad(p->dY, kMlpOutPad, kMlpOut, kOffB3)) != hipSuccess) return e;
-    // dZ2 = (dY W3) * gelu'(Z2)
-    ep = Epi{nullptr, p->Z[2], kMlpHid, p->dZa, kMlpHid};
-    if ((e = gemm_t<false, false, EPI_GELU_BWD>(st, M, kMlpHid, kMlpOutPad, p->dY, kMlpOutPad, p->w[3], kMlpHid,
-                                                nullptr, 0, 0, 0, ep)) != hipSuccess)
-        return e;
-    uint16_t *dZ = p->dZa, *dZn = p->dZb;
-    const int64_t woff[3] = {kOffW0, kOffW1, kOffW2};
-    for (int l = 2; l >= 0; l--) {
-        const uint16_t *Hin = l > 0 ? p->H[l - 1] : X;
-        const int kin_ = l > 0 ? kMlpHid : kMlpIn;
-        if ((e = wgrad(dZ, kMlpHid, kMlpHid, Hin, kin_, woff[l], (int64_t)kMlpHid * kin_)) != hipSuccess) return e;
-        if ((e = bgrad(dZ, kMlpHid, kMlpHid, boff[l])) != hipSuccess) return e;
-        if (l == 0) break;
-        // dZ_{l-1} = (dZ_l W_l) * gelu'(Z_{l-1})
-        ep = Epi{nullptr, p->Z[l - 1], kMlpHid, dZn, kMlpHid};
-        if ((e = gemm_t<false, false, EPI_GELU_BWD>(st, M, kMlpHid, kMlpHid, dZ, kMlpHid, p->w[l], kMlpHid, nullptr, 0,
-                                                    0, 0, ep)) != hipSuccess)
-            return e;
-        uint16_t *tmp = dZ;
-        dZ = dZn;
-        dZn = tmp;
-    }
-    return hipSuccess;
-}
-
-hipError_t mlp_adam_step(mavi_mlp *p, float lr, hipStream_t st) {
-    p->adam_t += 1;
+    hipLaunchKernelGGL(k_train_wgrad, dim3(kWgTiles / 4, nsplit), dim3(256), 0, st, O, p->ws);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.0f - powf(b1, (float)p->adam_t), c2 = 1.0f - powf(b2, (float)p->adam_t);
-    hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, p->params, p->grad, p->m1, p->m2,
-                       (int64_t)kMlpParams, lr, b1, b2, eps, c1, c2);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return mlp_sync_weights(p, st);
+    float c1 = 1.f, c2 = 1.f;
+    if (lr > 0.f) {
+        p->adam_t += 1;
+        c1 = 1.0f - powf(b1, (float)p->adam_t);
+        c2 = 1.0f - powf(b2, (float)p->adam_t);
+    }
+    hipLaunchKernelGGL(k_train_update, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, p->ws, nsplit, p->params,
+                       p->grad, p->m1, p->m2, lr, b1, b2, eps, c1, c2, bf_weights(p), p->loss_part, 2 * Mp / kTrRows, M,
+                       loss);
+    return hipGetLastError();
 }
 
 double mlp_loss_value(mavi_mlp *p, int M, hipStream_t st, hipError_t *err) {
-    const int nb = (M + 255) / 256;
+    const int nb = 2 * ((M + kSplitRows - 1) / kSplitRows * kSplitRows / kTrRows);
     std::vector<float> h(nb);
     *err = hipMemcpyAsync(h.data(), p->loss_part, sizeof(float) * nb, hipMemcpyDeviceToHost, st);
     if (*err == hipSuccess) *err = hipStreamSynchronize(st);
@@ -734,9 +952,8 @@ int mavi_mlp_create(mavi_ctx *ctx, uint64_t seed, mavi_mlp **out) {
     if (e == hipSuccess) e = dalloc(&p->w[1], (int64_t)kMlpHid * kMlpHid, st);
     if (e == hipSuccess) e = dalloc(&p->w[2], (int64_t)kMlpHid * kMlpHid, st);
     if (e == hipSuccess) e = dalloc(&p->w[3], (int64_t)kMlpOutPad * kMlpHid, st);
+    for (int l = 0; l < 2 && e == hipSuccess; l++) e = dalloc(&p->wt[l], (int64_t)kMlpHid * kMlpHid, st);
     if (e == hipSuccess) e = dalloc(&p->b3, kMlpOutPad, st);
-    p->ws_cap = (int64_t)64 * kMlpHid * kMlpIn;
-    if (e == hipSuccess) e = dalloc(&p->ws, p->ws_cap, st);
     int dev = 0, ncu = 256;
     if (e == hipSuccess) e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -782,13 +999,15 @@ static void mlp_free(mavi_mlp *p) {
     (void)hipStreamSynchronize(p->ctx->stream);
     dfree(p->params); dfree(p->grad); dfree(p->m1); dfree(p->m2);
     for (int l = 0; l < 4; l++) dfree(p->w[l]);
+    for (auto &q : p->wt) dfree(q);
     dfree(p->b3); dfree(p->ws);
     for (int l = 0; l < 3; l++) {
-        dfree(p->Z[l]);
         dfree(p->H[l]);
+        dfree(p->HT[l]);
+        dfree(p->dZT[l]);
     }
-    dfree(p->dZa); dfree(p->dZb); dfree(p->Yw); dfree(p->dY); dfree(p->loss_part); dfree(p->Xw); dfree(p->Tw);
-    dfree(p->dsX); dfree(p->dsT); dfree(p->bX); dfree(p->bT);
+    dfree(p->Yw); dfree(p->XT); dfree(p->dYT); dfree(p->loss_part); dfree(p->Xw); dfree(p->Tw); dfree(p->loss_hist);
+    dfree(p->dsX); dfree(p->dsT);
     mavi_ctx *ctx = p->ctx;
     const bool held = p->ctx_held;
     delete p;
@@ -873,12 +1092,20 @@ int mavi_mlp_loss_grad(mavi_mlp *p, int64_t m, const uint16_t *x, const float *t
     mavi_ctx *ctx = p->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    if ((int64_t)((m + kSplitRows - 1) / kSplitRows) * kMlpHid * kMlpIn > p->ws_cap)
+    if ((m + kSplitRows - 1) / kSplitRows > kMaxSplits)
         return set_err(ctx, MAVI_E_BADARG, "batch too large for the split-K work space");
-    HIPCHK(ctx, mavi::ensure_work(p, (int)m));
+    if (m > p->rows_cap) {
+        (void)hipStreamSynchronize(st);
+        dfree(p->Xw);
+        dfree(p->Tw);
+        p->rows_cap = 0;
+        HIPCHK(ctx, dalloc(&p->Xw, m * kMlpIn, st));
+        HIPCHK(ctx, dalloc(&p->Tw, m * kMlpOut, st));
+        p->rows_cap = (int)m;
+    }
     HIPCHK(ctx, hipMemcpyAsync(p->Xw, x, sizeof(uint16_t) * m * kMlpIn, hipMemcpyHostToDevice, st));
     HIPCHK(ctx, hipMemcpyAsync(p->Tw, t, sizeof(float) * m * kMlpOut, hipMemcpyHostToDevice, st));
-    HIPCHK(ctx, mavi::mlp_loss_grad_dev(p, p->Xw, p->Tw, (int)m, st));
+    HIPCHK(ctx, mavi::mlp_pass(p, TrainIn{p->Xw, p->Tw, 0, 0, 0}, (int)m, 0.f, nullptr, st));
     hipError_t e = hipSuccess;
     const double l = mavi::mlp_loss_value(p, (int)m, st, &e);
     HIPCHK(ctx, e);
@@ -940,36 +1167,18 @@ int mavi_mlp_train(mavi_mlp *p, int64_t steps, int32_t batch, float lr, uint64_t
     if (!p || steps < 0 || batch <= 0 || batch > (1 << 20) || !(lr > 0.f)) return MAVI_E_BADARG;
     mavi_ctx *ctx = p->ctx;
     if (p->ds_count <= 0) return set_err(ctx, MAVI_E_BADARG, "empty data set");
-    if ((int64_t)((batch + kSplitRows - 1) / kSplitRows) * kMlpHid * kMlpIn > p->ws_cap)
+    if ((batch + kSplitRows - 1) / kSplitRows > kMaxSplits)
         return set_err(ctx, MAVI_E_BADARG, "batch too large for the split-K work space");
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    if (batch > p->b_cap) {
-        dfree(p->bX);
-        dfree(p->bT);
-        p->b_cap = 0;
-        HIPCHK(ctx, dalloc(&p->bX, (int64_t)batch * kMlpIn, st));
-        HIPCHK(ctx, dalloc(&p->bT, (int64_t)batch * kMlpOut, st));
-        p->b_cap = batch;
-    }
     if (steps > p->loss_hist_cap) {
         dfree(p->loss_hist);
         p->loss_hist_cap = 0;
         HIPCHK(ctx, dalloc(&p->loss_hist, steps, st));
         p->loss_hist_cap = steps;
     }
-    HIPCHK(ctx, mavi::ensure_work(p, batch));
-    const int nchunk = batch * (kMlpIn / 8);
-    for (int64_t s = 0; s < steps; s++) {
-        hipLaunchKernelGGL(k_gather_batch, dim3((nchunk + 255) / 256), dim3(256), 0, st, p->dsX, p->dsT, p->ds_count,
-                           seed, s, batch, p->bX, p->bT);
-        HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, mavi::mlp_loss_grad_dev(p, p->bX, p->bT, batch, st));
-        hipLaunchKernelGGL(k_loss_finish, dim3(1), dim3(64), 0, st, p->loss_part, (batch + 255) / 256, batch,
-                           p->loss_hist + s);
-        HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, mavi::mlp_adam_step(p, lr, st));
-    }
+    for (int64_t k = 0; k < steps; k++)
+        HIPCHK(ctx, mavi::mlp_pass(p, TrainIn{p->dsX, p->dsT, p->ds_count, seed, k}, batch, lr, p->loss_hist + k, st));
     if (losses && steps > 0)
         HIPCHK(ctx, hipMemcpyAsync(losses, p->loss_hist, sizeof(float) * steps, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));

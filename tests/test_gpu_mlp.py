@@ -125,3 +125,35 @@ def test_training_reduces_loss_and_is_deterministic(gpu_ctx):
     mse = float(np.mean((yv - tv) ** 2))
     base = float(np.mean((tv - tv.mean(axis=0)) ** 2))
     assert mse < 0.2 * base, (mse, base)
+
+
+@pytest.mark.parametrize("m", [1, 31, 33, 256, 257, 16384])
+def test_gradients_at_the_edges_of_the_tiles(gpu_ctx, m):
+    """One row, around a workgroup's 32 rows, around a 256-row chunk and the
+    largest batch: every weight and bias block against the oracle, and the
+    minibatch drawn from a data set trains as the same rows handed over do."""
+    from mavi_hip import learned
+
+    say(f"[mlp grad edges] m={m}")
+    p, x, t = problem(40 + m % 97, m)
+    net = learned.MLP(ctx=gpu_ctx)
+    net.params = p
+    loss, g = net.loss_grad(x, t)
+    loss_ref, g_ref = mo.loss_grad(p.astype(np.float64), mo.bf16_bits_to_f64(x), t.astype(np.float64), bf16=True)
+    assert abs(loss - loss_ref) <= 1e-4 * abs(loss_ref)
+    for (ow, ob), (nout, nin) in zip(mo.OFFS, mo.SHAPES):
+        for lo, hi in ((ow, ow + nout * nin), (ob, ob + nout)):
+            d = np.linalg.norm(g[lo:hi] - g_ref[lo:hi])
+            assert d <= 5e-3 * np.linalg.norm(g_ref[lo:hi]) + 1e-12, (lo, hi, d, np.linalg.norm(g_ref[lo:hi]))
+    # one Adam step from zero moments moves every parameter by
+    # lr * g / (|g| + eps / sqrt-correction): its sign and size follow g
+    if m == 1:
+        net.dataset_append(x, t)
+        losses = net.train(steps=1, batch=1, lr=1e-3, seed=4)
+        assert abs(losses[0] - loss) <= 1e-6 * abs(loss)
+        # (1 - b2) g^2 / (1 - b2) = g^2 up to FP32 rounding of the corrections
+        want = p - 1e-3 * g / (np.abs(g) + 1e-8)
+        big = np.abs(g) > 1e-4
+        assert np.abs(net.params - want)[big].max() <= 1e-6
+    with pytest.raises(Exception):
+        net.loss_grad(np.zeros((16385, mo.N_IN), np.uint16), np.zeros((16385, 2), np.float32))
