@@ -392,6 +392,79 @@ __device__ __forceinline__ void scan_range(const SysParams &P, const RingCtx &R,
 }
 
 
+// The candidates of one particle as up to six slot ranges (two per chunk row
+// where a periodic grid's columns wrap), walked in order as one sequence, N at a
+// time: the N loads are in flight together.  For systems of few waves per SIMD,
+// where the two-candidate loops wait on memory ~20 times in a row and the waves
+// at the column edges, one candidate at a time, 40 times.
+template <int POT, int N>
+__device__ __forceinline__ void scan_deep(const SysParams &P, const RingCtx &R, PairAcc<POT> &acc,
+                                          const double2 *__restrict__ pin, int s, double xi, double yi, bool wrap,
+                                          const int (&a)[6], const int (&l)[6]) {
+    const int c1 = l[0], c2 = c1 + l[1], c3 = c2 + l[2], c4 = c3 + l[3], c5 = c4 + l[4], tot = c5 + l[5];
+    const int o0 = a[0], o1 = a[1] - c1, o2 = a[2] - c2, o3 = a[3] - c3, o4 = a[4] - c4, o5 = a[5] - c5;
+    for (int k = 0; k < tot; k += N) {
+        double2 p[N];
+        int j[N], idj[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int q = min(k + u, tot - 1);
+            j[u] = q + (q < c3 ? (q < c1 ? o0 : (q < c2 ? o1 : o2)) : (q < c4 ? o3 : (q < c5 ? o4 : o5)));
+            p[u] = load_slot(pin, j[u]);
+            idj[u] = POT == POT_RINGS ? R.ids[j[u]] - R.id_base : 0;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all N loads issued before the first is used
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const bool take = k + u < tot && j[u] != s;
+            double dx = xi - p[u].x, dy = yi - p[u].y;
+            if (wrap) {
+                dx = min_image(dx, P.L, P.halfL);
+                dy = min_image(dy, P.H, P.halfH);
+            }
+            if constexpr (POT == POT_LJ) {
+                const double f = lj_scale_masked(P, dx * dx + dy * dy, take);
+                acc.fx = __builtin_fma(f, dx, acc.fx);
+                acc.fy = __builtin_fma(f, dy, acc.fy);
+            } else {
+                acc.add(P, R, dx, dy, take, idj[u]);
+            }
+        }
+    }
+}
+
+// pair_gather_chunks with scan_deep: the same candidates in the same order.
+template <int POT>
+__device__ __forceinline__ void pair_gather_deep(const SysParams &P, const RingCtx &R, PairAcc<POT> &acc,
+                                                 const double2 *__restrict__ pin, const int c,
+                                                 const int32_t *__restrict__ start, const int s, const bool valid,
+                                                 const double2 pi) {
+    const int row = c / P.cols, col = c - row * P.cols;
+    const bool left = col == 0, right = col == P.cols - 1;
+    const bool wrap = valid && P.periodic && (row == 0 || row == P.rows - 1 || left || right);
+    int a[6], l[6];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        int r = row + d - 1;
+        bool ok = valid;
+        if (P.periodic) r = (r < 0) ? r + P.rows : (r >= P.rows ? r - P.rows : r);
+        else ok = ok && r >= 0 && r < P.rows;
+        const int32_t *sr = start + (ok ? r : 0) * P.cols;
+        // columns in slot order; the wrapped column of a periodic edge last
+        const int c0 = left ? 0 : col - 1, c1 = right ? P.cols : col + 2;
+        a[2 * d] = ok ? sr[c0] : 0;
+        l[2 * d] = ok ? sr[c1] - a[2 * d] : 0;
+        const bool two = ok && P.periodic && (left || right);
+        const int cw = left ? P.cols - 1 : 0;
+        a[2 * d + 1] = two ? sr[cw] : 0;
+        l[2 * d + 1] = two ? sr[cw + 1] - a[2 * d + 1] : 0;
+    }
+    // minimum images as pair_gather_chunks takes them: per wave, per lane in
+    // the waves that touch a wrapped column
+    const bool lanes = __any(valid && P.periodic && (left || right));
+    scan_deep<POT, POT == POT_RINGS ? 4 : 8>(P, R, acc, pin, s, pi.x, pi.y, lanes ? wrap : __any(wrap), a, l);
+}
+
 // Pair forces of sorted slot s over the 3x3 chunk block of chunk c (local
 // chunk index; `start` is the scan of this system's chunks, holding global
 // sorted slots).  Shared by the single-system and batch kernels.

@@ -35,6 +35,15 @@ void dfree(T *&p) {
     p = nullptr;
 }
 
+// Up to this many particles the chunk gather keeps eight candidates a lane in
+// flight (pair_gather_deep): there are few waves a SIMD, and a candidate's trip
+// to memory is what a step waits for.  Above, other waves hide it and the extra
+// registers (fewer waves) cost more.  us a step, two candidates in flight ->
+// eight: LJ 4k 39.5 -> 37.0, 66k 45.5 -> 40.0, 202k 59.0 -> 54.7, 393k 72.9 ->
+// 68.0, 787k 99.4 -> 99.9, 1M 115.9 -> 119.7; self-propelled 32k 23.2 -> 21.2,
+// 490k 49.0 -> 47.0; run-and-tumble 32k 20.3 -> 19.7, 490k 38.7 -> 40.3.
+constexpr int64_t kDeepGather = 300000;
+
 inline int nblk(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
 inline bool is_pow2_wg(int32_t w) { return w == 64 || w == 128 || w == 256 || w == 512 || w == 1024; }

@@ -128,8 +128,8 @@ struct NextBin {
     int32_t *stamp;
 };
 
-template <int MODE, int POT, bool ALLPAIRS, bool WALLS = false>
-__global__ __attribute__((amdgpu_waves_per_eu(WALLS ? 1 : 8))) void k_pair(SysParams P, RingCtx R, const double2 *__restrict__ pin, const int32_t *__restrict__ scell,
+template <int MODE, int POT, bool ALLPAIRS, bool WALLS = false, bool DEEP = false>
+__global__ __attribute__((amdgpu_waves_per_eu(WALLS || DEEP ? 1 : 8))) void k_pair(SysParams P, RingCtx R, const double2 *__restrict__ pin, const int32_t *__restrict__ scell,
                        const int32_t *__restrict__ start, double2 *__restrict__ Pst, double2 *__restrict__ Vst,
                        double2 *__restrict__ Fout, double2 *__restrict__ P2, double2 *__restrict__ F1,
                        double list2, const int32_t *__restrict__ needc, const uint32_t *__restrict__ epoch,
@@ -182,6 +182,8 @@ __global__ __attribute__((amdgpu_waves_per_eu(WALLS ? 1 : 8))) void k_pair(SysPa
     }
     if constexpr (ALLPAIRS) {
         if (valid) scan_range<POT>(P, R, acc, pin, s, pi.x, pi.y, P.periodic != 0, 0, P.na);
+    } else if constexpr (DEEP) {
+        pair_gather_deep<POT>(P, R, acc, pin, scell[sv], start, s, valid, pi);
     } else {
         pair_gather_chunks<POT>(P, R, acc, pin, scell[sv], start, s, valid, pi, list2, s_list);
     }
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(64 * kInvWaves) void k_invasions(
 // ---------------------------------------------------------------------------
 constexpr double kTwoPi = 2.0 * 3.141592653589793;  // 2*pi in Julia
 
-template <int MODE, int POT, bool ALLPAIRS, bool WALLS>
+template <int MODE, int POT, bool ALLPAIRS, bool WALLS, bool DEEP>
 __global__ void k_active(SysParams P, const double2 *__restrict__ pin, const double2 *__restrict__ ain,
                          const int32_t *__restrict__ idin, const int32_t *__restrict__ scell,
                          const int32_t *__restrict__ start, double2 *__restrict__ pout, double2 *__restrict__ aout,
@@ -514,6 +516,8 @@ __global__ void k_active(SysParams P, const double2 *__restrict__ pin, const dou
     PairAcc<POT> acc;
     if constexpr (ALLPAIRS) {
         if (valid) scan_range<POT>(P, R, acc, pin, s, pi.x, pi.y, P.periodic != 0, 0, P.na);
+    } else if constexpr (DEEP) {
+        pair_gather_deep<POT>(P, R, acc, pin, scell[sv], start, s, valid, pi);
     } else {
         pair_gather_chunks<POT>(P, R, acc, pin, scell[sv], start, s, valid, pi, INFINITY, nullptr);
     }
@@ -1031,16 +1035,25 @@ hipError_t launch_pair_t(mavi_sys *s, const double2 *pin, hipStream_t st, bool r
         nb = NextBin{s->key, s->rank, s->cnt, s->flags, fuse_stamp ? s->stamp : nullptr};
         s->keys_ready = true;
     }
+    const bool deep = !ALL && s->P.na <= kDeepGather && !(l2 < INFINITY);
     if constexpr (MODE == MODE_VERLET1 || MODE == MODE_VERLET2) {
         if (walls) {  // the walls list's forces and walls! in the epilogue
-            hipLaunchKernelGGL((k_pair<MODE, POT, ALL, true>), dim3(nblk(s->P.na, wgk)), dim3(wgk), lds, st, s->P,
+            auto k = &k_pair<MODE, POT, ALL, true, false>;
+            if constexpr (!ALL) {
+                if (deep) k = &k_pair<MODE, POT, ALL, true, true>;
+            }
+            hipLaunchKernelGGL(k, dim3(nblk(s->P.na, wgk)), dim3(wgk), lds, st, s->P,
                                ring_ctx(s), pin, s->scell, s->start, s->P_[c], s->V_[c], s->F, s->P2, s->F1, l2,
                                needc, s->epoch, perm, s->V_[1 - c], s->F,
                                (MODE == MODE_VERLET2 && !ALL) ? s->stamp : nullptr, nb);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((k_pair<MODE, POT, ALL>), dim3(nblk(s->P.na, wgk)), dim3(wgk), lds, st, s->P, ring_ctx(s), pin,
+    auto k = &k_pair<MODE, POT, ALL>;
+    if constexpr (!ALL) {
+        if (deep) k = &k_pair<MODE, POT, ALL, false, true>;
+    }
+    hipLaunchKernelGGL(k, dim3(nblk(s->P.na, wgk)), dim3(wgk), lds, st, s->P, ring_ctx(s), pin,
                        s->scell, s->start, s->P_[c], s->V_[c], s->F, s->P2, s->F1, l2, needc, s->epoch, perm,
                        s->V_[1 - c], s->F, nullptr, nb);
     return hipGetLastError();
@@ -1081,7 +1094,11 @@ void launch_active_k(mavi_sys *s, const double *noise_dev, hipStream_t st) {
         nb = NextBin{s->key, s->rank, s->cnt, s->flags, nullptr};
         s->keys_ready = true;
     }
-    hipLaunchKernelGGL((k_active<MODE, POT, ALL, WALLS>), dim3(nblk(s->P.na, wg)), dim3(wg), 0, st, s->P, s->P_[c],
+    auto k = &k_active<MODE, POT, ALL, WALLS, false>;
+    if constexpr (!ALL) {
+        if (s->P.na <= kDeepGather) k = &k_active<MODE, POT, ALL, WALLS, true>;
+    }
+    hipLaunchKernelGGL(k, dim3(nblk(s->P.na, wg)), dim3(wg), 0, st, s->P, s->P_[c],
                        s->V_[c], s->ID_[c], s->scell, s->start, s->P_[o], s->V_[o], s->ID_[o], s->F, noise_dev,
                        s->seed, s->counter, nb);
 }
