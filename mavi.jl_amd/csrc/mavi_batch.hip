@@ -13,11 +13,19 @@
 // concatenated too (nbase + local id), and ring arrays (rbase, even); a
 // wavefront of the ring kernel holds floor(64 / nmax) rings of one replica.
 //
-// A step is: binning of all replicas, one pair launch per kind and
-// evaluation (VERLET1 / VERLET2 for LJ and HarmTrunc replicas, FORCES for
-// rings), and the per-ring kernel for rings replicas.  Each replica runs the
-// same device functions as a single system (mavi_device.h), so its results
-// are bit-identical to mavi_step on the same descriptor.
+// The plain (LJ, HarmTrunc) and the rings replicas are two families with arrays
+// of their own, so that each steps by the kernels that suit it and, where both
+// are there, on a stream of its own beside the other.  A step of a family is:
+// binning of its replicas, one pair launch per kind and evaluation (VERLET1 /
+// VERLET2 for LJ and HarmTrunc, FORCES for rings), and the per-ring kernel for
+// rings.  Calls of 8 steps and more step the rings replicas on Verlet lists
+// instead (mavi_rlist.hip: one kernel a step, the same bits), if every one of
+// them may use lists.  Each replica runs the same device functions as a single
+// system (mavi_device.h), so its results are bit-identical to mavi_step on the
+// same descriptor.  48 replicas (1000 to 40000 particles, 200 steps with all
+// transfers): 25.0 ms with both families in one set of launches, 17.8 ms
+// now; the plain replicas' launches (60 us a step) are what it waits for, the
+// rings replicas' one kernel (16.6 us) runs beside them.
 //
 // Force reuse, as for a single system: the second evaluation of an LJ or
 // HarmTrunc replica does the next binning's first pass on the positions it
@@ -37,30 +45,11 @@
 #include <string>
 #include <vector>
 
+#include "mavi_batch.h"
 #include "mavi_device.h"
 #include "mavi_host.h"
 
 namespace {
-
-struct Replica {
-    SysParams P;
-    int32_t pbase, npad;  // first sorted slot (multiple of 64), padded slot count
-    int32_t nbase;        // first particle id
-    int32_t cbase;        // first chunk; cbase + P.ncell is the pad chunk
-    int32_t rbase;        // first ring (even; rings only)
-    int32_t tbase, ibase; // first ring type / interaction entry
-    int32_t abase;        // first entry of the active id list (rings only)
-    int64_t cpbase;       // first continuous position (rings only)
-    double list2;         // squared candidate-list range
-    uint64_t seed;
-    float inv_nmax;
-    int32_t kind;         // 0 LJ, 1 HarmTrunc, 2 rings
-    int32_t rwbase;       // first wave of the ring kernel (rings only)
-};
-
-enum { KIND_LJ = 0, KIND_HT = 1, KIND_RINGS = 2, NKIND = 3 };
-
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Chunk and arrival rank of every padded slot.  Padding slots go to their
 // replica's pad chunk.  nslots is a multiple of 64: whole waves leave.
@@ -164,7 +153,7 @@ __device__ __forceinline__ void mark_block(const SysParams &P, int32_t *needc, i
 // (global wave, replica).  The per-particle work is pair_gather_chunks /
 // pair_epilogue with the replica's parameters, as in k_pair; with U (Verlet
 // kinds), the force reuse and fused binning pass described at the top.
-template <int MODE, int POT>
+template <int MODE, int POT, bool DEEP>
 __global__ void kb_pair(const Replica *__restrict__ reps, const int2 *__restrict__ items, int32_t nitems,
                         const int32_t *__restrict__ ids, const int32_t *__restrict__ rtype,
                         const RingType *__restrict__ types, const RingInter *__restrict__ inter,
@@ -213,8 +202,11 @@ __global__ void kb_pair(const Replica *__restrict__ reps, const int2 *__restrict
         acc.ring_i = ring_of((uint32_t)acc.id_i, R);
         acc.type_i = P.typed ? R.rtype[acc.ring_i] : 0;
     }
-    pair_gather_chunks<POT>(P, R, acc, pin, scell[sv] - Q.cbase, start + Q.cbase, s, valid, pi,
-                            listed ? Q.list2 : INFINITY, s_list);
+    if constexpr (DEEP)
+        pair_gather_deep<POT>(P, R, acc, pin, scell[sv] - Q.cbase, start + Q.cbase, s, valid, pi);
+    else
+        pair_gather_chunks<POT>(P, R, acc, pin, scell[sv] - Q.cbase, start + Q.cbase, s, valid, pi,
+                                listed ? Q.list2 : INFINITY, s_list);
     if constexpr (MODE == MODE_VERLET2) {
         double2 xf = make_double2(0.0, 0.0);
         if (valid) pair_epilogue<MODE>(P, s, pi, acc.fx, acc.fy, Pst, Vst, Fout, P2, F1, &xf);
@@ -295,75 +287,29 @@ __global__ __launch_bounds__(256) void kb_rings(const Replica *__restrict__ reps
 struct mavi_batch {
     mavi_ctx *ctx = nullptr;
     std::vector<HostSys> hs;
-    std::vector<Replica> reps;
     bool finalized = false;
-    int64_t nids = 0, nactive = 0, nslots = 0, ncells = 0, nrings = 0;
-    SysParams G{};  // na = nslots, ncell = ncells: the sort over all replicas
-    // per-kind wave lists
-    int2 *items[NKIND] = {nullptr, nullptr, nullptr};
-    int32_t nitems[NKIND] = {0, 0, 0};
-    int32_t *ring_wave_rep = nullptr;
-    int32_t nring_waves = 0;
-    Replica *d_reps = nullptr;
-    int32_t *wave_rep = nullptr;
-    // state (same roles as in mavi_sys)
-    double2 *P_[2] = {nullptr, nullptr}, *V_[2] = {nullptr, nullptr};
-    int32_t *ID_[2] = {nullptr, nullptr};
-    double2 *F = nullptr, *P2 = nullptr, *F1 = nullptr;
-    int32_t *key = nullptr, *rank = nullptr, *src = nullptr, *scell = nullptr, *sid = nullptr, *slot_of = nullptr;
-    int32_t *cnt = nullptr, *start = nullptr;
-    unsigned long long *scan_state = nullptr, *scan_ticket = nullptr;
-    uint32_t *flags = nullptr;
-    // force reuse
-    int32_t *perm = nullptr, *needc = nullptr;
-    uint32_t *epoch = nullptr, *rvalid = nullptr;
-    bool keys_ready = false;  // the last second evaluation did the next binning's first pass
-    unsigned long long *counter = nullptr;
-    int32_t *active_ids = nullptr;
-    double2 *pos_id = nullptr, *vel_id = nullptr, *force_id = nullptr;
-    double *pol = nullptr, *areas = nullptr;
-    double2 *cms = nullptr, *cms_next = nullptr, *cpos = nullptr;
-    int32_t *rtype = nullptr;
-    RingType *types = nullptr;
-    RingInter *inter = nullptr;
-    int cur = 0;
+    // plain (LJ, HarmTrunc) and rings replicas; null if there are none
+    BatchSub *sub[2] = {nullptr, nullptr};
+    struct Where {
+        int32_t sub, local;
+    };
+    std::vector<Where> where;  // of each replica
     std::vector<char> uploaded;
-    // execution shape
-    int32_t wg[2] = {256, 256};      // plain, rings
+    hipStream_t side = nullptr;  // the plain replicas' steps where both families are there
+    hipEvent_t fork = nullptr, join = nullptr;
+    // execution shape: plain, rings
+    int32_t wg[2] = {256, 256};
     int32_t listed[2] = {0, 0};
     int32_t graph_steps = 100;
     bool use_graphs = true;
-    hipGraphExec_t graph = nullptr;
-    // profiling
     bool prof = false;
-    ProfSlot profs[MAVI_PROF_NCLASS];
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
 namespace {
 
-struct BatchProf {
-    mavi_batch *b;
-    int which;
-    hipStream_t st;
-    BatchProf(mavi_batch *b_, int w, hipStream_t st_) : b(b_), which(w), st(st_) {
-        if (b->prof) (void)hipEventRecord(b->ev0, st);
-    }
-    ~BatchProf() {
-        if (!b->prof) return;
-        (void)hipEventRecord(b->ev1, st);
-        if (hipEventSynchronize(b->ev1) == hipSuccess) {
-            float ms = 0.f;
-            if (hipEventElapsedTime(&ms, b->ev0, b->ev1) == hipSuccess) {
-                b->profs[which].ms += ms;
-                b->profs[which].launches += 1;
-            }
-        }
-    }
-};
-
-hipError_t batch_bin(mavi_batch *b, hipStream_t st) {
+hipError_t batch_bin(BatchSub *b, hipStream_t st) {
     BatchProf ps(b, MAVI_PROF_BIN, st);
+    if (b->rl) b->rl->valid = b->rl->ordered = false;  // the slots move
     const int c = b->cur, nc = 1 - c;
     const int ns = (int)b->nslots;
     const int n = (int)b->ncells + 1;
@@ -388,12 +334,10 @@ hipError_t batch_bin(mavi_batch *b, hipStream_t st) {
 }
 
 template <int MODE, int POT>
-void batch_pair_kind(mavi_batch *b, int kind, const double2 *pin, hipStream_t st) {
+void batch_pair_kind(BatchSub *b, int kind, const double2 *pin, hipStream_t st) {
     const int ni = b->nitems[kind];
     if (ni == 0) return;
-    const int slot = kind == KIND_RINGS ? 1 : 0;
-    const int wg = b->wg[slot];
-    const int listed = b->listed[slot];
+    const int wg = b->wg, listed = b->listed;
     const size_t lds = listed ? sizeof(uint16_t) * kListCap * (size_t)wg : 0;
     const int c = b->cur;
     BatchReuse U{};
@@ -413,12 +357,13 @@ void batch_pair_kind(mavi_batch *b, int kind, const double2 *pin, hipStream_t st
         U.cnt = b->cnt;
         U.flags = b->flags;
     }
-    hipLaunchKernelGGL((kb_pair<MODE, POT>), dim3(nblk(ni, wg / 64)), dim3(wg), lds, st, b->d_reps, b->items[kind],
+    auto k = !listed && b->nslots <= kDeepGather ? &kb_pair<MODE, POT, true> : &kb_pair<MODE, POT, false>;
+    hipLaunchKernelGGL(k, dim3(nblk(ni, wg / 64)), dim3(wg), lds, st, b->d_reps, b->items[kind],
                        ni, b->ID_[c], b->rtype, b->types, b->inter, pin, b->scell, b->start, b->P_[c], b->V_[c],
                        b->F, b->P2, b->F1, listed, U);
 }
 
-hipError_t batch_step(mavi_batch *b, hipStream_t st) {
+hipError_t batch_step(BatchSub *b, hipStream_t st) {
     hipError_t e = batch_bin(b, st);
     if (e != hipSuccess) return e;
     {
@@ -442,7 +387,7 @@ hipError_t batch_step(mavi_batch *b, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t batch_graph(mavi_batch *b, hipStream_t st) {
+hipError_t batch_graph(BatchSub *b, hipStream_t st) {
     if (b->graph) return hipSuccess;
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
@@ -458,26 +403,34 @@ hipError_t batch_graph(mavi_batch *b, hipStream_t st) {
     return e;
 }
 
-void drop_graph(mavi_batch *b) {
+void drop_graph(BatchSub *b) {
+    mavi::rlb_drop_graph(b);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     b->graph = nullptr;
 }
 
 int batch_check_flags(mavi_batch *b) {
     mavi_ctx *ctx = b->ctx;
-    const size_t nr = b->reps.size();
-    std::vector<uint32_t> h(nr, 0);
-    HIPCHK(ctx, hipMemcpyAsync(h.data(), b->flags, sizeof(uint32_t) * nr, hipMemcpyDeviceToHost, ctx->stream));
+    std::vector<uint32_t> h[2];
+    for (int k = 0; k < 2; k++) {
+        if (!b->sub[k]) continue;
+        h[k].assign(b->sub[k]->reps.size(), 0);
+        HIPCHK(ctx, hipMemcpyAsync(h[k].data(), b->sub[k]->flags, sizeof(uint32_t) * h[k].size(),
+                                   hipMemcpyDeviceToHost, ctx->stream));
+    }
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    for (size_t r = 0; r < nr; r++) {
-        if (!h[r]) continue;
-        HIPCHK(ctx, hipMemsetAsync(b->flags, 0, sizeof(uint32_t) * nr, ctx->stream));
+    for (size_t r = 0; r < b->where.size(); r++) {
+        const uint32_t f = h[b->where[r].sub][b->where[r].local];
+        if (!f) continue;
+        for (int k = 0; k < 2; k++)
+            if (b->sub[k])
+                HIPCHK(ctx, hipMemsetAsync(b->sub[k]->flags, 0, sizeof(uint32_t) * h[k].size(), ctx->stream));
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         const std::string who = "replica " + std::to_string(r) + ": ";
-        if (h[r] & MAVI_FLAG_SCAN_STALL) return set_err(ctx, MAVI_E_HIP, "chunk-count scan: look-back did not complete");
-        if (h[r] & MAVI_FLAG_NONFINITE)
+        if (f & MAVI_FLAG_SCAN_STALL) return set_err(ctx, MAVI_E_HIP, "chunk-count scan: look-back did not complete");
+        if (f & MAVI_FLAG_NONFINITE)
             return set_err(ctx, MAVI_E_NONFINITE, who + "non-finite particle position met while binning");
-        if (h[r] & MAVI_FLAG_OUT_OF_BOX)
+        if (f & MAVI_FLAG_OUT_OF_BOX)
             return set_err(ctx, MAVI_E_OUT_OF_BOX, who + "particle outside the chunk grid (BoundsError in update_chunks!)");
         return set_err(ctx, MAVI_E_CELL_OVERFLOW,
                        who + "a chunk holds more particles than its capacity nc (BoundsError in update_chunks!)");
@@ -487,11 +440,15 @@ int batch_check_flags(mavi_batch *b) {
 
 // Id-order staging of one replica -> its sorted slots in copy cur (+ ring
 // geometry), as mavi_sys_upload does for a single system.
-hipError_t batch_stage_in(mavi_batch *b, int r, hipStream_t st) {
+hipError_t batch_stage_in(BatchSub *b, int r, hipStream_t st) {
     const Replica &Q = b->reps[r];
     const int c = b->cur;
     // a replaced state: its forces are recomputed and every slot binned afresh
     b->keys_ready = false;
+    if (b->rl) {
+        b->rl->valid = b->rl->ordered = false;
+        b->rl->step_hist[0] = b->rl->step_hist[1] = b->rl->step_hist[2] = 0.0;
+    }
     hipError_t e0 = hipMemsetAsync(b->rvalid + r, 0, sizeof(uint32_t), st);
     if (e0 != hipSuccess) return e0;
     const bool rings = Q.kind == KIND_RINGS;
@@ -506,9 +463,9 @@ hipError_t batch_stage_in(mavi_batch *b, int r, hipStream_t st) {
     return hipGetLastError();
 }
 
-int run_impl(mavi_batch *b, int64_t nsteps) {
+// Steps of one family on stream st through the chunk gather.
+int sub_gather(BatchSub *b, int64_t nsteps, hipStream_t st) {
     mavi_ctx *ctx = b->ctx;
-    hipStream_t st = ctx->stream;
     int64_t k = 0;
     const bool graphs = b->use_graphs && !b->prof && nsteps >= b->graph_steps;
     // the graph holds steps that follow a step of these kernels (fused
@@ -522,78 +479,136 @@ int run_impl(mavi_batch *b, int64_t nsteps) {
         for (; k + b->graph_steps <= nsteps; k += b->graph_steps) HIPCHK(ctx, hipGraphLaunch(b->graph, st));
     }
     for (; k < nsteps; k++) HIPCHK(ctx, batch_step(b, st));
+    return MAVI_OK;
+}
+
+// Steps of the rings replicas on the context's stream: on lists, as a rings
+// system alone, where every replica may.
+int sub_rings(BatchSub *b, int64_t nsteps) {
+    int64_t left = nsteps;
+    if (b->rl && !b->rl->disabled && (b->rl->valid || nsteps >= kRlMinCall)) {
+        const int rc = mavi::rlb_steps(b, nsteps, &left);
+        if (rc != MAVI_OK) return rc;
+    }
+    return left > 0 ? sub_gather(b, left, b->ctx->stream) : MAVI_OK;
+}
+
+// The plain replicas' steps are queued ahead of the rings replicas', whose
+// block loop waits on the host; at most this many steps, so that the queue
+// does not fill.
+constexpr int64_t kAheadSteps = 512;
+
+int both_steps(mavi_batch *b, int64_t nsteps) {
+    mavi_ctx *ctx = b->ctx;
+    const int64_t ahead = nblk(kAheadSteps, b->graph_steps) * (int64_t)b->graph_steps;
+    for (int64_t k = 0; k < nsteps; k += ahead) {
+        const int64_t n = std::min(ahead, nsteps - k);
+        int rc = sub_gather(b->sub[0], n, b->side);
+        if (rc == MAVI_OK) rc = sub_rings(b->sub[1], n);
+        if (rc != MAVI_OK) return rc;
+        HIPCHK(ctx, hipStreamSynchronize(b->side));
+    }
+    return MAVI_OK;
+}
+
+int batch_steps(mavi_batch *b, int64_t nsteps) {
+    mavi_ctx *ctx = b->ctx;
+    if (!b->sub[1]) return sub_gather(b->sub[0], nsteps, ctx->stream);
+    if (!b->sub[0]) return sub_rings(b->sub[1], nsteps);
+    // the families share no memory: the plain replicas' steps run beside the
+    // rings replicas'
+    HIPCHK(ctx, hipEventRecord(b->fork, ctx->stream));
+    HIPCHK(ctx, hipStreamWaitEvent(b->side, b->fork, 0));
+    const int rc = both_steps(b, nsteps);
+    // also after an error: nothing of this call is left running on the side
+    const hipError_t e1 = hipEventRecord(b->join, b->side);
+    const hipError_t e2 = hipStreamWaitEvent(ctx->stream, b->join, 0);
+    if (rc != MAVI_OK) return rc;
+    HIPCHK(ctx, e1);
+    HIPCHK(ctx, e2);
+    return MAVI_OK;
+}
+
+hipError_t sub_unpermute(BatchSub *b, hipStream_t st) {
     const int ns = (int)b->nslots;
     hipLaunchKernelGGL(kb_unpermute, dim3(nblk(ns, 256)), dim3(256), 0, st, ns, b->ID_[b->cur], b->P_[b->cur],
                        b->V_[b->cur], b->F, b->pos_id, b->vel_id, b->force_id);
-    HIPCHK(ctx, hipGetLastError());
+    return hipGetLastError();
+}
+
+int run_impl(mavi_batch *b, int64_t nsteps) {
+    mavi_ctx *ctx = b->ctx;
+    const int rc = batch_steps(b, nsteps);
+    if (rc != MAVI_OK) return rc;
+    for (BatchSub *u : b->sub)
+        if (u) HIPCHK(ctx, sub_unpermute(u, ctx->stream));
     return batch_check_flags(b);
+}
+
+// Every slot of a replica in id order (rings: of its active ids), in copy 0;
+// the ids of both copies.
+__global__ void kb_ring_order(const Replica *__restrict__ reps, const int32_t *__restrict__ wave_rep, int32_t nslots,
+                              const int32_t *__restrict__ active_ids, const double2 *__restrict__ pos_id,
+                              double2 *__restrict__ P, int32_t *__restrict__ ID0, int32_t *__restrict__ ID1,
+                              int32_t *__restrict__ slot_of) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nslots) return;
+    const Replica &Q = reps[uniform(wave_rep[s >> 6])];
+    const int t = s - Q.pbase;
+    if (t >= Q.P.na) return;
+    const int id = Q.nbase + active_ids[Q.abase + t];
+    P[s] = pos_id[id];
+    ID0[s] = ID1[s] = id;
+    slot_of[id] = s;
 }
 
 }  // namespace
 
-extern "C" {
+namespace mavi {
 
-int mavi_batch_create(mavi_ctx *ctx, mavi_batch **out) {
-    if (!ctx || !out) return MAVI_E_BADARG;
-    *out = new mavi_batch();
-    (*out)->ctx = ctx;
-    ctx_retain(ctx);
-    return MAVI_OK;
+hipError_t launch_batch_ring_order(BatchSub *b, hipStream_t st) {
+    hipError_t e = sub_unpermute(b, st);
+    if (e != hipSuccess) return e;
+    b->cur = 0;
+    b->keys_ready = false;
+    const int ns = (int)b->nslots;
+    hipLaunchKernelGGL(kb_ring_order, dim3(nblk(ns, 256)), dim3(256), 0, st, b->d_reps, b->wave_rep, ns,
+                       b->active_ids, b->pos_id, b->P_[0], b->ID_[0], b->ID_[1], b->slot_of);
+    return hipGetLastError();
 }
 
-int mavi_batch_destroy(mavi_batch *b) {
-    if (!b) return MAVI_OK;
-    (void)hipSetDevice(b->ctx->device);
-    (void)hipStreamSynchronize(b->ctx->stream);
-    drop_graph(b);
-    for (int c = 0; c < 2; c++) {
-        dfree(b->P_[c]);
-        dfree(b->V_[c]);
-        dfree(b->ID_[c]);
-    }
-    for (int k = 0; k < NKIND; k++) dfree(b->items[k]);
-    dfree(b->ring_wave_rep); dfree(b->d_reps); dfree(b->wave_rep);
-    dfree(b->F); dfree(b->P2); dfree(b->F1);
-    dfree(b->perm); dfree(b->needc); dfree(b->epoch); dfree(b->rvalid);
-    dfree(b->key); dfree(b->rank); dfree(b->src); dfree(b->scell); dfree(b->sid); dfree(b->slot_of);
-    dfree(b->cnt); dfree(b->start); dfree(b->scan_state); dfree(b->scan_ticket); dfree(b->flags); dfree(b->counter);
-    dfree(b->active_ids); dfree(b->pos_id); dfree(b->vel_id); dfree(b->force_id);
-    dfree(b->pol); dfree(b->areas); dfree(b->cms); dfree(b->cms_next); dfree(b->cpos);
-    dfree(b->rtype); dfree(b->types); dfree(b->inter);
-    if (b->ev0) (void)hipEventDestroy(b->ev0);
-    if (b->ev1) (void)hipEventDestroy(b->ev1);
-    mavi_ctx *ctx = b->ctx;
-    delete b;
-    ctx_release(ctx);
-    return MAVI_OK;
+hipError_t launch_batch_cell_order(BatchSub *b, const Replica *greps, int64_t gcells, unsigned long long *ticket,
+                                   unsigned long long *state, hipStream_t st) {
+    BatchProf ps(b, MAVI_PROF_BIN, st);
+    const int ns = (int)b->nslots, n = (int)gcells + 1;
+    b->keys_ready = false;
+    hipError_t e = launch_fill_i32(b->cnt, 0, b->ncells + 1, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kb_bin_count, dim3(nblk(ns, 256)), dim3(256), 0, st, greps, b->wave_rep, ns, b->P_[b->cur],
+                       b->key, b->rank, b->cnt, b->flags);
+    launch_scan(b->cnt, n, b->start, ticket, state, b->flags, st);
+    SysParams G = b->G;
+    G.ncell = (int32_t)gcells;
+    hipLaunchKernelGGL(k_scatter, dim3(nblk(std::max(ns, n), 256)), dim3(256), 0, st, G, b->key, b->rank, b->start,
+                       b->src, b->scell, b->ID_[b->cur], b->sid, b->cnt, nullptr, nullptr, nullptr, nullptr);
+    return hipGetLastError();
 }
 
-int mavi_batch_add_replica(mavi_batch *b, const mavi_sys_desc *d, int32_t *index) {
-    if (!b || !d) return MAVI_E_BADARG;
-    mavi_ctx *ctx = b->ctx;
-    if (b->finalized) return set_err(ctx, MAVI_E_BADARG, "batch already finalized");
-    HostSys h;
-    std::string err;
-    int st = build_params(d, h, err);
-    if (st != MAVI_OK) return set_err(ctx, st, err);
-    if (h.P.cols == 0) return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas need chunks (cols, rows > 0)");
-    if (h.P.potential == MAVI_POT_SZABO || h.P.potential == MAVI_POT_RTP)
-        return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas are LJ / HarmTrunc gases or rings");
-    if (h.P.nwalls > 0) return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas take a single rectangle wall");
-    if (h.P.potential == MAVI_POT_RINGS && h.P.nmax > 32)
-        return set_err(ctx, MAVI_E_UNSUPPORTED, "batch rings replicas need nmax <= 32");
-    b->hs.push_back(std::move(h));
-    if (index) *index = (int32_t)(b->hs.size() - 1);
-    return MAVI_OK;
+}  // namespace mavi
+
+namespace {
+
+int32_t rings_uniform(const std::vector<RingInter> &I) {
+    for (const RingInter &x : I)
+        if (x.k_rep != I[0].k_rep || x.k_atr != I[0].k_atr || x.dist_eq != I[0].dist_eq || x.dist_max != I[0].dist_max)
+            return 0;
+    return 1;
 }
 
-int mavi_batch_finalize(mavi_batch *b) {
-    if (!b) return MAVI_E_BADARG;
+// Device arrays of one family.
+int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
     mavi_ctx *ctx = b->ctx;
-    if (b->finalized) return set_err(ctx, MAVI_E_BADARG, "batch already finalized");
-    if (b->hs.empty()) return set_err(ctx, MAVI_E_BADARG, "empty batch");
-    HIPCHK(ctx, hipSetDevice(ctx->device));
-    const int nr = (int)b->hs.size();
+    const int nr = (int)b->global.size();
     std::vector<int2> items[NKIND];
     std::vector<int32_t> wave_rep, ring_wave_rep, active, rtype;
     std::vector<RingType> types;
@@ -601,7 +616,7 @@ int mavi_batch_finalize(mavi_batch *b) {
     int64_t nslots = 0, nids = 0, nactive = 0, ncells = 0, nrings = 0, ncpos = 0, ntypes = 0, ninter = 0;
     b->reps.resize(nr);
     for (int r = 0; r < nr; r++) {
-        const HostSys &h = b->hs[r];
+        const HostSys &h = hs[b->global[r]];
         Replica &Q = b->reps[r];
         Q = Replica{};
         Q.P = h.P;
@@ -631,6 +646,7 @@ int mavi_batch_finalize(mavi_batch *b) {
             for (int q = 0; q < h.P.nrings; q++) rtype.push_back(h.rtype[q]);
             for (int64_t q = h.P.nrings; q < nrpad; q++) rtype.push_back(0);
             types.insert(types.end(), h.types.begin(), h.types.end());
+            Q.uniform = rings_uniform(h.inter);
             inter.insert(inter.end(), h.inter.begin(), h.inter.end());
             active.insert(active.end(), h.active.begin(), h.active.end());
             nrings += nrpad;
@@ -642,8 +658,6 @@ int mavi_batch_finalize(mavi_batch *b) {
         nslots += npad;
         nids += h.P.n;
         ncells += (int64_t)h.P.ncell + 1;
-        if (nslots > 0x3fffffff || nids > 0x3fffffff || ncells > 0x3fffffff)
-            return set_err(ctx, MAVI_E_BADARG, "batch too large (2^30 slots, ids or chunks)");
     }
     b->nslots = nslots;
     b->nids = nids;
@@ -654,7 +668,6 @@ int mavi_batch_finalize(mavi_batch *b) {
     b->G = SysParams{};
     b->G.na = (int32_t)nslots;
     b->G.ncell = (int32_t)ncells;
-    b->uploaded.assign(nr, 0);
 
     hipStream_t st = ctx->stream;
     hipError_t e = hipSuccess;
@@ -725,8 +738,128 @@ int mavi_batch_finalize(mavi_batch *b) {
     // padding slots carry id -1 in both state copies for good
     for (int c = 0; c < 2 && e == hipSuccess; c++) e = mavi::launch_fill_i32(b->ID_[c], -1, nslots, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess && b->rings) e = mavi::rlb_alloc(b, st);
     if (e != hipSuccess) return set_err(ctx, MAVI_E_HIP, std::string("batch allocation/upload failed: ") +
                                                              hipGetErrorString(e));
+    return MAVI_OK;
+}
+
+void sub_free(BatchSub *b) {
+    drop_graph(b);
+    mavi::rlb_free(b);
+    for (int c = 0; c < 2; c++) {
+        dfree(b->P_[c]);
+        dfree(b->V_[c]);
+        dfree(b->ID_[c]);
+    }
+    for (int k = 0; k < NKIND; k++) dfree(b->items[k]);
+    dfree(b->ring_wave_rep); dfree(b->d_reps); dfree(b->wave_rep);
+    dfree(b->F); dfree(b->P2); dfree(b->F1);
+    dfree(b->perm); dfree(b->needc); dfree(b->epoch); dfree(b->rvalid);
+    dfree(b->key); dfree(b->rank); dfree(b->src); dfree(b->scell); dfree(b->sid); dfree(b->slot_of);
+    dfree(b->cnt); dfree(b->start); dfree(b->scan_state); dfree(b->scan_ticket); dfree(b->flags); dfree(b->counter);
+    dfree(b->active_ids); dfree(b->pos_id); dfree(b->vel_id); dfree(b->force_id);
+    dfree(b->pol); dfree(b->areas); dfree(b->cms); dfree(b->cms_next); dfree(b->cpos);
+    dfree(b->rtype); dfree(b->types); dfree(b->inter);
+    if (b->ev0) (void)hipEventDestroy(b->ev0);
+    if (b->ev1) (void)hipEventDestroy(b->ev1);
+    delete b;
+}
+
+}  // namespace
+
+extern "C" {
+
+int mavi_batch_create(mavi_ctx *ctx, mavi_batch **out) {
+    if (!ctx || !out) return MAVI_E_BADARG;
+    *out = new mavi_batch();
+    (*out)->ctx = ctx;
+    ctx_retain(ctx);
+    return MAVI_OK;
+}
+
+int mavi_batch_destroy(mavi_batch *b) {
+    if (!b) return MAVI_OK;
+    (void)hipSetDevice(b->ctx->device);
+    if (b->side) (void)hipStreamSynchronize(b->side);
+    (void)hipStreamSynchronize(b->ctx->stream);
+    for (BatchSub *u : b->sub)
+        if (u) sub_free(u);
+    if (b->fork) (void)hipEventDestroy(b->fork);
+    if (b->join) (void)hipEventDestroy(b->join);
+    if (b->side) (void)hipStreamDestroy(b->side);
+    mavi_ctx *ctx = b->ctx;
+    delete b;
+    ctx_release(ctx);
+    return MAVI_OK;
+}
+
+int mavi_batch_add_replica(mavi_batch *b, const mavi_sys_desc *d, int32_t *index) {
+    if (!b || !d) return MAVI_E_BADARG;
+    mavi_ctx *ctx = b->ctx;
+    if (b->finalized) return set_err(ctx, MAVI_E_BADARG, "batch already finalized");
+    HostSys h;
+    std::string err;
+    int st = build_params(d, h, err);
+    if (st != MAVI_OK) return set_err(ctx, st, err);
+    if (h.P.cols == 0) return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas need chunks (cols, rows > 0)");
+    if (h.P.potential == MAVI_POT_SZABO || h.P.potential == MAVI_POT_RTP)
+        return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas are LJ / HarmTrunc gases or rings");
+    if (h.P.nwalls > 0) return set_err(ctx, MAVI_E_UNSUPPORTED, "batch replicas take a single rectangle wall");
+    if (h.P.potential == MAVI_POT_RINGS && h.P.nmax > 32)
+        return set_err(ctx, MAVI_E_UNSUPPORTED, "batch rings replicas need nmax <= 32");
+    b->hs.push_back(std::move(h));
+    if (index) *index = (int32_t)(b->hs.size() - 1);
+    return MAVI_OK;
+}
+
+int mavi_batch_finalize(mavi_batch *b) {
+    if (!b) return MAVI_E_BADARG;
+    mavi_ctx *ctx = b->ctx;
+    if (b->finalized) return set_err(ctx, MAVI_E_BADARG, "batch already finalized");
+    if (b->hs.empty()) return set_err(ctx, MAVI_E_BADARG, "empty batch");
+    HIPCHK(ctx, hipSetDevice(ctx->device));
+    // (again after a failed finalize: from the descriptors)
+    for (BatchSub *&u : b->sub) {
+        if (u) sub_free(u);
+        u = nullptr;
+    }
+    b->where.clear();
+    int64_t nslots = 0, nids = 0, ncells = 0;
+    for (size_t r = 0; r < b->hs.size(); r++) {
+        const HostSys &h = b->hs[r];
+        const int k = h.P.potential == MAVI_POT_RINGS ? 1 : 0;
+        BatchSub *&u = b->sub[k];
+        if (!u) {
+            u = new BatchSub();
+            u->ctx = ctx;
+            u->rings = k == 1;
+        }
+        b->where.push_back({k, (int32_t)u->global.size()});
+        u->global.push_back((int32_t)r);
+        nslots += ((int64_t)h.P.na + 63) / 64 * 64;
+        nids += h.P.n;
+        ncells += (int64_t)h.P.ncell + 1;
+        if (nslots > 0x3fffffff || nids > 0x3fffffff || ncells > 0x3fffffff)
+            return set_err(ctx, MAVI_E_BADARG, "batch too large (2^30 slots, ids or chunks)");
+    }
+    for (int k = 0; k < 2; k++) {
+        BatchSub *u = b->sub[k];
+        if (!u) continue;
+        u->wg = b->wg[k];
+        u->listed = b->listed[k];
+        u->graph_steps = b->graph_steps;
+        u->use_graphs = b->use_graphs;
+        u->prof = b->prof;
+        const int rc = sub_finalize(u, b->hs);
+        if (rc != MAVI_OK) return rc;
+    }
+    if (b->sub[0] && b->sub[1]) {
+        if (!b->side) HIPCHK(ctx, hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
+        if (!b->fork) HIPCHK(ctx, hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
+        if (!b->join) HIPCHK(ctx, hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
+    }
+    b->uploaded.assign(b->hs.size(), 0);
     b->hs.clear();
     b->hs.shrink_to_fit();
     b->finalized = true;
@@ -735,7 +868,7 @@ int mavi_batch_finalize(mavi_batch *b) {
 
 static int check_index(mavi_batch *b, int32_t i) {
     if (!b->finalized) return set_err(b->ctx, MAVI_E_BADARG, "batch not finalized");
-    if (i < 0 || i >= (int32_t)b->reps.size()) return set_err(b->ctx, MAVI_E_BADARG, "replica index out of range");
+    if (i < 0 || i >= (int32_t)b->where.size()) return set_err(b->ctx, MAVI_E_BADARG, "replica index out of range");
     return MAVI_OK;
 }
 
@@ -746,14 +879,15 @@ int mavi_batch_upload(mavi_batch *b, int32_t i, const double *pos, const double 
     mavi_ctx *ctx = b->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const Replica &Q = b->reps[i];
+    BatchSub *u = b->sub[b->where[i].sub];
+    const Replica &Q = u->reps[b->where[i].local];
     const size_t bytes = sizeof(double2) * (size_t)Q.P.n;
-    HIPCHK(ctx, hipMemcpyAsync(b->pos_id + Q.nbase, pos, bytes, hipMemcpyHostToDevice, st));
+    HIPCHK(ctx, hipMemcpyAsync(u->pos_id + Q.nbase, pos, bytes, hipMemcpyHostToDevice, st));
     if (vel && Q.kind != KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(b->vel_id + Q.nbase, vel, bytes, hipMemcpyHostToDevice, st));
+        HIPCHK(ctx, hipMemcpyAsync(u->vel_id + Q.nbase, vel, bytes, hipMemcpyHostToDevice, st));
     if (pol && Q.kind == KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(b->pol + Q.rbase, pol, sizeof(double) * Q.P.nrings, hipMemcpyHostToDevice, st));
-    HIPCHK(ctx, batch_stage_in(b, i, st));
+        HIPCHK(ctx, hipMemcpyAsync(u->pol + Q.rbase, pol, sizeof(double) * Q.P.nrings, hipMemcpyHostToDevice, st));
+    HIPCHK(ctx, batch_stage_in(u, b->where[i].local, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
     b->uploaded[i] = 1;
     return MAVI_OK;
@@ -766,13 +900,14 @@ int mavi_batch_download(mavi_batch *b, int32_t i, double *pos, double *vel, doub
     mavi_ctx *ctx = b->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const Replica &Q = b->reps[i];
+    BatchSub *u = b->sub[b->where[i].sub];
+    const Replica &Q = u->reps[b->where[i].local];
     const size_t bytes = sizeof(double2) * (size_t)Q.P.n;
-    if (pos) HIPCHK(ctx, hipMemcpyAsync(pos, b->pos_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
+    if (pos) HIPCHK(ctx, hipMemcpyAsync(pos, u->pos_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
     if (vel && Q.kind != KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(vel, b->vel_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
+        HIPCHK(ctx, hipMemcpyAsync(vel, u->vel_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
     if (pol && Q.kind == KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(pol, b->pol + Q.rbase, sizeof(double) * Q.P.nrings, hipMemcpyDeviceToHost, st));
+        HIPCHK(ctx, hipMemcpyAsync(pol, u->pol + Q.rbase, sizeof(double) * Q.P.nrings, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
     return MAVI_OK;
 }
@@ -783,8 +918,9 @@ int mavi_batch_get_forces(mavi_batch *b, int32_t i, double *forces) {
     if (rc != MAVI_OK) return rc;
     mavi_ctx *ctx = b->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    const Replica &Q = b->reps[i];
-    HIPCHK(ctx, hipMemcpyAsync(forces, b->force_id + Q.nbase, sizeof(double2) * (size_t)Q.P.n,
+    const BatchSub *u = b->sub[b->where[i].sub];
+    const Replica &Q = u->reps[b->where[i].local];
+    HIPCHK(ctx, hipMemcpyAsync(forces, u->force_id + Q.nbase, sizeof(double2) * (size_t)Q.P.n,
                                hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return MAVI_OK;
@@ -807,7 +943,7 @@ int mavi_batch_noise_get_counter(mavi_batch *b, uint64_t *counter) {
     if (!b->finalized) return set_err(ctx, MAVI_E_BADARG, "batch not finalized");
     HIPCHK(ctx, hipSetDevice(ctx->device));
     unsigned long long c = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&c, b->counter, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(&c, b->sub[b->sub[0] ? 0 : 1]->counter, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     *counter = c;
     return MAVI_OK;
@@ -820,17 +956,30 @@ int mavi_batch_noise_set_counter(mavi_batch *b, uint64_t counter) {
     HIPCHK(ctx, hipSetDevice(ctx->device));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     const unsigned long long c = counter;
-    HIPCHK(ctx, hipMemcpy(b->counter, &c, sizeof(c), hipMemcpyHostToDevice));
+    for (BatchSub *u : b->sub)
+        if (u) HIPCHK(ctx, hipMemcpy(u->counter, &c, sizeof(c), hipMemcpyHostToDevice));
     return MAVI_OK;
 }
 
 // A changed pair-kernel shape may visit candidates in another order: the
 // reused forces would not be its bits, so every replica recomputes once.
 static int batch_forget_forces(mavi_batch *b) {
-    if (!b->finalized || !b->rvalid) return MAVI_OK;
+    if (!b->finalized) return MAVI_OK;
     HIPCHK(b->ctx, hipSetDevice(b->ctx->device));
-    HIPCHK(b->ctx, hipMemsetAsync(b->rvalid, 0, sizeof(uint32_t) * b->reps.size(), b->ctx->stream));
+    for (BatchSub *u : b->sub)
+        if (u) HIPCHK(b->ctx, hipMemsetAsync(u->rvalid, 0, sizeof(uint32_t) * u->reps.size(), b->ctx->stream));
     return MAVI_OK;
+}
+
+// The options of a family (0 plain, 1 rings) changed.
+static void batch_set_shape(mavi_batch *b, int k) {
+    BatchSub *u = b->sub[k];
+    if (!u) return;
+    if (u->wg != b->wg[k] || u->listed != b->listed[k] || u->graph_steps != b->graph_steps) drop_graph(u);
+    u->wg = b->wg[k];
+    u->listed = b->listed[k];
+    u->graph_steps = b->graph_steps;
+    u->use_graphs = b->use_graphs;
 }
 
 int mavi_batch_set_option(mavi_batch *b, int32_t option, int32_t value) {
@@ -841,21 +990,22 @@ int mavi_batch_set_option(mavi_batch *b, int32_t option, int32_t value) {
         case MAVI_BOPT_WG_RINGS:
             if (value == 0) value = 256;
             if (!is_pow2_wg(value)) return set_err(ctx, MAVI_E_BADARG, "workgroup must be 64..1024, a power of 2");
-            if (b->wg[option - MAVI_BOPT_WG_PLAIN] != value) drop_graph(b);
             b->wg[option - MAVI_BOPT_WG_PLAIN] = value;
+            batch_set_shape(b, option - MAVI_BOPT_WG_PLAIN);
             return batch_forget_forces(b);
         case MAVI_BOPT_LIST_PLAIN:
         case MAVI_BOPT_LIST_RINGS:
-            if (b->listed[option - MAVI_BOPT_LIST_PLAIN] != (value != 0)) drop_graph(b);
             b->listed[option - MAVI_BOPT_LIST_PLAIN] = value != 0;
+            batch_set_shape(b, option - MAVI_BOPT_LIST_PLAIN);
             return batch_forget_forces(b);
         case MAVI_BOPT_GRAPH_STEPS:
             if (value < 2 || (value & 1)) return set_err(ctx, MAVI_E_BADARG, "graph steps must be even and >= 2");
-            if (value != b->graph_steps) drop_graph(b);
             b->graph_steps = value;
+            for (int k = 0; k < 2; k++) batch_set_shape(b, k);
             return MAVI_OK;
         case MAVI_BOPT_GRAPHS:
             b->use_graphs = value != 0;
+            for (int k = 0; k < 2; k++) batch_set_shape(b, k);
             return MAVI_OK;
         default:
             return set_err(ctx, MAVI_E_BADARG, "unknown batch option");
@@ -865,28 +1015,41 @@ int mavi_batch_set_option(mavi_batch *b, int32_t option, int32_t value) {
 int mavi_batch_info(mavi_batch *b, int64_t *info) {
     if (!b || !info) return MAVI_E_BADARG;
     if (!b->finalized) return set_err(b->ctx, MAVI_E_BADARG, "batch not finalized");
-    info[0] = (int64_t)b->reps.size();
-    info[1] = b->nids;
-    info[2] = b->nactive;
-    info[3] = b->nslots;
-    info[4] = b->ncells;
-    int64_t nr = 0;
-    for (const Replica &Q : b->reps) nr += Q.kind == KIND_RINGS ? Q.P.nrings : 0;
-    info[5] = nr;
+    info[0] = (int64_t)b->where.size();
+    for (int k = 1; k < 6; k++) info[k] = 0;
+    for (const BatchSub *u : b->sub) {
+        if (!u) continue;
+        info[1] += u->nids;
+        info[2] += u->nactive;
+        info[3] += u->nslots;
+        info[4] += u->ncells;
+        for (const Replica &Q : u->reps) info[5] += u->rings ? Q.P.nrings : 0;
+    }
     return MAVI_OK;
 }
 
 int mavi_batch_prof_enable(mavi_batch *b, int on) {
     if (!b) return MAVI_E_BADARG;
     b->prof = on != 0;
-    for (auto &p : b->profs) p = ProfSlot{};
+    for (BatchSub *u : b->sub) {
+        if (!u) continue;
+        u->prof = b->prof;
+        for (auto &p : u->profs) p = ProfSlot{};
+    }
     return MAVI_OK;
 }
 
 int mavi_batch_prof_get(mavi_batch *b, int which, double *ms_total, int64_t *launches) {
     if (!b || which < 0 || which >= MAVI_PROF_NCLASS) return MAVI_E_BADARG;
-    if (ms_total) *ms_total = b->profs[which].ms;
-    if (launches) *launches = b->profs[which].launches;
+    double ms = 0.0;
+    int64_t n = 0;
+    for (const BatchSub *u : b->sub) {
+        if (!u) continue;
+        ms += u->profs[which].ms;
+        n += u->profs[which].launches;
+    }
+    if (ms_total) *ms_total = ms;
+    if (launches) *launches = n;
     return MAVI_OK;
 }
 
@@ -899,55 +1062,62 @@ int mavi_batch_autotune(mavi_batch *b, int32_t trial_steps, double *best_us, int
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     // snapshot: id-order staging of every replica, polarisations, step counter
-    const int ns = (int)b->nslots;
-    hipLaunchKernelGGL(kb_unpermute, dim3(nblk(ns, 256)), dim3(256), 0, st, ns, b->ID_[b->cur], b->P_[b->cur],
-                       b->V_[b->cur], b->F, b->pos_id, b->vel_id, b->force_id);
-    HIPCHK(ctx, hipGetLastError());
-    double2 *pos0 = nullptr, *vel0 = nullptr;
-    double *pol0 = nullptr;
-    unsigned long long *cnt0 = nullptr;
-    const size_t bytes = sizeof(double2) * (size_t)b->nids;
-    hipError_t e = dalloc(&pos0, b->nids, st);
-    if (e == hipSuccess) e = dalloc(&vel0, b->nids, st);
-    if (e == hipSuccess) e = dalloc(&cnt0, 1, st);
-    if (e == hipSuccess && b->nrings) e = dalloc(&pol0, b->nrings, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(pos0, b->pos_id, bytes, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(vel0, b->vel_id, bytes, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(cnt0, b->counter, sizeof(unsigned long long), hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess && pol0) e = hipMemcpyAsync(pol0, b->pol, sizeof(double) * b->nrings, hipMemcpyDeviceToDevice, st);
-    auto restore = [&]() -> hipError_t {
-        hipError_t r = hipMemcpyAsync(b->pos_id, pos0, bytes, hipMemcpyDeviceToDevice, st);
-        if (r == hipSuccess) r = hipMemcpyAsync(b->vel_id, vel0, bytes, hipMemcpyDeviceToDevice, st);
-        if (r == hipSuccess)
-            r = hipMemcpyAsync(b->counter, cnt0, sizeof(unsigned long long), hipMemcpyDeviceToDevice, st);
-        if (r == hipSuccess && pol0)
-            r = hipMemcpyAsync(b->pol, pol0, sizeof(double) * b->nrings, hipMemcpyDeviceToDevice, st);
-        b->cur = 0;
-        for (int q = 0; q < (int)b->reps.size() && r == hipSuccess; q++) r = batch_stage_in(b, q, st);
-        if (r == hipSuccess) r = hipStreamSynchronize(st);
-        return r;
+    struct Snap {
+        double2 *pos = nullptr, *vel = nullptr;
+        double *pol = nullptr;
+        unsigned long long *cnt = nullptr;
+    } snap[2];
+    hipError_t e = hipSuccess;
+    auto copy = [&](void *dst, const void *src, size_t bytes) {
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, st);
+    };
+    for (int k = 0; k < 2; k++) {
+        BatchSub *u = b->sub[k];
+        if (!u) continue;
+        Snap &S = snap[k];
+        if (e == hipSuccess) e = sub_unpermute(u, st);
+        if (e == hipSuccess) e = dalloc(&S.pos, u->nids, st);
+        if (e == hipSuccess) e = dalloc(&S.vel, u->nids, st);
+        if (e == hipSuccess) e = dalloc(&S.cnt, 1, st);
+        if (e == hipSuccess && u->nrings) e = dalloc(&S.pol, u->nrings, st);
+        const size_t bytes = sizeof(double2) * (size_t)u->nids;
+        copy(S.pos, u->pos_id, bytes);
+        copy(S.vel, u->vel_id, bytes);
+        copy(S.cnt, u->counter, sizeof(unsigned long long));
+        if (S.pol) copy(S.pol, u->pol, sizeof(double) * u->nrings);
+    }
+    auto restore = [&](int k) {
+        BatchSub *u = b->sub[k];
+        const Snap &S = snap[k];
+        const size_t bytes = sizeof(double2) * (size_t)u->nids;
+        copy(u->pos_id, S.pos, bytes);
+        copy(u->vel_id, S.vel, bytes);
+        copy(u->counter, S.cnt, sizeof(unsigned long long));
+        if (S.pol) copy(u->pol, S.pol, sizeof(double) * u->nrings);
+        u->cur = 0;
+        for (int q = 0; q < (int)u->reps.size() && e == hipSuccess; q++) e = batch_stage_in(u, q, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
     };
     const int wgs[4] = {64, 128, 256, 512};
-    const bool saved_prof = b->prof;
-    b->prof = false;
-    double best_total = 1e300;
-    for (int slot = 0; slot < 2 && e == hipSuccess; slot++) {
-        const bool present = slot == 0 ? (b->nitems[KIND_LJ] + b->nitems[KIND_HT] > 0) : b->nitems[KIND_RINGS] > 0;
-        if (!present) continue;
+    for (BatchSub *u : b->sub)
+        if (u) u->prof = false;
+    for (int k = 0; k < 2 && e == hipSuccess; k++) {
+        BatchSub *u = b->sub[k];
+        if (!u) continue;
         double best = 1e300;
-        int bw = b->wg[slot], bl = b->listed[slot];
+        int bw = u->wg, bl = u->listed;
         for (int tp = 0; tp < 2 && e == hipSuccess; tp++) {
             for (int wi = 0; wi < 4 && e == hipSuccess; wi++) {
-                b->wg[slot] = wgs[wi];
-                b->listed[slot] = tp;
-                if ((e = restore()) != hipSuccess) break;
-                if ((e = batch_step(b, st)) != hipSuccess) break;  // warm-up
-                if ((e = hipEventRecord(b->ev0, st)) != hipSuccess) break;
-                for (int k = 0; k < trial_steps && e == hipSuccess; k++) e = batch_step(b, st);
-                if (e == hipSuccess) e = hipEventRecord(b->ev1, st);
-                if (e == hipSuccess) e = hipEventSynchronize(b->ev1);
+                u->wg = wgs[wi];
+                u->listed = tp;
+                restore(k);
+                if (e == hipSuccess) e = batch_step(u, st);  // warm-up
+                if (e == hipSuccess) e = hipEventRecord(u->ev0, st);
+                for (int t = 0; t < trial_steps && e == hipSuccess; t++) e = batch_step(u, st);
+                if (e == hipSuccess) e = hipEventRecord(u->ev1, st);
+                if (e == hipSuccess) e = hipEventSynchronize(u->ev1);
                 float ms = 0.f;
-                if (e == hipSuccess) e = hipEventElapsedTime(&ms, b->ev0, b->ev1);
+                if (e == hipSuccess) e = hipEventElapsedTime(&ms, u->ev0, u->ev1);
                 const double us = 1e3 * ms / trial_steps;
                 if (e == hipSuccess && us < best) {
                     best = us;
@@ -956,32 +1126,47 @@ int mavi_batch_autotune(mavi_batch *b, int32_t trial_steps, double *best_us, int
                 }
             }
         }
-        b->wg[slot] = bw;
-        b->listed[slot] = bl;
+        u->wg = b->wg[k] = bw;
+        u->listed = b->listed[k] = bl;
+        drop_graph(u);
     }
-    // the chosen shapes of both slots together: a mixed batch steps both
-    // kinds, so the time of one slot's search is not the step's time
-    if (e == hipSuccess) e = restore();
-    if (e == hipSuccess) e = batch_step(b, st);  // warm-up
-    if (e == hipSuccess) e = hipEventRecord(b->ev0, st);
-    for (int k = 0; k < trial_steps && e == hipSuccess; k++) e = batch_step(b, st);
-    if (e == hipSuccess) e = hipEventRecord(b->ev1, st);
-    if (e == hipSuccess) e = hipEventSynchronize(b->ev1);
-    if (e == hipSuccess) {
+    // the chosen shapes of both families together, as a run steps them (the
+    // rings replicas on lists where they may)
+    double best_total = 1e300;
+    int rc = MAVI_OK;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    for (int k = 0; k < 2; k++)
+        if (b->sub[k]) restore(k);
+    for (auto &v : ev)
+        if (e == hipSuccess) e = hipEventCreate(&v);
+    if (e == hipSuccess) rc = batch_steps(b, 1);  // warm-up
+    if (rc == MAVI_OK && e == hipSuccess) e = hipEventRecord(ev[0], st);
+    if (rc == MAVI_OK && e == hipSuccess) rc = batch_steps(b, trial_steps);
+    if (rc == MAVI_OK && e == hipSuccess) e = hipEventRecord(ev[1], st);
+    if (rc == MAVI_OK && e == hipSuccess) e = hipEventSynchronize(ev[1]);
+    if (rc == MAVI_OK && e == hipSuccess) {
         float ms = 0.f;
-        e = hipEventElapsedTime(&ms, b->ev0, b->ev1);
+        e = hipEventElapsedTime(&ms, ev[0], ev[1]);
         best_total = 1e3 * ms / trial_steps;
     }
-    b->prof = saved_prof;
-    drop_graph(b);
-    if (e == hipSuccess) e = restore();
-    if (e == hipSuccess) (void)hipMemsetAsync(b->flags, 0, sizeof(uint32_t) * b->reps.size(), st);
+    for (auto &v : ev)
+        if (v) (void)hipEventDestroy(v);
+    for (int k = 0; k < 2; k++) {
+        BatchSub *u = b->sub[k];
+        if (!u) continue;
+        u->prof = b->prof;
+        restore(k);
+        if (e == hipSuccess) (void)hipMemsetAsync(u->flags, 0, sizeof(uint32_t) * u->reps.size(), st);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    dfree(pos0);
-    dfree(vel0);
-    dfree(pol0);
-    dfree(cnt0);
+    for (Snap &S : snap) {
+        dfree(S.pos);
+        dfree(S.vel);
+        dfree(S.pol);
+        dfree(S.cnt);
+    }
     HIPCHK(ctx, e);
+    if (rc != MAVI_OK) return rc;
     if (best_us) *best_us = best_total;
     if (shape) {
         shape[0] = b->wg[0];

@@ -988,8 +988,6 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
     return MAVI_OK;
 }
 
-constexpr int64_t kRlMinCall = 8;
-
 static int steps_impl(mavi_sys *s, int64_t nsteps, const double *noise_host) {
     mavi_ctx *ctx = s->ctx;
     if (nsteps < 0) return set_err(ctx, MAVI_E_BADARG, "nsteps < 0");

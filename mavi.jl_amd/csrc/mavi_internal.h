@@ -215,6 +215,7 @@ struct NList {
 
 constexpr double kRlSkin = 0.3;      // default list skin of rings (fraction of the widest range)
 constexpr int kRlGraphSteps = 8;     // steps per captured graph (even)
+constexpr int64_t kRlMinCall = 8;    // a call that has to build lists needs this many steps to win the build
 
 // Verlet lists of a rings system with a fixed population (mavi_rlist.hip).
 struct RList {
@@ -223,7 +224,7 @@ struct RList {
     bool disabled = false;    // a list or a chunk overflowed: the chunk gather takes over
     bool ordered = false;     // the state lies in ring order, both copies' ids too
     bool valid = false;       // lists complete for the current state
-    bool uniform = false;     // one interaction for all type pairs
+    bool uniform = false;     // one interaction for all type pairs (a batch: every ring full)
     double rl2 = 0.0;         // list radius squared (range + skin)^2, with margin
     double half_skin = 0.0;   // displacement bound
     int32_t block = 0;        // steps between host checks (option; 0: as many as the bound allows, at most kNlBlockCap)
@@ -232,6 +233,9 @@ struct RList {
     int32_t step_i = 0;
     double d_start = 0.0;     // largest displacement from the build of the next block's first positions
     SysParams G{};            // list grid (cells >= range + skin)
+    void *greps = nullptr;    // a batch: its replica table with the list grids (device)
+    int64_t gcells = 0;       // and their cells
+    int per = 1;              // most rings of a wave of the step kernel
     int ph = 0;               // counter word of the current step
     int32_t *head = nullptr;  // int4 per slot: the first four entries, -1 past the end
     int32_t *more = nullptr;  // further entries
@@ -243,7 +247,7 @@ struct RList {
     double *polsnap = nullptr;
     uint32_t *fsnap = nullptr;
     double2 *polcs = nullptr; // cos, sin of the polarisations
-    uint32_t *bmax = nullptr; // per wave of the step kernel
+    uint32_t *bmax = nullptr; // per workgroup of the step kernel
     int32_t nbmax = 0;
     uint32_t *status = nullptr;
     unsigned long long *counter = nullptr;  // two words, alternating between steps

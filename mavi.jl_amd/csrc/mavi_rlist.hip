@@ -32,7 +32,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
+#include "mavi_batch.h"
 #include "mavi_device.h"
 #include "mavi_host.h"
 
@@ -40,7 +42,10 @@ namespace {
 
 constexpr int kRlHead = 4;    // list entries in the particle's int4
 constexpr int kRlMax = 16;    // list entries per particle
-constexpr int kRlWG = 256;    // step workgroup: four waves of floor(64 / nmax) rings
+// Step workgroup: waves of floor(64 / nmax) rings.  us a step at 2k / 800k
+// particles: 4 waves 11.7 / 48.6, 8 waves 12.8 / 51.7, 12 waves 14.0 / 54.8
+// (one wave does the ring stage of all while the others' places stay empty).
+constexpr int kRlWaves = 4, kRlWG = 64 * kRlWaves;
 constexpr uint32_t kRlOverflow = 1u;  // a list longer than kRlMax
 constexpr uint32_t kRlCapacity = 2u;  // a chunk count may have passed the capacity
 
@@ -67,12 +72,27 @@ struct RLArgs {
     const RingType *types;
     const RingInter *inter;     // matrix of interactions; null: `uni` for every pair
     RingInter uni;
-    uint32_t *bmax;             // per wave: high word of the largest squared step, rounded up
+    uint32_t *bmax;             // per workgroup: high word of the largest squared step, rounded up
     uint32_t *flags, *status;
     uint64_t seed;
     const unsigned long long *cin;  // the step counter before this step
     unsigned long long *cout;
+    int64_t stride;             // slots (stride of `more`)
+    int32_t per;                // most rings of a wave
+    // a batch: replicas by wave of the step kernel, and their table
+    const Replica *reps;
+    const int32_t *wave_rep;
+    int32_t nwaves;
 };
+
+// Where a system's arrays start in a batch (0 for a system alone).
+struct RLBase {
+    int32_t slot = 0, id = 0, chunk = 0, ring = 0, type = 0, inter = 0, flag = 0;
+    int64_t cpos = 0;
+};
+__device__ __forceinline__ RLBase rl_base(const Replica &Q, int rep) {
+    return RLBase{Q.pbase, Q.nbase, Q.cbase, Q.rbase, Q.tbase, Q.ibase, rep, Q.cpbase};
+}
 
 __device__ __forceinline__ void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -104,8 +124,10 @@ __device__ __forceinline__ uint32_t visit_rank(const SysParams &P, int ri, int c
     return (uint32_t)(d * 3 + c);
 }
 
-__device__ __forceinline__ RingInter rl_inter(const SysParams &P, const RLArgs &A, int ti, int32_t e) {
-    return A.inter ? A.inter[ti + P.ntypes * (e >> kRlSlotBits)] : A.uni;
+// The interaction of type ti with entry e's type (mat null: `uni` for every pair).
+__device__ __forceinline__ RingInter rl_inter(const SysParams &P, const RingInter *mat, const RingInter &uni, int ti,
+                                              int32_t e) {
+    return mat ? mat[ti + P.ntypes * (e >> kRlSlotBits)] : uni;
 }
 
 // calc_interaction_force (src/rings/integration.jl:47-77) of a listed pair in
@@ -113,8 +135,10 @@ __device__ __forceinline__ RingInter rl_inter(const SysParams &P, const RLArgs &
 __device__ __forceinline__ double2 rl_force(const RingInter &I, double2 d, double r2, bool same) {
     const double dist = sqrt(r2);
     double fmod;
-    if (r2 < I.eq2) fmod = -I.k_rep * (dist / I.dist_eq - 1.0);
-    else fmod = same ? 0.0 : -I.k_atr * (dist / I.dist_eq - 1.0);
+    double u = dist;
+    if (I.dist_eq != 1.0) u = dist / I.dist_eq;  // discs of unit diameter need no division
+    if (r2 < I.eq2) fmod = -I.k_rep * (u - 1.0);
+    else fmod = same ? 0.0 : -I.k_atr * (u - 1.0);
     const double q = fmod / dist;
     return make_double2(q * d.x, q * d.y);
 }
@@ -128,8 +152,9 @@ __device__ __forceinline__ unsigned long long visit_key(const SysParams &P, int 
 
 // The sum of a particle with a long list, by repeated selection of the next
 // pair in the gather's order.
-__device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs &A, int q, int t0, int t1, int ti,
-                                            double2 x, int ri, int ci) {
+__device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs &A, const RingInter *mat,
+                                               const RingInter &uni, int q, int t0, int t1, int ti, double2 x, int ri,
+                                               int ci) {
     const int n = A.count[q];
     const int4 h = A.head[q];
     double2 f = make_double2(0.0, 0.0);
@@ -139,12 +164,12 @@ __device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs 
         unsigned long long best = ~0ull;
         int32_t be = -1;
         for (int e = 0; e < n; e++) {
-            const int32_t w = e == 0 ? h.x : e == 1 ? h.y : e == 2 ? h.z : e == 3 ? h.w : A.more[(int64_t)(e - kRlHead) * P.na + q];
+            const int32_t w = e == 0 ? h.x : e == 1 ? h.y : e == 2 ? h.z : e == 3 ? h.w : A.more[(int64_t)(e - kRlHead) * A.stride + q];
             const int j = w & kRlSlotMask;
             const double2 pj = A.Pin[j];
             const double2 d = cdiff(P, x, pj);
             const double r2 = d.x * d.x + d.y * d.y;
-            if (r2 > rl_inter(P, A, ti, w).max2) continue;
+            if (r2 > rl_inter(P, mat, uni, ti, w).max2) continue;
             const unsigned long long k = visit_key(P, ri, ci, pj, j);
             if ((first || k > prev) && k < best) {
                 best = k;
@@ -154,12 +179,59 @@ __device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs 
         if (be < 0) return f;
         const int j = be & kRlSlotMask;
         const double2 d = cdiff(P, x, A.Pin[j]);
-        const double2 c = rl_force(rl_inter(P, A, ti, be), d, d.x * d.x + d.y * d.y, j >= t0 && j < t1);
+        const double2 c = rl_force(rl_inter(P, mat, uni, ti, be), d, d.x * d.x + d.y * d.y, j >= t0 && j < t1);
         f.x += c.x;
         f.y += c.y;
         prev = best;
         first = false;
     }
+}
+
+// What the polarisation update of ring k of a workgroup (place k % per of wave
+// k / per, per the most rings of a wave) needs from memory, and its noise.  np 0: no ring there.
+struct RingScalars {
+    double pol, cs, sn, rate, dt, noise;
+    int32_t np, rg;
+};
+template <bool BATCH>
+__device__ __forceinline__ RingScalars ring_scalars(const SysParams &P0, const RLArgs &A, int block, int k,
+                                                    unsigned long long step) {
+    const int w = k / A.per, wl = block * kRlWaves + w;
+    RingScalars R{};
+    if (BATCH && wl >= A.nwaves) return R;
+    const Replica *Q = BATCH ? A.reps + A.wave_rep[wl] : nullptr;
+    const SysParams &P = BATCH ? Q->P : P0;
+    const int own = BATCH ? 64 / P.nmax : A.per;  // rings of that wave
+    const int g = k - w * A.per;
+    const int ring = (BATCH ? wl - Q->rwbase : wl) * own + g;
+    if (g >= own || ring >= P.nrings) return R;
+    R.rg = (BATCH ? Q->rbase : 0) + ring;
+    const RingType *T = A.types + (BATCH ? Q->tbase : 0) + (P.typed ? A.rtype[R.rg] : 0);
+    const double2 cs = A.polcs[R.rg];
+    R.pol = A.pol[R.rg];
+    R.cs = cs.x;
+    R.sn = cs.y;
+    R.np = T->np;
+    R.dt = P.dt;
+    R.rate = 1.0 / T->relax;
+    const double rot = T->rot;
+    const double z = rot != 0.0 ? philox_normal(BATCH ? Q->seed : A.seed, step, (uint32_t)ring) : 0.0;
+    R.noise = sqrt(2.0 * rot * R.dt) * z;
+    return R;
+}
+
+// Largest value of the wave, in lane 63.
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+#define MAVI_DPP_MAX(ctrl, rows) \
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false))
+    MAVI_DPP_MAX(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane 15 of a row holds the row's
+    MAVI_DPP_MAX(0x112, 0xf);
+    MAVI_DPP_MAX(0x114, 0xf);
+    MAVI_DPP_MAX(0x118, 0xf);
+    MAVI_DPP_MAX(0x142, 0xa);  // row_bcast 15, 31
+    MAVI_DPP_MAX(0x143, 0xc);
+#undef MAVI_DPP_MAX
+    return v;
 }
 
 // One Rings step! of the rings of this workgroup.  LAST: the last step of a
@@ -171,33 +243,45 @@ __device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs 
 // once per ring and component on a few lanes (2 or 3 per ring) instead of as
 // masked loops of every lane, and the scalar work of a ring (noise, asin,
 // sincos of the new angle) once per workgroup on one lane per ring: as part of
-// every wave it was a third of the ring kernel's instructions.  45.9 us at
-// 800k particles (806 VALU instructions per wave) against 97 us for the five
-// launches it replaces (scan 12.1, scatter 8.7, finalize 11.1, pairs 26.2, ring
-// update 38.1); 11.8 against 33 us at 2k particles.
-template <bool LAST>
-__global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
+// every wave it was a third of the ring kernel's instructions.  That lane takes
+// its inputs and the noise, which do not depend on the forces, while the pairs'
+// positions are on their way.  With the rebuilds 46.3 us a step at 800k
+// particles (49.0 with the ring stage's loads at its end) against 97 us for the
+// five launches it replaces (scan 12.1, scatter 8.7, finalize 11.1, pairs 26.2,
+// ring update 38.1); 11.3 against 33 us at 2k particles.
+template <bool LAST, bool BATCH>
+__global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4 : 1))) void k_rl_step(SysParams P0, RLArgs A) {
     __shared__ double2 s_a[kRlWG + 32], s_b[kRlWG + 32], s_c[kRlWG + 32];
     __shared__ double s_t[kRlWG + 32];
-    __shared__ double s_r[4][64 * 3];  // per ring of a wave: sums
-    const int lane = (int)lane_id(), wave = (int)(threadIdx.x >> 6);
+    __shared__ double s_r[kRlWaves][64 * 3];  // per ring of a wave: sums
+    __shared__ uint32_t s_max[kRlWaves];
+    __shared__ RingScalars s_ring[64];  // wave 0: of the workgroup's first 64 rings
+    const int lane = (int)lane_id(), wave = uniform((int)(threadIdx.x >> 6));
+    const int block = xcd_block();
+    const int wl = block * kRlWaves + wave;
+    const int rep = BATCH ? uniform(A.wave_rep[min(wl, A.nwaves - 1)]) : 0;
+    const SysParams P = BATCH ? A.reps[rep].P : P0;
+    const RLBase B = BATCH ? rl_base(A.reps[rep], rep) : RLBase{};
+    const RingInter *mat = BATCH ? (A.reps[rep].uniform ? nullptr : A.inter + B.inter) : A.inter;
+    const RingInter &uni = BATCH ? A.inter[B.inter] : A.uni;
     const int per = 64 / P.nmax;
     const int grp = lane / P.nmax, i = lane - grp * P.nmax;
-    const int block = xcd_block();
-    const int r = (block * 4 + wave) * per + grp;
-    const bool ring_ok = grp < per && r < P.nrings;
+    const int first = (BATCH ? wl - A.reps[rep].rwbase : wl) * per;  // the wave's first ring
+    const int r = first + grp;
+    const bool ring_ok = (!BATCH || wl < A.nwaves) && grp < per && r < P.nrings;
     const int rr = ring_ok ? r : 0;
-    const int t = P.typed ? A.rtype[rr] : 0;
-    const RingType *T = A.types + t;
-    const int np = T->np;
+    const int t = P.typed ? A.rtype[B.ring + rr] : 0;
+    const RingType *T = A.types + B.type + t;
+    const bool full = !A.slot_of;  // every ring has nmax particles
+    const int np = full ? P.nmax : T->np;
     const bool act = ring_ok && i < np;
     const int id = rr * P.nmax + i;
-    const int q = act ? (A.slot_of ? A.slot_of[id] : id) : 0;
+    const int q = act ? (full ? B.slot + id : A.slot_of[B.id + id]) : B.slot;
     const int t0 = q - i, t1 = t0 + np;  // the ring's slots
     const double2 x = act ? A.Pin[q] : make_double2(0.0, 0.0);
     int4 h = act ? A.head[q] : make_int4(-1, -1, -1, -1);
     const int32_t ko = act ? A.key[q] : 0;
-    const double2 pcs = A.polcs[rr];
+    const double2 pcs = A.polcs[B.ring + rr];
     const unsigned long long step = A.cin[0] + 1ull;
     if (blockIdx.x == 0 && threadIdx.x == 0) A.cout[0] = step;
 
@@ -207,6 +291,13 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
 #pragma unroll
     for (int e = 0; e < kRlHead; e++)
         pj[e] = ent[e] >= 0 ? A.Pin[ent[e] & kRlSlotMask] : x;
+
+    // meanwhile: what the ring stage of wave 0 takes from memory and its noise
+    uint32_t hi0 = 0u;
+    if (wave == 0) {
+        hi0 = A.bmax[block];
+        if (lane < kRlWaves * A.per) s_ring[lane] = ring_scalars<BATCH>(P0, A, block, lane, step);
+    }
 
     // neighbours along the ring and the unwrap's steps, meanwhile
     const int me = (int)threadIdx.x, tb = me - i, wb = wave * 64;
@@ -237,7 +328,7 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
     }
     lds_sync();
     const double2 c = s_c[me], cn = s_c[tb + inext];
-    if (LAST && act) A.cpos[id] = c;
+    if (LAST && act) A.cpos[B.cpos + id] = c;
     s_t[me] = c.x * cn.y - c.y * cn.x;
     lds_sync();
     if (lane < 3 * per) {
@@ -262,7 +353,7 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
         if (!__any(ent[e] >= 0)) continue;
         const double2 d = wave_diff(P, x, pj[e]);
         const double r2 = d.x * d.x + d.y * d.y;
-        const RingInter I = rl_inter(P, A, t, ent[e] >= 0 ? ent[e] : 0);
+        const RingInter I = rl_inter(P, mat, uni, t, ent[e] >= 0 ? ent[e] : 0);
         in[e] = ent[e] >= 0 && !(r2 > I.max2);
         if (in[e]) {
             const int j = ent[e] & kRlSlotMask;
@@ -275,7 +366,7 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
     if (__any(order || longer)) {
         const int ri = ko >> 16, ci = ko & 0xffff;
         if (longer) {
-            f[0] = rl_long_sum(P, A, q, t0, t1, t, x, ri, ci);
+            f[0] = rl_long_sum(P, A, mat, uni, q, t0, t1, t, x, ri, ci);
             f[1] = f[2] = f[3] = make_double2(0.0, 0.0);
         } else if (order) {
             unsigned long long k[kRlHead];
@@ -316,9 +407,10 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
     const double area = s_r[wave][min(grp, per - 1) * 3 + 2] / 2.0;
     if (ring_ok && i == 0) {
         const double *s = &s_r[wave][grp * 3];
-        A.cms[r] = A.cms_next[r];  // update_cms! reads the previous continuous positions
-        A.cms_next[r] = make_double2(s[0] / (double)np, s[1] / (double)np);
-        A.areas[r] = area;
+        const int g = B.ring + r;
+        A.cms[g] = A.cms_next[g];  // update_cms! reads the previous continuous positions
+        A.cms_next[g] = make_double2(s[0] / (double)np, s[1] / (double)np);
+        A.areas[g] = area;
     }
     double area0 = (double)np * T->lspring / T->p0;
     area0 = area0 * area0;
@@ -368,84 +460,104 @@ __global__ __launch_bounds__(kRlWG) void k_rl_step(SysParams P, RLArgs A) {
             uint32_t flag = 0;
             int32_t rn, cc;
             cell_rc(P, P.rows, P.cols, P.cl, P.ch, px, py, &flag, MAVI_FLAG_OUT_OF_BOX, &rn, &cc);
-            if (flag) atomicOr(A.flags, flag);
+            if (flag) atomicOr(A.flags + B.flag, flag);
             const int32_t kn = (rn << 16) | cc;
             if (kn != ko) {
                 A.key[q] = kn;
-                atomicSub(&A.ccnt[r0 * P.cols + c0], 1);
-                if (atomicAdd(&A.ccnt[rn * P.cols + cc], 1) + 1 > P.nc) atomicOr(A.status, kRlCapacity);
+                atomicSub(&A.ccnt[B.chunk + r0 * P.cols + c0], 1);
+                if (atomicAdd(&A.ccnt[B.chunk + rn * P.cols + cc], 1) + 1 > P.nc) atomicOr(A.status, kRlCapacity);
             }
         }
     }
-    // largest squared step since the block began (high word, rounded up; a
-    // non-finite step keeps the largest word)
-    uint32_t hi = l2 == l2 ? min((uint32_t)__double2hiint(l2) + 1u, 0x7ff00000u) : 0x7ff00000u;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
-    if (lane == 0) {
-        uint32_t *slot = A.bmax + block * 4 + wave;
-        if (hi > *slot) *slot = hi;
-    }
+
+    // largest squared step (high word, rounded up; a non-finite step gives the
+    // largest word)
+    const uint32_t hi =
+        wave_umax(l2 == l2 ? min((uint32_t)__double2hiint(l2) + 1u, 0x7ff00000u) : 0x7ff00000u);
+    if (lane == 63) s_max[wave] = hi;
 
     // ---- polarisations: one lane per ring of the workgroup
     __syncthreads();
     if (wave != 0) return;
-    for (int k = lane; k < 4 * per; k += 64) {
-        const int w = k / per, g = k - w * per;
-        const int rg = (block * 4 + w) * per + g;
-        if (rg >= P.nrings) break;
-        const RingType *R = A.types + (P.typed ? A.rtype[rg] : 0);
-        const double vcx = s_r[w][2 * g] / (double)R->np, vcy = s_r[w][2 * g + 1] / (double)R->np;
-        const double2 cs = A.polcs[rg];
+    if (lane == 0) {  // the largest since the block began
+        uint32_t m = hi0;
+#pragma unroll
+        for (int w = 0; w < kRlWaves; w++) m = max(m, s_max[w]);
+        if (m > hi0) A.bmax[block] = m;
+    }
+    for (int k = lane; k < kRlWaves * A.per; k += 64) {
+        const RingScalars R = k < 64 ? s_ring[k] : ring_scalars<BATCH>(P0, A, block, k, step);
+        if (R.np == 0) continue;  // no ring
+        const int w = k / A.per, g = k - w * A.per;
+        const double vcx = s_r[w][2 * g] / (double)R.np, vcy = s_r[w][2 * g + 1] / (double)R.np;
         const double speed = sqrt(vcx * vcx + vcy * vcy);
         double cr = 0.0;
         if (speed != 0.0) {
-            cr = (cs.x * vcy - cs.y * vcx) / speed;
+            cr = (R.cs * vcy - R.sn * vcx) / speed;
             if (fabs(cr) > 1.0) cr = cr > 0.0 ? 1.0 : -1.0;
         }
-        const double z = R->rot != 0.0 ? philox_normal(A.seed, step, (uint32_t)rg) : 0.0;
-        const double d_theta = 1.0 / R->relax * asin(cr) * P.dt + sqrt(2.0 * R->rot * P.dt) * z;
-        const double th = A.pol[rg] + d_theta;
+        const double d_theta = R.rate * asin(cr) * R.dt + R.noise;
+        const double th = R.pol + d_theta;
         double sn, cn2;
         sincos(th, &sn, &cn2);
-        A.pol[rg] = th;
-        A.polcs[rg] = make_double2(cn2, sn);
+        A.pol[R.rg] = th;
+        A.polcs[R.rg] = make_double2(cn2, sn);
     }
 }
 
 // The lists: one thread per particle, in cell order of the list grid (src[t]:
-// the slot at place t), over the 3x3 cells around its own.
-__global__ __launch_bounds__(256) void k_rl_build(SysParams G, SysParams P, const double2 *__restrict__ pos,
-                                                  const int32_t *__restrict__ ID, const int32_t *__restrict__ rtype,
-                                                  const RingType *__restrict__ types,
-                                                  const int32_t *__restrict__ src, const int32_t *__restrict__ scell,
-                                                  const int32_t *__restrict__ start, double rl2,
-                                                  int4 *__restrict__ head, int32_t *__restrict__ more,
-                                                  uint8_t *__restrict__ count, uint32_t *__restrict__ status) {
+// the slot at place t), over the 3x3 cells around its own.  A batch's places
+// lie in their replica's slot range (waves of one replica), greps holds the
+// list grids and radii.
+struct RLBuild {
+    const double2 *pos;
+    const int32_t *ID, *rtype;
+    const RingType *types;
+    const int32_t *src, *scell, *start;
+    int32_t nslots;
+    double rl2;
+    int4 *head;
+    int32_t *more;
+    uint8_t *count;
+    uint32_t *status;
+    const Replica *reps, *greps;
+    const int32_t *wave_rep;  // replica of 64 slots
+};
+template <bool BATCH>
+__global__ __launch_bounds__(256) void k_rl_build(SysParams G0, SysParams P0, RLBuild A) {
     const int t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= P.na) return;
-    const int q = src[t], c = scell[t];
-    const double2 x = pos[q];
-    const int id = ID[q], ring = id / P.nmax;
-    const int np = types[P.typed ? rtype[ring] : 0].np;
+    if (t >= A.nslots) return;
+    const int rep = BATCH ? uniform(A.wave_rep[t >> 6]) : 0;
+    const SysParams &P = BATCH ? A.reps[rep].P : P0;
+    const SysParams &G = BATCH ? A.greps[rep].P : G0;
+    const RLBase B = BATCH ? rl_base(A.reps[rep], rep) : RLBase{};
+    const double rl2 = BATCH ? A.greps[rep].list2 : A.rl2;
+    const int gbase = BATCH ? A.greps[rep].cbase : 0;
+    const int32_t *start = A.start + gbase;
+    const int q = A.src[t], c = A.scell[t] - gbase;
+    const int id = A.ID[q] - B.id;
+    if (id < 0) return;  // a padding slot
+    const double2 x = A.pos[q];
+    const int ring = id / P.nmax;
+    const int np = A.types[B.type + (P.typed ? A.rtype[B.ring + ring] : 0)].np;
     const int row = c / G.cols, col = c - row * G.cols;
     int32_t h[kRlHead] = {-1, -1, -1, -1};
     int n = 0;
     auto run = [&](int a, int b) {
         for (int u = a; u < b; u++) {
-            const int j = src[u];
+            const int j = A.src[u];
             if (j == q) continue;
-            const double2 d = cdiff(P, x, pos[j]);
+            const double2 d = cdiff(P, x, A.pos[j]);
             if (!(d.x * d.x + d.y * d.y <= rl2)) continue;
-            const int idj = ID[j], rj = idj / P.nmax;
+            const int idj = A.ID[j] - B.id, rj = idj / P.nmax;
             if (rj == ring) {
                 const int diff = abs(id - idj);
                 if (diff == 1 || diff == np - 1) continue;  // bonded neighbours do not interact
             }
-            const int32_t e = j | ((P.typed ? rtype[rj] : 0) << kRlSlotBits);
+            const int32_t e = j | ((P.typed ? A.rtype[B.ring + rj] : 0) << kRlSlotBits);
 #pragma unroll
             for (int s = 0; s < kRlHead; s++) h[s] = n == s ? e : h[s];
-            if (n >= kRlHead && n < kRlMax) more[(int64_t)(n - kRlHead) * P.na + q] = e;
+            if (n >= kRlHead && n < kRlMax) A.more[(int64_t)(n - kRlHead) * A.nslots + q] = e;
             n++;
         }
     };
@@ -461,36 +573,42 @@ __global__ __launch_bounds__(256) void k_rl_build(SysParams G, SysParams P, cons
         }
     }
     if (n > kRlMax) {
-        atomicOr(status, kRlOverflow);
+        atomicOr(A.status, kRlOverflow);
         n = kRlMax;
     }
-    head[q] = make_int4(h[0], h[1], h[2], h[3]);
-    count[q] = (uint8_t)n;
+    A.head[q] = make_int4(h[0], h[1], h[2], h[3]);
+    A.count[q] = (uint8_t)n;
 }
 
 // After a build: reference chunks and counts (capacity as the binning checks
 // it), the build positions, cos and sin of the polarisations.
-__global__ void k_rl_keys(SysParams P, const double2 *__restrict__ pos, int32_t *__restrict__ key,
-                          int32_t *__restrict__ ccnt, double2 *__restrict__ xb, const double *__restrict__ pol,
-                          double2 *__restrict__ polcs, uint32_t *__restrict__ flags) {
+template <bool BATCH>
+__global__ void k_rl_keys(SysParams P0, int32_t nslots, int32_t nrings, const Replica *__restrict__ reps,
+                          const int32_t *__restrict__ wave_rep, const double2 *__restrict__ pos,
+                          int32_t *__restrict__ key, int32_t *__restrict__ ccnt, double2 *__restrict__ xb,
+                          const double *__restrict__ pol, double2 *__restrict__ polcs, uint32_t *__restrict__ flags) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = s < P.na;
+    if (s < nrings) {
+        double sn, cs;
+        sincos(pol[s], &sn, &cs);
+        polcs[s] = make_double2(cs, sn);
+    }
+    if ((s & ~63) >= nslots) return;  // whole waves
+    const int rep = BATCH ? uniform(wave_rep[s >> 6]) : 0;
+    const SysParams &P = BATCH ? reps[rep].P : P0;
+    const RLBase B = BATCH ? rl_base(reps[rep], rep) : RLBase{};
+    const bool valid = s - B.slot < P.na;
     uint32_t flag = 0;
     int32_t r = 0, c = 0, k = -1;
     double2 p = make_double2(0.0, 0.0);
     if (valid) {
         p = pos[s];
         cell_rc(P, P.rows, P.cols, P.cl, P.ch, p.x, p.y, &flag, MAVI_FLAG_OUT_OF_BOX, &r, &c);
-        k = r * P.cols + c;
+        k = B.chunk + r * P.cols + c;
     }
     const int32_t rank = wave_arrival_rank(valid, k, ccnt);
     if (valid && rank + 1 > P.nc) flag |= MAVI_FLAG_OVERFLOW;
-    if (flag) atomicOr(flags, flag);
-    if (s < P.nrings) {
-        double sn, cs;
-        sincos(pol[s], &sn, &cs);
-        polcs[s] = make_double2(cs, sn);
-    }
+    if (flag) atomicOr(flags + B.flag, flag);
     if (!valid) return;
     key[s] = (r << 16) | c;
     xb[s] = p;
@@ -506,8 +624,8 @@ struct RLSnap {
 __global__ void k_rl_block_start(int32_t na, int32_t nrings, const double2 *__restrict__ pos,
                                  const double *__restrict__ pol, const double2 *__restrict__ cms,
                                  const double2 *__restrict__ cms_next, RLSnap S, uint32_t *__restrict__ bmax,
-                                 int32_t nbmax, unsigned long long *__restrict__ out, uint32_t *__restrict__ status,
-                                 const uint32_t *__restrict__ flags, const unsigned long long *__restrict__ counter,
+                                 int32_t nbmax, unsigned long long *__restrict__ out,
+                                 const uint32_t *__restrict__ flags, int32_t nflags, const unsigned long long *__restrict__ counter,
                                  unsigned long long *__restrict__ c0) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < na) S.pos[i] = pos[i];
@@ -517,8 +635,8 @@ __global__ void k_rl_block_start(int32_t na, int32_t nrings, const double2 *__re
         S.cms_next[i] = cms_next[i];
     }
     if (i < nbmax) bmax[i] = 0u;
+    if (i < nflags) S.flags[i] = flags[i];
     if (i == 0) {
-        *S.flags = *flags;
         out[0] = out[1] = 0ull;
         *c0 = *counter;
     }
@@ -528,7 +646,10 @@ __global__ void k_rl_block_start(int32_t na, int32_t nrings, const double2 *__re
 // squared displacement from the build, out[2] <- the status.  At most 64
 // workgroups, so the maxima of one word take few atomics.
 constexpr int kRlMeasureBlocks = 64;
-__global__ __launch_bounds__(1024) void k_rl_measure(SysParams P, const double2 *__restrict__ pos,
+template <bool BATCH>
+__global__ __launch_bounds__(1024) void k_rl_measure(SysParams P0, int32_t nslots, const Replica *__restrict__ reps,
+                                                     const int32_t *__restrict__ wave_rep,
+                                                     const double2 *__restrict__ pos,
                                                      const double2 *__restrict__ xb,
                                                      const uint32_t *__restrict__ bmax, int32_t nbmax,
                                                      const uint32_t *__restrict__ status,
@@ -536,8 +657,10 @@ __global__ __launch_bounds__(1024) void k_rl_measure(SysParams P, const double2 
     double d2 = 0.0;
     uint32_t hi = 0u;
     const int g = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-    for (int s = g; s < P.na; s += stride) {
-        const double2 d = cdiff(P, pos[s], xb[s]);
+    for (int s = g; s < nslots; s += stride) {
+        const Replica *Q = BATCH ? reps + uniform(wave_rep[s >> 6]) : nullptr;
+        if (BATCH && s - Q->pbase >= Q->P.na) continue;  // padding
+        const double2 d = cdiff(BATCH ? Q->P : P0, pos[s], xb[s]);
         const double v = d.x * d.x + d.y * d.y;
         d2 = v == v ? fmax(d2, v) : INFINITY;
     }
@@ -560,7 +683,7 @@ __global__ void k_rl_copy_counter(const unsigned long long *__restrict__ src, un
 
 __global__ void k_rl_restore(int32_t na, int32_t nrings, RLSnap S, double2 *__restrict__ pos, double *__restrict__ pol,
                              double2 *__restrict__ cms, double2 *__restrict__ cms_next, uint32_t *__restrict__ flags,
-                             uint32_t *__restrict__ status) {
+                             int32_t nflags, uint32_t *__restrict__ status) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < na) pos[i] = S.pos[i];
     if (i < nrings) {
@@ -568,68 +691,110 @@ __global__ void k_rl_restore(int32_t na, int32_t nrings, RLSnap S, double2 *__re
         cms[i] = S.cms[i];
         cms_next[i] = S.cms_next[i];
     }
-    if (i == 0) {
-        *flags = *S.flags;
-        *status = 0u;
-    }
+    if (i < nflags) flags[i] = S.flags[i];
+    if (i == 0) *status = 0u;
 }
 
-int rl_waves(const SysParams &P) {
-    const int per = 64 / P.nmax;
-    return nblk(nblk(P.nrings, per), 4) * 4;
-}
+int rl_blocks(const SysParams &P) { return nblk(nblk(P.nrings, 64 / P.nmax), kRlWaves); }
 
 RLSnap rl_snap(const RList &N) { return RLSnap{N.psnap, N.csnap, N.nsnap, N.polsnap, N.fsnap}; }
 
-hipError_t rl_step(mavi_sys *s, bool last, hipStream_t st) {
-    RList &N = *s->rl;
-    ProfScope ps(s, MAVI_PROF_RINGS, st);
+// What the block loop needs of a system alone or of a batch's rings replicas.
+struct RLSys {
+    mavi_ctx *ctx;
+    RList *N;
+    SysParams P;  // alone; a batch: unused
+    int32_t nslots, nrings, nflags;
+    double2 **Pc;
+    int *cur;
+    double *pol;
+    double2 *cms, *cms_next;
+    uint32_t *flags;
+    unsigned long long *counter;
+    const Replica *reps;       // batch: replica table, replica of 64 slots
+    const int32_t *wave_rep;
+    bool graphs;
+    mavi_sys *s;
+    BatchSub *b;
+};
+RLSys rl_env(mavi_sys *s) {
+    return RLSys{s->ctx, s->rl, s->P, s->P.na, s->P.nrings, 1, s->P_, &s->cur, s->pol, s->cms, s->cms_next, s->flags,
+                 s->counter, nullptr, nullptr, s->use_graphs && !s->prof, s, nullptr};
+}
+RLSys rl_env(BatchSub *b) {
+    return RLSys{b->ctx, b->rl, SysParams{}, (int32_t)b->nslots, (int32_t)b->nrings, (int32_t)b->reps.size(), b->P_,
+                 &b->cur, b->pol, b->cms, b->cms_next, b->flags, b->counter, b->d_reps, b->wave_rep,
+                 b->use_graphs && !b->prof, nullptr, b};
+}
+
+hipError_t rl_step(const RLSys &E, bool last, hipStream_t st) {
+    RList &N = *E.N;
+    const int c = *E.cur;
     RLArgs A{};
-    const int c = s->cur;
-    A.Pin = s->P_[c];
-    A.Pout = s->P_[1 - c];
-    A.F = s->F;
-    A.slot_of = s->P.na == s->P.n ? nullptr : s->slot_of;
+    A.Pin = E.Pc[c];
+    A.Pout = E.Pc[1 - c];
     A.head = (const int4 *)N.head;
     A.more = N.more;
     A.count = N.count;
     A.key = N.key;
     A.ccnt = N.ccnt;
-    A.pol = s->pol;
+    A.pol = E.pol;
     A.polcs = N.polcs;
-    A.areas = s->areas;
-    A.cms = s->cms;
-    A.cms_next = s->cms_next;
-    A.cpos = s->cpos;
-    A.rtype = s->rtype;
-    A.types = s->types;
-    A.inter = N.uniform ? nullptr : s->inter;
-    A.uni = s->host_inter[0];
+    A.cms = E.cms;
+    A.cms_next = E.cms_next;
     A.bmax = N.bmax;
-    A.flags = s->flags;
+    A.flags = E.flags;
     A.status = N.status;
-    A.seed = s->seed;
     A.cin = N.counter + N.ph;
     A.cout = N.counter + (1 - N.ph);
-    const dim3 grid(rl_waves(s->P) / 4);
-    if (last) hipLaunchKernelGGL(k_rl_step<true>, grid, dim3(kRlWG), 0, st, s->P, A);
-    else hipLaunchKernelGGL(k_rl_step<false>, grid, dim3(kRlWG), 0, st, s->P, A);
+    A.stride = E.nslots;
+    A.per = N.per;
+    const dim3 grid(N.nbmax);
+    if (mavi_sys *s = E.s) {
+        ProfScope ps(s, MAVI_PROF_RINGS, st);
+        A.F = s->F;
+        A.slot_of = s->P.na == s->P.n ? nullptr : s->slot_of;
+        A.areas = s->areas;
+        A.cpos = s->cpos;
+        A.rtype = s->rtype;
+        A.types = s->types;
+        A.inter = N.uniform ? nullptr : s->inter;
+        A.uni = s->host_inter[0];
+        A.seed = s->seed;
+        if (last) hipLaunchKernelGGL((k_rl_step<true, false>), grid, dim3(kRlWG), 0, st, s->P, A);
+        else hipLaunchKernelGGL((k_rl_step<false, false>), grid, dim3(kRlWG), 0, st, s->P, A);
+    } else {
+        BatchSub *b = E.b;
+        BatchProf ps(b, MAVI_PROF_RINGS, st);
+        A.F = b->F;
+        A.slot_of = N.uniform ? nullptr : b->slot_of;  // (of a batch: every replica's rings are full)
+        A.areas = b->areas;
+        A.cpos = b->cpos;
+        A.rtype = b->rtype;
+        A.types = b->types;
+        A.inter = b->inter;
+        A.reps = b->d_reps;
+        A.wave_rep = b->ring_wave_rep;
+        A.nwaves = b->nring_waves;
+        if (last) hipLaunchKernelGGL((k_rl_step<true, true>), grid, dim3(kRlWG), 0, st, SysParams{}, A);
+        else hipLaunchKernelGGL((k_rl_step<false, true>), grid, dim3(kRlWG), 0, st, SysParams{}, A);
+    }
     N.ph = 1 - N.ph;
-    s->cur = 1 - c;
+    *E.cur = 1 - c;
     return hipGetLastError();
 }
 
 // Eight steps from (copy, counter word) captured once.
-hipError_t rl_graph(mavi_sys *s, hipStream_t st, hipGraphExec_t *out) {
-    RList &N = *s->rl;
+hipError_t rl_graph(const RLSys &E, hipStream_t st, hipGraphExec_t *out) {
+    RList &N = *E.N;
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    const int c0 = s->cur, ph0 = N.ph;
+    const int c0 = *E.cur, ph0 = N.ph;
     hipError_t e1 = hipSuccess;
-    for (int k = 0; k < kRlGraphSteps && e1 == hipSuccess; k++) e1 = rl_step(s, false, st);
+    for (int k = 0; k < kRlGraphSteps && e1 == hipSuccess; k++) e1 = rl_step(E, false, st);
     e = hipStreamEndCapture(st, &g);
-    s->cur = c0;
+    *E.cur = c0;
     N.ph = ph0;
     if (e1 != hipSuccess) e = e1;
     if (e == hipSuccess) e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
@@ -638,34 +803,63 @@ hipError_t rl_graph(mavi_sys *s, hipStream_t st, hipGraphExec_t *out) {
 }
 
 // State in ring order (both copies' ids, slot_of the identity over active ids).
-hipError_t rl_ring_order(mavi_sys *s, hipStream_t st) {
-    RList &N = *s->rl;
+hipError_t rl_ring_order(const RLSys &E, hipStream_t st) {
+    RList &N = *E.N;
     if (N.ordered) return hipSuccess;
-    hipError_t e = mavi::launch_unpermute(s, false, false, st);
-    s->cur = 0;
-    if (e == hipSuccess) e = mavi::launch_iota_state(s, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(s->ID_[1], s->ID_[0], sizeof(int32_t) * (size_t)s->P.na, hipMemcpyDeviceToDevice, st);
-    s->sorted = false;
+    hipError_t e;
+    if (mavi_sys *s = E.s) {
+        e = mavi::launch_unpermute(s, false, false, st);
+        s->cur = 0;
+        if (e == hipSuccess) e = mavi::launch_iota_state(s, st);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(s->ID_[1], s->ID_[0], sizeof(int32_t) * (size_t)s->P.na, hipMemcpyDeviceToDevice, st);
+        s->sorted = false;
+    } else {
+        e = mavi::launch_batch_ring_order(E.b, st);
+    }
     N.ordered = e == hipSuccess;
     return e;
 }
 
-hipError_t rl_rebuild(mavi_sys *s, hipStream_t st) {
-    RList &N = *s->rl;
-    const SysParams &P = s->P;
-    hipError_t e = mavi::drop_keys(s, st);
-    if (e == hipSuccess) e = rl_ring_order(s, st);
-    if (e == hipSuccess) e = mavi::launch_cell_order(s, N.G, N.scan_ticket, N.scan_state, st);
+hipError_t rl_rebuild(const RLSys &E, hipStream_t st) {
+    RList &N = *E.N;
+    mavi_sys *s = E.s;
+    BatchSub *b = E.b;
+    hipError_t e = s ? mavi::drop_keys(s, st) : hipSuccess;
+    if (e == hipSuccess) e = rl_ring_order(E, st);
+    if (e == hipSuccess)
+        e = s ? mavi::launch_cell_order(s, N.G, N.scan_ticket, N.scan_state, st)
+              : mavi::launch_batch_cell_order(b, (const Replica *)N.greps, N.gcells, N.scan_ticket, N.scan_state, st);
     if (e != hipSuccess) return e;
-    ProfScope ps(s, MAVI_PROF_BIN, st);
-    const int c = s->cur;
-    hipLaunchKernelGGL(k_rl_build, dim3(nblk(P.na, 256)), dim3(256), 0, st, N.G, P, s->P_[c], s->ID_[c], s->rtype,
-                       s->types, s->src, s->scell, s->start, N.rl2, (int4 *)N.head, N.more, N.count, N.status);
+    const int c = *E.cur;
+    RLBuild A{};
+    A.pos = E.Pc[c];
+    A.ID = s ? s->ID_[c] : b->ID_[c];
+    A.rtype = s ? s->rtype : b->rtype;
+    A.types = s ? s->types : b->types;
+    A.src = s ? s->src : b->src;
+    A.scell = s ? s->scell : b->scell;
+    A.start = s ? s->start : b->start;
+    A.nslots = E.nslots;
+    A.rl2 = N.rl2;
+    A.head = (int4 *)N.head;
+    A.more = N.more;
+    A.count = N.count;
+    A.status = N.status;
+    A.reps = E.reps;
+    A.greps = (const Replica *)N.greps;
+    A.wave_rep = E.wave_rep;
+    const dim3 gb(nblk(E.nslots, 256)), gk(nblk(std::max(E.nslots, E.nrings), 256));
+    if (s) hipLaunchKernelGGL(k_rl_build<false>, gb, dim3(256), 0, st, N.G, s->P, A);
+    else hipLaunchKernelGGL(k_rl_build<true>, gb, dim3(256), 0, st, SysParams{}, SysParams{}, A);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = mavi::launch_fill_i32(N.ccnt, 0, P.ncell, st)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_rl_keys, dim3(nblk(std::max(P.na, P.nrings), 256)), dim3(256), 0, st, P, s->P_[c], N.key,
-                       N.ccnt, N.xb, s->pol, N.polcs, s->flags);
+    if ((e = mavi::launch_fill_i32(N.ccnt, 0, s ? s->P.ncell : b->ncells, st)) != hipSuccess) return e;
+    if (s)
+        hipLaunchKernelGGL(k_rl_keys<false>, gk, dim3(256), 0, st, s->P, E.nslots, E.nrings, nullptr, nullptr,
+                           E.Pc[c], N.key, N.ccnt, N.xb, E.pol, N.polcs, E.flags);
+    else
+        hipLaunchKernelGGL(k_rl_keys<true>, gk, dim3(256), 0, st, SysParams{}, E.nslots, E.nrings, E.reps, E.wave_rep,
+                           E.Pc[c], N.key, N.ccnt, N.xb, E.pol, N.polcs, E.flags);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     N.valid = true;
     N.d_start = 0.0;
@@ -685,147 +879,49 @@ int64_t rl_room(const RList &N) {
 
 constexpr int64_t kRlMinBlock = 6;  // shorter blocks cost more than the rebuild they put off
 
-}  // namespace
-
-namespace mavi {
-
-bool rl_eligible(const mavi_sys *s) {
-    const SysParams &P = s->P;
-    if (P.potential != MAVI_POT_RINGS || P.nwalls > 0 || !P.periodic || P.na <= 0 || P.nmax > 32) return false;
-    if (P.na > kRlSlotMask || P.ntypes > 32) return false;
-    if (P.cols < 3 || P.rows < 3 || P.rows > 32767 || P.cols > 65535) return false;
-    const double range = sqrt(s->list2);
-    if (!(range > 0.0) || !(range < INFINITY)) return false;
-    // every pair within range is in adjacent chunks at the binned positions
-    return P.cl >= range * (1.0 + 1e-12) && P.ch >= range * (1.0 + 1e-12);
-}
-
-// skin as a fraction of the range; false: the box holds fewer than three cells
-// of the list grid a side
-bool rl_set_skin(mavi_sys *s, double skin_frac) {
-    RList &N = *s->rl;
-    const SysParams &P = s->P;
-    const double range = sqrt(s->list2), skin = skin_frac * range;
-    const double rl = (range + skin) * (1.0 + 1e-9);
-    N.rl2 = rl * rl;
-    N.half_skin = 0.5 * skin * (1.0 - 1e-9);
-    SysParams G = P;
-    G.cols = P.cl >= rl ? P.cols : (int32_t)floor(P.L / rl);
-    G.rows = P.ch >= rl ? P.rows : (int32_t)floor(P.H / rl);
-    G.cl = P.L / (double)std::max(G.cols, 1);
-    G.ch = P.H / (double)std::max(G.rows, 1);
-    G.ncell = G.cols * G.rows;
-    G.nc = P.na;
-    N.G = G;
-    N.valid = false;
-    N.fits = G.cols >= 3 && G.rows >= 3;
-    return N.fits;
-}
-
-hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
-    s->rl = new RList();
-    RList &N = *s->rl;
-    rl_set_skin(s, kRlSkin);
-    const int64_t na = s->P.na, nr = s->P.nrings;
-    N.uniform = true;
-    for (const RingInter &I : s->host_inter) {
-        const RingInter &J = s->host_inter[0];
-        N.uniform = N.uniform && I.k_rep == J.k_rep && I.k_atr == J.k_atr && I.dist_eq == J.dist_eq &&
-                    I.dist_max == J.dist_max;
-    }
-    N.nbmax = rl_waves(s->P);
-    N.scan_words = (s->P.ncell + 1 + kScanTileMin - 1) / kScanTileMin + 1;
-    hipError_t e = dalloc(&N.head, 4 * na, st);
-    if (e == hipSuccess) e = dalloc(&N.more, (int64_t)(kRlMax - kRlHead) * na, st);
-    if (e == hipSuccess) e = dalloc(&N.count, na, st);
-    if (e == hipSuccess) e = dalloc(&N.key, na, st);
-    if (e == hipSuccess) e = dalloc(&N.ccnt, (int64_t)s->P.ncell, st);
-    if (e == hipSuccess) e = dalloc(&N.xb, na, st);
-    if (e == hipSuccess) e = dalloc(&N.psnap, na, st);
-    if (e == hipSuccess) e = dalloc(&N.csnap, nr, st);
-    if (e == hipSuccess) e = dalloc(&N.nsnap, nr, st);
-    if (e == hipSuccess) e = dalloc(&N.polsnap, nr, st);
-    if (e == hipSuccess) e = dalloc(&N.fsnap, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.polcs, nr, st);
-    if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
-    if (e == hipSuccess) e = dalloc(&N.status, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.counter, 2, st);
-    if (e == hipSuccess) e = dalloc(&N.out, 3, st);
-    if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.scan_state, N.scan_words, st);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&N.host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
-    return e;
-}
-
-void rl_drop_graph(mavi_sys *s) {
-    if (!s->rl) return;
-    for (auto &row : s->rl->graph)
-        for (auto &g : row) {
-            if (!g) continue;
-            (void)hipStreamSynchronize(s->ctx->stream);
-            (void)hipGraphExecDestroy(g);
-            g = nullptr;
-        }
-}
-
-void rl_free(mavi_sys *s) {
-    if (!s->rl) return;
-    RList &N = *s->rl;
-    rl_drop_graph(s);
-    dfree(N.head); dfree(N.more); dfree(N.count); dfree(N.key); dfree(N.ccnt); dfree(N.xb); dfree(N.psnap);
-    dfree(N.csnap); dfree(N.nsnap); dfree(N.polsnap); dfree(N.fsnap); dfree(N.polcs); dfree(N.bmax); dfree(N.status);
-    dfree(N.counter); dfree(N.out); dfree(N.scan_ticket); dfree(N.scan_state);
-    if (N.host) (void)hipHostFree(N.host);
-    delete s->rl;
-    s->rl = nullptr;
-}
-
-bool rl_active(const mavi_sys *s) {
-    return s->rl && s->rl->on && s->rl->fits && !s->rl->disabled && !s->neigh_on && !s->var;
-}
-
-int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
-    mavi_ctx *ctx = s->ctx;
+// Blocks of steps with one read back each (see the top); *left > 0: the chunk
+// gather runs the rest.
+int rl_run(const RLSys &E, int64_t nsteps, int64_t *left) {
+    mavi_ctx *ctx = E.ctx;
     hipStream_t st = ctx->stream;
-    RList &N = *s->rl;
-    const SysParams &P = s->P;
+    RList &N = *E.N;
     *left = 0;
-    const int span = std::max(std::max(P.na, P.nrings), N.nbmax);
+    const int span = std::max(std::max(E.nslots, E.nrings), std::max(N.nbmax, E.nflags));
     int64_t k = 0;
     while (k < nsteps) {
         const bool fresh = !N.valid;
-        if (fresh) HIPCHK(ctx, rl_rebuild(s, st));
+        if (fresh) HIPCHK(ctx, rl_rebuild(E, st));
         int64_t want = N.block_now;
         if (N.block == 0) {
             if (rl_step_est(N) > 0.0) want = std::min(want, std::max<int64_t>(1, rl_room(N)));
             else want = std::min<int64_t>(want, 8);  // no step length measured yet
         }
         const int64_t blk = std::min<int64_t>(want, nsteps - k);
-        const int cur0 = s->cur;
+        const int cur0 = *E.cur;
         N.ph = 0;
-        hipLaunchKernelGGL(k_rl_block_start, dim3(nblk(span, 256)), dim3(256), 0, st, P.na, P.nrings, s->P_[s->cur],
-                           s->pol, s->cms, s->cms_next, rl_snap(N), N.bmax, N.nbmax, N.out, N.status, s->flags,
-                           s->counter, N.counter);
+        hipLaunchKernelGGL(k_rl_block_start, dim3(nblk(span, 256)), dim3(256), 0, st, E.nslots, E.nrings, E.Pc[cur0],
+                           E.pol, E.cms, E.cms_next, rl_snap(N), N.bmax, N.nbmax, N.out, E.flags, E.nflags, E.counter,
+                           N.counter);
         HIPCHK(ctx, hipGetLastError());
-        const bool graphs = s->use_graphs && !s->prof;
         const bool ends = k + blk == nsteps;  // the block's last step leaves the call's outputs
         const int64_t plain = ends ? blk - 1 : blk;
         int64_t done = 0;
         while (done < plain) {
-            if (graphs && done + kRlGraphSteps <= plain) {
-                hipGraphExec_t &g = N.graph[s->cur][N.ph];
-                if (!g) HIPCHK(ctx, rl_graph(s, st, &g));
+            if (E.graphs && done + kRlGraphSteps <= plain) {
+                hipGraphExec_t &g = N.graph[*E.cur][N.ph];
+                if (!g) HIPCHK(ctx, rl_graph(E, st, &g));
                 HIPCHK(ctx, hipGraphLaunch(g, st));
                 done += kRlGraphSteps;  // an even number: the copies and the counter words are where they were
             } else {
-                HIPCHK(ctx, rl_step(s, false, st));
+                HIPCHK(ctx, rl_step(E, false, st));
                 done++;
             }
         }
-        if (ends) HIPCHK(ctx, rl_step(s, true, st));
-        const int mb = std::min(nblk(std::max(P.na, N.nbmax), 1024), kRlMeasureBlocks);
-        hipLaunchKernelGGL(k_rl_measure, dim3(mb), dim3(1024), 0, st, P, s->P_[s->cur], N.xb, N.bmax, N.nbmax,
-                           N.status, N.out);
+        if (ends) HIPCHK(ctx, rl_step(E, true, st));
+        const int mb = std::min(nblk(std::max(E.nslots, N.nbmax), 1024), kRlMeasureBlocks);
+        auto measure = E.reps ? &k_rl_measure<true> : &k_rl_measure<false>;
+        hipLaunchKernelGGL(measure, dim3(mb), dim3(1024), 0, st, E.P, E.nslots, E.reps, E.wave_rep, E.Pc[*E.cur], N.xb,
+                           N.bmax, N.nbmax, N.status, N.out);
         HIPCHK(ctx, hipGetLastError());
         HIPCHK(ctx, hipMemcpyAsync(N.host, N.out, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
         HIPCHK(ctx, hipStreamSynchronize(st));
@@ -840,9 +936,9 @@ int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
         const bool finite = std::isfinite(step) && std::isfinite(d_end);
         const double bound = std::min(N.d_start + (T - 1.0) * step, 0.5 * (N.d_start + d_end + T * step));
         if (status || !finite || !(bound <= N.half_skin)) {
-            s->cur = cur0;
-            hipLaunchKernelGGL(k_rl_restore, dim3(nblk(span, 256)), dim3(256), 0, st, P.na, P.nrings, rl_snap(N),
-                               s->P_[s->cur], s->pol, s->cms, s->cms_next, s->flags, N.status);
+            *E.cur = cur0;
+            hipLaunchKernelGGL(k_rl_restore, dim3(nblk(span, 256)), dim3(256), 0, st, E.nslots, E.nrings, rl_snap(N),
+                               E.Pc[cur0], E.pol, E.cms, E.cms_next, E.flags, E.nflags, N.status);
             HIPCHK(ctx, hipGetLastError());
             N.valid = false;
             N.rollbacks++;
@@ -859,7 +955,7 @@ int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
             if (N.block != 0 && N.block_now > 1) N.block_now = std::max(1, N.block_now / 2);
             continue;
         }
-        hipLaunchKernelGGL(k_rl_copy_counter, dim3(1), dim3(64), 0, st, N.counter + N.ph, s->counter);
+        hipLaunchKernelGGL(k_rl_copy_counter, dim3(1), dim3(64), 0, st, N.counter + N.ph, E.counter);
         HIPCHK(ctx, hipGetLastError());
         k += blk;
         N.d_start = d_end;
@@ -876,8 +972,177 @@ int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
         const int32_t cap = N.block == 0 ? kNlBlockCap : N.block;
         if (N.block_now < cap) N.block_now = std::min(cap, 2 * N.block_now);
     }
-    s->sorted = false;  // not in chunk order
     return MAVI_OK;
 }
+
+}  // namespace
+
+namespace mavi {
+
+// Whether a rings system can run on lists.
+static bool rl_fits(const SysParams &P, double list2) {
+    if (P.potential != MAVI_POT_RINGS || P.nwalls > 0 || !P.periodic || P.na <= 0 || P.nmax > 32) return false;
+    if (P.na > kRlSlotMask || P.ntypes > 32) return false;
+    if (P.cols < 3 || P.rows < 3 || P.rows > 32767 || P.cols > 65535) return false;
+    const double range = sqrt(list2);
+    if (!(range > 0.0) || !(range < INFINITY)) return false;
+    // every pair within range is in adjacent chunks at the binned positions
+    return P.cl >= range * (1.0 + 1e-12) && P.ch >= range * (1.0 + 1e-12);
+}
+
+// The list grid: cells at least range + skin wide.  false: the box holds fewer
+// than three a side.
+static bool rl_grid(const SysParams &P, double range, double skin_frac, SysParams &G, double &rl2, double &half_skin) {
+    const double skin = skin_frac * range;
+    const double rl = (range + skin) * (1.0 + 1e-9);
+    rl2 = rl * rl;
+    half_skin = 0.5 * skin * (1.0 - 1e-9);
+    G = P;
+    G.cols = P.cl >= rl ? P.cols : (int32_t)floor(P.L / rl);
+    G.rows = P.ch >= rl ? P.rows : (int32_t)floor(P.H / rl);
+    G.cl = P.L / (double)std::max(G.cols, 1);
+    G.ch = P.H / (double)std::max(G.rows, 1);
+    G.ncell = G.cols * G.rows;
+    G.nc = P.na;
+    return G.cols >= 3 && G.rows >= 3;
+}
+
+bool rl_eligible(const mavi_sys *s) { return rl_fits(s->P, s->list2); }
+
+// skin as a fraction of the range
+bool rl_set_skin(mavi_sys *s, double skin_frac) {
+    RList &N = *s->rl;
+    N.fits = rl_grid(s->P, sqrt(s->list2), skin_frac, N.G, N.rl2, N.half_skin);
+    N.valid = false;
+    return N.fits;
+}
+
+static hipError_t rl_buffers(RList &N, int64_t nslots, int64_t nrings, int64_t ncells, int64_t nflags,
+                             hipStream_t st) {
+    N.scan_words = (int32_t)((ncells + 1 + kScanTileMin - 1) / kScanTileMin) + 1;
+    hipError_t e = dalloc(&N.head, 4 * nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.more, (int64_t)(kRlMax - kRlHead) * nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.count, nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.key, nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.ccnt, ncells, st);
+    if (e == hipSuccess) e = dalloc(&N.xb, nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.psnap, nslots, st);
+    if (e == hipSuccess) e = dalloc(&N.csnap, nrings, st);
+    if (e == hipSuccess) e = dalloc(&N.nsnap, nrings, st);
+    if (e == hipSuccess) e = dalloc(&N.polsnap, nrings, st);
+    if (e == hipSuccess) e = dalloc(&N.fsnap, nflags, st);
+    if (e == hipSuccess) e = dalloc(&N.polcs, nrings, st);
+    if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
+    if (e == hipSuccess) e = dalloc(&N.status, 1, st);
+    if (e == hipSuccess) e = dalloc(&N.counter, 2, st);
+    if (e == hipSuccess) e = dalloc(&N.out, 3, st);
+    if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);
+    if (e == hipSuccess) e = dalloc(&N.scan_state, N.scan_words, st);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&N.host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
+    return e;
+}
+
+static bool rl_uniform(const RingInter *I, int n) {
+    for (int k = 1; k < n; k++)
+        if (I[k].k_rep != I[0].k_rep || I[k].k_atr != I[0].k_atr || I[k].dist_eq != I[0].dist_eq ||
+            I[k].dist_max != I[0].dist_max)
+            return false;
+    return true;
+}
+
+static void rl_drop_graphs(RList &N, hipStream_t st) {
+    for (auto &row : N.graph)
+        for (auto &g : row) {
+            if (!g) continue;
+            (void)hipStreamSynchronize(st);
+            (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
+}
+
+static void rl_release(RList *&rl, hipStream_t st) {
+    if (!rl) return;
+    RList &N = *rl;
+    rl_drop_graphs(N, st);
+    dfree(N.head); dfree(N.more); dfree(N.count); dfree(N.key); dfree(N.ccnt); dfree(N.xb); dfree(N.psnap);
+    dfree(N.csnap); dfree(N.nsnap); dfree(N.polsnap); dfree(N.fsnap); dfree(N.polcs); dfree(N.bmax); dfree(N.status);
+    dfree(N.counter); dfree(N.out); dfree(N.scan_ticket); dfree(N.scan_state);
+    if (N.greps) (void)hipFree(N.greps);
+    if (N.host) (void)hipHostFree(N.host);
+    delete rl;
+    rl = nullptr;
+}
+
+hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
+    s->rl = new RList();
+    RList &N = *s->rl;
+    rl_set_skin(s, kRlSkin);
+    N.uniform = rl_uniform(s->host_inter.data(), (int)s->host_inter.size());
+    N.per = 64 / s->P.nmax;
+    N.nbmax = rl_blocks(s->P);
+    return rl_buffers(N, s->P.na, s->P.nrings, s->P.ncell, 1, st);
+}
+
+void rl_drop_graph(mavi_sys *s) {
+    if (s->rl) rl_drop_graphs(*s->rl, s->ctx->stream);
+}
+
+void rl_free(mavi_sys *s) { rl_release(s->rl, s->ctx->stream); }
+
+void rlb_drop_graph(BatchSub *b) {
+    if (b->rl) rl_drop_graphs(*b->rl, b->ctx->stream);
+}
+
+void rlb_free(BatchSub *b) { rl_release(b->rl, b->ctx->stream); }
+
+// The lists of a batch's rings replicas: one block length and one displacement
+// bound for all (the smallest half skin), a list grid per replica.  No lists
+// if some replica is not eligible.
+hipError_t rlb_alloc(BatchSub *b, hipStream_t st) {
+    if (b->nslots > kRlSlotMask) return hipSuccess;
+    std::vector<Replica> g(b->reps);
+    int64_t gcells = 0;
+    double half = INFINITY;
+    bool full = true;
+    int per = 1;
+    for (Replica &Q : g) {
+        const double range = sqrt(Q.list2);
+        SysParams G = Q.P;
+        double rl2, hs;
+        if (!rl_fits(Q.P, Q.list2) || !rl_grid(Q.P, range, kRlSkin, G, rl2, hs)) return hipSuccess;
+        full = full && Q.P.na == Q.P.n;
+        per = std::max(per, 64 / Q.P.nmax);
+        half = std::min(half, hs);
+        Q.P = G;
+        Q.list2 = rl2;
+        Q.cbase = (int32_t)gcells;
+        gcells += G.ncell + 1;  // and its pad cell
+    }
+    b->rl = new RList();
+    RList &N = *b->rl;
+    N.half_skin = half;
+    N.per = per;
+    N.gcells = gcells;
+    N.fits = true;
+    N.uniform = full;
+    N.nbmax = nblk(b->nring_waves, kRlWaves);
+    hipError_t e = rl_buffers(N, b->nslots, b->nrings, b->ncells, (int64_t)b->reps.size(), st);
+    if (e == hipSuccess) e = hipMalloc(&N.greps, sizeof(Replica) * g.size());
+    if (e == hipSuccess) e = hipMemcpyAsync(N.greps, g.data(), sizeof(Replica) * g.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    return e;
+}
+
+bool rl_active(const mavi_sys *s) {
+    return s->rl && s->rl->on && s->rl->fits && !s->rl->disabled && !s->neigh_on && !s->var;
+}
+
+int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
+    const int rc = rl_run(rl_env(s), nsteps, left);
+    s->sorted = false;  // not in chunk order
+    return rc;
+}
+
+int rlb_steps(BatchSub *b, int64_t nsteps, int64_t *left) { return rl_run(rl_env(b), nsteps, left); }
 
 }  // namespace mavi

@@ -215,3 +215,38 @@ def test_batch_errors(gpu_ctx):
     state, space, cfg, ic = normal_case(True, n=40, cols=5, rows=4)
     with pytest.raises(mv.UnsupportedOnGPU):
         b2.add(state, space, cfg, ic)
+
+
+@pytest.mark.parametrize("names", [
+    ("normal", "smallest_rings", "largest_rings", "types", "mixture"),  # ring sizes and counts that share workgroups
+    ("normal", "smallest_rings", "normal_ragged"),  # every ring full: slots by place
+    ("types", "few_cells"),  # a box too small for lists: all through the chunk gather
+])
+def test_batch_rings_on_lists_bitexact(gpu_ctx, names):
+    """Rings replicas on Verlet lists beside plain ones (their steps overlap):
+    calls too short to build lists, with rebuilds, odd, after a replica's
+    state is replaced and with the noise counter moved, against each system
+    alone."""
+    from test_gpu_rlist import CASES
+
+    specs = [("lj_periodic_small_cut", "plain", next(s for s in replica_cases() if s[0] == "lj_periodic_small_cut")[2])]
+    specs += [(nm, "rings", CASES[nm]) for nm in names]
+    steps_list = [3, 61, 5, 260]
+    want = [single_run(kind, mk(), 50 + i, steps_list) for i, (_, kind, mk) in enumerate(specs)]
+    b = build_batch([(spec, spec[2](), 50 + i) for i, spec in enumerate(specs)], gpu_ctx)
+    for j, k in enumerate(steps_list):
+        say(f"[batch lists] {names}: {k} steps")
+        b.run(k)
+        for i, (name, _, _) in enumerate(specs):
+            pos, vel, pol = b.download(i)
+            assert_same(f"{name} after {sum(steps_list[:j + 1])} steps", (pos, vel, pol, b.get_forces(i)), want[i][j])
+    # replica 1 back to its start, all others go on: the replica's run repeats
+    # with the counter where it began
+    state = specs[1][2]()[0]
+    assert b.noise_counter() == sum(steps_list)
+    b.upload(1, state.pos.copy(), None, state.pol.copy())
+    b.set_noise_counter(0)
+    b.run(steps_list[0])
+    b.run(steps_list[1])
+    pos, vel, pol = b.download(1)
+    assert_same("replaced replica", (pos, vel, pol, b.get_forces(1)), want[1][1])
