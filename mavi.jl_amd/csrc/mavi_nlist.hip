@@ -81,6 +81,7 @@ struct NLArgs {
     double2 *Px_next;     // x_{n+2}
     uint32_t *flags;
     uint32_t *status;
+    int32_t small_grid;   // the chunks between the first and last column (row) span less than a pair can close
     int32_t reuse;        // 0: every particle sums its next first evaluation afresh
 };
 
@@ -110,9 +111,14 @@ __device__ __forceinline__ bool chunks_adjacent(const SysParams &P, int ri, int 
     return dr <= 1 && dc <= 1;
 }
 
+// The same of packed chunks without the periodic edges.
+__device__ __forceinline__ bool chunks_touch(int32_t ki, int32_t kj) {
+    const uint32_t d = (uint32_t)(kj - ki) + 0x10001u;  // (row difference + 1) << 16 | column difference + 1
+    return d < 0x30000u && (d & 0xffffu) < 3u;
+}
+
 // One pair.  A list pad is the particle itself (its offsets are 0 and the LJ
-// factor is masked), so it adds nothing.  STALE: with `test`, the pair counts
-// only when the step-start chunks are adjacent.
+// factor is masked), so it adds nothing.
 // Slots of a group's two entries packed in one word: 16-bit offsets from s
 // taken modulo na (periodic rows put partners about na slots away).
 __device__ __forceinline__ int wrap_slot(int j, int na) { return j < 0 ? j + na : (j >= na ? j - na : j); }
@@ -129,17 +135,15 @@ __device__ __forceinline__ int32_t slot_offset(int s, int j, int na) {
     return d;
 }
 
-template <int POT, bool WRAP, bool STALE>
+template <int POT, bool WRAP>
 __device__ __forceinline__ void nl_pair(const SysParams &P, const double2 pj, const int32_t j, const int s,
-                                        double xi, double yi, bool test, int ri, int ci,
-                                        const int32_t *__restrict__ kcur, PairAcc<POT> &acc) {
+                                        double xi, double yi, PairAcc<POT> &acc) {
     double dx = xi - pj.x, dy = yi - pj.y;
     if constexpr (WRAP) {
         dx = min_image(dx, P.L, P.halfL);
         dy = min_image(dy, P.H, P.halfH);
     }
-    bool take = j != s;
-    if constexpr (STALE) take = take && (!test || chunks_adjacent(P, ri, ci, kcur[wrap_slot(j, P.na)]));
+    const bool take = j != s;
     if constexpr (POT == POT_LJ) {
         const double f = lj_scale_masked(P, dx * dx + dy * dy, take);
         acc.fx = __builtin_fma(f, dx, acc.fx);
@@ -150,32 +154,33 @@ __device__ __forceinline__ void nl_pair(const SysParams &P, const double2 pj, co
     }
 }
 
+// A group's slots in an array with ghost copies.
+__device__ __forceinline__ void ghost_slots(int s, int2 c, int (&j)[4]) {
+    j[0] = s + (int32_t)(int16_t)(c.x & 0xffff);
+    j[1] = s + (c.x >> 16);
+    j[2] = s + (int32_t)(int16_t)(c.y & 0xffff);
+    j[3] = s + (c.y >> 16);
+}
+
 // The sum over one particle's list in list order (ascending partner id),
-// four entries per iteration; the next group is loaded one iteration ahead,
-// so the list and position loads of consecutive groups overlap.  WRAPIN: pin
-// holds drifted positions, taken through state_pos.  GHOST: pin holds
+// four entries per iteration; q is the first group, the next is loaded one
+// iteration ahead, so the list and position loads of consecutive groups overlap.  GHOST: pin holds
 // kGhost copies of the other end's positions on each side of the slots
 // (pin[j - na] = pin[j] for j >= na - kGhost, pin[j + na] = pin[j] for
 // j < kGhost), so a partner is read at s + offset without the wrap modulo na
 // (|offset| <= min(32768, na / 2)).
-template <int POT, bool WRAP, bool STALE, bool WRAPIN = false, bool GHOST = false>
+template <int POT, bool WRAP, bool GHOST>
 __device__ __forceinline__ void nl_sum(const SysParams &P, const double2 *__restrict__ pin,
-                                       const int2 *__restrict__ nbr, int s, int groups, double xi, double yi,
-                                       bool test, int ri, int ci, const int32_t *__restrict__ kcur,
-                                       PairAcc<POT> &acc) {
-    if (groups <= 0) return;
+                                       const int2 *__restrict__ nbr, int2 q, int s, int groups, double xi,
+                                       double yi, PairAcc<POT> &acc) {
     const int na = P.na;
     const double2 *pb = GHOST ? pin - kGhost : pin;  // indexed from 0 with kGhost added
-    int2 q = nbr[s];
     for (int g = 0; g < groups; g++) {
         const int2 c = q;
         if (g + 1 < groups) q = nbr[(g + 1) * na + s];
         int j[4];
         if constexpr (GHOST) {
-            j[0] = s + (int32_t)(int16_t)(c.x & 0xffff);
-            j[1] = s + (c.x >> 16);
-            j[2] = s + (int32_t)(int16_t)(c.y & 0xffff);
-            j[3] = s + (c.y >> 16);
+            ghost_slots(s, c, j);
         } else {
             j[0] = lo_slot(s, c.x, na);
             j[1] = hi_slot(s, c.x, na);
@@ -185,12 +190,94 @@ __device__ __forceinline__ void nl_sum(const SysParams &P, const double2 *__rest
         double2 p[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) p[e] = load_slot(pb, GHOST ? j[e] + kGhost : j[e]);
-        if constexpr (WRAPIN) {  // after all four loads are in flight
 #pragma unroll
-            for (int e = 0; e < 4; e++) p[e] = state_pos(P, p[e]);
+        for (int e = 0; e < 4; e++) nl_pair<POT, WRAP>(P, p[e], j[e], s, xi, yi, acc);
+    }
+}
+
+// Both sums of a wave with a marked particle in one walk of the lists: acc, the
+// second evaluation at the drifted positions (for the marked, `test`, only the
+// pairs of adjacent step-start chunks), and acc1, the next first evaluation:
+// every pair at the positions after walls!.  A pair's force is evaluated once
+// where the periodic wrap moves neither particle (the same differences, the
+// same bits) and twice in the groups where it moves one for some lane.
+template <int POT, bool WRAP>
+__device__ __forceinline__ void nl_sum_both(const SysParams &P, const double2 *__restrict__ pin,
+                                            const int2 *__restrict__ nbr, int2 q, int s, int groups, double2 pu,
+                                            double2 pw, bool test, int32_t ki, const int32_t *__restrict__ kcur,
+                                            bool small_grid, PairAcc<POT> &acc, PairAcc<POT> &acc1) {
+    const int na = P.na;
+    const double2 *pb = pin - kGhost;
+    const bool self = pu.x != pw.x || pu.y != pw.y;
+    // chunks adjacent across the periodic edges: of pairs near them, or in a grid
+    // that a pair in range could span the other way
+    const bool across = P.periodic && (WRAP || small_grid);
+    auto load = [&](const int (&j)[4], double2 (&p)[4], int32_t (&k)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            p[e] = load_slot(pb, j[e] + kGhost);
+            k[e] = test ? kcur[wrap_slot(j[e], na)] : 0;
+        }
+    };
+    auto add = [&](const int (&j)[4], const double2 (&p)[4], const int32_t (&k)[4]) {
+        bool twice = false;
+        if constexpr (WRAP) {
+            bool moved = self;
+#pragma unroll
+            for (int e = 0; e < 4; e++)  // as periodic_wrap tests it
+                moved = moved || (P.periodic && (fabs(p[e].x - (P.blx + P.halfL)) > P.halfL ||
+                                                 fabs(p[e].y - (P.bly + P.halfH)) > P.halfH));
+            twice = __any(moved);
+        }
+        bool adj[4];
+        bool apart = false;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            adj[e] = !test || chunks_touch(ki, k[e]);
+            apart = apart || !adj[e];
+        }
+        if (across && __any(apart)) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) adj[e] = adj[e] || chunks_adjacent(P, ki >> 16, ki & 0xffff, k[e]);
         }
 #pragma unroll
-        for (int e = 0; e < 4; e++) nl_pair<POT, WRAP, STALE>(P, p[e], j[e], s, xi, yi, test, ri, ci, kcur, acc);
+        for (int e = 0; e < 4; e++) {
+            double dx = pu.x - p[e].x, dy = pu.y - p[e].y;
+            if constexpr (WRAP) {
+                dx = min_image(dx, P.L, P.halfL);
+                dy = min_image(dy, P.H, P.halfH);
+            }
+            const bool take = j[e] != s;
+            double dx1 = dx, dy1 = dy;
+            if (WRAP && twice) {
+                const double2 w = state_pos(P, p[e]);
+                dx1 = min_image(pw.x - w.x, P.L, P.halfL);
+                dy1 = min_image(pw.y - w.y, P.H, P.halfH);
+            }
+            if constexpr (POT == POT_LJ) {
+                const double f = lj_scale_masked(P, dx * dx + dy * dy, take);
+                const double fa = adj[e] ? f : 0.0;
+                acc.fx = __builtin_fma(fa, dx, acc.fx);
+                acc.fy = __builtin_fma(fa, dy, acc.fy);
+                const double f1 = WRAP && twice ? lj_scale_masked(P, dx1 * dx1 + dy1 * dy1, take) : f;
+                acc1.fx = __builtin_fma(f1, dx1, acc1.fx);
+                acc1.fy = __builtin_fma(f1, dy1, acc1.fy);
+            } else {
+                RingCtx R{};
+                if (take && adj[e]) acc.add(P, R, dx, dy, true, 0);
+                if (take) acc1.add(P, R, dx1, dy1, true, 0);
+            }
+        }
+    };
+    for (int g = 0; g < groups; g++) {
+        const int2 c = q;
+        if (g + 1 < groups) q = nbr[(g + 1) * na + s];
+        int j[4];
+        double2 p[4];
+        int32_t k[4];
+        ghost_slots(s, c, j);
+        load(j, p, k);
+        add(j, p, k);
     }
 }
 
@@ -520,16 +607,20 @@ __global__ void k_nl_keys(SysParams P, const double2 *__restrict__ pos, int32_t 
 // The drift of one particle (update_verlet!, src/integration.jl:424) from
 // start position pi with velocity v and force f into pout, the reference
 // chunk of its final position (after walls!'s periodic wrap) into knew and,
-// if it differs from kold (the chunks the next second evaluation keeps), the
-// chunk counts and the marks in chg of the pairs that evaluation could treat
-// differently from the first evaluation after it: a list partner whose kold
-// chunk is not adjacent to this particle's (1) and then the particle (2);
-// all partners if the wrap moved the particle (the first evaluation sums the
-// wrapped positions).
-__device__ __forceinline__ double nl_drift(const SysParams &P, const NLArgs &A, int s, double2 pi, double2 v,
-                                           double fx, double fy, double2 *__restrict__ pout,
-                                           const int32_t *__restrict__ kold, int32_t *__restrict__ knew,
-                                           uint8_t *__restrict__ chg) {
+// if it differs from ko (the chunk the next second evaluation keeps), the
+// chunk counts.  A particle that changed chunk marks (nl_marks) the pairs that
+// evaluation could treat differently from the first evaluation after it: a list
+// partner whose kept chunk is not adjacent to this particle's (1) and then the
+// particle (2); all partners if the wrap moved the particle (the first
+// evaluation sums the wrapped positions).
+struct Drift {
+    double l2 = 0.0;  // squared step length
+    bool moved = false, wrapped = false;
+};
+__device__ __forceinline__ Drift nl_drift(const SysParams &P, const NLArgs &A, int s, double2 pi, double2 v,
+                                          double fx, double fy, double2 *__restrict__ pout, int32_t ko,
+                                          int32_t *__restrict__ knew) {
+    Drift D;
     const double px = pi.x + (v.x * P.dt + fx * P.term), py = pi.y + (v.y * P.dt + fy * P.term);
     pout[s] = make_double2(px, py);
     // the copies the list sums read across the ends of the slot range
@@ -537,7 +628,6 @@ __device__ __forceinline__ double nl_drift(const SysParams &P, const NLArgs &A, 
     if (s >= P.na - kGhost) pout[s - P.na] = make_double2(px, py);
     double wx = px, wy = py;
     if (P.periodic) periodic_wrap(P, wx, wy);  // walls! moves it there after the kick
-    const int32_t ko = kold[s];
     // still clear inside its chunk (by far more than the rounding of the
     // chunk edges): the same chunk, without the exact division
     const int r0 = ko >> 16, c0 = ko & 0xffff;
@@ -553,24 +643,9 @@ __device__ __forceinline__ double nl_drift(const SysParams &P, const NLArgs &A, 
         kn = pack_rc(r, c);
     }
     knew[s] = kn;
-    if (kn != ko) {
-        const bool wrapped = wx != px || wy != py;
-        bool any = false;
-        const int groups = (int)(((uint32_t)A.ncount[s] & ~kEdgeBit) + 3u) >> 2;
-        for (int g = 0; g < groups; g++) {
-            const int2 q = A.nbr[g * P.na + s];
-            const int j4[4] = {lo_slot(s, q.x, P.na), hi_slot(s, q.x, P.na), lo_slot(s, q.y, P.na),
-                               hi_slot(s, q.y, P.na)};
-            for (int e = 0; e < 4; e++) {
-                const int j = j4[e];
-                if (j == s) continue;  // list pad
-                if (wrapped || !chunks_adjacent(P, r0, c0, kold[j])) {
-                    mark(chg, j, 1u);
-                    any = true;
-                }
-            }
-        }
-        if (any) mark(chg, s, 2u);
+    D.moved = kn != ko;
+    D.wrapped = wx != px || wy != py;
+    if (D.moved) {
         atomicSub(&A.ccnt[r0 * P.cols + c0], 1);
         // while one step's moves are applied a count runs through values at
         // least as large as its final one
@@ -578,7 +653,33 @@ __device__ __forceinline__ double nl_drift(const SysParams &P, const NLArgs &A, 
             atomicOr(A.status, kStatusCapacity);
     }
     const double lx = px - pi.x, ly = py - pi.y;  // the step's length, squared
-    return lx * lx + ly * ly;
+    D.l2 = lx * lx + ly * ly;
+    return D;
+}
+
+// The marks of the wave's particles whose chunk changed in their drift
+// (`moved`, from chunk ko of kold), one particle after another, the wave's
+// lanes on the entries of its list.
+__device__ __forceinline__ void nl_marks(const SysParams &P, const NLArgs &A, int s, bool moved, bool wrapped,
+                                         int groups, int32_t ko, const int32_t *__restrict__ kold,
+                                         uint8_t *__restrict__ chg) {
+    static_assert(kNlMax <= 64, "a list entry per lane");
+    const int lane = (int)lane_id();
+    for (unsigned long long m = __ballot(moved); m; m &= m - 1) {
+        const int l = __ffsll(m) - 1;
+        const int sl = __builtin_amdgcn_readlane(s, l), k = __builtin_amdgcn_readlane(ko, l);
+        const bool all = __builtin_amdgcn_readlane((int)wrapped, l) != 0;
+        bool any = false;
+        if (lane < 4 * __builtin_amdgcn_readlane(groups, l)) {
+            const int16_t *row = (const int16_t *)(A.nbr + (int64_t)(lane >> 2) * P.na + sl);
+            const int j = wrap_slot(sl + row[lane & 3], P.na);
+            if (j != sl && (all || !chunks_adjacent(P, k >> 16, k & 0xffff, kold[j]))) {  // (not a list pad)
+                mark(chg, j, 1u);
+                any = true;
+            }
+        }
+        if (__any(any) && lane == 0) mark(chg, sl, 2u);
+    }
 }
 
 // max of v over the wave into slot[blockIdx.x] (kept across launches: the
@@ -586,9 +687,18 @@ __device__ __forceinline__ double nl_drift(const SysParams &P, const NLArgs &A, 
 // retires without waiting for the rest of its workgroup; squared lengths are
 // non-negative doubles, ordered as their bit patterns).
 __device__ __forceinline__ void block_max_into(double v, double *__restrict__ slot) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    if (lane_id() == 0)
+    // (DPP: row_shr 1, 2, 4, 8, row_bcast 15, 31; the maximum in lane 63)
+#define MAVI_DPP_FMAX(ctrl, rows)                                                                                \
+    v = fmax(v, __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, rows, 0xf, false),      \
+                                 __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, rows, 0xf, false)))
+    MAVI_DPP_FMAX(0x111, 0xf);
+    MAVI_DPP_FMAX(0x112, 0xf);
+    MAVI_DPP_FMAX(0x114, 0xf);
+    MAVI_DPP_FMAX(0x118, 0xf);
+    MAVI_DPP_FMAX(0x142, 0xa);
+    MAVI_DPP_FMAX(0x143, 0xc);
+#undef MAVI_DPP_FMAX
+    if (lane_id() == 63)
         atomicMax((unsigned long long *)&slot[blockIdx.x], (unsigned long long)__double_as_longlong(v));
 }
 
@@ -602,19 +712,23 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_start(SysParams P, NLArgs A) 
     const int sv = valid ? s : 0;
     const double2 pi = A.Pst[sv];
     const uint32_t m = valid ? (uint32_t)A.ncount[s] : 0u;
+    const int2 q0 = A.nbr[sv];
+    const int32_t k0 = A.kcur[sv];
+    const double2 v = A.V[sv];
     const int groups = (int)((m & ~kEdgeBit) + 3u) >> 2;
     PairAcc<POT> acc;
     if (__any((m & kEdgeBit) != 0u))
-        nl_sum<POT, true, false>(P, A.Pst, A.nbr, sv, groups, pi.x, pi.y, false, 0, 0, nullptr, acc);
+        nl_sum<POT, true, false>(P, A.Pst, A.nbr, q0, sv, groups, pi.x, pi.y, acc);
     else
-        nl_sum<POT, false, false>(P, A.Pst, A.nbr, sv, groups, pi.x, pi.y, false, 0, 0, nullptr, acc);
-    double l2 = 0.0;
+        nl_sum<POT, false, false>(P, A.Pst, A.nbr, q0, sv, groups, pi.x, pi.y, acc);
+    Drift dr;
     if (valid) {
         A.F[s] = make_double2(acc.fx, acc.fy);
         A.fk_on[s] = 0;
-        l2 = nl_drift(P, A, s, pi, A.V[s], acc.fx, acc.fy, A.Px, A.kcur, A.knext, A.chg);
+        dr = nl_drift(P, A, s, pi, v, acc.fx, acc.fy, A.Px, k0, A.knext);
     }
-    block_max_into(l2, A.bmax);
+    nl_marks(P, A, sv, dr.moved, dr.wrapped, groups, k0, A.kcur, A.chg);
+    block_max_into(dr.l2, A.bmax);
 }
 
 // Second evaluation at the drifted positions with the step-start chunks,
@@ -622,6 +736,20 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_start(SysParams P, NLArgs A) 
 // then the next step: its first evaluation (this one, or for the marked
 // particles every pair within range at the wrapped positions) and its drift.
 // Records the largest drift step.
+//
+// Bound: up to ~200k particles the longest wave, not the chip: its FP64
+// instructions with little beside it to fill the gaps (a plain wave takes ~10k
+// cycles, half of them in the sum).  About 2% of the waves hold a marked
+// particle, so every launch beyond a few thousand particles has one; with both
+// sums in one walk it takes 14k cycles (near a periodic edge 20k, where pairs
+// are evaluated twice) instead of 22k for two walks that test chunks and wrap
+// every position, and a particle that changed chunk has its list walked by the
+// whole wave instead of by its lane.  What the kick and the drift need is loaded
+// with the first positions.  us a step with the rebuilds, before -> after: 10k
+// particles 13.5 -> 10.2, 102k 19.1 -> 14.0, 200k 23.0 -> 17.8, 1M (bound by
+// issue and the L1's gathers) 48.8 -> 45.2.  More list groups or positions in
+// flight measured nothing (14.0 -> 14.4), more waves a SIMD by fewer registers
+// cost (14.0 -> 15.9).
 template <int POT>
 __global__ __launch_bounds__(kNeedBlock) void k_nl_second(SysParams P, NLArgs A) {
     const int s = xcd_block() * blockDim.x + threadIdx.x;
@@ -631,6 +759,11 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_second(SysParams P, NLArgs A)
     const double2 pw = state_pos(P, pu);
     const uint32_t c = valid ? A.chg[s] : 0u;
     const uint32_t m = valid ? (uint32_t)A.ncount[s] : 0u;
+    const int2 q0 = A.nbr[sv];
+    const int32_t k0 = A.knext[sv];
+    const double2 v = A.V[sv];
+    const double2 f = A.F[sv];
+    const uint32_t on = A.fk_on[sv];
     const int groups = (int)((m & ~kEdgeBit) + 3u) >> 2;
     const bool stale = c != 0u;
     const bool fresh = stale || !A.reuse;  // the next first evaluation is summed afresh
@@ -638,28 +771,17 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_second(SysParams P, NLArgs A)
     PairAcc<POT> acc, acc1;
     if (__any(fresh)) {
         const int32_t ki = A.kcur[sv];
-        const int ri = ki >> 16, ci = ki & 0xffff;
-        const int g1 = fresh ? groups : 0;
-        if (wrap) {
-            nl_sum<POT, true, true, false, true>(P, A.Px, A.nbr, sv, groups, pu.x, pu.y, stale, ri, ci, A.kcur, acc);
-            nl_sum<POT, true, false, true, true>(P, A.Px, A.nbr, sv, g1, pw.x, pw.y, false, 0, 0, nullptr, acc1);
-        } else {
-            nl_sum<POT, false, true, false, true>(P, A.Px, A.nbr, sv, groups, pu.x, pu.y, stale, ri, ci, A.kcur,
-                                                  acc);
-            nl_sum<POT, false, false, true, true>(P, A.Px, A.nbr, sv, g1, pw.x, pw.y, false, 0, 0, nullptr, acc1);
-        }
+        if (wrap) nl_sum_both<POT, true>(P, A.Px, A.nbr, q0, sv, groups, pu, pw, stale, ki, A.kcur, A.small_grid, acc, acc1);
+        else nl_sum_both<POT, false>(P, A.Px, A.nbr, q0, sv, groups, pu, pw, stale, ki, A.kcur, A.small_grid, acc, acc1);
     } else {
-        if (wrap)
-            nl_sum<POT, true, false, false, true>(P, A.Px, A.nbr, sv, groups, pu.x, pu.y, false, 0, 0, nullptr, acc);
-        else
-            nl_sum<POT, false, false, false, true>(P, A.Px, A.nbr, sv, groups, pu.x, pu.y, false, 0, 0, nullptr, acc);
+        if (wrap) nl_sum<POT, true, true>(P, A.Px, A.nbr, q0, sv, groups, pu.x, pu.y, acc);
+        else nl_sum<POT, false, true>(P, A.Px, A.nbr, q0, sv, groups, pu.x, pu.y, acc);
     }
-    double l2 = 0.0;
+    Drift dr;
     if (valid) {
         const double fx = acc.fx, fy = acc.fy;                     // this second evaluation
         const double gx = fresh ? acc1.fx : fx, gy = fresh ? acc1.fy : fy;  // the next first one
-        const double2 v = A.V[s];
-        const double2 fo = A.fk_on[s] ? A.Fk[s] : A.F[s];           // this step's first one
+        const double2 fo = on ? A.Fk[s] : f;                       // this step's first one
         // vel += dt/2 * (forces + old_forces) (src/integration.jl:430), then walls!
         double vx = v.x + P.hdt * (fx + fo.x);
         double vy = v.y + P.hdt * (fy + fo.y);
@@ -677,10 +799,11 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_second(SysParams P, NLArgs A)
         if (fresh) A.Fk[s] = make_double2(gx, gy);
         A.fk_on[s] = fresh ? 1 : 0;
         A.chg[s] = 0;
-        l2 = nl_drift(P, A, s, pw, make_double2(vx, vy), gx, gy, A.Px_next, A.knext, A.knn, A.chg_next);
+        dr = nl_drift(P, A, s, pw, make_double2(vx, vy), gx, gy, A.Px_next, k0, A.knn);
     }
+    nl_marks(P, A, sv, dr.moved, dr.wrapped, groups, k0, A.knext, A.chg_next);
     // the largest step since the block began, per workgroup slot
-    block_max_into(l2, A.bmax);
+    block_max_into(dr.l2, A.bmax);
 }
 
 // out[0] <- max of bmax, out[1] <- max of dpend (the doubles' bits), out[2]
@@ -777,6 +900,9 @@ NLArgs nl_args(mavi_sys *s) {
     A.flags = s->flags;
     A.status = N.status;
     A.reuse = s->reuse ? 1 : 0;
+    // range + 2 skin: more than a pair can close between the build and any position
+    const double reach = sqrt(N.rl2) + 2.0 * sqrt(N.thr2);
+    A.small_grid = (s->P.cols - 2) * s->P.cl < reach || (s->P.rows - 2) * s->P.ch < reach;
     return A;
 }
 

@@ -234,3 +234,48 @@ def test_block_sized_by_stale_step_rolls_back(gpu_ctx, oracle_mod):
     p_ref, v_ref, _, _, _ = o.newton_steps(pos1, vel1, 100)
     ep, ev = traj_err(s.state.pos, s.state.vel, p_ref, v_ref, space.geometry_cfg.length)
     assert ep <= TRAJ_RTOL and ev <= TRAJ_RTOL
+
+
+@pytest.mark.parametrize("kind", ["lj", "ht"])
+@pytest.mark.parametrize("cols,rows,periodic", [(3, 3, True), (4, 3, True), (9, 11, True), (3, 4, False)])
+def test_marked_particles_one_walk(gpu_ctx, oracle_mod, cols, rows, periodic, kind):
+    """The second evaluation and the next first one of marked particles, summed
+    in one walk of the list: hot gases that change chunk and cross the periodic
+    edges in most steps, on the smallest chunk grids (chunks adjacent across
+    the box both ways), inside and near the edges.  Force reuse off sums every
+    particle both ways: the same bits; and the oracle."""
+    import mavi_hip as mv
+    from mavi_hip import _lib
+
+    rng = np.random.default_rng(17 * cols + rows)
+    L, H = 2.0 * cols, 2.0 * rows
+    nx, ny = int(1.3 * L), int(1.3 * H)
+    n = nx * ny
+    ix = np.arange(n)
+    pos = np.stack([(ix % nx + 0.5) * L / nx, (ix // nx + 0.5) * H / ny], axis=1) + 0.05 * rng.uniform(-1, 1, (n, 2))
+    vel = 6.0 * rng.normal(size=(n, 2))
+    if kind == "lj":
+        dyn = mv.LenJonesCfg(sigma=0.7, epsilon=0.5, cutoff=1.7)
+    else:
+        dyn = mv.HarmTruncCfg(k_rep=40.0, k_atr=3.0, dist_eq=0.8, dist_max=1.2)
+    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls() if periodic else mv.RigidWalls(),
+                        geometry_cfg=mv.RectangleCfg(length=L, height=H))
+    ic = mv.IntCfg(dt=1e-3, chunks_cfg=mv.ChunksCfg(num_cols=cols, num_rows=rows), device=mv.GPU())
+    runs = []
+    for reuse, block in ((1, 0), (0, 0), (1, 5)):
+        s = mv.System(state=mv.SecondLawState(pos=pos.copy(), vel=vel.copy()), space_cfg=space, dynamic_cfg=dyn,
+                      int_cfg=ic)
+        s.dev.set_option(_lib.MAVI_OPT_REUSE_FORCES, reuse)
+        s.dev.set_option(_lib.MAVI_OPT_NLIST_BLOCK, block)
+        s.advance(40)
+        s.download()
+        assert s.dev.nlist_info()["active"]
+        runs.append((s.state.pos.copy(), s.state.vel.copy(), s.forces.copy()))
+    for r in runs[1:]:
+        for a, b in zip(r, runs[0]):
+            assert np.array_equal(a, b)
+    o = oracle_mod.from_system(n, space, dyn, ic)
+    p_ref, v_ref, _, _, _ = o.newton_steps(pos, vel, 40)
+    ep, ev = traj_err(runs[0][0], runs[0][1], p_ref, v_ref, L, periodic=periodic)
+    say(f"[marked] {kind} {cols}x{rows} n={n} pos {ep:.2e} vel {ev:.2e}")
+    assert ep <= TRAJ_RTOL and ev <= TRAJ_RTOL
