@@ -295,6 +295,7 @@ struct mavi_batch {
     };
     std::vector<Where> where;  // of each replica
     std::vector<char> uploaded;
+    PinBuf pin;
     hipStream_t side = nullptr;  // the plain replicas' steps where both families are there
     hipEvent_t fork = nullptr, join = nullptr;
     // execution shape: plain, rings
@@ -785,6 +786,7 @@ int mavi_batch_destroy(mavi_batch *b) {
     (void)hipStreamSynchronize(b->ctx->stream);
     for (BatchSub *u : b->sub)
         if (u) sub_free(u);
+    if (b->pin.p) (void)hipHostFree(b->pin.p);
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
     if (b->side) (void)hipStreamDestroy(b->side);
@@ -859,6 +861,7 @@ int mavi_batch_finalize(mavi_batch *b) {
         if (!b->fork) HIPCHK(ctx, hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
         if (!b->join) HIPCHK(ctx, hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     }
+    for (const HostSys &h : b->hs) b->pin.fit(h.P.n);
     b->uploaded.assign(b->hs.size(), 0);
     b->hs.clear();
     b->hs.shrink_to_fit();
@@ -882,11 +885,11 @@ int mavi_batch_upload(mavi_batch *b, int32_t i, const double *pos, const double 
     BatchSub *u = b->sub[b->where[i].sub];
     const Replica &Q = u->reps[b->where[i].local];
     const size_t bytes = sizeof(double2) * (size_t)Q.P.n;
-    HIPCHK(ctx, hipMemcpyAsync(u->pos_id + Q.nbase, pos, bytes, hipMemcpyHostToDevice, st));
-    if (vel && Q.kind != KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(u->vel_id + Q.nbase, vel, bytes, hipMemcpyHostToDevice, st));
-    if (pol && Q.kind == KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(u->pol + Q.rbase, pol, sizeof(double) * Q.P.nrings, hipMemcpyHostToDevice, st));
+    const bool rings = Q.kind == KIND_RINGS;
+    HIPCHK(ctx, mavi::copy_in(ctx, b->pin,
+                              {{(void *)pos, u->pos_id + Q.nbase, bytes},
+                               {(void *)vel, u->vel_id + Q.nbase, vel && !rings ? bytes : 0},
+                               {(void *)pol, u->pol + Q.rbase, pol && rings ? sizeof(double) * Q.P.nrings : 0}}));
     HIPCHK(ctx, batch_stage_in(u, b->where[i].local, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
     b->uploaded[i] = 1;
@@ -899,16 +902,14 @@ int mavi_batch_download(mavi_batch *b, int32_t i, double *pos, double *vel, doub
     if (rc != MAVI_OK) return rc;
     mavi_ctx *ctx = b->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
     BatchSub *u = b->sub[b->where[i].sub];
     const Replica &Q = u->reps[b->where[i].local];
     const size_t bytes = sizeof(double2) * (size_t)Q.P.n;
-    if (pos) HIPCHK(ctx, hipMemcpyAsync(pos, u->pos_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
-    if (vel && Q.kind != KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(vel, u->vel_id + Q.nbase, bytes, hipMemcpyDeviceToHost, st));
-    if (pol && Q.kind == KIND_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(pol, u->pol + Q.rbase, sizeof(double) * Q.P.nrings, hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
+    const bool rings = Q.kind == KIND_RINGS;
+    HIPCHK(ctx, mavi::copy_out(ctx, b->pin,
+                               {{pos, u->pos_id + Q.nbase, pos ? bytes : 0},
+                                {vel, u->vel_id + Q.nbase, vel && !rings ? bytes : 0},
+                                {pol, u->pol + Q.rbase, pol && rings ? sizeof(double) * Q.P.nrings : 0}}));
     return MAVI_OK;
 }
 
@@ -920,9 +921,7 @@ int mavi_batch_get_forces(mavi_batch *b, int32_t i, double *forces) {
     HIPCHK(ctx, hipSetDevice(ctx->device));
     const BatchSub *u = b->sub[b->where[i].sub];
     const Replica &Q = u->reps[b->where[i].local];
-    HIPCHK(ctx, hipMemcpyAsync(forces, u->force_id + Q.nbase, sizeof(double2) * (size_t)Q.P.n,
-                               hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    HIPCHK(ctx, mavi::copy_out(ctx, b->pin, {{forces, u->force_id + Q.nbase, sizeof(double2) * (size_t)Q.P.n}}));
     return MAVI_OK;
 }
 

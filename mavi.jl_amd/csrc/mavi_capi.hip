@@ -22,8 +22,7 @@ bool is_active(const mavi_sys *s) {
 int check_flags(mavi_sys *s) {
     mavi_ctx *ctx = s->ctx;
     uint32_t h = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&h, s->flags, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    HIPCHK(ctx, mavi::copy_out(ctx, s->pin, {{&h, s->flags, sizeof(uint32_t)}}));
     if (h == 0) return MAVI_OK;
     HIPCHK(ctx, hipMemsetAsync(s->flags, 0, sizeof(uint32_t), ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -158,6 +157,7 @@ static void sys_free(mavi_sys *s) {
     dfree(s->rmask); dfree(s->dsinks); dfree(s->dboxes); dfree(s->box_mask);
     if (s->vrb) (void)hipFree(s->vrb);
     if (s->vstage) (void)hipHostFree(s->vstage);
+    if (s->pin.p) (void)hipHostFree(s->pin.p);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     mavi_ctx *ctx = s->ctx;
@@ -386,6 +386,7 @@ int mavi_sys_create(mavi_ctx *ctx, const mavi_sys_desc *d, mavi_sys **out) {
     mavi_sys *s = new mavi_sys();
     s->ctx = ctx;
     s->P = h.P;
+    s->pin.fit(h.P.n);
     s->list2 = h.list2;
     SysParams &P = s->P;
     std::vector<int32_t> &active = h.active;
@@ -487,22 +488,18 @@ int mavi_sys_upload(mavi_sys *s, const double *pos, const double *vel, const dou
     if (!s || !pos) return MAVI_E_BADARG;
     mavi_ctx *ctx = s->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    const size_t bytes = sizeof(double2) * (size_t)s->P.n;
-    HIPCHK(ctx, hipMemcpyAsync(s->pos_id, pos, bytes, hipMemcpyHostToDevice, ctx->stream));
-    if (is_active(s)) {
+    const size_t n = (size_t)s->P.n, bytes = sizeof(double2) * n;
+    const bool rings = s->P.potential == MAVI_POT_RINGS, active = is_active(s);
+    HIPCHK(ctx, mavi::copy_in(ctx, s->pin,
+                              {{(void *)pos, s->pos_id, bytes},
+                               {(void *)vel, s->vel_id, vel && s->vel_id && !active ? bytes : 0},
+                               {(void *)pol, active ? s->ang_id : s->pol,
+                                pol ? sizeof(double) * (active ? n : rings ? (size_t)s->P.nrings : 0) : 0}}));
+    if (active) {
         // pol_angle (n) -> the x components of the velocity staging
-        if (pol) {
-            HIPCHK(ctx, hipMemcpyAsync(s->ang_id, pol, sizeof(double) * (size_t)s->P.n, hipMemcpyHostToDevice,
-                                       ctx->stream));
-            HIPCHK(ctx, mavi::launch_spread_angles(s, ctx->stream));
-        } else {
-            HIPCHK(ctx, hipMemsetAsync(s->vel_id, 0, bytes, ctx->stream));
-        }
-    } else if (vel && s->vel_id) {
-        HIPCHK(ctx, hipMemcpyAsync(s->vel_id, vel, bytes, hipMemcpyHostToDevice, ctx->stream));
+        if (pol) HIPCHK(ctx, mavi::launch_spread_angles(s, ctx->stream));
+        else HIPCHK(ctx, hipMemsetAsync(s->vel_id, 0, bytes, ctx->stream));
     }
-    if (pol && s->P.potential == MAVI_POT_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(s->pol, pol, sizeof(double) * s->P.nrings, hipMemcpyHostToDevice, ctx->stream));
     s->cur = 0;
     if (s->nl) s->nl->valid = false;  // a new state in id order
     mavi::rl_invalidate(s);
@@ -528,20 +525,14 @@ int mavi_sys_download(mavi_sys *s, double *pos, double *vel, double *pol) {
     if (!s) return MAVI_E_BADARG;
     mavi_ctx *ctx = s->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    const size_t bytes = sizeof(double2) * (size_t)s->P.n;
-    if (pos) HIPCHK(ctx, hipMemcpyAsync(pos, s->pos_id, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    if (is_active(s)) {
-        if (pol) {
-            HIPCHK(ctx, mavi::launch_pack_angles(s, ctx->stream));
-            HIPCHK(ctx, hipMemcpyAsync(pol, s->ang_id, sizeof(double) * (size_t)s->P.n, hipMemcpyDeviceToHost,
-                                       ctx->stream));
-        }
-    } else if (vel && s->vel_id) {
-        HIPCHK(ctx, hipMemcpyAsync(vel, s->vel_id, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    }
-    if (pol && s->P.potential == MAVI_POT_RINGS)
-        HIPCHK(ctx, hipMemcpyAsync(pol, s->pol, sizeof(double) * s->P.nrings, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    const size_t n = (size_t)s->P.n, bytes = sizeof(double2) * n;
+    const bool rings = s->P.potential == MAVI_POT_RINGS, active = is_active(s);
+    if (active && pol) HIPCHK(ctx, mavi::launch_pack_angles(s, ctx->stream));
+    HIPCHK(ctx, mavi::copy_out(ctx, s->pin,
+                               {{pos, s->pos_id, pos ? bytes : 0},
+                                {vel, s->vel_id, vel && s->vel_id && !active ? bytes : 0},
+                                {pol, active ? s->ang_id : s->pol,
+                                 pol ? sizeof(double) * (active ? n : rings ? (size_t)s->P.nrings : 0) : 0}}));
     return MAVI_OK;
 }
 
@@ -591,7 +582,7 @@ int mavi_forces(mavi_sys *s, double *forces) {
     if (st == MAVI_OK) st = check_flags(s);
     if (st != MAVI_OK) return st;
     if (forces)
-        HIPCHK(ctx, hipMemcpy(forces, s->force_id, sizeof(double2) * (size_t)s->P.n, hipMemcpyDeviceToHost));
+        HIPCHK(ctx, mavi::copy_out(ctx, s->pin, {{forces, s->force_id, sizeof(double2) * (size_t)s->P.n}}));
     return MAVI_OK;
 }
 
@@ -599,8 +590,7 @@ int mavi_get_forces(mavi_sys *s, double *forces) {
     if (!s || !forces) return MAVI_E_BADARG;
     mavi_ctx *ctx = s->ctx;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    HIPCHK(ctx, hipMemcpy(forces, s->force_id, sizeof(double2) * (size_t)s->P.n, hipMemcpyDeviceToHost));
+    HIPCHK(ctx, mavi::copy_out(ctx, s->pin, {{forces, s->force_id, sizeof(double2) * (size_t)s->P.n}}));
     return MAVI_OK;
 }
 
@@ -930,7 +920,6 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
             }
         }
         HIPCHK(ctx, mavi::nl_measure(s, st));
-        HIPCHK(ctx, hipMemcpyAsync(N.host, N.dmax, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
         HIPCHK(ctx, hipStreamSynchronize(st));
         const double step = sqrt(__builtin_bit_cast(double, N.host[0]));
         const double d_end = sqrt(__builtin_bit_cast(double, N.host[1]));
@@ -1424,11 +1413,10 @@ int mavi_rings_info(mavi_sys *s, double *areas, double *cms, double *continuous_
     mavi_ctx *ctx = s->ctx;
     if (s->P.potential != MAVI_POT_RINGS) return set_err(ctx, MAVI_E_BADARG, "not a rings system");
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (areas) HIPCHK(ctx, hipMemcpy(areas, s->areas, sizeof(double) * s->P.nrings, hipMemcpyDeviceToHost));
-    if (cms) HIPCHK(ctx, hipMemcpy(cms, s->cms, sizeof(double2) * s->P.nrings, hipMemcpyDeviceToHost));
-    if (continuous_pos)
-        HIPCHK(ctx, hipMemcpy(continuous_pos, s->cpos, sizeof(double2) * s->P.n, hipMemcpyDeviceToHost));
+    HIPCHK(ctx, mavi::copy_out(ctx, s->pin,
+                               {{areas, s->areas, areas ? sizeof(double) * s->P.nrings : 0},
+                                {cms, s->cms, cms ? sizeof(double2) * s->P.nrings : 0},
+                                {continuous_pos, s->cpos, continuous_pos ? sizeof(double2) * s->P.n : 0}}));
     return MAVI_OK;
 }
 

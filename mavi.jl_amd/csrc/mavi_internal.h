@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -200,14 +201,13 @@ struct NList {
     double2 *xb = nullptr;    // positions at build
     double2 *vsnap = nullptr;  // block-start velocities (rollback; positions are written after the check)
     uint32_t *fsnap = nullptr;
-    unsigned long long *dmax = nullptr;  // reduced per block (bits): [0] largest drift step^2, [1] largest pending displacement^2, [2] status
     double *bmax = nullptr;              // per workgroup of the evaluations: largest drift step^2 since the block began
     double *dpend = nullptr;             // per workgroup: largest displacement^2 of the pending positions (block end)
     int32_t nbmax = 0;
     uint32_t *status = nullptr;          // bit 0: a list overflowed kmax; bit 1: a chunk count may have passed the capacity
     unsigned long long *scan_ticket = nullptr, *scan_state = nullptr;  // the list grid's scan (cleared per build)
     int32_t scan_words = 0;
-    unsigned long long *host = nullptr;  // pinned read back: dmax[0..1], status
+    unsigned long long *host = nullptr;  // pinned, per block (bits): [0] largest drift step^2, [1] largest pending displacement^2, [2] status
     double d_start = 0.0;     // largest displacement from the build of the next block's first positions
     int64_t rebuilds = 0, rollbacks = 0;
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // six steps from ph = 0 on state copy 0 / 1 (a rebuild's sort flips it)
@@ -258,7 +258,28 @@ struct RList {
     hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [state copy][counter word]
 };
 
+// Transfers of up to kPinBytes go through a pinned buffer of the system's (or
+// batch's) own and one kernel, larger ones by a copy each: a copy from or to
+// pageable memory costs over 10 us however small.  1k particles: download 44 -> 21
+// us, the flags word after a step 15 us less; at 256 KiB the copy through the
+// buffer takes about what it saves.
+constexpr size_t kPinBytes = 256 * 1024;
+struct PinBuf {
+    void *p = nullptr;    // hipHostMalloc, at the first use
+    size_t bytes = 4096;  // its size
+    // room for the state of n particles, if that is small
+    void fit(int64_t n) {
+        const int64_t want = 40 * n + 4096;
+        if (want <= (int64_t)kPinBytes && want > (int64_t)bytes) bytes = (size_t)want;
+    }
+};
+struct Xfer {
+    void *host, *dev;
+    size_t bytes;  // a multiple of 4; 0: skipped
+};
+
 struct mavi_sys {
+    PinBuf pin;
     mavi_ctx *ctx = nullptr;
     int refs = 0;          // learned propagators bound to this system
     bool closing = false;  // destroyed while referenced: freed at the last release
@@ -426,7 +447,7 @@ hipError_t nl_rebuild(mavi_sys *s, hipStream_t st);
 hipError_t nl_step(mavi_sys *s, hipStream_t st);
 // block start: step maxima cleared (clear) and the flags word kept
 hipError_t nl_block_start(mavi_sys *s, hipStream_t st, bool clear);
-// block end: dmax <- the largest drift step, the largest displacement of the
+// block end: host <- the largest drift step, the largest displacement of the
 // pending positions from the build, the status word
 hipError_t nl_measure(mavi_sys *s, hipStream_t st);
 // after an accepted block: the state's positions <- the wrap of the last
@@ -450,6 +471,8 @@ inline void rl_invalidate(mavi_sys *s) {
 // left where it is: s->src, s->scell, s->start.
 hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,
                              hipStream_t st);
+hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
+hipError_t copy_out(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
 hipError_t launch_export_chunks(mavi_sys *s, int64_t *d_cp, int64_t *d_counts, hipStream_t st);
 hipError_t launch_forces_only(mavi_sys *s, hipStream_t st);
 // One newton_step!; reuse = the previous call was a Verlet step of this

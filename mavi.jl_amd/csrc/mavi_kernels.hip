@@ -23,6 +23,8 @@
 // The library is compiled with -ffp-contract=off: a*b+c is only fused where
 // the code calls __builtin_fma, so the arithmetic that follows Julia's
 // rounding (positions, velocities, HarmTrunc forces, ring updates) does.
+#include <string.h>
+
 #include "mavi_device.h"
 #include "mavi_host.h"
 
@@ -1385,6 +1387,94 @@ hipError_t launch_observables(mavi_sys *s, double *d_out, hipStream_t st) {
     hipLaunchKernelGGL(k_observables, dim3(nblk(s->P.na, kObsThreads)), dim3(kObsThreads), 0, st, s->P,
                        s->P_[s->cur], has_vel ? s->V_[s->cur] : nullptr, with_pe, d_out);
     return hipGetLastError();
+}
+
+// Up to three arrays copied by one launch, in 4-byte words (one side is pinned
+// host memory).
+struct CopyArgs {
+    const uint32_t *src[3];
+    uint32_t *dst[3];
+    int32_t n[3];
+};
+__global__ void k_copy3(CopyArgs A) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        if (i >= 0 && i < A.n[k]) A.dst[k][i] = A.src[k][i];
+        i -= A.n[k];
+    }
+}
+
+static hipError_t copy3(mavi_ctx *ctx, char *pin, std::initializer_list<Xfer> list, bool in) {
+    CopyArgs A{};
+    int k = 0, total = 0;
+    size_t at = 0;
+    for (const Xfer &x : list) {
+        A.n[k] = (int32_t)(x.bytes / 4);
+        A.src[k] = (const uint32_t *)(in ? (void *)(pin + at) : x.dev);
+        A.dst[k] = (uint32_t *)(in ? x.dev : (void *)(pin + at));
+        total += A.n[k];
+        at += (x.bytes + 63) / 64 * 64;
+        k++;
+    }
+    if (total == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_copy3, dim3(nblk(total, 256)), dim3(256), 0, ctx->stream, A);
+    return hipGetLastError();
+}
+
+// The pinned buffer, or null if the transfer is larger (or there is none to be had).
+static char *pin_for(PinBuf &pin, std::initializer_list<Xfer> list) {
+    size_t need = 0;
+    for (const Xfer &x : list) need += (x.bytes + 63) / 64 * 64;
+    if (need > pin.bytes || list.size() > 3) return nullptr;
+    if (!pin.p && hipHostMalloc(&pin.p, pin.bytes, hipHostMallocDefault) != hipSuccess) {
+        pin.p = nullptr;
+        (void)hipGetLastError();
+    }
+    return (char *)pin.p;
+}
+
+// Host arrays to the device on the context's stream.  The pinned buffer is free:
+// every use of it ends with a wait for the stream, in copy_out here, after a
+// copy_in in its caller.
+hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list) {
+    char *p = pin_for(pin, list);
+    if (p) {
+        size_t at = 0;
+        for (const Xfer &x : list) {
+            if (x.bytes) memcpy(p + at, x.host, x.bytes);
+            at += (x.bytes + 63) / 64 * 64;
+        }
+        return copy3(ctx, p, list, true);
+    }
+    for (const Xfer &x : list) {
+        if (!x.bytes) continue;
+        hipError_t e = hipMemcpyAsync(x.dev, x.host, x.bytes, hipMemcpyHostToDevice, ctx->stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// Device arrays to the host, complete on return.
+hipError_t copy_out(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list) {
+    char *p = pin_for(pin, list);
+    hipError_t e = hipSuccess;
+    if (p) {
+        e = copy3(ctx, p, list, false);
+    } else {
+        for (const Xfer &x : list)
+            if (x.bytes && e == hipSuccess)
+                e = hipMemcpyAsync(x.host, x.dev, x.bytes, hipMemcpyDeviceToHost, ctx->stream);
+    }
+    const hipError_t e2 = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = e2;
+    if (e != hipSuccess || !p) return e;
+    size_t at = 0;
+    for (const Xfer &x : list) {
+        if (x.bytes) memcpy(x.host, p + at, x.bytes);
+        at += (x.bytes + 63) / 64 * 64;
+    }
+    return hipSuccess;
 }
 
 }  // namespace mavi

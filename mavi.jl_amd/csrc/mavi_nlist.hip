@@ -819,7 +819,8 @@ __global__ __launch_bounds__(kNeedBlock) void k_nl_second(SysParams P, NLArgs A)
 }
 
 // out[0] <- max of bmax, out[1] <- max of dpend (the doubles' bits), out[2]
-// <- the status word (one workgroup of 1024 threads).
+// <- the status word (one workgroup of 1024 threads).  out is pinned host
+// memory: the host waits for the launch and reads.
 __global__ __launch_bounds__(1024) void k_nl_reduce(const double *__restrict__ bmax, const double *__restrict__ dpend,
                                                     int32_t n, const uint32_t *__restrict__ status,
                                                     unsigned long long *__restrict__ out) {
@@ -987,7 +988,6 @@ hipError_t nl_alloc(mavi_sys *s, hipStream_t st) {
     if (e == hipSuccess) e = dalloc(&N.xb, na, st);
     if (e == hipSuccess) e = dalloc(&N.vsnap, na, st);
     if (e == hipSuccess) e = dalloc(&N.fsnap, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.dmax, 3, st);
     N.nbmax = nblk(s->P.na, kNeedBlock);  // workgroups of the second evaluation
     if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
     if (e == hipSuccess) e = dalloc(&N.dpend, N.nbmax, st);
@@ -1015,7 +1015,7 @@ void nl_free(mavi_sys *s) {
         p = nullptr;
     }
     dfree(N.fk); dfree(N.fk_on); dfree(N.xb); dfree(N.vsnap); dfree(N.fsnap);
-    dfree(N.dmax); dfree(N.bmax); dfree(N.dpend); dfree(N.status); dfree(N.scan_ticket); dfree(N.scan_state);
+    dfree(N.bmax); dfree(N.dpend); dfree(N.status); dfree(N.scan_ticket); dfree(N.scan_state);
     if (N.host) (void)hipHostFree(N.host);
     delete s->nl;
     s->nl = nullptr;
@@ -1076,7 +1076,7 @@ hipError_t nl_measure(mavi_sys *s, hipStream_t st) {
     hipLaunchKernelGGL(k_nl_measure, dim3(N.nbmax), dim3(kNeedBlock), 0, st, s->P, N.px[N.ph % 2], N.xb, N.dpend);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_nl_reduce, dim3(1), dim3(1024), 0, st, N.bmax, N.dpend, N.nbmax, N.status, N.dmax);
+    hipLaunchKernelGGL(k_nl_reduce, dim3(1), dim3(1024), 0, st, N.bmax, N.dpend, N.nbmax, N.status, N.host);
     return hipGetLastError();
 }
 

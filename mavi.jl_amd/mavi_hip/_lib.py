@@ -312,10 +312,18 @@ class DeviceSystem:
         self._call("mavi_forces", dptr(f))
         return f
 
-    def get_forces(self):
-        f = np.zeros((self.n, 2))
+    def get_forces(self, out=None):
+        """Forces by particle id, into ``out`` if it can take them."""
+        f = out if self._takes(out) else np.zeros((self.n, 2))
         self._call("mavi_get_forces", dptr(f))
+        if out is not None and f is not out:
+            out[:] = f
+            return out
         return f
+
+    def _takes(self, a) -> bool:
+        return (isinstance(a, np.ndarray) and a.dtype == np.float64 and a.shape == (self.n, 2)
+                and a.flags.c_contiguous and a.flags.writeable)
 
     def step(self, nsteps: int):
         self._call("mavi_step", C.c_int64(int(nsteps)))

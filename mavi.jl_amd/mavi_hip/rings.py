@@ -590,7 +590,7 @@ class RingsSystem:
 
     def download(self):
         self.dev.download(self.state.pos, None, self.state.pol)
-        self.forces[:] = self.dev.get_forces()
+        self.dev.get_forces(self.forces)
         self.areas, self.cms, self.continuos_pos = self.dev.rings_info()
         self._sync_var()
 

@@ -280,7 +280,7 @@ class System:
             self.dev.download(self.state.pos, None, self.state.pol_angle)
         else:
             self.dev.download(self.state.pos, self.state.vel)
-        self.forces[:] = self.dev.get_forces()
+        self.dev.get_forces(self.forces)
 
     # --- reference operations ----------------------------------------------
     def update_chunks(self):
