@@ -235,6 +235,7 @@ struct RList {
     SysParams G{};            // list grid (cells >= range + skin)
     void *greps = nullptr;    // a batch: its replica table with the list grids (device)
     int64_t gcells = 0;       // and their cells
+    bool scan_stale = false;  // the list grid changed: its scan starts from a cleared ticket and states
     int per = 1;              // most rings of a wave of the step kernel
     int ph = 0;               // counter word of the current step
     int32_t *head = nullptr;  // int4 per slot: the first four entries, -1 past the end

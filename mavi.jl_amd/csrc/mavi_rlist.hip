@@ -826,6 +826,11 @@ hipError_t rl_rebuild(const RLSys &E, hipStream_t st) {
     mavi_sys *s = E.s;
     BatchSub *b = E.b;
     hipError_t e = s ? mavi::drop_keys(s, st) : hipSuccess;
+    if (N.scan_stale) {
+        if (e == hipSuccess) e = mavi::launch_fill_i32((int32_t *)N.scan_ticket, 0, 2, st);
+        if (e == hipSuccess) e = mavi::launch_fill_i32((int32_t *)N.scan_state, 0, 2 * (int64_t)N.scan_words, st);
+        N.scan_stale = e != hipSuccess;
+    }
     if (e == hipSuccess) e = rl_ring_order(E, st);
     if (e == hipSuccess)
         e = s ? mavi::launch_cell_order(s, N.G, N.scan_ticket, N.scan_state, st)
@@ -1014,6 +1019,7 @@ bool rl_set_skin(mavi_sys *s, double skin_frac) {
     RList &N = *s->rl;
     N.fits = rl_grid(s->P, sqrt(s->list2), skin_frac, N.G, N.rl2, N.half_skin);
     N.valid = false;
+    N.scan_stale = true;
     return N.fits;
 }
 

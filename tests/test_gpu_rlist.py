@@ -186,3 +186,22 @@ def test_errors_are_the_gathers(gpu_ctx):
             dev.step(20)
         dev.upload(state.pos, None, state.pol)  # a good state runs again
         dev.step(20)
+
+
+def test_skin_changes_on_a_grid_of_several_scan_tiles(gpu_ctx):
+    """A list grid of several scan tiles whose number changes with the skin:
+    each grid's scan starts afresh."""
+    from mavi_hip import _lib, rings
+
+    def one():
+        state, space, cfg, ic = normal_case(True, n=10, cols=64, rows=60, seed=12)
+        return rings.RingsSystem(state=state, space_cfg=space, dynamic_cfg=cfg, int_cfg=ic, seed=3)
+
+    a, b = one(), one()
+    b.dev.set_option(_lib.MAVI_OPT_NLIST, 0)
+    for skin in (0, 100, 350, 0):
+        a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, skin)
+        a.advance(20)
+        b.advance(20)
+        assert a.dev.nlist_info()["active"]
+        same(skin, a, b)
