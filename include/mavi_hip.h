@@ -316,8 +316,13 @@ int mavi_sys_noise_set(mavi_sys *sys, uint64_t seed, uint64_t counter);
  *                       kept for the second evaluation (pairs whose
  *                       step-start chunks are not adjacent left out), forces
  *                       summed in ascending partner id; lists rebuilt when a
- *                       particle has moved half the skin.  0: the chunk gather
- *   MAVI_OPT_NLIST_SKIN skin in thousandths of the range (0: 150)
+ *                       particle has moved half the skin.  Rings step! of a
+ *                       fixed population on a periodic chunk grid whose chunks
+ *                       are at least the range wide runs on lists too (calls of
+ *                       8 steps and more), with the chunk gather's bits.
+ *                       0: the chunk gather
+ *   MAVI_OPT_NLIST_SKIN skin in thousandths of the range (0: LJ 150, HarmTrunc
+ *                       300, or 150 if those lists overflow, rings 300)
  *   MAVI_OPT_NLIST_BLOCK steps between displacement checks (0: as many as
  *                       the displacement bound allows at the last measured
  *                       step length, at most 60) */

@@ -890,7 +890,7 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
     NList &N = *s->nl;
     const SysParams &P = s->P;
     const size_t bytes = sizeof(double2) * (size_t)P.na;
-    const double half_skin = sqrt(N.thr2);
+    double half_skin = sqrt(N.thr2);
     *left = 0;
     int64_t k = 0;
     while (k < nsteps) {
@@ -945,6 +945,14 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
             // a list overflowed, a chunk count may have passed the capacity
             // (the chunk gather checks it exactly), or one step from a fresh
             // build moved a particle more than skin / 2
+            if (status && !N.skin_set && N.skin_frac > kNlSkin) {
+                // lists that a thinner skin may hold
+                nl_drop_graph(s);
+                mavi::nl_set_skin(s, kNlSkin);
+                half_skin = sqrt(N.thr2);
+                HIPCHK(ctx, hipMemsetAsync(N.status, 0, sizeof(uint32_t), st));
+                continue;
+            }
             if (status || (fresh && blk == 1)) {
                 // the chunk gather takes over
                 N.disabled = true;
@@ -1566,7 +1574,8 @@ int mavi_sys_set_option(mavi_sys *s, int32_t option, int32_t value) {
             if (value < 0 || value > 2000) return set_err(s->ctx, MAVI_E_BADARG, "skin: 0 (default) .. 2000 thousandths");
             if (s->nl) {
                 nl_drop_graph(s);
-                mavi::nl_set_skin(s, value == 0 ? 0.15 : value / 1000.0);
+                mavi::nl_set_skin(s, value == 0 ? mavi::nl_default_skin(s) : value / 1000.0);
+                s->nl->skin_set = value != 0;
             }
             if (s->rl) (void)mavi::rl_set_skin(s, value == 0 ? kRlSkin : value / 1000.0);
             break;

@@ -173,12 +173,15 @@ constexpr int32_t kNlBlockCap = 60;  // most steps between host checks of the li
 
 // Verlet neighbour lists of a finite-range plain system (LJ with a cutoff,
 // HarmTrunc) whose chunks are at least the interaction range wide (mavi_nlist.hip).
+constexpr double kNlSkin = 0.15, kNlWideSkin = 0.3;  // default skins of plain systems (nl_default_skin)
+
 struct NList {
     bool on = true;           // option MAVI_OPT_NLIST
     bool valid = false;       // built for the current slot order and still complete
     bool disabled = false;    // a list overflowed: the chunk gather takes over
     double range = 0.0;       // interaction range (rcut / dist_max)
-    double skin_frac = 0.15;  // skin = skin_frac * range (option, thousandths)
+    double skin_frac = kNlSkin;  // skin = skin_frac * range (option, thousandths)
+    bool skin_set = false;    // by the option: kept when a list overflows
     double rl2 = 0.0;         // list radius squared (range + skin)^2, with margin
     double thr2 = 0.0;        // displacement bound squared (skin / 2)^2, with margin
     double edge = 0.0;        // within this distance of a periodic edge: minimum image
@@ -455,6 +458,7 @@ hipError_t nl_measure(mavi_sys *s, hipStream_t st);
 // evaluated drift
 hipError_t nl_settle(mavi_sys *s, hipStream_t st);
 void nl_set_skin(mavi_sys *s, double skin_frac);
+double nl_default_skin(const mavi_sys *s);
 // Lists of a rings system (mavi_rlist.hip).  rl_active: the next steps may run
 // on them; rl_steps: up to nsteps steps (*left > 0: the chunk gather runs the
 // rest); rl_invalidate: the state was moved or reordered by other kernels.

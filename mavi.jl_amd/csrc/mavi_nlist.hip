@@ -941,6 +941,14 @@ bool nl_eligible(const mavi_sys *s) {
     return P.cl >= range * (1.0 + 1e-12) && P.ch >= range * (1.0 + 1e-12);
 }
 
+// The skin without an option.  HarmTrunc lists are short (a few partners at a
+// range of about the particles' size), so a wider skin costs a step little and
+// halves the rebuilds: 0.15 -> 0.3, us a step with the rebuilds: 22k walled discs
+// 11.2 -> 9.6, 160k 18.5 -> 15.6, 490k 37.8 -> 28.4, 1M 66.2 -> 47.8 (0.25: 51.2,
+// 0.4: 46.0 there, 9.9 at 22k).  Lennard-Jones lists hold ~20 partners: 0.15
+// against 0.2 and 0.3: 1k 8.9, 9.4, 10.1, 102k 13.9, 14.5, 15.7.
+double nl_default_skin(const mavi_sys *s) { return s->P.potential == MAVI_POT_HARMTRUNC ? kNlWideSkin : kNlSkin; }
+
 void nl_set_skin(mavi_sys *s, double skin_frac) {
     NList &N = *s->nl;
     const SysParams &P = s->P;
@@ -970,7 +978,7 @@ hipError_t nl_alloc(mavi_sys *s, hipStream_t st) {
     s->nl = new NList();
     NList &N = *s->nl;
     N.range = nl_range(s);
-    nl_set_skin(s, N.skin_frac);
+    nl_set_skin(s, nl_default_skin(s));
     const int64_t na = s->P.na;
     N.kmax = kNlMax;
     hipError_t e = dalloc(&N.nbr, (int64_t)(N.kmax / 2) * na, st);  // 16-bit entries

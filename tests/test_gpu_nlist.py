@@ -279,3 +279,33 @@ def test_marked_particles_one_walk(gpu_ctx, oracle_mod, cols, rows, periodic, ki
     ep, ev = traj_err(runs[0][0], runs[0][1], p_ref, v_ref, L, periodic=periodic)
     say(f"[marked] {kind} {cols}x{rows} n={n} pos {ep:.2e} vel {ev:.2e}")
     assert ep <= TRAJ_RTOL and ev <= TRAJ_RTOL
+
+
+def test_default_skin_falls_back_before_the_gather(gpu_ctx):
+    """HarmTrunc lists at the default skin overflow (more than 128 stencil
+    candidates) where those at 150 thousandths hold: the lists go on with the
+    thinner skin, with the same bits as that skin set by the option."""
+    import mavi_hip as mv
+    from mavi_hip import _lib
+
+    rng = np.random.default_rng(3)
+    side = 40
+    ix = np.arange(side * side)
+    pos = np.stack([ix % side + 0.5, ix // side + 0.5], axis=1) + 0.02 * rng.uniform(-1, 1, (side * side, 2))
+    vel = 2.0 * rng.normal(size=pos.shape)
+    dyn = mv.HarmTruncCfg(k_rep=0.5, k_atr=0.05, dist_eq=2.0, dist_max=3.05)
+    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=float(side), height=float(side)))
+    ic = mv.IntCfg(dt=1e-4, chunks_cfg=mv.ChunksCfg(num_cols=13, num_rows=13), device=mv.GPU())
+    runs = []
+    for skin in (0, 150):
+        s = mv.System(state=mv.SecondLawState(pos=pos.copy(), vel=vel.copy()), space_cfg=space, dynamic_cfg=dyn,
+                      int_cfg=ic)
+        s.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, skin)
+        s.advance(40)
+        s.download()
+        info = s.dev.nlist_info()
+        say(f"[skin fallback] {skin}: {info}")
+        assert info["active"] and info["rollbacks"] == (1 if skin == 0 else 0)
+        runs.append((s.state.pos.copy(), s.state.vel.copy(), s.forces.copy()))
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
