@@ -17,6 +17,7 @@
 //   scan_state   u64[ntiles]   published tile states of the one-pass scan
 //                              (4096 or 16384 chunks per tile), scan_ticket its counter
 //   pos_id, vel_id, force_id   double2[n] id-order staging for the host
+//   ang_id       double[n]     self-propelled: the angles as the host holds them
 // na = number of active ids (get_particles_ids); the chunk index is
 // row0*cols + col0 with row0 = reference row - 1 (row 1 = top of the box,
 // src/chunks.jl:129) and col0 = reference col - 1.  Row-major chunks make the
@@ -171,10 +172,10 @@ struct RingRates {
 
 constexpr int32_t kNlBlockCap = 60;  // most steps between host checks of the list validity
 
-// Verlet neighbour lists of a finite-range plain system (LJ with a cutoff,
-// HarmTrunc) whose chunks are at least the interaction range wide (mavi_nlist.hip).
 constexpr double kNlSkin = 0.15, kNlWideSkin = 0.3;  // default skins of plain systems (nl_default_skin)
 
+// Verlet neighbour lists of a finite-range plain system (LJ with a cutoff,
+// HarmTrunc) whose chunks are at least the interaction range wide (mavi_nlist.hip).
 struct NList {
     bool on = true;           // option MAVI_OPT_NLIST
     bool valid = false;       // built for the current slot order and still complete
@@ -253,9 +254,11 @@ struct RList {
     double2 *polcs = nullptr; // cos, sin of the polarisations
     uint32_t *bmax = nullptr; // per workgroup of the step kernel
     int32_t nbmax = 0;
+    uint8_t *arena = nullptr; // holds all of the above and below
     uint32_t *status = nullptr;
     unsigned long long *counter = nullptr;  // two words, alternating between steps
     unsigned long long *out = nullptr, *host = nullptr;  // block-end maxima and status, pinned copy
+    unsigned long long *own_host = nullptr;  // a batch: the copy is an allocation of its own
     unsigned long long *scan_ticket = nullptr, *scan_state = nullptr;
     int32_t scan_words = 0;
     int64_t rebuilds = 0, rollbacks = 0;
@@ -267,14 +270,14 @@ struct RList {
 // pageable memory costs over 10 us however small.  1k particles: download 44 -> 21
 // us, the flags word after a step 15 us less; at 256 KiB the copy through the
 // buffer takes about what it saves.
-constexpr size_t kPinBytes = 256 * 1024;
+constexpr size_t kPinBytes = 256 * 1024, kPinWords = 8;
 struct PinBuf {
-    void *p = nullptr;    // hipHostMalloc, at the first use
+    void *p = nullptr;    // hipHostMalloc, at the first use, with kPinWords words behind it
     size_t bytes = 4096;  // its size
     // room for the state of n particles, if that is small
     void fit(int64_t n) {
         const int64_t want = 40 * n + 4096;
-        if (want <= (int64_t)kPinBytes && want > (int64_t)bytes) bytes = (size_t)want;
+        if (!p && want <= (int64_t)kPinBytes && want > (int64_t)bytes) bytes = (size_t)want;
     }
 };
 struct Xfer {
@@ -476,6 +479,8 @@ inline void rl_invalidate(mavi_sys *s) {
 // left where it is: s->src, s->scell, s->start.
 hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,
                              hipStream_t st);
+// Eight words of pinned memory behind the buffer (null: none to be had).
+unsigned long long *pin_words(PinBuf &pin);
 hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
 hipError_t copy_out(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
 hipError_t launch_export_chunks(mavi_sys *s, int64_t *d_cp, int64_t *d_counts, hipStream_t st);

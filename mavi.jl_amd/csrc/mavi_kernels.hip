@@ -18,6 +18,8 @@
 //                   k_rings<UPDATE> (one ring per
 //                   thread, any size): unwrap, shoelace area, springs, area
 //                   force and overdamped update (src/rings/integration.jl:79-351).
+//                   (Finite-range plain systems and fixed ring populations step
+//                   on Verlet lists instead: mavi_nlist.hip, mavi_rlist.hip.)
 //   K7 observables  k_observables (src/quantities.jl:12-18, 46-66).
 //
 // The library is compiled with -ffp-contract=off: a*b+c is only fused where
@@ -1422,16 +1424,22 @@ static hipError_t copy3(mavi_ctx *ctx, char *pin, std::initializer_list<Xfer> li
     return hipGetLastError();
 }
 
+unsigned long long *pin_words(PinBuf &pin) {
+    pin.bytes = (pin.bytes + 63) / 64 * 64;
+    if (!pin.p && hipHostMalloc(&pin.p, pin.bytes + 8 * kPinWords, hipHostMallocDefault) != hipSuccess) {
+        pin.p = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return (unsigned long long *)((char *)pin.p + pin.bytes);
+}
+
 // The pinned buffer, or null if the transfer is larger (or there is none to be had).
 static char *pin_for(PinBuf &pin, std::initializer_list<Xfer> list) {
     size_t need = 0;
     for (const Xfer &x : list) need += (x.bytes + 63) / 64 * 64;
     if (need > pin.bytes || list.size() > 3) return nullptr;
-    if (!pin.p && hipHostMalloc(&pin.p, pin.bytes, hipHostMallocDefault) != hipSuccess) {
-        pin.p = nullptr;
-        (void)hipGetLastError();
-    }
-    return (char *)pin.p;
+    return pin_words(pin) ? (char *)pin.p : nullptr;
 }
 
 // Host arrays to the device on the context's stream.  The pinned buffer is free:

@@ -1000,7 +1000,7 @@ hipError_t nl_alloc(mavi_sys *s, hipStream_t st) {
     if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
     if (e == hipSuccess) e = dalloc(&N.dpend, N.nbmax, st);
     if (e == hipSuccess) e = dalloc(&N.status, 1, st);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&N.host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
+    if (e == hipSuccess && (N.host = pin_words(s->pin)) == nullptr) e = hipErrorOutOfMemory;
     // scan states of the list grid (no more cells than the chunk grid)
     N.scan_words = (s->P.ncell + 1 + kScanTileMin - 1) / kScanTileMin + 1;
     if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);
@@ -1024,7 +1024,6 @@ void nl_free(mavi_sys *s) {
     }
     dfree(N.fk); dfree(N.fk_on); dfree(N.xb); dfree(N.vsnap); dfree(N.fsnap);
     dfree(N.bmax); dfree(N.dpend); dfree(N.status); dfree(N.scan_ticket); dfree(N.scan_state);
-    if (N.host) (void)hipHostFree(N.host);
     delete s->nl;
     s->nl = nullptr;
 }

@@ -670,7 +670,19 @@ __global__ __launch_bounds__(1024) void k_rl_measure(SysParams P0, int32_t nslot
         d2 = fmax(d2, __shfl_xor(d2, o, 64));
         hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
     }
+    // one atomic per workgroup and word (one per wave, 1024 on an address: 30 us)
+    __shared__ double s_d[16];
+    __shared__ uint32_t s_h[16];
     if (lane_id() == 0) {
+        s_d[threadIdx.x >> 6] = d2;
+        s_h[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) {
+            d2 = fmax(d2, s_d[w]);
+            hi = max(hi, s_h[w]);
+        }
         atomicMax(&out[0], (unsigned long long)hi << 32);
         atomicMax(&out[1], (unsigned long long)__double_as_longlong(d2));
     }
@@ -1026,25 +1038,38 @@ bool rl_set_skin(mavi_sys *s, double skin_frac) {
 static hipError_t rl_buffers(RList &N, int64_t nslots, int64_t nrings, int64_t ncells, int64_t nflags,
                              hipStream_t st) {
     N.scan_words = (int32_t)((ncells + 1 + kScanTileMin - 1) / kScanTileMin) + 1;
-    hipError_t e = dalloc(&N.head, 4 * nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.more, (int64_t)(kRlMax - kRlHead) * nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.count, nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.key, nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.ccnt, ncells, st);
-    if (e == hipSuccess) e = dalloc(&N.xb, nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.psnap, nslots, st);
-    if (e == hipSuccess) e = dalloc(&N.csnap, nrings, st);
-    if (e == hipSuccess) e = dalloc(&N.nsnap, nrings, st);
-    if (e == hipSuccess) e = dalloc(&N.polsnap, nrings, st);
-    if (e == hipSuccess) e = dalloc(&N.fsnap, nflags, st);
-    if (e == hipSuccess) e = dalloc(&N.polcs, nrings, st);
-    if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
-    if (e == hipSuccess) e = dalloc(&N.status, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.counter, 2, st);
-    if (e == hipSuccess) e = dalloc(&N.out, 3, st);
-    if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);
-    if (e == hipSuccess) e = dalloc(&N.scan_state, N.scan_words, st);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&N.host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
+    // one allocation for all: a system is made with few calls
+    struct Part {
+        void **p;
+        size_t bytes;
+    } parts[] = {
+        {(void **)&N.head, sizeof(int32_t) * 4 * nslots},
+        {(void **)&N.more, sizeof(int32_t) * (kRlMax - kRlHead) * nslots},
+        {(void **)&N.count, sizeof(*N.count) * nslots},
+        {(void **)&N.key, sizeof(*N.key) * nslots},
+        {(void **)&N.ccnt, sizeof(*N.ccnt) * ncells},
+        {(void **)&N.xb, sizeof(*N.xb) * nslots},
+        {(void **)&N.psnap, sizeof(*N.psnap) * nslots},
+        {(void **)&N.csnap, sizeof(*N.csnap) * nrings},
+        {(void **)&N.nsnap, sizeof(*N.nsnap) * nrings},
+        {(void **)&N.polsnap, sizeof(*N.polsnap) * nrings},
+        {(void **)&N.fsnap, sizeof(*N.fsnap) * nflags},
+        {(void **)&N.polcs, sizeof(*N.polcs) * nrings},
+        {(void **)&N.bmax, sizeof(*N.bmax) * N.nbmax},
+        {(void **)&N.status, sizeof(*N.status)},
+        {(void **)&N.counter, sizeof(*N.counter) * 2},
+        {(void **)&N.out, sizeof(*N.out) * 3},
+        {(void **)&N.scan_ticket, sizeof(*N.scan_ticket)},
+        {(void **)&N.scan_state, sizeof(*N.scan_state) * N.scan_words},
+    };
+    size_t total = 0;
+    for (const Part &q : parts) total += (q.bytes + 255) / 256 * 256;
+    hipError_t e = dalloc(&N.arena, (int64_t)total, st);
+    size_t at = 0;
+    for (const Part &q : parts) {
+        if (e == hipSuccess) *q.p = N.arena + at;
+        at += (q.bytes + 255) / 256 * 256;
+    }
     return e;
 }
 
@@ -1070,11 +1095,9 @@ static void rl_release(RList *&rl, hipStream_t st) {
     if (!rl) return;
     RList &N = *rl;
     rl_drop_graphs(N, st);
-    dfree(N.head); dfree(N.more); dfree(N.count); dfree(N.key); dfree(N.ccnt); dfree(N.xb); dfree(N.psnap);
-    dfree(N.csnap); dfree(N.nsnap); dfree(N.polsnap); dfree(N.fsnap); dfree(N.polcs); dfree(N.bmax); dfree(N.status);
-    dfree(N.counter); dfree(N.out); dfree(N.scan_ticket); dfree(N.scan_state);
+    dfree(N.arena);
     if (N.greps) (void)hipFree(N.greps);
-    if (N.host) (void)hipHostFree(N.host);
+    if (N.own_host) (void)hipHostFree(N.own_host);
     delete rl;
     rl = nullptr;
 }
@@ -1086,6 +1109,7 @@ hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
     N.uniform = rl_uniform(s->host_inter.data(), (int)s->host_inter.size());
     N.per = 64 / s->P.nmax;
     N.nbmax = rl_blocks(s->P);
+    if ((N.host = pin_words(s->pin)) == nullptr) return hipErrorOutOfMemory;
     return rl_buffers(N, s->P.na, s->P.nrings, s->P.ncell, 1, st);
 }
 
@@ -1132,7 +1156,9 @@ hipError_t rlb_alloc(BatchSub *b, hipStream_t st) {
     N.fits = true;
     N.uniform = full;
     N.nbmax = nblk(b->nring_waves, kRlWaves);
-    hipError_t e = rl_buffers(N, b->nslots, b->nrings, b->ncells, (int64_t)b->reps.size(), st);
+    hipError_t e = hipHostMalloc((void **)&N.own_host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
+    N.host = N.own_host;
+    if (e == hipSuccess) e = rl_buffers(N, b->nslots, b->nrings, b->ncells, (int64_t)b->reps.size(), st);
     if (e == hipSuccess) e = hipMalloc(&N.greps, sizeof(Replica) * g.size());
     if (e == hipSuccess) e = hipMemcpyAsync(N.greps, g.data(), sizeof(Replica) * g.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
