@@ -905,7 +905,6 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
         // the block's start state, to roll back to (the state's positions are
         // written only after the check)
         HIPCHK(ctx, mavi::nl_block_start(s, st, !fresh));
-        HIPCHK(ctx, hipMemcpyAsync(N.vsnap, s->V_[s->cur], bytes, hipMemcpyDeviceToDevice, st));
         int64_t done = 0;
         const bool graphs = s->use_graphs && !s->prof;
         while (done < blk) {

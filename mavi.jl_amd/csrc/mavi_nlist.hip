@@ -48,6 +48,8 @@
 // chunk gather, whose binning checks it exactly.
 #include <math.h>
 
+#include <algorithm>
+
 #include "mavi_device.h"
 #include "mavi_host.h"
 
@@ -846,13 +848,29 @@ __global__ __launch_bounds__(1024) void k_nl_reduce(const double *__restrict__ b
     if (threadIdx.x == 2) out[2] = *status;
 }
 
+// Four arrays of words cleared by one launch (blockIdx.y: the array): a launch
+// each took 2.3 us, and a single step of 1k particles builds its lists.
+struct ClearArgs {
+    int32_t *p[4];
+    int32_t n[4];
+};
+__global__ void k_nl_clear(ClearArgs A) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if ((int)blockIdx.y == k && i < A.n[k]) A.p[k][i] = 0;
+}
+
 // At a block's start: the step maxima cleared (not after a build, whose drift
-// counts among the block's steps) and the flags word kept for a rollback.
+// counts among the block's steps), the velocities and the flags word kept for a
+// rollback (a copy of 16 MB by the runtime takes 18 us, a third of the rate).
 __global__ void k_nl_block_start(double *__restrict__ bmax, int32_t n, int32_t clear,
-                                 const uint32_t *__restrict__ flags, uint32_t *__restrict__ fsnap) {
+                                 const uint32_t *__restrict__ flags, uint32_t *__restrict__ fsnap, int32_t na,
+                                 const double2 *__restrict__ V, double2 *__restrict__ vsnap) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (clear && i < n) bmax[i] = 0.0;
     if (i == 0) *fsnap = *flags;
+    if (i < na) vsnap[i] = V[i];
 }
 
 // At a block's end, per workgroup: the largest squared displacement of the
@@ -1032,9 +1050,15 @@ hipError_t nl_rebuild(mavi_sys *s, hipStream_t st) {
     NList &N = *s->nl;
     hipError_t e = drop_keys(s, st);  // counts a fused first pass left on the chunk grid
     // the list grid's scan starts from a cleared ticket and states (its tile
-    // count changes with the skin)
-    if (e == hipSuccess) e = launch_fill_i32((int32_t *)N.scan_ticket, 0, 2, st);
-    if (e == hipSuccess) e = launch_fill_i32((int32_t *)N.scan_state, 0, 2 * (int64_t)N.scan_words, st);
+    // count changes with the skin); the chunk counts and step maxima with them
+    if (e == hipSuccess) {
+        const ClearArgs C{{(int32_t *)N.scan_ticket, (int32_t *)N.scan_state, N.ccnt, (int32_t *)N.bmax},
+                          {2, 2 * N.scan_words, s->P.ncell, 2 * N.nbmax}};
+        int32_t words = 0;
+        for (const int32_t n : C.n) words = std::max(words, n);
+        hipLaunchKernelGGL(k_nl_clear, dim3(nblk(words, 256), 4), dim3(256), 0, st, C);
+        e = hipGetLastError();
+    }
     if (e == hipSuccess) e = launch_bin(s, st, false, false, false, &N.G, N.scan_ticket, N.scan_state);
     if (e != hipSuccess) return e;
     s->sorted = false;   // not in reference chunk order: the chunk gather's stamps start over
@@ -1046,11 +1070,9 @@ hipError_t nl_rebuild(mavi_sys *s, hipStream_t st) {
         hipLaunchKernelGGL(k_nl_build, dim3(nblk(N.G.cols, kBuildWaves), N.G.rows), dim3(64 * kBuildWaves), 0, st, N.G, P, s->P_[c], s->ID_[c],
                            s->start, (int2 *)N.nbr, N.ncount, N.rl2, N.edge, N.status);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = launch_fill_i32(N.ccnt, 0, P.ncell, st)) != hipSuccess) return e;
         hipLaunchKernelGGL(k_nl_keys, dim3(nblk(P.na, 256)), dim3(256), 0, st, P, s->P_[c], N.key[0], N.ccnt,
                            N.chg[0], N.chg[1], N.xb, s->flags);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = launch_fill_i32((int32_t *)N.bmax, 0, 2 * (int64_t)N.nbmax, st)) != hipSuccess) return e;
     }
     // the first evaluation and drift of the first step
     N.ph = 0;
@@ -1071,8 +1093,8 @@ hipError_t nl_rebuild(mavi_sys *s, hipStream_t st) {
 
 hipError_t nl_block_start(mavi_sys *s, hipStream_t st, bool clear) {
     NList &N = *s->nl;
-    hipLaunchKernelGGL(k_nl_block_start, dim3(nblk(N.nbmax, 256)), dim3(256), 0, st, N.bmax, N.nbmax,
-                       clear ? 1 : 0, s->flags, N.fsnap);
+    hipLaunchKernelGGL(k_nl_block_start, dim3(nblk(s->P.na, 256)), dim3(256), 0, st, N.bmax, N.nbmax, clear ? 1 : 0,
+                       s->flags, N.fsnap, s->P.na, s->V_[s->cur], N.vsnap);
     return hipGetLastError();
 }
 
