@@ -45,19 +45,25 @@ CASES = {
     "normal": lambda: normal_case(True),
     "normal_ragged": lambda: normal_case(True, n=21, cols=7, rows=5, seed=3),
     "smallest_rings": lambda: normal_case(True, n=4, cols=6, rows=7, seed=4),
+    "rings_of_two": lambda: normal_case(True, n=2, cols=12, rows=11, seed=13),  # 32 rings a wave: 96 sums
+    "rings_of_three": lambda: normal_case(True, n=3, cols=11, rows=9, seed=14),
     "largest_rings": lambda: normal_case(True, n=32, cols=5, rows=3, seed=5),
     "few_cells": lambda: normal_case(True, n=9, cols=2, rows=2, seed=6),
     "types": lambda: types_case(True),
     "mixture": lambda: mixture(nrings=120, seed=8),
     "dense": lambda: squeezed(normal_case(True, n=10, cols=9, rows=8), 0.62, 1e-4),
     "dense_types": lambda: squeezed(types_case(True), 0.7, 1e-4),
+    "touching": lambda: squeezed(normal_case(True, n=10, cols=9, rows=8), 0.66, 1e-4),
 }
 
 
-def make(case, lists, seed=11):
+def make(case, lists, seed=11, dt=None):
+    import mavi_hip as mv
     from mavi_hip import _lib, rings
 
     state, space, cfg, ic = CASES[case]()
+    if dt is not None:
+        ic = mv.IntCfg(dt=dt, chunks_cfg=ic.chunks_cfg, device=mv.GPU())
     s = rings.RingsSystem(state=state, space_cfg=space, dynamic_cfg=cfg, int_cfg=ic, seed=seed)
     if not lists:
         s.dev.set_option(_lib.MAVI_OPT_NLIST, 0)
@@ -85,6 +91,46 @@ def test_same_bits_as_the_gather(gpu_ctx, case):
         same((case, k), a, b)
     say(f"[rings lists] {case} {a.dev.nlist_info()}")
     assert a.dev.nlist_info()["rebuilds"] >= 1 or case == "few_cells"
+
+
+def partners(s, reach):
+    """Particles within `reach` of each particle, bonded neighbours left out."""
+    pos = s.state.pos.reshape(-1, 2)
+    g = s.space_cfg.geometry_cfg
+    n = s.state.rings_pos.shape[1]
+    d = pos[:, None, :] - pos[None, :, :]
+    box = np.array([g.length, g.height])
+    d -= box * np.round(d / box)
+    near = (d ** 2).sum(axis=2) <= reach ** 2
+    ring, k = np.arange(len(pos)) // n, np.arange(len(pos)) % n
+    gap = np.abs(k[:, None] - k[None, :])
+    near &= ~((ring[:, None] == ring[None, :]) & ((gap <= 1) | (gap == n - 1)))
+    return near.sum(axis=1)
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if c != "few_cells"])
+def test_same_bits_with_every_step_on_lists(gpu_ctx, case):
+    """At a time step short enough for the lists not one step goes to the
+    gather: a third system with the launch counters on says so."""
+    from mavi_hip import _lib
+
+    dt = min(1e-3, CASES[case]()[3].dt)
+    a, b, c = make(case, True, dt=dt), make(case, False, dt=dt), make(case, True, dt=dt)
+    if case == "dense":  # more pairs in range than the first four entries hold
+        assert partners(a, 1.2).max() > 4
+    if case == "touching":  # three or four pairs in range, all among the first entries: put in order there
+        assert partners(a, 1.2).max() >= 3 and partners(a, 1.2 * 1.02).max() <= 4
+        for s in (a, c):
+            s.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, 20)
+    c.dev.prof_enable(True)
+    for k in (8, 61, 31):
+        for s in (a, b, c):
+            s.advance(k)
+        same((case, k), a, b)
+        same((case, k, "direct launches"), c, b)
+    gathers, steps = c.dev.prof_get(_lib.MAVI_PROF_FORCE)[1], c.dev.prof_get(_lib.MAVI_PROF_RINGS)[1]
+    say(f"[rings lists] {case} gathers {gathers} list steps {steps} {a.dev.nlist_info()} {c.dev.nlist_info()}")
+    assert gathers == 0 and steps >= 100 and a.dev.nlist_info()["active"]
 
 
 @pytest.mark.parametrize("skin,block,graphs", [(0, 0, 0), (50, 64, 1), (100, 7, 1), (600, 0, 1), (1000, 1, 1)])
