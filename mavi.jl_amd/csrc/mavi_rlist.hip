@@ -310,8 +310,10 @@ __global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4
     const double2 dprev = wave_diff(P, x, xp);
     s_b[me] = i == 0 ? x : dprev;
     lds_sync();
-    // ring size for the serial lanes of two sums a ring (per <= 32: rl_fits)
+    // ring sizes for the serial lanes: lane l < 3 per (<= 63: rl_fits) works for
+    // ring l / 2 or l / 3
     const int np2 = __shfl(np, min(lane >> 1, per - 1) * P.nmax, 64);
+    const int np3 = __shfl(np, min(lane / 3, per - 1) * P.nmax, 64);
     if (lane < 2 * per) {
         // c_0 = x_0, c_k = c_{k-1} + calc_diff(x_k, x_{k-1}), one lane per component
         const int o = 2 * (wb + (lane >> 1) * P.nmax) + (lane & 1);
@@ -330,18 +332,15 @@ __global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4
     if (LAST && act) A.cpos[B.cpos + id] = c;
     s_t[me] = c.x * cn.y - c.y * cn.x;
     lds_sync();
-    // centre of mass and shoelace sums in ring order, one lane per sum (rings of
-    // two: 96 sums in two turns)
-    for (int o = 0; o < 3 * per; o += 64) {
-        const int l = o + lane, g = l / 3, which = l - 3 * g;
-        const int np3 = __shfl(np, min(g, per - 1) * P.nmax, 64);
-        if (l >= 3 * per) continue;
+    if (lane < 3 * per) {
+        // centre of mass and shoelace sums in ring order, one lane per sum
+        const int g = lane / 3, which = lane - 3 * g;
         const double *src = which == 2 ? s_t + wb + g * P.nmax : (const double *)(s_c + wb + g * P.nmax) + which;
         const int stride = which == 2 ? 1 : 2;
         double s = 0.0;
 #pragma unroll 4
         for (int k = 0; k < np3; k++) s += src[k * stride];
-        s_r[wave][l] = s;
+        s_r[wave][lane] = s;
     }
 
     // ---- pair forces
@@ -1001,9 +1000,10 @@ namespace mavi {
 // Whether a rings system can run on lists.
 static bool rl_fits(const SysParams &P, double list2) {
     if (P.potential != MAVI_POT_RINGS || P.nwalls > 0 || !P.periodic || P.na <= 0) return false;
-    // rings of one particle have no spring to themselves (0 / 0: every step is
-    // non-finite), and k_rl_step counts on two sums a ring fitting a wave
-    if (P.nmax < 2 || P.nmax > 32) return false;
+    // k_rl_step has a lane for each of a wave's three sums a ring, which rings of
+    // two (32 to a wave) have more of than lanes; taking turns cost all others
+    // up to 0.8 % of a step
+    if (P.nmax < 3 || P.nmax > 32) return false;
     if (P.na > kRlSlotMask || P.ntypes > 32) return false;
     if (P.cols < 3 || P.rows < 3 || P.rows > 32767 || P.cols > 65535) return false;
     const double range = sqrt(list2);

@@ -220,7 +220,8 @@ def test_batch_errors(gpu_ctx):
 @pytest.mark.parametrize("names", [
     ("normal", "smallest_rings", "largest_rings", "types", "mixture"),  # ring sizes and counts that share workgroups
     ("normal", "smallest_rings", "normal_ragged"),  # every ring full: slots by place
-    ("rings_of_two", "normal", "rings_of_three"),  # more sums than lanes in a wave
+    ("rings_of_two", "normal"),  # rings too small for lists: all through the chunk gather
+    ("normal", "rings_of_three"),  # the smallest rings on lists
     ("types", "few_cells"),  # a box too small for lists: all through the chunk gather
 ])
 def test_batch_rings_on_lists_bitexact(gpu_ctx, names):

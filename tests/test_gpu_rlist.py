@@ -41,11 +41,12 @@ def squeezed(case, factor, dt):
     return state, space, cfg, ic
 
 
+OFF_LISTS = ("few_cells", "rings_of_two")  # a box too small; more sums in a wave than lanes
 CASES = {
     "normal": lambda: normal_case(True),
     "normal_ragged": lambda: normal_case(True, n=21, cols=7, rows=5, seed=3),
     "smallest_rings": lambda: normal_case(True, n=4, cols=6, rows=7, seed=4),
-    "rings_of_two": lambda: normal_case(True, n=2, cols=12, rows=11, seed=13),  # 32 rings a wave: 96 sums
+    "rings_of_two": lambda: normal_case(True, n=2, cols=12, rows=11, seed=13),
     "rings_of_three": lambda: normal_case(True, n=3, cols=11, rows=9, seed=14),
     "largest_rings": lambda: normal_case(True, n=32, cols=5, rows=3, seed=5),
     "few_cells": lambda: normal_case(True, n=9, cols=2, rows=2, seed=6),
@@ -84,13 +85,13 @@ def test_same_bits_as_the_gather(gpu_ctx, case):
     a, b = make(case, True), make(case, False)
     info = a.dev.nlist_info()
     say(f"[rings lists] {case} {info}")
-    assert info["eligible"] and not b.dev.nlist_info()["active"]
+    assert info["eligible"] == (case != "rings_of_two") and not b.dev.nlist_info()["active"]
     for k in (8, 61, 1, 30):
         a.advance(k)
         b.advance(k)
         same((case, k), a, b)
     say(f"[rings lists] {case} {a.dev.nlist_info()}")
-    assert a.dev.nlist_info()["rebuilds"] >= 1 or case == "few_cells"
+    assert a.dev.nlist_info()["rebuilds"] >= 1 or case in OFF_LISTS
 
 
 def partners(s, reach):
@@ -108,7 +109,7 @@ def partners(s, reach):
     return near.sum(axis=1)
 
 
-@pytest.mark.parametrize("case", [c for c in CASES if c != "few_cells"])
+@pytest.mark.parametrize("case", [c for c in CASES if c not in OFF_LISTS])
 def test_same_bits_with_every_step_on_lists(gpu_ctx, case):
     """At a time step short enough for the lists not one step goes to the
     gather: a third system with the launch counters on says so."""
