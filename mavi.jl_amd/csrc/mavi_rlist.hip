@@ -150,40 +150,71 @@ __device__ __forceinline__ unsigned long long visit_key(const SysParams &P, int 
     return ((unsigned long long)visit_rank(P, ri, ci, rj, cj) << 32) | (uint32_t)j;
 }
 
-// The sum of a particle with a long list, by repeated selection of the next
-// pair in the gather's order.
-__device__ __forceinline__ double2 rl_long_sum(const SysParams &P, const RLArgs &A, const RingInter *mat,
-                                               const RingInter &uni, int q, int t0, int t1, int ti, double2 x, int ri,
-                                               int ci) {
-    const int n = A.count[q];
-    const int4 h = A.head[q];
-    double2 f = make_double2(0.0, 0.0);
-    unsigned long long prev = 0ull;
-    bool first = true;
-    for (;;) {
-        unsigned long long best = ~0ull;
-        int32_t be = -1;
-        for (int e = 0; e < n; e++) {
-            const int32_t w = e == 0 ? h.x : e == 1 ? h.y : e == 2 ? h.z : e == 3 ? h.w : A.more[(int64_t)(e - kRlHead) * A.stride + q];
+// The sums of the wave's particles with long lists (`longer`), into their f: four
+// particles at a time, a row of 16 lanes to each, a lane to each entry.  A lane's
+// pair in range goes to its place in the gather's order (the number of its row's
+// smaller keys) in the row's part of `place`, which the particle's own lane sums
+// from the front.  Bound: the trip of a row's entries and positions to memory, once
+// per four particles; with each such lane selecting its pairs one by one, its list
+// walked for every pair, it was that trip for every entry of every walk.  us a step
+// of jammed mixtures, before -> after: 20k particles 25.2 -> 16.4, 200k 41.4 ->
+// 24.1; 2k pressed to 0.6 of the box's side 59 -> 25 (the gather 47).  Out of the
+// way of the step's straight line (builtin_expect): 1 % of a step where no list is long.
+__device__ __forceinline__ void rl_long_sums(const SysParams &P, const RLArgs &A, const RingInter *mat,
+                                             const RingInter &uni, bool longer, int q, int cnt, int t0, int np, int ti,
+                                             int32_t ko, const double2 *xs, double2 *place, double2 &f) {
+    static_assert(kRlMax == 16, "a lane of a row per entry");
+    const int lane = (int)lane_id(), e = lane & 15, row = lane >> 4;
+    for (unsigned long long m = __ballot(longer); m;) {
+        // the next four
+        int l[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            l[k] = m ? __ffsll(m) - 1 : -1;
+            m &= m - 1;
+        }
+        const int from = row == 0 ? l[0] : row == 1 ? l[1] : row == 2 ? l[2] : l[3];
+        const int src = max(from, 0);
+        const int qs = __shfl(q, src, 64), cs = __shfl(cnt, src, 64), n = from < 0 ? 0 : cs;
+        const int ts = __shfl(t0, src, 64), nps = __shfl(np, src, 64), tis = __shfl(ti, src, 64);
+        const int32_t ks = __shfl(ko, src, 64);
+        bool in = false;
+        unsigned long long key = ~0ull;
+        double2 c = make_double2(0.0, 0.0);
+        if (e < n) {
+            const int32_t w = e < kRlHead ? ((const int32_t *)A.head)[(int64_t)kRlHead * qs + e]
+                                          : A.more[(int64_t)(e - kRlHead) * A.stride + qs];
             const int j = w & kRlSlotMask;
             const double2 pj = A.Pin[j];
-            const double2 d = cdiff(P, x, pj);
+            const double2 d = cdiff(P, xs[src], pj);
             const double r2 = d.x * d.x + d.y * d.y;
-            if (r2 > rl_inter(P, mat, uni, ti, w).max2) continue;
-            const unsigned long long k = visit_key(P, ri, ci, pj, j);
-            if ((first || k > prev) && k < best) {
-                best = k;
-                be = w;
+            const RingInter I = rl_inter(P, mat, uni, tis, w);
+            in = !(r2 > I.max2);
+            if (in) {
+                key = visit_key(P, ks >> 16, ks & 0xffff, pj, j);
+                c = rl_force(I, d, r2, j >= ts && j < ts + nps);
             }
         }
-        if (be < 0) return f;
-        const int j = be & kRlSlotMask;
-        const double2 d = cdiff(P, x, A.Pin[j]);
-        const double2 c = rl_force(rl_inter(P, mat, uni, ti, be), d, d.x * d.x + d.y * d.y, j >= t0 && j < t1);
-        f.x += c.x;
-        f.y += c.y;
-        prev = best;
-        first = false;
+        int at = 0;
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            const unsigned long long o = __shfl(key, (lane & 48) + k, 64);
+            at += o < key ? 1 : 0;
+        }
+        if (in) place[(lane & 48) + at] = c;
+        const unsigned long long hits = __ballot(in);
+        lds_sync();
+        if (lane == l[0] || lane == l[1] || lane == l[2] || lane == l[3]) {
+            const int r = lane == l[0] ? 0 : lane == l[1] ? 1 : lane == l[2] ? 2 : 3;
+            const int k1 = __popcll((hits >> (16 * r)) & 0xffffull);
+            double2 s = make_double2(0.0, 0.0);
+            for (int k = 0; k < k1; k++) {
+                s.x += place[16 * r + k].x;
+                s.y += place[16 * r + k].y;
+            }
+            f = s;
+        }
+        lds_sync();  // before the places are written again
     }
 }
 
@@ -250,7 +281,7 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
 // five launches it replaces (scan 12.1, scatter 8.7, finalize 11.1, pairs 26.2,
 // ring update 38.1); 11.3 against 33 us at 2k particles.
 template <bool LAST, bool BATCH>
-__global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4 : 1))) void k_rl_step(SysParams P0, RLArgs A) {
+__global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(4))) void k_rl_step(SysParams P0, RLArgs A) {
     __shared__ double2 s_a[kRlWG + 32], s_b[kRlWG + 32], s_c[kRlWG + 32];
     __shared__ double s_t[kRlWG + 32];
     __shared__ double s_r[kRlWaves][64 * 3];  // per ring of a wave: sums
@@ -291,6 +322,8 @@ __global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4
 #pragma unroll
     for (int e = 0; e < kRlHead; e++)
         pj[e] = ent[e] >= 0 ? A.Pin[ent[e] & kRlSlotMask] : x;
+    int cnt = 0;  // of a list that the head may not hold
+    if (ent[kRlHead - 1] >= 0) cnt = A.count[q];
 
     // meanwhile: what the ring stage of wave 0 takes from memory and its noise
     uint32_t hi0 = 0u;
@@ -362,14 +395,11 @@ __global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4
             m++;
         }
     }
-    const bool longer = ent[kRlHead - 1] >= 0 && A.count[q] > kRlHead;
+    const bool longer = cnt > kRlHead;
     const bool order = m > 2 && !longer;
-    if (__any(order || longer)) {
-        const int ri = ko >> 16, ci = ko & 0xffff;
-        if (longer) {
-            f[0] = rl_long_sum(P, A, mat, uni, q, t0, t1, t, x, ri, ci);
-            f[1] = f[2] = f[3] = make_double2(0.0, 0.0);
-        } else if (order) {
+    if (__builtin_expect(__any(order), 0)) {
+        if (order) {
+            const int ri = ko >> 16, ci = ko & 0xffff;
             unsigned long long k[kRlHead];
 #pragma unroll
             for (int e = 0; e < kRlHead; e++)
@@ -396,6 +426,7 @@ __global__ __launch_bounds__(kRlWG) __attribute__((amdgpu_waves_per_eu(BATCH ? 4
         Fi.x += f[e].x;
         Fi.y += f[e].y;
     }
+    if (__builtin_expect(__any(longer), 0)) rl_long_sums(P, A, mat, uni, longer, q, cnt, t0, np, t, ko, s_a + wb, s_b + wb, Fi);
 
     // ---- springs and area force
     const double2 ds = wave_diff(P, x, xn);
