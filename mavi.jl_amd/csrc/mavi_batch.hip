@@ -446,10 +446,7 @@ hipError_t batch_stage_in(BatchSub *b, int r, hipStream_t st) {
     const int c = b->cur;
     // a replaced state: its forces are recomputed and every slot binned afresh
     b->keys_ready = false;
-    if (b->rl) {
-        b->rl->valid = b->rl->ordered = false;
-        b->rl->step_hist[0] = b->rl->step_hist[1] = b->rl->step_hist[2] = 0.0;
-    }
+    mavi::rl_renew(b->rl);
     hipError_t e0 = hipMemsetAsync(b->rvalid + r, 0, sizeof(uint32_t), st);
     if (e0 != hipSuccess) return e0;
     const bool rings = Q.kind == KIND_RINGS;
@@ -486,12 +483,19 @@ int sub_gather(BatchSub *b, int64_t nsteps, hipStream_t st) {
 // Steps of the rings replicas on the context's stream: on lists, as a rings
 // system alone, where every replica may.
 int sub_rings(BatchSub *b, int64_t nsteps) {
-    int64_t left = nsteps;
-    if (b->rl && !b->rl->disabled && (b->rl->valid || nsteps >= kRlMinCall)) {
-        const int rc = mavi::rlb_steps(b, nsteps, &left);
+    while (nsteps > 0) {
+        if (b->rl && mavi::rl_take(*b->rl, nsteps)) {
+            const int rc = mavi::rlb_steps(b, nsteps, &nsteps);
+            if (rc != MAVI_OK) return rc;
+            continue;
+        }
+        // (in whole graphs: a step of direct launches costs the host more)
+        const int64_t n = b->rl ? mavi::rl_turn(*b->rl, nsteps, b->graph_steps) : nsteps;
+        const int rc = sub_gather(b, n, b->ctx->stream);
         if (rc != MAVI_OK) return rc;
+        nsteps -= n;
     }
-    return left > 0 ? sub_gather(b, left, b->ctx->stream) : MAVI_OK;
+    return MAVI_OK;
 }
 
 // The plain replicas' steps are queued ahead of the rings replicas', whose

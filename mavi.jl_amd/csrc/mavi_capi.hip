@@ -502,8 +502,7 @@ int mavi_sys_upload(mavi_sys *s, const double *pos, const double *vel, const dou
     }
     s->cur = 0;
     if (s->nl) s->nl->valid = false;  // a new state in id order
-    mavi::rl_invalidate(s);
-    if (s->rl) s->rl->step_hist[0] = s->rl->step_hist[1] = s->rl->step_hist[2] = 0.0;  // its steps may be longer
+    mavi::rl_renew(s->rl);
     HIPCHK(ctx, mavi::drop_keys(s, ctx->stream));
     HIPCHK(ctx, mavi::launch_iota_state(s, ctx->stream));
     if (s->P.potential == MAVI_POT_RINGS) HIPCHK(ctx, mavi::launch_rings_init(s, ctx->stream));
@@ -1009,35 +1008,35 @@ static int steps_impl(mavi_sys *s, int64_t nsteps, const double *noise_host) {
         }
         nsteps = left;  // lists disabled (a list overflowed): the chunk gather runs the rest
     }
-    // Rings on lists: the same bits as the gather, so the choice is free.  A
-    // call that has to build them needs kRlMinCall steps to win the build
-    // back (a build and its checks cost about six gather steps' launches).
-    if (!noise_host && mavi::rl_active(s) && (nsteps >= kRlMinCall || (nsteps > 0 && s->rl->valid))) {
-        while (nsteps > 0) {
-            // up to and including the next step that checks invasions
-            const int64_t until = s->inv_sched ? std::max<int64_t>(s->inv_every - s->inv_since, 0) + 1 : nsteps;
-            const int64_t seg = std::min(nsteps, until);
-            int64_t left = 0;
-            const int rc = mavi::rl_steps(s, seg, &left);
-            if (rc != MAVI_OK) return rc;
-            const int64_t ran = seg - left;
-            nsteps -= ran;
-            if (s->inv_sched) {
-                const bool due = ran > 0 && s->inv_since + ran - 1 >= s->inv_every;
-                s->inv_since = due ? 1 : s->inv_since + ran;
-                const int rc2 = due ? run_invasions(s) : MAVI_OK;
-                if (rc2 != MAVI_OK) return rc2;
+    auto gather = [&](int64_t n) -> int {
+        // only Verlet steps carry forces from one step to the next; the
+        // two-step graph replays from state copy 0 and holds no invasion check
+        const bool rings = s->P.potential == MAVI_POT_RINGS || is_active(s);
+        const bool graphs = s->use_graphs && !s->prof && n >= 4 && !s->var;
+        int64_t k = 0;
+        while (k < n) {
+            // (a rings or self-propelled graph starts from the keys its
+            // update passes leave)
+            const bool keys_ok = !mavi::update_fuses_bin(s) || s->keys_ready;
+            if (graphs && k + 2 <= n && s->cur == 0 && (rings || s->f_valid) && keys_ok && !invasions_due(s, 1)) {
+                HIPCHK(ctx, ensure_graph(s, st));
+                HIPCHK(ctx, hipGraphLaunch(s->graph2, st));
+                if (s->inv_sched) s->inv_since += 2;
+                k += 2;
+                continue;
             }
-            if (left > 0) break;  // the chunk gather runs the rest
-        }
-        if (nsteps == 0) {
-            const int rc = sync_staging(s, true);
+            const bool due = invasions_due(s, 0);
+            const int rc0 = before_step();
+            if (rc0 != MAVI_OK) return rc0;
+            HIPCHK(ctx, launch_step(s, st, s->f_valid));
+            const int rc = after_step(due);
             if (rc != MAVI_OK) return rc;
-            return check_flags(s);
+            k++;
         }
-    }
-    mavi::rl_invalidate(s);  // (a captured graph moves the state without passing launch_bin's host side)
+        return MAVI_OK;
+    };
     if (noise_host) {
+        mavi::rl_invalidate(s);
         // draws per step: one per ring (rings), one (Szabo) or two (RTP) per particle
         const int64_t nr = s->P.potential == MAVI_POT_RINGS ? s->P.nrings
                            : s->P.potential == MAVI_POT_RTP ? 2 * (int64_t)s->P.n
@@ -1060,30 +1059,29 @@ static int steps_impl(mavi_sys *s, int64_t nsteps, const double *noise_host) {
             if (rc != MAVI_OK) return rc;
         }
     } else {
-        // only Verlet steps carry forces from one step to the next; the
-        // two-step graph replays from state copy 0 and holds no invasion check
-        const bool rings = s->P.potential == MAVI_POT_RINGS || is_active(s);
-        const bool graphs = s->use_graphs && !s->prof && nsteps >= 4 && !s->var;
-        int64_t k = 0;
-        while (k < nsteps) {
-            // (a rings or self-propelled graph starts from the keys its
-            // update passes leave)
-            const bool keys_ok = !mavi::update_fuses_bin(s) || s->keys_ready;
-            if (graphs && k + 2 <= nsteps && s->cur == 0 && (rings || s->f_valid) && keys_ok &&
-                !invasions_due(s, 1)) {
-                HIPCHK(ctx, ensure_graph(s, st));
-                HIPCHK(ctx, hipGraphLaunch(s->graph2, st));
-                if (s->inv_sched) s->inv_since += 2;
-                k += 2;
+        // Rings on lists: the same bits as the gather, so the choice is free
+        while (nsteps > 0) {
+            if (mavi::rl_allowed(s) && mavi::rl_take(*s->rl, nsteps)) {
+                // up to and including the next step that checks invasions
+                const int64_t until = s->inv_sched ? std::max<int64_t>(s->inv_every - s->inv_since, 0) + 1 : nsteps;
+                const int64_t seg = std::min(nsteps, until);
+                int64_t left = 0;
+                int rc = mavi::rl_steps(s, seg, &left);
+                if (rc != MAVI_OK) return rc;
+                const int64_t ran = seg - left;
+                nsteps -= ran;
+                if (s->inv_sched) {
+                    const bool due = ran > 0 && s->inv_since + ran - 1 >= s->inv_every;
+                    s->inv_since = due ? 1 : s->inv_since + ran;
+                    if (due && (rc = run_invasions(s)) != MAVI_OK) return rc;
+                }
                 continue;
             }
-            const bool due = invasions_due(s, 0);
-            const int rc0 = before_step();
-            if (rc0 != MAVI_OK) return rc0;
-            HIPCHK(ctx, launch_step(s, st, s->f_valid));
-            const int rc = after_step(due);
+            mavi::rl_invalidate(s);  // (a captured graph moves the state without passing launch_bin's host side)
+            const int64_t n = mavi::rl_allowed(s) ? mavi::rl_turn(*s->rl, nsteps, 2) : nsteps;
+            const int rc = gather(n);
             if (rc != MAVI_OK) return rc;
-            k++;
+            nsteps -= n;
         }
     }
     int rc = sync_staging(s, true);
@@ -1566,6 +1564,7 @@ int mavi_sys_set_option(mavi_sys *s, int32_t option, int32_t value) {
             if (s->rl) {
                 s->rl->on = value != 0;
                 mavi::rl_invalidate(s);
+                mavi::rl_reset(*s->rl);
             }
             changed = true;
             break;

@@ -219,13 +219,24 @@ struct NList {
 
 constexpr double kRlSkin = 0.3;      // default list skin of rings (fraction of the widest range)
 constexpr int kRlGraphSteps = 8;     // steps per captured graph (even)
-constexpr int64_t kRlMinCall = 8;    // a call that has to build lists needs this many steps to win the build
+// A call that has to build the rings lists has at least this many steps (a
+// build and its checks cost about 100 us at any size; us a call with an upload,
+// gather and lists: 8 steps of 2k particles 316, 198, of 800k 1250, 903).
+constexpr int64_t kRlMinCall = 8;
+// Steps that go to the gather after the lists had to give up on a state (steps
+// too long, a chunk that may be over its capacity), doubled while that repeats:
+// a try that fails costs 100 to 300 us.
+constexpr int64_t kRlWaitMin = 64, kRlWaitMax = 2048;
 
 // Verlet lists of a rings system with a fixed population (mavi_rlist.hip).
 struct RList {
     bool on = true;           // option MAVI_OPT_NLIST
     bool fits = false;        // the list grid has at least 3 x 3 cells
-    bool disabled = false;    // a list or a chunk overflowed: the chunk gather takes over
+    bool disabled = false;    // a list overflowed: the chunk gather takes over, until a new state or skin
+    int32_t skip = 0, skip_next = 1;  // calls on new states until a disabled list is tried again (doubling, at most 64)
+    int64_t wait = 0, backoff = 0;    // gather steps before the lists are tried again, and the last such turn
+    int64_t ran = 0;          // steps since the last such turn
+    bool renewed = true, first = false;  // a new state since rl_take; since the last steps on lists
     bool ordered = false;     // the state lies in ring order, both copies' ids too
     bool valid = false;       // lists complete for the current state
     bool uniform = false;     // one interaction for all type pairs (a batch: every ring full)
@@ -462,19 +473,29 @@ hipError_t nl_measure(mavi_sys *s, hipStream_t st);
 hipError_t nl_settle(mavi_sys *s, hipStream_t st);
 void nl_set_skin(mavi_sys *s, double skin_frac);
 double nl_default_skin(const mavi_sys *s);
-// Lists of a rings system (mavi_rlist.hip).  rl_active: the next steps may run
-// on them; rl_steps: up to nsteps steps (*left > 0: the chunk gather runs the
-// rest); rl_invalidate: the state was moved or reordered by other kernels.
+// Lists of a rings system (mavi_rlist.hip).  rl_allowed: steps may run on them
+// (rl_active: and no list overflowed); rl_take: the next ones do, of a call that
+// has n to go; rl_steps: up to nsteps steps (*left > 0: they gave up on the
+// state); rl_turn: how many of n steps the gather takes (in whole units) before
+// the lists are asked again; rl_invalidate: the state was moved or reordered by
+// other kernels; rl_renew: it was replaced; rl_reset: forget that they gave up.
 bool rl_eligible(const mavi_sys *s);
 hipError_t rl_alloc(mavi_sys *s, hipStream_t st);
 void rl_free(mavi_sys *s);
 bool rl_set_skin(mavi_sys *s, double skin_frac);
 void rl_drop_graph(mavi_sys *s);
+bool rl_allowed(const mavi_sys *s);
 bool rl_active(const mavi_sys *s);
+bool rl_take(RList &N, int64_t n);
 int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left);
+int64_t rl_turn(RList &N, int64_t n, int64_t unit);
 inline void rl_invalidate(mavi_sys *s) {
     if (s->rl) s->rl->valid = s->rl->ordered = false;
 }
+inline void rl_renew(RList *N) {
+    if (N) N->renewed = true, N->valid = N->ordered = false;
+}
+void rl_reset(RList &N);
 // Counting sort of the slots on another grid over the same space, the state
 // left where it is: s->src, s->scell, s->start.
 hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,

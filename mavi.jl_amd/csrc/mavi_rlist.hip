@@ -918,15 +918,29 @@ hipError_t rl_rebuild(const RLSys &E, hipStream_t st) {
 
 double rl_step_est(const RList &N) { return std::max(N.step_hist[0], std::max(N.step_hist[1], N.step_hist[2])); }
 
-// Steps from a block start that keep d_start + (steps - 1) x step within
-// half_skin, at a step 1.08 times the estimate.
-int64_t rl_room(const RList &N) {
-    const double r = (N.half_skin - N.d_start) / (1.08 * rl_step_est(N));
+// Steps from a block start that keep d + (steps - 1) x step within half_skin, at
+// a step 1.08 times the estimate; d: the largest displacement there.
+int64_t rl_fit(const RList &N, double d) {
+    const double r = (N.half_skin - d) / (1.08 * rl_step_est(N));
     if (!(r < 1e9)) return INT64_MAX;
     return (int64_t)floor(r) + 1;
 }
+int64_t rl_room(const RList &N) { return rl_fit(N, N.d_start); }
 
+// Lists that would serve fewer steps go to the gather.  us for 200 steps of
+// jammed mixtures with 6, 3, 2 and 1 here (gather: 6890 .. 11470): 2k particles
+// at dt 0.01 6060, 6040, 3970, 4360; 20k at 0.005 6590, 4910, 4940, 5090, at 0.02
+// 6780, 6770, 6760, 8420; 200k at 0.005 10560, 7490, 7440, 7650.
+constexpr int64_t kRlMinFit = 2;
 constexpr int64_t kRlMinBlock = 6;  // shorter blocks cost more than the rebuild they put off
+constexpr int64_t kRlNewBlock = 8;  // most steps of the first block on a new state
+
+// The lists give the state to the gather for a while.
+void rl_back_off(RList &N) {
+    N.backoff = N.ran > 4 * N.backoff ? kRlWaitMin : std::clamp(2 * N.backoff, kRlWaitMin, kRlWaitMax);
+    N.wait = N.backoff;
+    N.ran = 0;
+}
 
 // Blocks of steps with one read back each (see the top); *left > 0: the chunk
 // gather runs the rest.
@@ -937,13 +951,26 @@ int rl_run(const RLSys &E, int64_t nsteps, int64_t *left) {
     *left = 0;
     const int span = std::max(std::max(E.nslots, E.nrings), std::max(N.nbmax, E.nflags));
     int64_t k = 0;
+    bool first = N.first;  // on a new state
+    N.first = false;
     while (k < nsteps) {
-        const bool fresh = !N.valid;
-        if (fresh) HIPCHK(ctx, rl_rebuild(E, st));
+        const double est = rl_step_est(N);
+        if (N.block == 0 && N.valid && est > 0.0) {
+            // lists that serve few more steps are rebuilt, unless these are the
+            // call's last or new ones would serve few
+            const int64_t few = std::min(std::min(kRlMinBlock, nsteps - k), std::max<int64_t>(1, rl_fit(N, 0.0) / 4));
+            if (rl_room(N) < few) N.valid = false;
+        }
+        if (N.block == 0 && !N.valid && !first && est > 0.0 && rl_fit(N, 0.0) <= kRlMinFit) {
+            rl_back_off(N);
+            *left = nsteps - k;
+            return MAVI_OK;
+        }
+        if (!N.valid) HIPCHK(ctx, rl_rebuild(E, st));
         int64_t want = N.block_now;
         if (N.block == 0) {
-            if (rl_step_est(N) > 0.0) want = std::min(want, std::max<int64_t>(1, rl_room(N)));
-            else want = std::min<int64_t>(want, 8);  // no step length measured yet
+            if (first || !(est > 0.0)) want = std::min<int64_t>(want, kRlNewBlock);
+            if (est > 0.0) want = std::min(want, std::max<int64_t>(1, rl_room(N)));
         }
         const int64_t blk = std::min<int64_t>(want, nsteps - k);
         const int cur0 = *E.cur;
@@ -977,6 +1004,8 @@ int rl_run(const RLSys &E, int64_t nsteps, int64_t *left) {
         const double step = sqrt(__builtin_bit_cast(double, N.host[0]));
         const double d_end = sqrt(__builtin_bit_cast(double, N.host[1]));
         const uint32_t status = (uint32_t)N.host[2];
+        if (first) N.step_hist[0] = N.step_hist[1] = N.step_hist[2] = 0.0;  // of the state before
+        first = false;
         N.step_hist[N.step_i] = step;
         N.step_i = (N.step_i + 1) % 3;
         // The block evaluated y_0 .. y_{T-1} and moved to y_T: y_t is within
@@ -994,11 +1023,22 @@ int rl_run(const RLSys &E, int64_t nsteps, int64_t *left) {
             // (one step from a fresh build evaluates the build positions: its
             // bound is 0, so a block can always shrink to one that passes)
             if (status || !finite) {
-                // the chunk gather takes over, for good if a list or a chunk
-                // overflowed, for this call if the state is not finite
-                N.disabled = status != 0;
-                if (!finite) N.step_hist[0] = N.step_hist[1] = N.step_hist[2] = 0.0;
+                // the chunk gather takes over: until a new state if a list
+                // overflowed, for a while if a chunk may have (it checks
+                // exactly: a particle may have been counted in before another
+                // of its step was counted out), for this call if the state is
+                // not finite
                 *left = nsteps - k;
+                if (status & kRlOverflow) {
+                    N.disabled = true;
+                    N.skip = N.skip_next;
+                    N.skip_next = std::min(2 * N.skip_next, 64);
+                } else if (!finite) {
+                    N.wait = *left;
+                } else {
+                    rl_back_off(N);
+                }
+                if (!finite) N.step_hist[0] = N.step_hist[1] = N.step_hist[2] = 0.0;
                 return MAVI_OK;
             }
             if (N.block != 0 && N.block_now > 1) N.block_now = std::max(1, N.block_now / 2);
@@ -1007,17 +1047,10 @@ int rl_run(const RLSys &E, int64_t nsteps, int64_t *left) {
         hipLaunchKernelGGL(k_rl_copy_counter, dim3(1), dim3(64), 0, st, N.counter + N.ph, E.counter);
         HIPCHK(ctx, hipGetLastError());
         k += blk;
+        N.ran += blk;
+        N.skip_next = 1;
         N.d_start = d_end;
-        if (N.block == 0) {
-            if (rl_room(N) < kRlMinBlock) N.valid = false;
-            // steps so long that a fresh list would serve only a few: the gather
-            if (!N.valid && 1.08 * rl_step_est(N) * (double)kRlMinBlock > N.half_skin && k < nsteps) {
-                *left = nsteps - k;
-                return MAVI_OK;
-            }
-        } else if (d_end + 1.2 * step * (double)N.block_now > N.half_skin) {
-            N.valid = false;
-        }
+        if (N.block != 0 && d_end + 1.2 * step * (double)N.block_now > N.half_skin) N.valid = false;
         const int32_t cap = N.block == 0 ? kNlBlockCap : N.block;
         if (N.block_now < cap) N.block_now = std::min(cap, 2 * N.block_now);
     }
@@ -1067,6 +1100,7 @@ bool rl_set_skin(mavi_sys *s, double skin_frac) {
     RList &N = *s->rl;
     N.fits = rl_grid(s->P, sqrt(s->list2), skin_frac, N.G, N.rl2, N.half_skin);
     N.valid = false;
+    rl_reset(N);
     N.scan_stale = true;
     return N.fits;
 }
@@ -1201,8 +1235,31 @@ hipError_t rlb_alloc(BatchSub *b, hipStream_t st) {
     return e;
 }
 
-bool rl_active(const mavi_sys *s) {
-    return s->rl && s->rl->on && s->rl->fits && !s->rl->disabled && !s->neigh_on && !s->var;
+bool rl_allowed(const mavi_sys *s) { return s->rl && s->rl->on && s->rl->fits && !s->neigh_on && !s->var; }
+
+bool rl_active(const mavi_sys *s) { return rl_allowed(s) && !s->rl->disabled; }
+
+bool rl_take(RList &N, int64_t n) {
+    if (N.renewed) {
+        N.renewed = false;
+        N.first = true;
+        if (N.disabled && --N.skip <= 0) N.disabled = false;
+    }
+    if (N.disabled || N.wait > 0) return false;
+    return n >= kRlMinCall || (N.valid && (N.block != 0 || rl_room(N) >= n));
+}
+
+int64_t rl_turn(RList &N, int64_t n, int64_t unit) {
+    if (N.disabled || N.wait <= 0) return n;
+    n = std::min(n, (N.wait + unit - 1) / unit * unit);
+    N.wait -= n;
+    return n;
+}
+
+void rl_reset(RList &N) {
+    N.disabled = false;
+    N.skip_next = 1;
+    N.wait = N.backoff = 0;
 }
 
 int rl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {

@@ -252,3 +252,70 @@ def test_skin_changes_on_a_grid_of_several_scan_tiles(gpu_ctx):
         b.advance(20)
         assert a.dev.nlist_info()["active"]
         same(skin, a, b)
+
+
+def test_lists_come_back_after_a_full_chunk(gpu_ctx):
+    """Chunks over their capacity fail the call; a good state uploaded after it
+    runs on lists again, and so does a thinner skin after lists that were too
+    long."""
+    import mavi_hip as mv
+    from mavi_hip import _lib, rings
+
+    state, space, cfg, ic = CASES["normal"]()
+    ic = mv.IntCfg(dt=1e-3, chunks_cfg=ic.chunks_cfg, device=mv.GPU())
+    d, _, keep = rings.describe(state, space, cfg, ic, 1)
+    d.nc = 6
+    crowd = state.pos.copy().reshape(-1, 10, 2)
+    box, num = space.geometry_cfg, ic.chunks_cfg
+    ang = np.arange(10) * 2 * np.pi / 10
+    for k in range(4):  # four rings drawn together about the corner of four chunks
+        at = np.array([box.length / num.num_cols, box.height / num.num_rows]) * 4
+        crowd[k] = at + (0.35 * (2 * (k % 2) - 1), 0.35 * (2 * (k // 2) - 1)) + \
+            0.3 * np.stack([np.cos(ang), np.sin(ang)], axis=1)
+    out = []
+    for lists in (1, 0):
+        dev = _lib.DeviceSystem(gpu_ctx, d, keep=keep)
+        dev.set_option(_lib.MAVI_OPT_NLIST, lists)
+        dev.upload(crowd.reshape(-1, 2), None, state.pol)
+        with pytest.raises(mv.CellOverflowError):
+            dev.step(30)
+        dev.set_noise_state(1, 0)
+        dev.upload(state.pos, None, state.pol)
+        dev.step(40)
+        say(f"[rings lists] after a full chunk: {dev.nlist_info()}")
+        assert dev.nlist_info()["active"] == bool(lists)
+        pos, pol = np.zeros_like(state.pos), np.zeros_like(state.pol)
+        dev.download(pos, None, pol)
+        out.append((pos, pol))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+
+    a, b = make("dense", True), make("dense", False)
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, 2000)
+    for s in (a, b):
+        s.dev.step(20)
+    assert not a.dev.nlist_info()["active"]
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, 0)
+    for s in (a, b):
+        s.dev.step(20)
+    assert a.dev.nlist_info()["active"]
+    same("after long lists", a, b)
+
+
+def test_steps_too_long_for_lists_go_to_the_gather(gpu_ctx):
+    """Runs whose particles cross half the skin in a step or two: the lists are
+    tried now and then, not once or twice in every call."""
+    from mavi_hip import _lib
+
+    a, b = make("normal", True, dt=0.02), make("normal", False, dt=0.02)
+    a.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, 100)
+    start = a.state.pos.copy()
+    for s in (a, b):
+        for _ in range(30):
+            s.state.pos[...] = start
+            s.upload()
+            s.dev.step(10)
+    info = a.dev.nlist_info()
+    say(f"[rings lists] long steps {info}")
+    assert info["active"] and info["rebuilds"] <= 8
+    same("long steps", a, b)
