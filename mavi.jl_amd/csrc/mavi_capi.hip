@@ -943,8 +943,8 @@ static int nl_steps(mavi_sys *s, int64_t nsteps, int64_t *left) {
             // a list overflowed, a chunk count may have passed the capacity
             // (the chunk gather checks it exactly), or one step from a fresh
             // build moved a particle more than skin / 2
-            if (status && !N.skin_set && N.skin_frac > kNlSkin) {
-                // lists that a thinner skin may hold
+            if (status == kNlOverflow && !N.skin_set && N.skin_frac > kNlSkin) {
+                // lists that a thinner skin may hold (a full chunk it does not help)
                 nl_drop_graph(s);
                 mavi::nl_set_skin(s, kNlSkin);
                 half_skin = sqrt(N.thr2);

@@ -173,6 +173,10 @@ struct RingRates {
 constexpr int32_t kNlBlockCap = 60;  // most steps between host checks of the list validity
 
 constexpr double kNlSkin = 0.15, kNlWideSkin = 0.3;  // default skins of plain systems (nl_default_skin)
+// status word of the lists of a plain system
+constexpr uint32_t kNlOverflow = 1u;  // a list held more than kmax entries, or a partner more
+                                      // than 32767 slots away
+constexpr uint32_t kNlCapacity = 2u;  // a chunk count passed the capacity during a step's moves
 
 // Verlet neighbour lists of a finite-range plain system (LJ with a cutoff,
 // HarmTrunc) whose chunks are at least the interaction range wide (mavi_nlist.hip).

@@ -56,9 +56,6 @@
 namespace {
 
 constexpr uint32_t kEdgeBit = 0x80000000u;  // ncount: minimum image needed
-constexpr uint32_t kStatusOverflow = 1u;    // a list held more than kmax entries, or a partner more
-                                            // than 32767 slots away (modulo na)
-constexpr uint32_t kStatusCapacity = 2u;    // a chunk count passed the capacity during a step's moves
 constexpr int kNlMax = 48;                  // list entries per particle (12 groups of 4)
 constexpr int kNeedBlock = 64;              // workgroup of the evaluation kernels: one wave, so waves of
                                             // unequal length free and take CU slots one at a time
@@ -463,7 +460,7 @@ __device__ __forceinline__ void build_cell(const SysParams &P, const int32_t *__
             const int pad = (((cw + 3) >> 2) << 2) - cw;
             *(lane < pad ? &w_list[p][cw + lane] : &w_dump[lane]) = 0;
             if (__any(far) || over) {
-                if (lane == 0) atomicOr(status, kStatusOverflow);
+                if (lane == 0) atomicOr(status, kNlOverflow);
             }
             my_count = lane == p ? cw : my_count;
             ng_max = max(ng_max, (cw + 3) >> 2);
@@ -549,7 +546,7 @@ __global__ __launch_bounds__(64 * kBuildWaves) void k_nl_build(SysParams G, SysP
     }
     if (M > kBuildCand) {
         for (int i = t0 + lane; i < t1; i += 64) ncount[i] = 0;
-        if (lane == 0) atomicOr(status, kStatusOverflow);
+        if (lane == 0) atomicOr(status, kNlOverflow);
         return;
     }
     // On a periodic list grid of at least 7 x 7 cells the image of a
@@ -664,7 +661,7 @@ __device__ __forceinline__ Drift nl_drift(const SysParams &P, const NLArgs &A, i
         // while one step's moves are applied a count runs through values at
         // least as large as its final one
         if (atomicAdd(&A.ccnt[(kn >> 16) * P.cols + (kn & 0xffff)], 1) + 1 > P.nc)
-            atomicOr(A.status, kStatusCapacity);
+            atomicOr(A.status, kNlCapacity);
     }
     const double lx = px - pi.x, ly = py - pi.y;  // the step's length, squared
     D.l2 = lx * lx + ly * ly;

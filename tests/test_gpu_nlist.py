@@ -309,3 +309,33 @@ def test_default_skin_falls_back_before_the_gather(gpu_ctx):
         runs.append((s.state.pos.copy(), s.state.vel.copy(), s.forces.copy()))
     for a, b in zip(*runs):
         assert np.array_equal(a, b)
+
+
+def test_full_chunk_leaves_the_skin(gpu_ctx):
+    """A chunk over its capacity hands HarmTrunc steps to the chunk gather at
+    once: a thinner skin, for lists that are too long, would not help."""
+    import mavi_hip as mv
+    from mavi_hip import _lib
+
+    side = 24
+    ix = np.arange(side * side)
+    pos = np.stack([(ix % side + 0.5) * 1.2, (ix // side + 0.5) * 1.2], axis=1)
+    L = 1.2 * side
+    # a clump on the corner of four chunks, from one into the next
+    pos[:36] = 5 * L / 23 + 0.3 * np.stack([np.arange(36) % 6 - 2.5, np.arange(36) // 6 - 2.5], axis=1)
+    vel = 0.1 * np.random.default_rng(2).normal(size=pos.shape)
+    vel[:36] = (3.0, 0.0)
+    dyn = mv.HarmTruncCfg(k_rep=1.0, k_atr=0.0, dist_eq=1.0, dist_max=1.2)
+    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=L, height=L))
+    ic = mv.IntCfg(dt=1e-3, chunks_cfg=mv.ChunksCfg(num_cols=23, num_rows=23), device=mv.GPU())
+    from mavi_hip.systems import describe
+
+    d, _ = describe(mv.SecondLawState(pos=pos, vel=vel), space, dyn, ic)
+    d.nc = 4
+    dev = _lib.DeviceSystem(gpu_ctx, d)
+    dev.upload(pos, vel)
+    with pytest.raises(mv.CellOverflowError):
+        dev.step(100)
+    info = dev.nlist_info()
+    say(f"[full chunk] {info}")
+    assert info["rollbacks"] == 1 and not info["active"]
