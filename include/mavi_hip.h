@@ -322,7 +322,9 @@ int mavi_sys_noise_set(mavi_sys *sys, uint64_t seed, uint64_t counter);
  *                       8 steps and more), with the chunk gather's bits.
  *                       0: the chunk gather
  *   MAVI_OPT_NLIST_SKIN skin in thousandths of the range (0: LJ 150, HarmTrunc
- *                       300, or 150 if those lists overflow, rings 300)
+ *                       300 with fewer than 5 partners within the range at the
+ *                       mean density unless those lists overflow, else 150,
+ *                       rings 300)
  *   MAVI_OPT_NLIST_BLOCK steps between displacement checks (0: as many as
  *                       the displacement bound allows at the last measured
  *                       step length, at most 60) */

@@ -956,13 +956,19 @@ bool nl_eligible(const mavi_sys *s) {
     return P.cl >= range * (1.0 + 1e-12) && P.ch >= range * (1.0 + 1e-12);
 }
 
-// The skin without an option.  HarmTrunc lists are short (a few partners at a
-// range of about the particles' size), so a wider skin costs a step little and
-// halves the rebuilds: 0.15 -> 0.3, us a step with the rebuilds: 22k walled discs
-// 11.2 -> 9.6, 160k 18.5 -> 15.6, 490k 37.8 -> 28.4, 1M 66.2 -> 47.8 (0.25: 51.2,
-// 0.4: 46.0 there, 9.9 at 22k).  Lennard-Jones lists hold ~20 partners: 0.15
-// against 0.2 and 0.3: 1k 8.9, 9.4, 10.1, 102k 13.9, 14.5, 15.7.
-double nl_default_skin(const mavi_sys *s) { return s->P.potential == MAVI_POT_HARMTRUNC ? kNlWideSkin : kNlSkin; }
+// The skin without an option.  HarmTrunc lists with few partners within the range
+// (about the particles' size): a wider skin costs a step little and halves the
+// rebuilds.  With more it lengthens lists that are the step's cost.  us for 300
+// steps at skins 0.15 and 0.3, by partners at the mean density: 2.7 (density 0.6,
+// range 1.2) 1k particles 2620, 2470, 22k 3396, 2996, 202k 6201, 5027; 4.1 (0.9,
+// 1.2) 2708, 2692, 3244, 3227, 5789, 5245; 5.6 (0.7, 1.6) 2695, 2838, 3457, 3594,
+// 5721, 5798; 8.8 (0.7, 2) 3148, 3527, 4077, 4511, 6714, 7243; 20 (0.7, 3) 4205,
+// 5319, 6284, 7420, 10293, 12282.  Lennard-Jones lists hold ~20: 0.15 against 0.2
+// and 0.3: 1k 8.9, 9.4, 10.1 us a step, 102k 13.9, 14.5, 15.7.
+double nl_default_skin(const mavi_sys *s) {
+    const double r = nl_range(s), partners = M_PI * r * r * (double)s->P.na / (s->P.L * s->P.H);
+    return s->P.potential == MAVI_POT_HARMTRUNC && partners < 5.0 ? kNlWideSkin : kNlSkin;
+}
 
 void nl_set_skin(mavi_sys *s, double skin_frac) {
     NList &N = *s->nl;

@@ -294,8 +294,9 @@ def test_default_skin_falls_back_before_the_gather(gpu_ctx):
     pos = np.stack([ix % side + 0.5, ix // side + 0.5], axis=1) + 0.02 * rng.uniform(-1, 1, (side * side, 2))
     vel = 2.0 * rng.normal(size=pos.shape)
     dyn = mv.HarmTruncCfg(k_rep=0.5, k_atr=0.05, dist_eq=2.0, dist_max=3.05)
-    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=float(side), height=float(side)))
-    ic = mv.IntCfg(dt=1e-4, chunks_cfg=mv.ChunksCfg(num_cols=13, num_rows=13), device=mv.GPU())
+    box = 3.0 * side  # mostly empty: the mean density takes the wide skin
+    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=box, height=box))
+    ic = mv.IntCfg(dt=1e-4, chunks_cfg=mv.ChunksCfg(num_cols=39, num_rows=39), device=mv.GPU())
     runs = []
     for skin in (0, 150):
         s = mv.System(state=mv.SecondLawState(pos=pos.copy(), vel=vel.copy()), space_cfg=space, dynamic_cfg=dyn,
@@ -339,3 +340,31 @@ def test_full_chunk_leaves_the_skin(gpu_ctx):
     info = dev.nlist_info()
     say(f"[full chunk] {info}")
     assert info["rollbacks"] == 1 and not info["active"]
+
+
+@pytest.mark.parametrize("reach,wide", [(1.2, True), (2.5, False)])
+def test_default_skin_by_partners(gpu_ctx, reach, wide):
+    """Few partners within the range take the wide skin, many the thin one: the
+    run rebuilds its lists as often as with that skin by the option."""
+    import mavi_hip as mv
+    from mavi_hip import _lib
+
+    rng = np.random.default_rng(6)
+    side, a = 30, 1.15
+    ix = np.arange(side * side)
+    pos = a * np.stack([ix % side + 0.5, ix // side + 0.5], axis=1)
+    vel = 2.0 * rng.normal(size=pos.shape)
+    dyn = mv.HarmTruncCfg(k_rep=10.0, k_atr=0.01, dist_eq=1.0, dist_max=reach)
+    L = a * side
+    space = mv.SpaceCfg(wall_type=mv.PeriodicWalls(), geometry_cfg=mv.RectangleCfg(length=L, height=L))
+    ic = mv.IntCfg(dt=1e-3, chunks_cfg=mv.ChunksCfg(num_cols=int(L // reach), num_rows=int(L // reach)), device=mv.GPU())
+    builds = {}
+    for skin in (0, 150, 300):
+        s = mv.System(state=mv.SecondLawState(pos=pos.copy(), vel=vel.copy()), space_cfg=space, dynamic_cfg=dyn,
+                      int_cfg=ic)
+        if skin:
+            s.dev.set_option(_lib.MAVI_OPT_NLIST_SKIN, skin)
+        s.advance(300)
+        builds[skin] = s.dev.nlist_info()["rebuilds"]
+    say(f"[skin by partners] {reach}: {builds}")
+    assert builds[150] != builds[300] and builds[0] == builds[300 if wide else 150]
