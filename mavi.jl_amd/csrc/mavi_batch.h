@@ -28,11 +28,13 @@ enum { KIND_LJ = 0, KIND_HT = 1, KIND_RINGS = 2, NKIND = 3 };
 // numbered from 0.
 struct BatchSub {
     mavi_ctx *ctx = nullptr;
+    PinBuf *pin = nullptr;  // the batch's
     bool rings = false;
     std::vector<int32_t> global;  // batch index of each replica
     std::vector<Replica> reps;
     int64_t nids = 0, nactive = 0, nslots = 0, ncells = 0, nrings = 0;
     SysParams G{};  // na = nslots, ncell = ncells: the sort over all replicas
+    uint8_t *arena = nullptr;  // holds all device arrays below
     // per-kind wave lists
     int2 *items[NKIND] = {nullptr, nullptr, nullptr};
     int32_t nitems[NKIND] = {0, 0, 0};

@@ -42,6 +42,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -296,7 +297,7 @@ struct mavi_batch {
     std::vector<Where> where;  // of each replica
     std::vector<char> uploaded;
     PinBuf pin;
-    hipStream_t side = nullptr;  // the plain replicas' steps where both families are there
+    hipStream_t side = nullptr;  // the context's, for the plain replicas' steps where both families are there
     hipEvent_t fork = nullptr, join = nullptr;
     // execution shape: plain, rings
     int32_t wg[2] = {256, 256};
@@ -675,9 +676,19 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
     b->G.ncell = (int32_t)ncells;
 
     hipStream_t st = ctx->stream;
-    hipError_t e = hipSuccess;
-#define ALLOC(ptr, cnt) \
-    if (e == hipSuccess) e = dalloc(&(ptr), (cnt), st)
+    // all arrays in one allocation: forty for a family, and two families, took
+    // longer than a short run of a small batch
+    struct Part {
+        void **p;
+        size_t at;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+#define ALLOC(ptr, cnt)                                                                            \
+    do {                                                                                           \
+        parts.push_back({(void **)&(ptr), total});                                                 \
+        total += (sizeof(*(ptr)) * (size_t)std::max<int64_t>((cnt), 1) + 255) / 256 * 256;         \
+    } while (0)
     for (int c = 0; c < 2; c++) {
         ALLOC(b->P_[c], nslots);
         ALLOC(b->V_[c], nslots);
@@ -725,6 +736,8 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
         ALLOC(b->inter, (int64_t)inter.size());
     }
 #undef ALLOC
+    hipError_t e = dalloc(&b->arena, (int64_t)total, st);
+    for (const Part &q : parts) *q.p = e == hipSuccess ? b->arena + q.at : nullptr;
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     auto up = [&](void *dst, const void *srcp, size_t bytes) {
@@ -752,20 +765,7 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
 void sub_free(BatchSub *b) {
     drop_graph(b);
     mavi::rlb_free(b);
-    for (int c = 0; c < 2; c++) {
-        dfree(b->P_[c]);
-        dfree(b->V_[c]);
-        dfree(b->ID_[c]);
-    }
-    for (int k = 0; k < NKIND; k++) dfree(b->items[k]);
-    dfree(b->ring_wave_rep); dfree(b->d_reps); dfree(b->wave_rep);
-    dfree(b->F); dfree(b->P2); dfree(b->F1);
-    dfree(b->perm); dfree(b->needc); dfree(b->epoch); dfree(b->rvalid);
-    dfree(b->key); dfree(b->rank); dfree(b->src); dfree(b->scell); dfree(b->sid); dfree(b->slot_of);
-    dfree(b->cnt); dfree(b->start); dfree(b->scan_state); dfree(b->scan_ticket); dfree(b->flags); dfree(b->counter);
-    dfree(b->active_ids); dfree(b->pos_id); dfree(b->vel_id); dfree(b->force_id);
-    dfree(b->pol); dfree(b->areas); dfree(b->cms); dfree(b->cms_next); dfree(b->cpos);
-    dfree(b->rtype); dfree(b->types); dfree(b->inter);
+    dfree(b->arena);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     delete b;
@@ -790,10 +790,9 @@ int mavi_batch_destroy(mavi_batch *b) {
     (void)hipStreamSynchronize(b->ctx->stream);
     for (BatchSub *u : b->sub)
         if (u) sub_free(u);
-    if (b->pin.p) (void)hipHostFree(b->pin.p);
+    mavi::pin_give(b->ctx, b->pin);
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
-    if (b->side) (void)hipStreamDestroy(b->side);
     mavi_ctx *ctx = b->ctx;
     delete b;
     ctx_release(ctx);
@@ -831,6 +830,7 @@ int mavi_batch_finalize(mavi_batch *b) {
         u = nullptr;
     }
     b->where.clear();
+    for (const HostSys &h : b->hs) b->pin.fit(h.P.n);
     int64_t nslots = 0, nids = 0, ncells = 0;
     for (size_t r = 0; r < b->hs.size(); r++) {
         const HostSys &h = b->hs[r];
@@ -839,6 +839,7 @@ int mavi_batch_finalize(mavi_batch *b) {
         if (!u) {
             u = new BatchSub();
             u->ctx = ctx;
+            u->pin = &b->pin;
             u->rings = k == 1;
         }
         b->where.push_back({k, (int32_t)u->global.size()});
@@ -861,11 +862,13 @@ int mavi_batch_finalize(mavi_batch *b) {
         if (rc != MAVI_OK) return rc;
     }
     if (b->sub[0] && b->sub[1]) {
-        if (!b->side) HIPCHK(ctx, hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
+        // (a stream takes up to 3 ms to make: one for all batches of the context)
+        std::lock_guard<std::mutex> hold(ctx->pins_lock);
+        if (!ctx->side) HIPCHK(ctx, hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
+        b->side = ctx->side;
         if (!b->fork) HIPCHK(ctx, hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
         if (!b->join) HIPCHK(ctx, hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     }
-    for (const HostSys &h : b->hs) b->pin.fit(h.P.n);
     b->uploaded.assign(b->hs.size(), 0);
     b->hs.clear();
     b->hs.shrink_to_fit();

@@ -93,6 +93,8 @@ int mavi_ctx_create(int device, mavi_ctx **out) {
 
 static void ctx_free(mavi_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
+    for (PinBuf &q : ctx->pins) (void)hipHostFree(q.p);
+    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -157,7 +159,7 @@ static void sys_free(mavi_sys *s) {
     dfree(s->rmask); dfree(s->dsinks); dfree(s->dboxes); dfree(s->box_mask);
     if (s->vrb) (void)hipFree(s->vrb);
     if (s->vstage) (void)hipHostFree(s->vstage);
-    if (s->pin.p) (void)hipHostFree(s->pin.p);
+    mavi::pin_give(s->ctx, s->pin);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     mavi_ctx *ctx = s->ctx;

@@ -27,6 +27,7 @@
 #include <stdint.h>
 
 #include <initializer_list>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -45,12 +46,24 @@
 // an object that something still references only marks it; the last release
 // frees it.  Callers (and garbage collectors, which finalize in any order)
 // may therefore destroy objects in any order.
+struct PinBuf {
+    void *p = nullptr;    // pinned, from the context at the first use, with kPinWords words behind it
+    size_t bytes = 4096;  // its size
+    // room for the state of n particles, if that is small
+    void fit(int64_t n);
+};
+
 struct mavi_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
     int refs = 0;
     bool closing = false;
+    // pinned buffers that systems and batches gave back
+    std::mutex pins_lock;  // of what follows
+    std::vector<PinBuf> pins;
+    size_t pins_bytes = 0;
+    hipStream_t side = nullptr;  // batches' plain replicas where rings step beside them
 };
 #define MAVI_HIDDEN __attribute__((visibility("hidden")))
 extern "C" {
@@ -273,7 +286,6 @@ struct RList {
     uint32_t *status = nullptr;
     unsigned long long *counter = nullptr;  // two words, alternating between steps
     unsigned long long *out = nullptr, *host = nullptr;  // block-end maxima and status, pinned copy
-    unsigned long long *own_host = nullptr;  // a batch: the copy is an allocation of its own
     unsigned long long *scan_ticket = nullptr, *scan_state = nullptr;
     int32_t scan_words = 0;
     int64_t rebuilds = 0, rollbacks = 0;
@@ -285,16 +297,16 @@ struct RList {
 // pageable memory costs over 10 us however small.  1k particles: download 44 -> 21
 // us, the flags word after a step 15 us less; at 256 KiB the copy through the
 // buffer takes about what it saves.
-constexpr size_t kPinBytes = 256 * 1024, kPinWords = 8;
-struct PinBuf {
-    void *p = nullptr;    // hipHostMalloc, at the first use, with kPinWords words behind it
-    size_t bytes = 4096;  // its size
-    // room for the state of n particles, if that is small
-    void fit(int64_t n) {
-        const int64_t want = 40 * n + 4096;
-        if (!p && want <= (int64_t)kPinBytes && want > (int64_t)bytes) bytes = (size_t)want;
-    }
-};
+// The buffers, of 4 KiB doubled up to kPinBytes, come from the context and go back
+// to it for the next system, up to kPinKeep in all: the runtime takes 28 us to
+// make one and 240 to free it, a sixth of the life of a 1k system that is made,
+// steps once and goes.
+constexpr size_t kPinBytes = 256 * 1024, kPinWords = 8, kPinKeep = 4 << 20;
+inline void PinBuf::fit(int64_t n) {
+    const int64_t want = 40 * n + 4096;
+    if (p || want > (int64_t)kPinBytes) return;
+    while ((int64_t)bytes < want) bytes *= 2;
+}
 struct Xfer {
     void *host, *dev;
     size_t bytes;  // a multiple of 4; 0: skipped
@@ -504,8 +516,10 @@ void rl_reset(RList &N);
 // left where it is: s->src, s->scell, s->start.
 hipError_t launch_cell_order(mavi_sys *s, const SysParams &G, unsigned long long *ticket, unsigned long long *state,
                              hipStream_t st);
-// Eight words of pinned memory behind the buffer (null: none to be had).
-unsigned long long *pin_words(PinBuf &pin);
+// Eight words of pinned memory behind the buffer (null: none to be had); pin_give:
+// the buffer back to the context, all work on it done.
+unsigned long long *pin_words(mavi_ctx *ctx, PinBuf &pin);
+void pin_give(mavi_ctx *ctx, PinBuf &pin);
 hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
 hipError_t copy_out(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list);
 hipError_t launch_export_chunks(mavi_sys *s, int64_t *d_cp, int64_t *d_counts, hipStream_t st);

@@ -1424,8 +1424,18 @@ static hipError_t copy3(mavi_ctx *ctx, char *pin, std::initializer_list<Xfer> li
     return hipGetLastError();
 }
 
-unsigned long long *pin_words(PinBuf &pin) {
-    pin.bytes = (pin.bytes + 63) / 64 * 64;
+unsigned long long *pin_words(mavi_ctx *ctx, PinBuf &pin) {
+    if (!pin.p) {
+        std::lock_guard<std::mutex> hold(ctx->pins_lock);
+        for (PinBuf &q : ctx->pins) {
+            if (q.bytes != pin.bytes) continue;
+            pin.p = q.p;
+            ctx->pins_bytes -= q.bytes;
+            q = ctx->pins.back();
+            ctx->pins.pop_back();
+            break;
+        }
+    }
     if (!pin.p && hipHostMalloc(&pin.p, pin.bytes + 8 * kPinWords, hipHostMallocDefault) != hipSuccess) {
         pin.p = nullptr;
         (void)hipGetLastError();
@@ -1434,19 +1444,33 @@ unsigned long long *pin_words(PinBuf &pin) {
     return (unsigned long long *)((char *)pin.p + pin.bytes);
 }
 
+void pin_give(mavi_ctx *ctx, PinBuf &pin) {
+    if (!pin.p) return;
+    {
+        std::lock_guard<std::mutex> hold(ctx->pins_lock);
+        if (ctx->pins_bytes + pin.bytes <= kPinKeep) {
+            ctx->pins.push_back(pin);
+            ctx->pins_bytes += pin.bytes;
+            pin.p = nullptr;
+        }
+    }
+    if (pin.p) (void)hipHostFree(pin.p);
+    pin.p = nullptr;
+}
+
 // The pinned buffer, or null if the transfer is larger (or there is none to be had).
-static char *pin_for(PinBuf &pin, std::initializer_list<Xfer> list) {
+static char *pin_for(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list) {
     size_t need = 0;
     for (const Xfer &x : list) need += (x.bytes + 63) / 64 * 64;
     if (need > pin.bytes || list.size() > 3) return nullptr;
-    return pin_words(pin) ? (char *)pin.p : nullptr;
+    return pin_words(ctx, pin) ? (char *)pin.p : nullptr;
 }
 
 // Host arrays to the device on the context's stream.  The pinned buffer is free:
 // every use of it ends with a wait for the stream, in copy_out here, after a
 // copy_in in its caller.
 hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list) {
-    char *p = pin_for(pin, list);
+    char *p = pin_for(ctx, pin, list);
     if (p) {
         size_t at = 0;
         for (const Xfer &x : list) {
@@ -1465,7 +1489,7 @@ hipError_t copy_in(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list)
 
 // Device arrays to the host, complete on return.
 hipError_t copy_out(mavi_ctx *ctx, PinBuf &pin, std::initializer_list<Xfer> list) {
-    char *p = pin_for(pin, list);
+    char *p = pin_for(ctx, pin, list);
     hipError_t e = hipSuccess;
     if (p) {
         e = copy3(ctx, p, list, false);

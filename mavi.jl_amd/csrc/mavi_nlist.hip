@@ -1021,7 +1021,7 @@ hipError_t nl_alloc(mavi_sys *s, hipStream_t st) {
     if (e == hipSuccess) e = dalloc(&N.bmax, N.nbmax, st);
     if (e == hipSuccess) e = dalloc(&N.dpend, N.nbmax, st);
     if (e == hipSuccess) e = dalloc(&N.status, 1, st);
-    if (e == hipSuccess && (N.host = pin_words(s->pin)) == nullptr) e = hipErrorOutOfMemory;
+    if (e == hipSuccess && (N.host = pin_words(s->ctx, s->pin)) == nullptr) e = hipErrorOutOfMemory;
     // scan states of the list grid (no more cells than the chunk grid)
     N.scan_words = (s->P.ncell + 1 + kScanTileMin - 1) / kScanTileMin + 1;
     if (e == hipSuccess) e = dalloc(&N.scan_ticket, 1, st);

@@ -1167,7 +1167,6 @@ static void rl_release(RList *&rl, hipStream_t st) {
     rl_drop_graphs(N, st);
     dfree(N.arena);
     if (N.greps) (void)hipFree(N.greps);
-    if (N.own_host) (void)hipHostFree(N.own_host);
     delete rl;
     rl = nullptr;
 }
@@ -1179,7 +1178,7 @@ hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
     N.uniform = rl_uniform(s->host_inter.data(), (int)s->host_inter.size());
     N.per = 64 / s->P.nmax;
     N.nbmax = rl_blocks(s->P);
-    if ((N.host = pin_words(s->pin)) == nullptr) return hipErrorOutOfMemory;
+    if ((N.host = pin_words(s->ctx, s->pin)) == nullptr) return hipErrorOutOfMemory;
     return rl_buffers(N, s->P.na, s->P.nrings, s->P.ncell, 1, st);
 }
 
@@ -1226,8 +1225,8 @@ hipError_t rlb_alloc(BatchSub *b, hipStream_t st) {
     N.fits = true;
     N.uniform = full;
     N.nbmax = nblk(b->nring_waves, kRlWaves);
-    hipError_t e = hipHostMalloc((void **)&N.own_host, 3 * sizeof(unsigned long long), hipHostMallocDefault);
-    N.host = N.own_host;
+    N.host = pin_words(b->ctx, *b->pin);
+    hipError_t e = N.host ? hipSuccess : hipErrorOutOfMemory;
     if (e == hipSuccess) e = rl_buffers(N, b->nslots, b->nrings, b->ncells, (int64_t)b->reps.size(), st);
     if (e == hipSuccess) e = hipMalloc(&N.greps, sizeof(Replica) * g.size());
     if (e == hipSuccess) e = hipMemcpyAsync(N.greps, g.data(), sizeof(Replica) * g.size(), hipMemcpyHostToDevice, st);
