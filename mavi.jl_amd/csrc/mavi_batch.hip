@@ -414,13 +414,13 @@ void drop_graph(BatchSub *b) {
 int batch_check_flags(mavi_batch *b) {
     mavi_ctx *ctx = b->ctx;
     std::vector<uint32_t> h[2];
+    Xfer x[2] = {};
     for (int k = 0; k < 2; k++) {
         if (!b->sub[k]) continue;
         h[k].assign(b->sub[k]->reps.size(), 0);
-        HIPCHK(ctx, hipMemcpyAsync(h[k].data(), b->sub[k]->flags, sizeof(uint32_t) * h[k].size(),
-                                   hipMemcpyDeviceToHost, ctx->stream));
+        x[k] = Xfer{h[k].data(), b->sub[k]->flags, sizeof(uint32_t) * h[k].size()};
     }
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    HIPCHK(ctx, mavi::copy_out(ctx, b->pin, {x[0], x[1]}));
     for (size_t r = 0; r < b->where.size(); r++) {
         const uint32_t f = h[b->where[r].sub][b->where[r].local];
         if (!f) continue;
@@ -512,7 +512,7 @@ int both_steps(mavi_batch *b, int64_t nsteps) {
         int rc = sub_gather(b->sub[0], n, b->side);
         if (rc == MAVI_OK) rc = sub_rings(b->sub[1], n);
         if (rc != MAVI_OK) return rc;
-        HIPCHK(ctx, hipStreamSynchronize(b->side));
+        if (k + ahead < nsteps) HIPCHK(ctx, hipStreamSynchronize(b->side));
     }
     return MAVI_OK;
 }
