@@ -222,7 +222,8 @@ def test_batch_errors(gpu_ctx):
     ("normal", "smallest_rings", "normal_ragged"),  # every ring full: slots by place
     ("rings_of_two", "normal"),  # rings too small for lists: all through the chunk gather
     ("normal", "rings_of_three"),  # the smallest rings on lists
-    ("types", "few_cells"),  # a box too small for lists: all through the chunk gather
+    ("types", "few_cells"),  # a box of few list cells
+    ("types", "tiny_box"),  # a box too small for lists: all through the chunk gather
 ])
 def test_batch_rings_on_lists_bitexact(gpu_ctx, names):
     """Rings replicas on Verlet lists beside plain ones (their steps overlap):
@@ -252,3 +253,43 @@ def test_batch_rings_on_lists_bitexact(gpu_ctx, names):
     b.run(steps_list[1])
     pos, vel, pol = b.download(1)
     assert_same("replaced replica", (pos, vel, pol, b.get_forces(1)), want[1][1])
+
+
+@pytest.mark.parametrize("names,lists", [
+    (("normal", "smallest_rings", "largest_rings", "types", "mixture"), True),
+    (("normal", "rings_of_three", "normal_ragged"), True),  # every ring full: slots by place
+    (("types", "few_cells"), True),
+    (("types", "tiny_box"), False),
+    (("normal", "rings_of_two"), False),
+])
+def test_batch_rings_run_on_lists(gpu_ctx, names, lists):
+    """That rings replicas do run on lists, by the launch counters: no gather
+    launch where every replica may, gathers only where one may not; against
+    each system alone on the chunk gather."""
+    import mavi_hip as mv
+    from mavi_hip import _lib, rings
+    from test_gpu_rlist import CASES
+
+    def case(nm):  # at a time step whose displacements suit the lists
+        state, space, cfg, ic = CASES[nm]()
+        return state, space, cfg, mv.IntCfg(dt=1e-3, chunks_cfg=ic.chunks_cfg, device=mv.GPU())
+
+    steps = 70
+    want = []
+    for i, nm in enumerate(names):
+        state, space, cfg, ic = case(nm)
+        s = rings.RingsSystem(state=state, space_cfg=space, dynamic_cfg=cfg, int_cfg=ic, seed=50 + i)
+        s.dev.set_option(_lib.MAVI_OPT_NLIST, 0)
+        s.advance(steps)
+        s.download()
+        want.append((s.state.pos.copy(), None, s.state.pol.copy(), s.forces.copy()))
+    for counted in (False, True):  # with graphs, and with direct launches that are counted
+        b = build_batch([((nm, "rings", None), case(nm), 50 + i) for i, nm in enumerate(names)], gpu_ctx)
+        b.prof_enable(counted)
+        b.run(steps)
+        for i, nm in enumerate(names):
+            pos, vel, pol = b.download(i)
+            assert_same(f"{nm} counted {counted}", (pos, vel, pol, b.get_forces(i)), want[i])
+    gathers, ring = b.prof_get(_lib.MAVI_PROF_FORCE)[1], b.prof_get(_lib.MAVI_PROF_RINGS)[1]
+    say(f"[batch lists] {names}: {gathers} gather launches, {ring} steps")
+    assert (gathers == 0) == lists and ring >= steps
