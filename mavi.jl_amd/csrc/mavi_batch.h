@@ -34,7 +34,7 @@ struct BatchSub {
     std::vector<Replica> reps;
     int64_t nids = 0, nactive = 0, nslots = 0, ncells = 0, nrings = 0;
     SysParams G{};  // na = nslots, ncell = ncells: the sort over all replicas
-    uint8_t *arena = nullptr;  // holds all device arrays below
+    std::vector<uint8_t *> blocks;  // the allocations that hold all device arrays below
     // per-kind wave lists
     int2 *items[NKIND] = {nullptr, nullptr, nullptr};
     int32_t nitems[NKIND] = {0, 0, 0};

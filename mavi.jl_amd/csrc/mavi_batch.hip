@@ -42,7 +42,6 @@
 #include <math.h>
 
 #include <algorithm>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -297,7 +296,10 @@ struct mavi_batch {
     std::vector<Where> where;  // of each replica
     std::vector<char> uploaded;
     PinBuf pin;
-    hipStream_t side = nullptr;  // the context's, for the plain replicas' steps where both families are there
+    // the plain replicas' steps where both families are there (not kept past the
+    // batch: with another stream about, all launches of the process take longer,
+    // 40 training steps 1430 -> 1475 us)
+    hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     // execution shape: plain, rings
     int32_t wg[2] = {256, 256};
@@ -512,7 +514,10 @@ int both_steps(mavi_batch *b, int64_t nsteps) {
         int rc = sub_gather(b->sub[0], n, b->side);
         if (rc == MAVI_OK) rc = sub_rings(b->sub[1], n);
         if (rc != MAVI_OK) return rc;
-        if (k + ahead < nsteps) HIPCHK(ctx, hipStreamSynchronize(b->side));
+        // the join in the context's stream would do, but while that waits the side
+        // stream's launches take longer (200 steps of 48 replicas 12.7 -> 13.0 ms);
+        // a few steps are over before this wait of the host's pays (one step 8 us)
+        if (nsteps >= kRlMinCall) HIPCHK(ctx, hipStreamSynchronize(b->side));
     }
     return MAVI_OK;
 }
@@ -611,6 +616,8 @@ int32_t rings_uniform(const std::vector<RingInter> &I) {
     return 1;
 }
 
+constexpr size_t kOwnBytes = 1 << 20;  // arrays from this size on are allocations of their own
+
 // Device arrays of one family.
 int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
     mavi_ctx *ctx = b->ctx;
@@ -676,19 +683,29 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
     b->G.ncell = (int32_t)ncells;
 
     hipStream_t st = ctx->stream;
-    // all arrays in one allocation: forty for a family, and two families, took
+    // small arrays in one allocation: forty for a family, and two families, took
     // longer than a short run of a small batch
+    hipError_t e = hipSuccess;
     struct Part {
         void **p;
         size_t at;
     };
     std::vector<Part> parts;
     size_t total = 0;
-#define ALLOC(ptr, cnt)                                                                            \
-    do {                                                                                           \
-        parts.push_back({(void **)&(ptr), total});                                                 \
-        total += (sizeof(*(ptr)) * (size_t)std::max<int64_t>((cnt), 1) + 255) / 256 * 256;         \
-    } while (0)
+    auto alloc = [&](void **p, size_t bytes) {
+        *p = nullptr;
+        bytes = (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+        if (bytes < kOwnBytes) {
+            parts.push_back({p, total});
+            total += bytes;
+        } else if (e == hipSuccess) {
+            uint8_t *own = nullptr;
+            e = dalloc(&own, (int64_t)bytes, st);
+            b->blocks.push_back(own);
+            *p = own;
+        }
+    };
+#define ALLOC(ptr, cnt) alloc((void **)&(ptr), sizeof(*(ptr)) * (size_t)(cnt))
     for (int c = 0; c < 2; c++) {
         ALLOC(b->P_[c], nslots);
         ALLOC(b->V_[c], nslots);
@@ -736,8 +753,10 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
         ALLOC(b->inter, (int64_t)inter.size());
     }
 #undef ALLOC
-    hipError_t e = dalloc(&b->arena, (int64_t)total, st);
-    for (const Part &q : parts) *q.p = e == hipSuccess ? b->arena + q.at : nullptr;
+    uint8_t *small = nullptr;
+    if (e == hipSuccess) e = dalloc(&small, (int64_t)total, st);
+    b->blocks.push_back(small);
+    for (const Part &q : parts) *q.p = small ? small + q.at : nullptr;
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     auto up = [&](void *dst, const void *srcp, size_t bytes) {
@@ -765,7 +784,7 @@ int sub_finalize(BatchSub *b, const std::vector<HostSys> &hs) {
 void sub_free(BatchSub *b) {
     drop_graph(b);
     mavi::rlb_free(b);
-    dfree(b->arena);
+    for (uint8_t *&q : b->blocks) dfree(q);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     delete b;
@@ -793,6 +812,7 @@ int mavi_batch_destroy(mavi_batch *b) {
     mavi::pin_give(b->ctx, b->pin);
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
+    if (b->side) (void)hipStreamDestroy(b->side);
     mavi_ctx *ctx = b->ctx;
     delete b;
     ctx_release(ctx);
@@ -862,10 +882,7 @@ int mavi_batch_finalize(mavi_batch *b) {
         if (rc != MAVI_OK) return rc;
     }
     if (b->sub[0] && b->sub[1]) {
-        // (a stream takes up to 3 ms to make: one for all batches of the context)
-        std::lock_guard<std::mutex> hold(ctx->pins_lock);
-        if (!ctx->side) HIPCHK(ctx, hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
-        b->side = ctx->side;
+        if (!b->side) HIPCHK(ctx, hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
         if (!b->fork) HIPCHK(ctx, hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
         if (!b->join) HIPCHK(ctx, hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
     }

@@ -94,7 +94,6 @@ int mavi_ctx_create(int device, mavi_ctx **out) {
 static void ctx_free(mavi_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     for (PinBuf &q : ctx->pins) (void)hipHostFree(q.p);
-    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

@@ -60,10 +60,9 @@ struct mavi_ctx {
     int refs = 0;
     bool closing = false;
     // pinned buffers that systems and batches gave back
-    std::mutex pins_lock;  // of what follows
+    std::mutex pins_lock;
     std::vector<PinBuf> pins;
     size_t pins_bytes = 0;
-    hipStream_t side = nullptr;  // batches' plain replicas where rings step beside them
 };
 #define MAVI_HIDDEN __attribute__((visibility("hidden")))
 extern "C" {
