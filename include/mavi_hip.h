@@ -317,9 +317,10 @@ int mavi_sys_noise_set(mavi_sys *sys, uint64_t seed, uint64_t counter);
  *                       step-start chunks are not adjacent left out), forces
  *                       summed in ascending partner id; lists rebuilt when a
  *                       particle has moved half the skin.  Rings step! of a
- *                       fixed population on a periodic chunk grid whose chunks
- *                       are at least the range wide runs on lists too (calls of
- *                       8 steps and more), with the chunk gather's bits.
+ *                       fixed population of rings of 3 to 32 particles on a
+ *                       periodic chunk grid whose chunks are at least the range
+ *                       wide runs on lists too (calls of 8 steps and more), with
+ *                       the chunk gather's bits.
  *                       0: the chunk gather
  *   MAVI_OPT_NLIST_SKIN skin in thousandths of the range (0: LJ 150, HarmTrunc
  *                       300 with fewer than 5 partners within the range at the

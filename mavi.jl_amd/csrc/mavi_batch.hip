@@ -20,10 +20,10 @@
 // VERLET2 for LJ and HarmTrunc, FORCES for rings), and the per-ring kernel for
 // rings.  Calls of 8 steps and more step the rings replicas on Verlet lists
 // instead (mavi_rlist.hip: one kernel a step, the same bits), if every one of
-// them may use lists.  Each replica runs the same device functions as a single
+// them may use lists (one that may not sends all to the gather).  Each replica runs the same device functions as a single
 // system (mavi_device.h), so its results are bit-identical to mavi_step on the
 // same descriptor.  48 replicas (1000 to 40000 particles, 200 steps with all
-// transfers): 25.0 ms with both families in one set of launches, 17.8 ms
+// transfers): 25.0 ms with both families in one set of launches, 16.7 ms
 // now; the plain replicas' launches (60 us a step) are what it waits for, the
 // rings replicas' one kernel (16.6 us) runs beside them.
 //

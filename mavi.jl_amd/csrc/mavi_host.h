@@ -36,12 +36,16 @@ void dfree(T *&p) {
 }
 
 // Up to this many particles the chunk gather keeps eight candidates a lane in
-// flight (pair_gather_deep): there are few waves a SIMD, and a candidate's trip
-// to memory is what a step waits for.  Above, other waves hide it and the extra
-// registers (fewer waves) cost more.  us a step, two candidates in flight ->
-// eight: LJ 4k 39.5 -> 37.0, 66k 45.5 -> 40.0, 202k 59.0 -> 54.7, 393k 72.9 ->
-// 68.0, 787k 99.4 -> 99.9, 1M 115.9 -> 119.7; self-propelled 32k 23.2 -> 21.2,
-// 490k 49.0 -> 47.0; run-and-tumble 32k 20.3 -> 19.7, 490k 38.7 -> 40.3.
+// flight (pair_gather_deep; rings four): there are few waves a SIMD, and a
+// candidate's trip to memory is what a step waits for.  Above, other waves hide it
+// and the extra registers (fewer waves) cost more.  us a step, two candidates in
+// flight -> eight: LJ 4k 39.5 -> 37.0, 66k 45.5 -> 40.0, 202k 59.0 -> 54.7, 393k
+// 72.9 -> 68.0, 787k 99.4 -> 99.9, 1M 115.9 -> 119.7; with a walls list 160k 66.9
+// -> 62.5, 292k 82.2 -> 82.8; self-propelled 32k 23.2 -> 21.2, 490k 49.0 -> 47.0;
+// run-and-tumble 32k 20.3 -> 19.7, 131k 25.5 -> 25.2, 292k 34.5 -> 34.4, 490k 38.7
+// -> 40.3; rings 2k 31.7 -> 28.6, 20k 34.3 -> 30.8, 200k 50.2 -> 47.2, 298k 58.3 ->
+// 55.5; a batch's plain replicas, by the family's slots: 16 of 1k 36.5 -> 31.4, 16
+// of 10k 54.5 -> 50.6.
 constexpr int64_t kDeepGather = 300000;
 
 inline int nblk(int64_t n, int t) { return (int)((n + t - 1) / t); }

@@ -255,7 +255,8 @@ struct RList {
     bool renewed = true, first = false;  // a new state since rl_take; since the last steps on lists
     bool ordered = false;     // the state lies in ring order, both copies' ids too
     bool valid = false;       // lists complete for the current state
-    bool uniform = false;     // one interaction for all type pairs (a batch: every ring full)
+    bool uniform = false;     // a system alone: one interaction for all type pairs (a batch: Replica.uniform)
+    bool full = false;        // every ring has nmax particles: a particle's slot is its id's place
     double rl2 = 0.0;         // list radius squared (range + skin)^2, with margin
     double half_skin = 0.0;   // displacement bound
     int32_t block = 0;        // steps between host checks (option; 0: as many as the bound allows, at most kNlBlockCap)

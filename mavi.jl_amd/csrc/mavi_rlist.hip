@@ -1,7 +1,7 @@
 // mavi_rlist.hip -- Verlet lists for Rings step! (src/rings/integration.jl:
-// 522-543) of a fixed ring population on a periodic chunk grid whose chunks
-// are at least the interaction range wide: one kernel per step instead of a
-// binning (three launches), the pair gather and the ring update.
+// 522-543) of a fixed population of rings (of 3 to 32 particles) on a periodic
+// chunk grid whose chunks are at least the interaction range wide: one kernel per
+// step instead of a binning (three launches), the pair gather and the ring update.
 //
 // State.  While the lists run the state lies in ring order (slot = position of
 // the particle's id among the active ids), so a ring's particles are
@@ -28,6 +28,11 @@
 // Errors.  Chunks and chunk counts of the reference grid follow every particle
 // (out of box, non-finite); a count that may have passed the capacity, or a
 // list that is too long, hands the block to the gather, which checks exactly.
+//
+// Handing over.  The lists give a state to the gather for a while when a list
+// would serve at most two of its steps or a chunk may be full (rl_back_off), and
+// until a new state or skin when a list is too long; the gather's steps are the
+// same bits.
 #include <math.h>
 
 #include <algorithm>
@@ -269,7 +274,8 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
 // call, which leaves the forces and the continuous positions (every step
 // recomputes both before it uses them).
 //
-// Bound: FP64 VALU issue and the length of its dependent chain.  The ring's
+// Bound: FP64 VALU issue (817 instructions a wave, 45 % of the issue cycles at 800k
+// particles) and the length of its dependent chain.  The ring's
 // left-to-right sums (unwrap, centre of mass, shoelace, mean velocity) run
 // once per ring and component on a few lanes (2 or 3 per ring) instead of as
 // masked loops of every lane, and the scalar work of a ring (noise, asin,
@@ -797,7 +803,7 @@ hipError_t rl_step(const RLSys &E, bool last, hipStream_t st) {
     if (mavi_sys *s = E.s) {
         ProfScope ps(s, MAVI_PROF_RINGS, st);
         A.F = s->F;
-        A.slot_of = s->P.na == s->P.n ? nullptr : s->slot_of;
+        A.slot_of = N.full ? nullptr : s->slot_of;
         A.areas = s->areas;
         A.cpos = s->cpos;
         A.rtype = s->rtype;
@@ -811,7 +817,7 @@ hipError_t rl_step(const RLSys &E, bool last, hipStream_t st) {
         BatchSub *b = E.b;
         BatchProf ps(b, MAVI_PROF_RINGS, st);
         A.F = b->F;
-        A.slot_of = N.uniform ? nullptr : b->slot_of;  // (of a batch: every replica's rings are full)
+        A.slot_of = N.full ? nullptr : b->slot_of;
         A.areas = b->areas;
         A.cpos = b->cpos;
         A.rtype = b->rtype;
@@ -1176,6 +1182,7 @@ hipError_t rl_alloc(mavi_sys *s, hipStream_t st) {
     RList &N = *s->rl;
     rl_set_skin(s, kRlSkin);
     N.uniform = rl_uniform(s->host_inter.data(), (int)s->host_inter.size());
+    N.full = s->P.na == s->P.n;
     N.per = 64 / s->P.nmax;
     N.nbmax = rl_blocks(s->P);
     if ((N.host = pin_words(s->ctx, s->pin)) == nullptr) return hipErrorOutOfMemory;
@@ -1223,7 +1230,7 @@ hipError_t rlb_alloc(BatchSub *b, hipStream_t st) {
     N.per = per;
     N.gcells = gcells;
     N.fits = true;
-    N.uniform = full;
+    N.full = full;
     N.nbmax = nblk(b->nring_waves, kRlWaves);
     N.host = pin_words(b->ctx, *b->pin);
     hipError_t e = N.host ? hipSuccess : hipErrorOutOfMemory;
