@@ -241,8 +241,9 @@ constexpr int kRlGraphSteps = 8;     // steps per captured graph (even)
 constexpr int64_t kRlMinCall = 8;
 // Steps that go to the gather after the lists had to give up on a state (steps
 // too long, a chunk that may be over its capacity), doubled while that repeats:
-// a try that fails costs 100 to 300 us.
-constexpr int64_t kRlWaitMin = 64, kRlWaitMax = 2048;
+// a try that fails costs 100 to 300 us.  A new state waits no longer than
+// kRlWaitNew: it may be a calmer one.
+constexpr int64_t kRlWaitMin = 64, kRlWaitMax = 2048, kRlWaitNew = 256;
 
 // Verlet lists of a rings system with a fixed population (mavi_rlist.hip).
 struct RList {

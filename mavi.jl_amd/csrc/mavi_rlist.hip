@@ -933,8 +933,8 @@ int64_t rl_fit(const RList &N, double d) {
 }
 int64_t rl_room(const RList &N) { return rl_fit(N, N.d_start); }
 
-// Lists that would serve fewer steps go to the gather.  us for 200 steps of
-// jammed mixtures with 6, 3, 2 and 1 here (gather: 6890 .. 11470): 2k particles
+// A state whose lists would serve no more steps than this goes to the gather.  us for
+// 200 steps of jammed mixtures with 6, 3, 2 and 1 here (gather: 6890 .. 11470): 2k particles
 // at dt 0.01 6060, 6040, 3970, 4360; 20k at 0.005 6590, 4910, 4940, 5090, at 0.02
 // 6780, 6770, 6760, 8420; 200k at 0.005 10560, 7490, 7440, 7650.
 constexpr int64_t kRlMinFit = 2;
@@ -1249,6 +1249,7 @@ bool rl_take(RList &N, int64_t n) {
     if (N.renewed) {
         N.renewed = false;
         N.first = true;
+        N.wait = std::min(N.wait, kRlWaitNew);
         if (N.disabled && --N.skip <= 0) N.disabled = false;
     }
     if (N.disabled || N.wait > 0) return false;
